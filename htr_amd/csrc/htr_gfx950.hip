@@ -447,9 +447,14 @@ int htr_anchor_decode(int K, int with_mfma, int iters, int workgroups, void* out
   return HTR_OK;
 }
 
+// workgroups of a search: one per compute unit at most, each takes tiles in turn and keeps its stored arrays in a slot of its own
+static unsigned viterbi_grid(int64_t tiles) { const int cus = num_cu(); return (unsigned)(tiles < cus ? tiles : cus); }
+
 size_t htr_viterbi_workspace_bytes(int64_t tiles, int T, int K) {
   if (tiles <= 0 || T < 1 || T > 256 || K < 2 || K > 8) return 0;
-  return align256((size_t)tiles * (size_t)(T > 1 ? T - 1 : 1) * (65536u >> K));
+  size_t rows = 0;
+  HTR_FOR_K_OR(K, rows = (size_t)vit_rows(T, VitCfg<KK>::C), return 0);
+  return align256(viterbi_grid(tiles) * (rows > 0 ? rows : 1) * (65536u >> K) * sizeof(float));
 }
 
 int htr_viterbi(const void* x, const void* w, int64_t tiles, int T, int K, int tailbite, void* states_u16, void* workspace,
@@ -459,25 +464,17 @@ int htr_viterbi(const void* x, const void* w, int64_t tiles, int T, int K, int t
   if (tiles <= 0 || tiles > 0x7FFFFFFF || T < 1 || T > 256) return HTR_ERR_SHAPE;
   if (((uintptr_t)x & 3) || ((uintptr_t)w & 3) || ((uintptr_t)states_u16 & 1)) return HTR_ERR_ALIGN;
   const size_t need = htr_viterbi_workspace_bytes(tiles, T, K);
-  if (!workspace || workspace_bytes < need) return HTR_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15)) return HTR_ERR_WORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const double rms = __builtin_sqrt(MEAN_SQ);
 #define HTR_LAUNCH_VIT(KK_)                                                                                              \
   {                                                                                                                      \
-    const size_t lds = ((size_t)2 * VitCfg<KK_>::SJ + 2048 + 1024 + 512 + 64) * sizeof(float);                           \
     HTR_CHECK_HIP((allow_full_lds<k_viterbi<KK_>>()));                                                                   \
-    HTR_CHECK_HIP(launch_kernel(k_viterbi<KK_>, dim3((unsigned)tiles), dim3(VitCfg<KK_>::THREADS), lds, st, (const float*)x, \
-                                (const float*)w, T, tailbite ? 1 : 0, (uint8_t*)workspace, (uint16_t*)states_u16, rms)); \
+    HTR_CHECK_HIP(launch_kernel(k_viterbi<KK_>, dim3(viterbi_grid(tiles)), dim3(VitCfg<KK_>::THREADS), VitCfg<KK_>::LDS, st, \
+                                (const float*)x, (const float*)w, (int)tiles, T, tailbite ? 1 : 0, (float*)workspace,    \
+                                (uint16_t*)states_u16, rms));                                                            \
   }
-  switch (K) {
-    case 2: HTR_LAUNCH_VIT(2); break;
-    case 3: HTR_LAUNCH_VIT(3); break;
-    case 4: HTR_LAUNCH_VIT(4); break;
-    case 5: HTR_LAUNCH_VIT(5); break;
-    case 6: HTR_LAUNCH_VIT(6); break;
-    case 7: HTR_LAUNCH_VIT(7); break;
-    default: HTR_LAUNCH_VIT(8); break;
-  }
+  HTR_FOR_K(K, HTR_LAUNCH_VIT(KK));
 #undef HTR_LAUNCH_VIT
   return HTR_OK;
 }

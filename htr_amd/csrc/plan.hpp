@@ -388,7 +388,7 @@ inline hipError_t launch_rotation(const void* x, const uint8_t* su, int n, int M
                        (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, (const htr_group_entry*)nullptr, 0ull);
 }
 
-#define HTR_FOR_K(K, EXPR)                 \
+#define HTR_FOR_K_OR(K, EXPR, OTHERWISE)   \
   switch (K) {                             \
     case 2: { constexpr int KK = 2; EXPR; } break; \
     case 3: { constexpr int KK = 3; EXPR; } break; \
@@ -397,8 +397,9 @@ inline hipError_t launch_rotation(const void* x, const uint8_t* su, int n, int M
     case 6: { constexpr int KK = 6; EXPR; } break; \
     case 7: { constexpr int KK = 7; EXPR; } break; \
     case 8: { constexpr int KK = 8; EXPR; } break; \
-    default: return HTR_ERR_K;             \
+    default: OTHERWISE;                    \
   }
+#define HTR_FOR_K(K, EXPR) HTR_FOR_K_OR(K, EXPR, return HTR_ERR_K)
 
 inline bool dtype_ok(int d) { return d == HTR_BF16 || d == HTR_F16 || d == HTR_F32; }
 

@@ -2,137 +2,301 @@
 // ------------------------------------------------------------------------------------------------ encoder search
 // Tail-biting bitshift-trellis Viterbi over the 65536 codec states (htr/reference.py:6-50 of the reference; its GPU
 // versions are htr/vit_v1.py and htr/vit_v2.py): per 256-weight tile, minimise sum_t w_t (x_t - cb[s_t])^2 with
-// s_t = ((s_{t-1} << K) & 0xFFFF) | bits.  One workgroup per tile.  Only the minima over the 2^K predecessors,
-// M_t[low] = min_j cost_{t-1}[j * Sj + low] (Sj = 65536 >> K entries), need to live between steps, and
+// s_t = ((s_{t-1} << K) & 0xFFFF) | bits.  One workgroup works on one tile at a time.  Only the minima over the 2^K
+// predecessors, M_t[low] = min_j cost_{t-1}[j * Sj + low] (Sj = 65536 >> K entries), need to live between steps, and
 // cost_t[s] = M_t[s >> K] + w_t (x_t - cb[s])^2, so two M arrays in LDS carry a whole tile (128 KB at K2, 32 KB at K4)
-// and no cost array ever goes to memory.  The value of a state is the procedural codebook, cb[s] = f32(v(s) / rms) with
-// 1021 distinct v, so a step's 65536 penalty terms are 1021 distinct numbers: they are computed once per step into an
-// LDS table that every candidate indexes with v(s) (two integer instructions).
-// Backpointers (one byte per M entry and step) go to global memory during the deciding pass only; thread 0 walks
-// them back.  Arithmetic and tie-breaking are the reference's: float32, d = (x - cb)^2, m + w * d without fusing,
-// the first index among equal values in every min / argmin.
+// and no cost array ever goes to memory.
+// A thread owns 64 states for the whole launch and keeps their codebook values in registers (1024 threads x 64 = all
+// 65536), so a candidate costs a subtraction, two multiplications and an addition, which this chip issues every 2.35
+// cycles from vector registers, and half a v_min3 (4.2).  (Looking the penalty up in a 1021-entry LDS table, as the first
+// version did, costs 5.4 cycles of the one LDS per 64 candidates plus the address arithmetic at the 4.2-cycle rate.)
+// The forward passes keep no backpointers at all: comparing and selecting an index costs 8.4 cycles per candidate against
+// 2.1 for the minimum alone.  Instead the deciding pass writes every C-th M array to memory, and the trace back
+// recomputes the C steps in between for the predecessors of the ONE state it is at (2^(K C) entries of M_{t-C}, 32 to 512
+// of them, one wave), with the same arithmetic, so the indices it finds are those the forward pass would have recorded.
+// Which array comes next does not depend on the state, so the other waves fetch it into LDS meanwhile.
+// Bound: vector issue in the forward passes (K4: 2890 cycles a step, 2944 by the rates above; 0.74 M cycles a pass), then
+// the trace back, 13 % of a tile: with every CU at it, the stored arrays (2 MB a tile) arrive at 5 TB/s.  C: a larger one
+// stores less and recomputes more (K3: C = 2 439 k cycles, C = 3 281 k; K5: C = 1 290 k, C = 2 327 k).
+// 1024 tiles at K4: 7.46 ms with the table and one byte of backpointer per entry and step, 3.25 ms now; 176 tiles at K3,
+// one per CU: 2.60 -> 0.87 ms.
+// Arithmetic and tie-breaking are the reference's: float32, d = (x - cb)^2, m + w * d without fusing, the first index
+// among equal values in every min / argmin.
 template <int K> struct VitCfg {
-  static constexpr int NB = 1 << K, SJ = 65536 >> K;
-  static constexpr int THREADS = K == 2 ? 1024 : (K == 8 ? 256 : 512);   // at most one thread per M entry
-  static constexpr int ITEMS = SJ / THREADS;         // M entries per thread
+  static constexpr int NB = 1 << K, SJ = 65536 >> K, PB = SJ / NB;
+  static constexpr int THREADS = 1024;
+  static constexpr int LOWS = SJ >= THREADS ? SJ / THREADS : 1;       // M entries of a thread, in runs of consecutive ones
+  static constexpr int RUN = LOWS < NB ? (LOWS < 8 ? LOWS : 8) : (NB < 8 ? NB : 8), RUNS = LOWS / RUN;
+  static constexpr int LANES = SJ >= THREADS ? 1 : THREADS / SJ;      // threads that share one M entry (K = 7, 8)
+  static constexpr int NJ = NB / LANES;                               // predecessors a thread looks at: LOWS * NJ = 64
+  static constexpr int C = K == 2 ? 4 : (K == 3 ? 3 : (K == 4 ? 2 : 1));  // steps per stored M array
+  static constexpr int ROW = SJ + SJ / 16;                            // floats of an M array in LDS (the trace back shifts every 16)
+  static constexpr size_t LDS = ((size_t)2 * ROW + 1024 + 512 + 32) * 4;
 };
+// stored M arrays of one tile: M_t for t = T - 1 - C, T - 1 - 2 C, ... > 0
+inline __host__ __device__ int vit_rows(int T, int C) { return T >= 2 ? (T - 2) / C : 0; }
 
-template <int K>
-__global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __restrict__ x, const float* __restrict__ w, int T,
-                                                               int tailbite, uint8_t* __restrict__ bps, uint16_t* __restrict__ states,
-                                                               double rms) {
-  using C = VitCfg<K>;
-  constexpr int NB = C::NB, SJ = C::SJ, THREADS = C::THREADS, ITEMS = C::ITEMS;
-  extern __shared__ __align__(16) unsigned char lds[];
-  float* M0 = (float*)lds;                 // [SJ]
-  float* M1 = M0 + SJ;                     // [SJ]
-  float* tl = M1 + SJ;                     // [2][1024] penalty of each v for the current / next step
-  float* cbv = tl + 2048;                  // [1024] codebook value of each v
-  float* xs = cbv + 1024;                  // [T] targets, then [T] weights (T <= 256)
-  float* ws = xs + 256;
-  float* red_v = ws + 256;                 // [32] reduction scratch
-  uint32_t* red_i = (uint32_t*)(red_v + 32);
-  const int tid = threadIdx.x;
-  const size_t tile = blockIdx.x;
-  const float* xg = x + tile * T;
-  const float* wg = w + tile * T;
-  uint8_t* bp = bps + tile * (size_t)(T - 1) * SJ;
-
-  for (int i = tid; i < 1024; i += THREADS) cbv[i] = i <= 1020 ? (float)((double)(i - 510) / rms) : 0.f;
-  for (int i = tid; i < T; i += THREADS) { xs[i] = xg[i]; ws[i] = wg[i]; }
-  // table index v + 510 of state s: two integer instructions, cheaper to recompute than to keep
-  auto vidx = [&](uint32_t s) { return __builtin_amdgcn_sad_u8(s * GEN_A + GEN_B, 0u, 0u); };
-  __syncthreads();
-  auto fill_terms = [&](int t, float* dst) {          // dst[v] = w_t * (x_t - cb(v))^2, unfused
-    const float xt = xs[t], wt = ws[t];
-    for (int i = tid; i < 1024; i += THREADS) {
-      const float diff = __fsub_rn(xt, cbv[i]);
-      dst[i] = __fmul_rn(wt, __fmul_rn(diff, diff));
-    }
-  };
-
-  uint32_t j0 = 0;
-  const int passes = tailbite ? 2 : 1;
-  uint32_t final_state = 0;
-  for (int pass = 0; pass < passes; ++pass) {
-    const bool constrained = pass == 1;               // second pass: start and end tied to j0
-    const bool record = pass == passes - 1;
-    // cost_0[s] = M_0[s >> K] + term_0(s) with M_0 = 0 (free start) or 0 at j0 and infinity elsewhere
-    for (int i = tid; i < SJ; i += THREADS) M0[i] = (!constrained || (uint32_t)i == j0) ? 0.f : __builtin_inff();
-    fill_terms(0, tl);
-    __syncthreads();
-    float* Mold = M0;
-    float* Mnew = M1;
-    for (int t = 0; t < T - 1; ++t) {
-      const float* tcur = tl + (t & 1) * 1024;
-      fill_terms(t + 1, tl + ((t + 1) & 1) * 1024);   // the next step's table, behind this step's barrier
-#pragma unroll 1
-      for (int i = 0; i < ITEMS; ++i) {
-        const int low = tid + i * THREADS;
-        float best = 0.f;
-        uint32_t bj = 0;
-#pragma unroll 8
-        for (int j = 0; j < NB; ++j) {
-          // state s = j * SJ + low; its own predecessor minimum is M[s >> K]
-          const float c = __fadd_rn(Mold[j * (SJ / NB) + (low >> K)], tcur[vidx((uint32_t)j * SJ + (uint32_t)low)]);
-          if (j == 0 || c < best) { best = c; bj = j; }
-        }
-        Mnew[low] = best;
-        if (record) bp[(size_t)t * SJ + low] = (uint8_t)bj;
-      }
-      __syncthreads();
-      float* tmp = Mold; Mold = Mnew; Mnew = tmp;
-    }
-    // last step: argmin over all states of cost_{T-1}, first index among equals; second pass: only states whose
-    // lower part is j0
-    const float* tcur = tl + ((T - 1) & 1) * 1024;
-    float best = __builtin_inff();
-    uint32_t bs = 0xFFFFFFFFu;
-#pragma unroll 1
-    for (int i = 0; i < ITEMS; ++i) {
-      const int low = tid + i * THREADS;
-#pragma unroll 8
-      for (int j = 0; j < NB; ++j) {
-        const uint32_t s = (uint32_t)j * SJ + (uint32_t)low;
-        float c = __fadd_rn(Mold[j * (SJ / NB) + (low >> K)], tcur[vidx(s)]);
-        if (constrained && (uint32_t)low != j0) c = __builtin_inff();
-        if (c < best || (c == best && s < bs)) { best = c; bs = s; }
-      }
-    }
-    // wave, then workgroup reduction of (value, index)
-    for (int off = 32; off > 0; off >>= 1) {
-      const float ov = __shfl_xor(best, off);
-      const uint32_t oi = (uint32_t)__shfl_xor((int)bs, off);
-      if (ov < best || (ov == best && oi < bs)) { best = ov; bs = oi; }
-    }
-    __syncthreads();
-    if ((tid & 63) == 0) { red_v[tid >> 6] = best; red_i[tid >> 6] = bs; }
-    __syncthreads();
-    if (tid == 0) {
-      float b = red_v[0]; uint32_t bi = red_i[0];
-      for (int k = 1; k < THREADS / 64; ++k)
-        if (red_v[k] < b || (red_v[k] == b && red_i[k] < bi)) { b = red_v[k]; bi = red_i[k]; }
-      red_i[0] = bi == 0xFFFFFFFFu ? 0u : bi;         // every cost infinite or NaN: the reference's argmin gives 0
-    }
-    __syncthreads();
-    final_state = red_i[0];
-    j0 = final_state & (SJ - 1);
-    __syncthreads();
-  }
-  // trace back (htr/reference.py:43-49): the backpointers of this tile were written by this workgroup; make them
-  // visible to the reading thread
-  __threadfence();
-  __syncthreads();
-  if (tid == 0) {
-    uint16_t* st = states + tile * T;
-    uint32_t s = final_state;
-    st[T - 1] = (uint16_t)s;
-    for (int t = T - 1; t > 0; --t) {
-      const uint32_t low = s >> K;
-      const uint32_t top = bp[(size_t)(t - 1) * SJ + low];
-      s = top * SJ + low;
-      st[t - 1] = (uint16_t)s;
-    }
+// one stage of an argmin over lanes: (v, k) becomes the better of this lane's and lane ^ H's, the smaller k among equals
+template <int H> __device__ __forceinline__ void argmin_stage(float& v, uint32_t& k) {
+  if constexpr (H <= 8) {
+    const float ov = lane_xor_dpp<H>(v);
+    const uint32_t ok = __float_as_uint(lane_xor_dpp<H>(__uint_as_float(k)));
+    if (ov < v || (ov == v && ok < k)) { v = ov; k = ok; }
+  } else {
+    const uint32_t u = __float_as_uint(v);
+    u2s rv, rk;
+    if constexpr (H == 16) { rv = __builtin_amdgcn_permlane16_swap(u, u, false, false); rk = __builtin_amdgcn_permlane16_swap(k, k, false, false); }
+    else { rv = __builtin_amdgcn_permlane32_swap(u, u, false, false); rk = __builtin_amdgcn_permlane32_swap(k, k, false, false); }
+    const float a = __uint_as_float(rv.x), b = __uint_as_float(rv.y);
+    const bool second = b < a || (b == a && rk.y < rk.x);
+    v = second ? b : a; k = second ? rk.y : rk.x;
   }
 }
+template <int SPAN> __device__ __forceinline__ void argmin_lanes(float& v, uint32_t& k) {      // over groups of SPAN adjacent lanes
+  if constexpr (SPAN >= 2) argmin_stage<1>(v, k);
+  if constexpr (SPAN >= 4) argmin_stage<2>(v, k);
+  if constexpr (SPAN >= 8) argmin_stage<4>(v, k);
+  if constexpr (SPAN >= 16) argmin_stage<8>(v, k);
+  if constexpr (SPAN >= 32) argmin_stage<16>(v, k);
+  if constexpr (SPAN >= 64) argmin_stage<32>(v, k);
+}
 
+template <int K>
+__global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __restrict__ x, const float* __restrict__ w, int tiles,
+                                                               int T, int tailbite, float* __restrict__ rows_g,
+                                                               uint16_t* __restrict__ states, double rms) {
+#pragma clang fp contract(off)          // m + w d^2 stays a multiplication and an addition (the __f*_rn functions do not keep the compiler from fusing)
+  using V = VitCfg<K>;
+  constexpr int SJ = V::SJ, PB = V::PB, THREADS = V::THREADS, RUN = V::RUN, RUNS = V::RUNS, LANES = V::LANES,
+                NJ = V::NJ, C = V::C;
+  extern __shared__ __align__(16) unsigned char lds[];
+  float* M0 = (float*)lds;                 // [ROW]
+  float* M1 = M0 + V::ROW;                 // [ROW]
+  float* cbv = M1 + V::ROW;                // [1024] codebook value of each v
+  float* xs = cbv + 1024;                  // [256] targets, [256] weights
+  float* ws = xs + 256;
+  float* red_v = ws + 256;                 // [16] reduction scratch
+  uint32_t* red_i = (uint32_t*)(red_v + 16);
+  const int tid = threadIdx.x, lane = tid & 63;
+  // this thread's M entries low(r, i) and predecessors pj(j)
+  auto low = [&](int r, int i) { return LANES == 1 ? (r * THREADS + tid) * RUN + i : tid / LANES; };
+  auto pj = [&](int j) { return LANES == 1 ? j : j * LANES + tid % LANES; };
+
+  for (int i = tid; i < 1024; i += THREADS) cbv[i] = i <= 1020 ? (float)((double)(i - 510) / rms) : 0.f;
+  __syncthreads();
+  auto cb_of = [&](uint32_t s) { return cbv[__builtin_amdgcn_sad_u8(s * GEN_A + GEN_B, 0u, 0u)]; };
+  float cb[RUNS][RUN][NJ];
+#pragma unroll
+  for (int r = 0; r < RUNS; ++r)
+#pragma unroll
+    for (int i = 0; i < RUN; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) cb[r][i][j] = cb_of((uint32_t)(pj(j) * SJ + low(r, i)));
+
+  const int nrows = vit_rows(T, C);
+  float* my_rows = rows_g + (size_t)blockIdx.x * nrows * SJ;          // one set of stored arrays per workgroup, reused tile by tile
+  for (size_t tile = blockIdx.x; tile < (size_t)tiles; tile += gridDim.x) {
+    for (int i = tid; i < T; i += THREADS) { xs[i] = x[tile * T + i]; ws[i] = w[tile * T + i]; }
+    uint32_t j0 = 0, final_state = 0;
+    const int passes = tailbite ? 2 : 1;
+    for (int pass = 0; pass < passes; ++pass) {
+      const bool constrained = pass == 1;             // second pass: start and end tied to j0
+      const bool record = pass == passes - 1;
+      // cost_0[s] = M_0[s >> K] + term_0(s) with M_0 = 0 (free start) or 0 at j0 and infinity elsewhere
+      for (int i = tid; i < SJ; i += THREADS) M0[i] = (!constrained || (uint32_t)i == j0) ? 0.f : __builtin_inff();
+      __syncthreads();
+      float* Mold = M0;
+      float* Mnew = M1;
+      int until = T - 2 < 0 ? 0 : (T - 2) % C;         // steps until the next stored array: M_{t+1} with (T - 2 - t) % C == 0
+      float* row = my_rows;
+      for (int t = 0; t < T - 1; ++t) {
+        const float xt = xs[t], wt = ws[t];
+        const bool keep = record && until == 0 && t + 1 < T - 1;
+#pragma unroll
+        for (int r = 0; r < RUNS; ++r) {
+          float best[RUN];
+#pragma unroll
+          for (int i = 0; i < RUN; ++i) best[i] = __builtin_inff();
+          const float* m_in = Mold + (low(r, 0) >> K);          // a run lies inside one predecessor group
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            const float m = m_in[pj(j) * PB];
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) {
+              const float d = xt - cb[r][i][j];
+              best[i] = fminf(best[i], m + wt * (d * d));
+            }
+          }
+          if constexpr (LANES >= 2) best[0] = fminf(best[0], lane_xor_dpp<1>(best[0]));
+          if constexpr (LANES >= 4) best[0] = fminf(best[0], lane_xor_dpp<2>(best[0]));
+          float* m_out = Mnew + low(r, 0);
+          float* g_out = row + low(r, 0);
+          if constexpr (RUN % 4 == 0) {
+#pragma unroll
+            for (int i = 0; i < RUN; i += 4) {
+              const f4 q = {best[i], best[i + 1], best[i + 2], best[i + 3]};
+              *(f4*)(m_out + i) = q;
+              if (keep) *(f4*)(g_out + i) = q;
+            }
+          } else if (LANES == 1 || tid % LANES == 0) {
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) {
+              m_out[i] = best[i];
+              if (keep) g_out[i] = best[i];
+            }
+          }
+        }
+        if (keep) row += SJ;
+        until = until == 0 ? C - 1 : until - 1;
+        __syncthreads();
+        float* tmp = Mold; Mold = Mnew; Mnew = tmp;
+      }
+      // last step: argmin over all states of cost_{T-1}, first index among equals; second pass: only states whose
+      // lower part is j0
+      const float xt = xs[T - 1], wt = ws[T - 1];
+      float best = __builtin_inff();
+      uint32_t bs = 0xFFFFFFFFu;
+#pragma unroll
+      for (int r = 0; r < RUNS; ++r)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const float m = Mold[pj(j) * PB + (low(r, 0) >> K)];
+#pragma unroll
+          for (int i = 0; i < RUN; ++i) {
+            const uint32_t s = (uint32_t)(pj(j) * SJ + low(r, i));
+            const float d = xt - cb[r][i][j];
+            float c = m + wt * (d * d);
+            if (constrained && (uint32_t)low(r, i) != j0) c = __builtin_inff();
+            if (c < best || (c == best && s < bs)) { best = c; bs = s; }
+          }
+        }
+      // wave, then workgroup reduction of (value, index)
+      argmin_lanes<64>(best, bs);
+      if (lane == 0) { red_v[tid >> 6] = best; red_i[tid >> 6] = bs; }
+      __syncthreads();
+      float b = red_v[lane & 15];
+      uint32_t bi = red_i[lane & 15];
+      argmin_lanes<16>(b, bi);
+      final_state = bi == 0xFFFFFFFFu ? 0u : bi;        // every cost infinite or NaN: the reference's argmin gives 0
+      __syncthreads();
+      if (!record) j0 = final_state & (SJ - 1);
+    }
+    // ---- trace back (htr/reference.py:43-49): from s_t to s_{t-1} .. s_{t-n}, n = min(C, t), in one turn.  With p_0 = s_t >> K
+    // and predecessors j_1, j_2, .., the state s_{t-d-1} is (j_{d+1}, p_d), p_d = (j_d, .., j_1, upper bits of p_0), and
+    // M_{t-d}[p_d] = min over j_{d+1} of M_{t-d-1}[(j_{d+1}, p_d) >> K] + term.  A lane stands for one (j_n, .., j_1), j_n in its
+    // lowest bits (and the upper bits of j_n, if the lanes do not suffice, in PER registers): level n - 1 reads M_{t-n},
+    // each level is a minimum over the lanes of one digit, which leaves the next level's values where they are needed.
+    // The lanes that attain a level's minimum are kept as a mask, and the digits are read off the masks at the end.
+    uint16_t* st = states + tile * T;
+    if (tid == 0) st[T - 1] = (uint16_t)final_state;
+    if (T > 1) {
+      constexpr int RL = SJ >= THREADS ? SJ / THREADS : 1;             // row elements per thread
+      auto lds_pos = [](uint32_t e) { return e + (e >> 4); };
+      const float* row = my_rows + (size_t)nrows * SJ;
+      int left = nrows;                                                // stored arrays not yet requested
+      auto request = [&](float (&reg)[RL]) {
+        if (left > 0) {
+          row -= SJ;
+#pragma unroll
+          for (int i = 0; i < RL; ++i) if (SJ >= THREADS || tid < SJ) reg[i] = row[i * THREADS + tid];
+        } else {
+#pragma unroll
+          for (int i = 0; i < RL; ++i) reg[i] = (!tailbite || (uint32_t)(i * THREADS + tid) == j0) ? 0.f : __builtin_inff();      // M_0
+        }
+        --left;
+      };
+      auto place = [&](const float (&reg)[RL], float* buf) {
+#pragma unroll
+        for (int i = 0; i < RL; ++i) if (SJ >= THREADS || tid < SJ) buf[lds_pos((uint32_t)(i * THREADS + tid))] = reg[i];
+      };
+      uint32_t s = final_state;
+      int t = T - 1;
+      auto turn = [&](auto nc, const float* buf) {
+        constexpr int n = decltype(nc)::value;
+        constexpr int PERB = K * n > 6 ? K * n - 6 : 0, PER = 1 << PERB, NBITS = K - PERB;      // lane bits of j_n
+        const uint32_t p0 = s >> K;
+        auto digit = [&](int i) { return i == n ? (uint32_t)lane & ((1u << NBITS) - 1) : ((uint32_t)lane >> (NBITS + K * (n - 1 - i))) & ((1u << K) - 1); };
+        unsigned long long mask[n][PER];
+        float v = 0.f;
+#pragma unroll
+        for (int d = n - 1; d >= 0; --d) {
+          uint32_t p = p0 >> (K * d);
+#pragma unroll
+          for (int i = 1; i <= d; ++i) p |= digit(i) << (16 - K - K * (d - i + 1));
+          const float xt = xs[t - d - 1], wt = ws[t - d - 1];
+          float c[PER];
+          const int per = d == n - 1 ? PER : 1;
+#pragma unroll
+          for (int k = 0; k < per; ++k) {
+            const uint32_t state = ((digit(d + 1) | (d == n - 1 ? (uint32_t)k << NBITS : 0u)) << (16 - K)) | p;
+            const float m = d == n - 1 ? buf[lds_pos(state >> K)] : v;
+            const float dd = xt - cb_of(state);
+            c[k] = m + wt * (dd * dd);
+          }
+          v = c[0];
+#pragma unroll
+          for (int k = 1; k < per; ++k) v = fminf(v, c[k]);
+          // over the lane bits of digit d + 1; the lower bits hold equal values already, so a mirror is as good as an xor
+          const int lo = d == n - 1 ? 0 : NBITS + K * (n - 2 - d), hi = d == n - 1 ? NBITS : lo + K;
+#pragma unroll
+          for (int bit = lo; bit < hi; ++bit) {
+            if (bit == 0) v = fminf(v, dpp_mov<0xB1>(v));
+            if (bit == 1) v = fminf(v, dpp_mov<0x4E>(v));
+            if (bit == 2) v = fminf(v, dpp_mov<0x141>(v));
+            if (bit == 3) v = fminf(v, dpp_mov<0x140>(v));
+            if (bit == 4) { float e, o; halves16(v, e, o); v = fminf(e, o); }
+            if (bit == 5) { float e, o; halves32(v, e, o); v = fminf(e, o); }
+          }
+#pragma unroll
+          for (int k = 0; k < per; ++k) mask[d][k] = __ballot(c[k] == v);
+        }
+        uint32_t base = 0u;                                            // first lane of the digits found so far
+#pragma unroll
+        for (int d = 0; d < n; ++d) {
+          const int shift = d == n - 1 ? 0 : NBITS + K * (n - 2 - d), width = d == n - 1 ? NBITS : K;
+          const int span = 1 << (shift + width);                       // lanes that share those digits
+          const unsigned long long in_span = span >= 64 ? ~0ull : ((1ull << (span & 63)) - 1);
+          uint32_t j = 0u;
+          bool found = false;
+#pragma unroll
+          for (int k = 0; k < (d == n - 1 ? PER : 1); ++k) {
+            const unsigned long long mk = (mask[d][k] >> base) & in_span;
+            if (!found && mk != 0ull) { j = ((uint32_t)__builtin_ctzll(mk) >> shift) | ((uint32_t)k << width); found = true; }
+          }
+          if (d < n - 1) base += j << shift;
+          s = j * SJ + (s >> K);
+          if (lane == 0) st[t - d - 1] = (uint16_t)s;
+        }
+      };
+      // arrays travel three turns ahead, two in registers and one in the other LDS buffer (K = 2, whose arrays are the
+      // largest: two turns, one in registers)
+      constexpr bool TWO = RL <= 8;
+      float ra[RL], rb[TWO ? RL : 1];
+      request(ra);
+      place(ra, M0);
+      request(ra);
+      if constexpr (TWO) request(rb);
+      __syncthreads();
+      auto one = [&](float (&reg)[RL], float* cur, float* nxt) {
+        place(reg, nxt);
+        request(reg);
+        if (tid < 64) {
+          if (t >= C) turn(std::integral_constant<int, C>{}, cur);
+          else if (C >= 4 && t == 3) turn(std::integral_constant<int, (C >= 4 ? 3 : 1)>{}, cur);
+          else if (C >= 3 && t == 2) turn(std::integral_constant<int, (C >= 3 ? 2 : 1)>{}, cur);
+          else turn(std::integral_constant<int, 1>{}, cur);
+        }
+        t -= C;
+        __syncthreads();
+      };
+      while (t > 0) {
+        one(ra, M0, M1);
+        if (t > 0) {
+          if constexpr (TWO) one(rb, M1, M0);
+          else one(ra, M1, M0);
+        }
+      }
+    }
+    __syncthreads();                                    // xs, ws and the M arrays are free for the next tile
+  }
+}

@@ -13,8 +13,6 @@ from . import _native, wire
 
 # callable(x[B, 256], w[B, 256], cb[65536], K) -> int64 states [B, 256]; None = the library's search on the GPU
 VITERBI = None
-# tiles per launch: bounds the backpointer scratch (tiles * 255 * (65536 >> K) bytes)
-MAX_SCRATCH_BYTES = 1 << 30
 _SCRATCH = {}
 _CHECKED_CB = set()          # data pointers of codebook tensors already compared with the procedural codebook
 
@@ -39,26 +37,21 @@ def viterbi(x, w, cb=None, K=4, tailbite=True):
     if w.shape != x.shape or not 1 <= T <= 256:
         raise RuntimeError("viterbi wants x and w of one shape [B, T <= 256]")
     L = _native.lib()
-    per_tile = L.htr_viterbi_workspace_bytes(1, T, K)
-    if per_tile == 0:
-        raise RuntimeError(f"viterbi: unsupported K {K} (2..8)")
-    out = torch.empty((B, T), dtype=torch.int16, device=x.device)
-    batch = max(1, min(B, MAX_SCRATCH_BYTES // per_tile))
-    cus = torch.cuda.get_device_properties(x.device).multi_processor_count
-    if B > batch >= cus:
-        batch -= batch % cus        # one workgroup per tile: whole rounds over the CUs, no launch with a few stragglers
+    if B == 0:
+        return torch.empty((0, T), dtype=torch.int64, device=x.device)
     with torch.cuda.device(x.device):
+        need = L.htr_viterbi_workspace_bytes(B, T, K)
+        if need == 0:
+            raise RuntimeError(f"viterbi: unsupported K {K} (2..8)")
+        out = torch.empty((B, T), dtype=torch.int16, device=x.device)
         stream = torch.cuda.current_stream(x.device)
-        need = L.htr_viterbi_workspace_bytes(batch, T, K)
         key = (x.device.index, stream.cuda_stream)
         ws = _SCRATCH.get(key)
         if ws is None or ws.numel() < need:
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
             _SCRATCH[key] = ws
-        for b0 in range(0, B, batch):
-            nb = min(batch, B - b0)
-            _native.check(L.htr_viterbi(x[b0:].data_ptr(), w[b0:].data_ptr(), nb, T, K, 1 if tailbite else 0,
-                                        out[b0:].data_ptr(), ws.data_ptr(), ws.numel(), stream.cuda_stream))
+        _native.check(L.htr_viterbi(x.data_ptr(), w.data_ptr(), B, T, K, 1 if tailbite else 0, out.data_ptr(), ws.data_ptr(),
+                                    ws.numel(), stream.cuda_stream))
     return out.long() & 0xFFFF
 
 

@@ -162,6 +162,23 @@ def test_gpu_search_matches_oracle(dev, oracle, K, B, T, tailbite):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,B,lengths", [(2, 3, (2, 3, 4, 5, 6, 8, 9, 30)), (3, 3, (2, 3, 4, 5, 7, 8, 29)), (4, 3, (2, 3, 4, 5, 6, 31)),
+                                         (5, 2, (2, 3, 20)), (6, 2, (2, 21)), (7, 2, (2, 22)), (8, 2, (2, 23)), (4, 600, (11,))])
+@pytest.mark.parametrize("tailbite", [True, False])
+def test_gpu_search_at_the_edges_of_its_trace_back(dev, oracle, K, B, lengths, tailbite):
+    """Lengths around multiples of the steps that the trace back resolves in one turn (4, 3, 2, 1 at K = 2, 3, 4, 5 and
+    more), and more tiles than workgroups, so that a workgroup takes several in turn.  Whole numbers: exact."""
+    from htr_amd import encode
+    for T in lengths:
+        print(f"viterbi K={K} B={B} T={T} tailbite={tailbite}", flush=True)
+        g = torch.Generator().manual_seed(77 * K + B + T)
+        x = torch.randn(B, T, generator=g)
+        w = torch.rand(B, T, generator=g) + 0.25
+        st = encode.viterbi(x.to(dev), w.to(dev), None, K, tailbite=tailbite).cpu().numpy()
+        assert np.array_equal(st.astype(np.uint32), oracle.c_viterbi(x.numpy(), w.numpy(), K, tailbite=tailbite))
+
+
+@pytest.mark.gpu
 def test_gpu_search_refuses_another_codebook(dev):
     from htr_amd import encode, wire
     print("viterbi: codebook check", flush=True)
