@@ -38,6 +38,7 @@ namespace {
 #include "decode.hpp"
 #include "linear.hpp"
 #include "linear_batch.hpp"
+#include "linear_tile.hpp"
 #include "linear_gemm.hpp"
 #include "dequant.hpp"
 #include "viterbi.hpp"
@@ -80,7 +81,7 @@ size_t htr_workspace_bytes(int m, int n, int K, int M, int nsplit) {
   if (wants_batch(M, nsplit, m, n)) {
     BatchPlan bp;
     if (!make_batch_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return 0;
-    return ws_need((size_t)bp.wgs * M * 128 * sizeof(float), prerot_bytes(n, M));
+    return ws_need((size_t)bp.wgs * M * 128 * sizeof(float), prerot_bytes(n, batch_prerot_rows(M)));
   }
   if (M > HTR_MAX_GROUP_ROWS) return 0;          // the chunked kernel takes up to 32 rows
   Plan pl;
@@ -207,9 +208,7 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     unsigned char* wsp = (unsigned char*)workspace + ws_half(workspace_bytes);
     LinearTail t;
     t.scales = (const uint16_t*)scales; t.sv = (const uint8_t*)sv; t.bias = bias; t.y = y;
-    t.xt_g = (const _Float16*)wsp;
-    t.xs_g = (const float*)(wsp + align256((size_t)M * n * 2));
-    t.sc_g = (const float*)(wsp + align256((size_t)M * n * 2) + align256((size_t)M * (n / 128) * 16));
+    place_prerot(t, wsp, n, batch_prerot_rows(M));
     t.status = (uint32_t*)workspace;
     t.cbscale = htr_cbscale();
     t.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
@@ -218,11 +217,11 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     hipStream_t st = (hipStream_t)stream;
     // the workgroups rotate their own activations where the plan allows it (16-bit rows on 16-byte boundaries)
     const bool rot = bp.rot && x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0;
-    if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st));
+    if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, tile_rows(M)));
     BatchArgs ba;
     ba.qw = (const uint32_t*)qweight; ba.part = (float*)((unsigned char*)workspace + WS_HEADER); ba.x = x; ba.su = (const uint8_t*)su;
     ba.m = m; ba.n = n; ba.M = M; ba.flags = x_dtype | (y_dtype << 2) | (bp.last_finishes ? FLAG_LAST_FINISHES : 0);
-    if (bp.rot && !rot) bp.lds = batch_lds_bytes(M);            // the staged kernel's layout
+    if (bp.rot && !rot) bp.lds = batch_lds_bytes(M);            // the layout of the kernel for pre-rotated activations
     HTR_FOR_K(K, return launch_batch_k<KK>(ba, rot, t, bp, st));
     return HTR_OK;
   }
@@ -330,6 +329,7 @@ static bool make_group_plan(int count, int m, int n, int max_M, Plan& pl) {
 
 size_t htr_grouped_workspace_bytes(int count, int m, int n, int K, int max_M) {
   if (K < 2 || K > 8 || !shape_ok(m, n) || max_M < 1 || max_M > HTR_MAX_GROUP_ROWS || count < 1 || count > HTR_MAX_GROUP) return 0;
+  if (max_M > 8) return ws_need(0, prerot_bytes(n, (size_t)32 * count));      // k_linear_tile: no partials, one row tile per problem
   Plan pl;
   if (!make_group_plan(count, m, n, max_M, pl)) return 0;
   return ws_need((size_t)count * pl.wgs * max_M * 128 * sizeof(float), (size_t)count * prerot_bytes(n, max_M));
@@ -344,12 +344,26 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
   if (max_M < 1 || max_M > HTR_MAX_GROUP_ROWS) return HTR_ERR_BATCH;
   if (!dtype_ok(x_dtype) || !dtype_ok(y_dtype)) return HTR_ERR_DTYPE;
   if ((uintptr_t)entries & 7) return HTR_ERR_ALIGN;
-  Plan pl;
-  if (!make_group_plan(count, m, n, max_M, pl)) return HTR_ERR_SPLIT;
   const size_t need = htr_grouped_workspace_bytes(count, m, n, K, max_M);
+  if (need == 0) return HTR_ERR_SPLIT;
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
 
   unsigned char* wsp = (unsigned char*)workspace + ws_half(workspace_bytes);      // scratch half
+  if (max_M > 8) {
+    // 9 to 32 rows per problem: one tile of 32 rows each
+    LinearTail t = {};
+    place_prerot(t, wsp, n, (size_t)32 * count);
+    t.status = (uint32_t*)workspace;
+    t.cbscale = htr_cbscale();
+    t.group = entries;
+    hipStream_t st = (hipStream_t)stream;
+    HTR_CHECK_HIP(launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, max_M, count), dim3(WG_THREADS), 0, st, (const void*)nullptr,
+                                (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries, 0ull, 1));
+    BatchArgs ba = {nullptr, nullptr, nullptr, nullptr, m, n, 0, x_dtype | (y_dtype << 2)};
+    HTR_FOR_K(K, return (launch_tile_v<KK, 1>(ba, t, 1, count, st)));
+  }
+  Plan pl;
+  if (!make_group_plan(count, m, n, max_M, pl)) return HTR_ERR_SPLIT;
   const size_t pre = prerot_bytes(n, max_M);
   LinearLaunch a;
   a.qw = nullptr; a.x = nullptr; a.su = nullptr;
@@ -370,7 +384,7 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
   hipStream_t st = (hipStream_t)stream;
   HTR_CHECK_HIP(launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, max_M, count), dim3(WG_THREADS), 0, st, (const void*)nullptr,
                               (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries,
-                              (unsigned long long)pre));
+                              (unsigned long long)pre, 0));
   HTR_FOR_K(K, return launch_linear_k<KK>(a, true, pl.mb, pl.wgs, pl.lds, st));
   return HTR_OK;
 }

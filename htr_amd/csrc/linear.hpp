@@ -48,6 +48,14 @@ __host__ __device__ inline size_t lds_bytes(int M, int nbl, int segfin) {
   return lds_fin_offset(M, nbl) + (size_t)segfin * M * 128 * 4;
 }
 
+// Order of the rotated activations for k_linear_tile: fragments of 32 rows x 16 columns, 1 KB each, as the lanes of a matrix
+// instruction want them.  Fragment (row tile jt, 32-column unit u, half hf): lane (kg = lane / 32, l32) holds row 32 jt + l32, columns
+// 32 u + 16 kg + 8 hf .. + 7.
+__host__ __device__ inline size_t frag_half(int n, size_t row, int col) {      // half-index of an element in the fragment order
+  const size_t unit = (row >> 5) * (size_t)(n >> 5) + (col >> 5);
+  return ((unit * 2 + ((col >> 3) & 1)) * 64 + ((col >> 4) & 1) * 32 + (row & 31)) * 8 + (col & 7);
+}
+
 // power-of-two activation scale 2^e with sqrt(128) * amax / 2^e in (8192, 16384]: |H128 x| / sqrt(128) <= sqrt(128) * max|x|,
 // so the rotated activations neither overflow f16 nor fall into its denormals
 __device__ __forceinline__ int scale_exponent(float amax) {
@@ -113,19 +121,20 @@ __device__ __forceinline__ void rotate4_mfma(const u4& xr, uint32_t sb, bool is_
 // (n / 512 loads per thread), which is cheaper than a second launch or an exchange between workgroups.
 __global__ __launch_bounds__(WG_THREADS) void k_rotate(const void* __restrict__ x, const uint8_t* __restrict__ su, int n, int x_dtype,
                                                        _Float16* __restrict__ xt_g, float* __restrict__ xs_g, float* __restrict__ sc_g,
-                                                       const htr_group_entry* __restrict__ group, unsigned long long group_stride) {
+                                                       const htr_group_entry* __restrict__ group, unsigned long long group_stride, int frag) {
   __shared__ float s_max[WG_WAVES];
   if (group != nullptr) {                  // grouped: blockIdx.z = problem, outputs shifted by the problem's stride
     const htr_group_entry& ge = group[blockIdx.z];
     if ((int)blockIdx.y >= ge.M) return;
     x = ge.x; su = (const uint8_t*)ge.su;
-    const size_t shift = (size_t)blockIdx.z * group_stride;
+    const size_t shift = (size_t)blockIdx.z * group_stride;        // fragment order: 0, problem z has the rows from 32 z on
     xt_g = (_Float16*)((unsigned char*)xt_g + shift);
     xs_g = (float*)((unsigned char*)xs_g + shift);
     sc_g = (float*)((unsigned char*)sc_g + shift);
   }
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, mrow = blockIdx.y, nblk = n >> 7;
   const size_t row = (size_t)mrow * n;
+  const size_t orow = frag ? (size_t)blockIdx.z * 32 + mrow : (size_t)mrow;      // row of the outputs
   const int blk = blockIdx.x * WG_WAVES + w;
   const int col = blk * 128;
   // Every load of the kernel goes out back to back, through descriptors over the activation row and the sign bytes:
@@ -187,19 +196,19 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate(const void* __restrict__ 
   for (int k = 0; k < WG_WAVES; ++k) amax = fmaxf(amax, s_max[k]);
   const int e = scale_exponent(amax);
   const float inv_sc = pow2f(-e);
-  if (threadIdx.x == 0 && blockIdx.x == 0) sc_g[mrow] = pow2f(e);
+  if (threadIdx.x == 0 && blockIdx.x == 0) sc_g[orow] = pow2f(e);
   if (blk < nblk) {
     va *= inv_sc; vb *= inv_sc;
     fwht128_wave(va, vb, lane);
     const _Float16 ha = (_Float16)(va * INV_SQRT128), hb = (_Float16)(vb * INV_SQRT128);
-    xt_g[row + col + lane] = ha;
-    xt_g[row + col + lane + 64] = hb;
+    xt_g[frag ? frag_half(n, orow, col + lane) : row + col + lane] = ha;
+    xt_g[frag ? frag_half(n, orow, col + lane + 64) : row + col + lane + 64] = hb;
     // sums of the rounded values: the lane's first element lies in tile lane / 16, its second in tile 4 + lane / 16, so the
     // 16-lane row parity is the tile parity of both, and the two elements are the two halves of the block
     float ea, oa, eb, ob;
     wave_sum_by_row_parity((float)ha, ea, oa);
     wave_sum_by_row_parity((float)hb, eb, ob);
-    if (lane == 0) *(f4*)(xs_g + ((size_t)mrow * nblk + blk) * 4) = f4{ea + eb, oa + ob, ea + oa, eb + ob};
+    if (lane == 0) *(f4*)(xs_g + (orow * nblk + blk) * 4) = f4{ea + eb, oa + ob, ea + oa, eb + ob};
   }
 }
 
@@ -208,7 +217,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate(const void* __restrict__ 
 // seventh of the vector instructions of the butterfly version per block, which shows where the rotation is not just
 // latency: 128 rows of 14336 columns take 8.6 us there.
 __global__ __launch_bounds__(WG_THREADS) void k_rotate_mfma(const void* __restrict__ x, const uint8_t* __restrict__ su, int n, int is_bf16,
-                                                            _Float16* __restrict__ xt_g, float* __restrict__ xs_g, float* __restrict__ sc_g) {
+                                                            _Float16* __restrict__ xt_g, float* __restrict__ xs_g, float* __restrict__ sc_g, int frag) {
   __shared__ uint32_t s_amax[WG_WAVES];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int mrow = blockIdx.y, nblk = n >> 7;
@@ -251,14 +260,16 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate_mfma(const void* __restri
   rotate4_mfma(xr, sb, is_bf16 != 0, lane, y);
   const int b_o = b0 + gk;                                 // lane (p = lane / 16, j) holds elements 32 a' + 16 h + j of block b0 + p
   const bool live_o = b_o < nblk;
-  HTR_GLOBAL _Float16* dst = (HTR_GLOBAL _Float16*)xt_g + (size_t)mrow * n + b_o * 128 + j;
+  // element 32 a + 16 h of the lane: row-major, or in fragment order (unit 4 b_o + a, half j / 8, lane 32 h + row % 32, j % 8)
+  HTR_GLOBAL _Float16* dst = (HTR_GLOBAL _Float16*)xt_g + (frag ? frag_half(n, mrow, b_o * 128 + j) : (size_t)mrow * n + b_o * 128 + j);
+  const int step_a = frag ? 1024 : 32, step_h = frag ? 256 : 16;
   float r[2][4];
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       const _Float16 hv = (_Float16)(y[h][a] * f);
-      if (live_o) dst[32 * a + 16 * h] = hv;
+      if (live_o) dst[step_a * a + step_h * h] = hv;
       r[h][a] = (float)hv;
     }
   // sums of the rounded values: even tiles (h = 0), odd tiles (h = 1), columns 0..63 (a < 2), columns 64..127

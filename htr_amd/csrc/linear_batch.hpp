@@ -1,4 +1,185 @@
 // Part of htr_gfx950.hip, included inside its anonymous namespace: k_linear_batch: 9 to 128 activation rows.
+// ------------------------------------------------------------------------------------------------ output side of a row block
+// Raw bits of the row constants (scale, output sign, bias) of rows lane and lane + 64 of a row block: requested early, converted late.
+struct RowBits { uint32_t sc0, sc1, sv0, sv1, b0, b1; };
+__device__ __forceinline__ RowBits load_row_bits(const LinearTail& t, int y_dtype, int r0) {
+  const int r1 = r0 + 64;
+  RowBits r = {0u, 0u, 0u, 0u, 0u, 0u};
+  r.sc0 = ((const HTR_GLOBAL uint16_t*)t.scales)[r0];
+  r.sc1 = ((const HTR_GLOBAL uint16_t*)t.scales)[r1];
+  r.sv0 = ((const HTR_GLOBAL uint8_t*)t.sv)[r0 >> 3];
+  r.sv1 = ((const HTR_GLOBAL uint8_t*)t.sv)[r1 >> 3];
+  if (t.bias != nullptr) {
+    if (y_dtype == HTR_F32) { r.b0 = ((const HTR_GLOBAL uint32_t*)t.bias)[r0]; r.b1 = ((const HTR_GLOBAL uint32_t*)t.bias)[r1]; }
+    else { r.b0 = ((const HTR_GLOBAL uint16_t*)t.bias)[r0]; r.b1 = ((const HTR_GLOBAL uint16_t*)t.bias)[r1]; }
+  }
+  return r;
+}
+// Who finishes which activation rows of a row block that S workgroups share.
+struct SplitRole { int S, s_idx; bool spread, finisher; };
+__device__ __forceinline__ SplitRole split_role(int M, int S, int s_idx, int flags) {
+  // the splits share the output side (below), unless the host found that the grid does not fit the chip at once: splits
+  // that wait for each other must all be resident, a last split that waits for the earlier ones need not be
+  const bool spread = (M > 16 || (M > 8 && S > 2)) && !(flags & FLAG_LAST_FINISHES);
+  return {S, s_idx, spread, spread ? s_idx < ((M + 7) >> 3) : s_idx == S - 1};
+}
+
+// The workgroup's partial of the row block is in LDS as two copies (to be added) of `ld` floats per activation row, the
+// second `copy` floats behind the first; output rows lane and lane + 64 sit at pos0 and pos1.  RPW = activation rows a
+// wave finishes at most.
+template <int RPW>
+__device__ __forceinline__ void finish_row_block(const LinearTail& t, float* __restrict__ part, int rb, int m, int M, const SplitRole& role,
+                                                 const RowBits& raw, const float* s_fin, int ld, int copy, int pos0, int pos1, int w,
+                                                 int lane, int y_dtype) {
+  const int S = role.S, s_idx = role.s_idx, RG = (M + 7) >> 3;      // RG: groups of eight activation rows
+  const bool spread = role.spread, finisher = role.finisher;
+  const int r0 = rb * 128 + lane, r1 = r0 + 64;
+  // ---- exchange between the splits of the row block.  The activation rows are dealt to the splits in groups of eight
+  // (group rg = rows 8 rg .. 8 rg + 7, one row per wave): split rg mod S finishes group rg, every other split leaves
+  // its partial of those rows in its slot.  So the output side of many rows is spread over the splits instead of
+  // falling to one workgroup (32 rows on 4096x14336, 8 splits: 23.0 -> 19.7 us; 128 rows: 56.6 -> 38.5).  The
+  // workgroups of one row block are neighbours in dispatch order and the grid fits the chip (the host checks it against
+  // the device's CU count and otherwise sets FLAG_LAST_FINISHES), so they run together; the wait is bounded all the same.  Up to 8 rows (one group), and up to 16 rows with two splits, the last split
+  // finishes everything, as in k_linear: two workgroups that wait for each other cost 0.3 us more than one that waits.
+  for (int rg = 0, owner = spread ? 0 : S - 1; rg < RG; ++rg, owner = !spread ? owner : (owner + 1 == S ? 0 : owner + 1)) {
+    const int mrow = 8 * rg + w;
+    if (owner != s_idx && mrow < M) {
+      const float* own = s_fin + mrow * ld;
+      const float* oth = own + copy;
+      uint32_t* dst = (uint32_t*)(part + (((size_t)rb * S + s_idx) * M + mrow) * 128);
+      __hip_atomic_store(dst + lane, __float_as_uint(own[pos0] + oth[pos0]) | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(dst + lane + 64, __float_as_uint(own[pos1] + oth[pos1]) | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  if (!finisher) return;
+  const uint32_t stale = t.status != nullptr ? load_status(t.status) : 0u;     // non-zero: an earlier launch on this workspace gave up
+
+  // ---- output side of this split's row groups: add the other splits' partials (fixed order), finish
+  const float rs0 = f16_bits_to_float((uint16_t)raw.sc0) * t.cbscale * INV_SQRT128;
+  const float rs1 = f16_bits_to_float((uint16_t)raw.sc1) * t.cbscale * INV_SQRT128;
+  const float sg0 = ((raw.sv0 >> (lane & 7)) & 1u) ? -1.f : 1.f, sg1 = ((raw.sv1 >> (lane & 7)) & 1u) ? -1.f : 1.f;
+  auto cvt_bias = [&](uint32_t b) {
+    return y_dtype == HTR_F32 ? __uint_as_float(b) : y_dtype == HTR_BF16 ? bf16_bits_to_float((uint16_t)b) : f16_bits_to_float((uint16_t)b);
+  };
+  const float b0v = cvt_bias(raw.b0), b1v = cvt_bias(raw.b1);
+  // slot of the k-th other split (k = 0 .. S - 2, own split skipped) for activation row mrow
+  auto slot_of = [&](int k, int mrow) { return (uint32_t*)(part + (((size_t)rb * S + (k + (k >= s_idx ? 1 : 0))) * M + mrow) * 128); };
+  // waits (bounded) until every other split's partial of activation row mrow is there; their sum in fixed order
+  auto wait_for_row = [&](int mrow, float& v0s, float& v1s) {
+    int tries = 0;
+    for (;;) {
+      bool missing = false;
+      v0s = 0.f; v1s = 0.f;
+      for (int jb = 0; jb < S - 1; jb += 8) {
+        uint32_t u0[8], u1[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const uint32_t* pp = slot_of(min(jb + k, S - 2), mrow);
+          u0[k] = __hip_atomic_load(pp + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          u1[k] = __hip_atomic_load(pp + lane + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (jb + k < S - 1) {
+            missing |= (u0[k] == 0u) | (u1[k] == 0u);
+            v0s += __uint_as_float(u0[k]); v1s += __uint_as_float(u1[k]);
+          }
+      }
+      if (!__any(missing)) return false;
+      if (++tries >= t.spin_limit) return true;
+      __builtin_amdgcn_s_sleep(2);
+    }
+  };
+  // the rest of a row: slots back to zero for the next call (or the failure noted), own partial, output side
+  auto finish_row = [&](int mrow, float v0s, float v1s, bool failed) {
+    if (S > 1) {
+      if (!failed) {
+        for (int k = 0; k < S - 1; ++k) {
+          uint32_t* pp = slot_of(k, mrow);
+          __hip_atomic_store(pp + lane, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(pp + lane + 64, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      } else if (lane == 0) {
+        report_give_up(t.status);
+      }
+    }
+    failed |= stale != 0u;
+    const float* own = s_fin + mrow * ld;
+    const float* oth = own + copy;
+    v0s += own[pos0] + oth[pos0]; v1s += own[pos1] + oth[pos1];
+    v0s *= rs0; v1s *= rs1;
+    fwht128_wave(v0s, v1s, lane);
+    v0s = __builtin_fmaf(v0s, sg0, b0v);
+    v1s = __builtin_fmaf(v1s, sg1, b1v);
+    if (failed) { v0s = __builtin_nanf(""); v1s = v0s; }
+    store_elem_g(t.y, y_dtype, (size_t)mrow * m + r0, v0s);
+    store_elem_g(t.y, y_dtype, (size_t)mrow * m + r1, v1s);
+  };
+  // Wave w finishes row w of this split's groups s_idx, s_idx + S, ...: its i-th row is 8 (s_idx + i S) + w (all groups
+  // if the last split finishes everything).
+  auto my_row = [&](int i) { return spread ? 8 * (s_idx + i * S) + w : 8 * i + w; };
+  // With up to eight other splits the slots of several of the wave's rows are requested together (at most 2 x 32
+  // registers of them), so that the rows behind the first cost no memory round trip of their own.  JW = slots
+  // requested per row (the next power of two from S - 1; the surplus repeats the last slot).
+  auto finish_rows_together = [&](auto jw) {
+    constexpr int JW = decltype(jw)::value;
+    constexpr int RB = RPW * JW <= 32 ? RPW : 32 / JW;      // rows per request
+#pragma unroll
+    for (int rbase = 0; rbase < RPW; rbase += RB) {
+      if (my_row(rbase) >= M) break;
+      float a0[RB], a1[RB];
+      int tries = 0;
+      bool failed = false;
+      for (;;) {
+        uint32_t u0[RB][JW], u1[RB][JW];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          // a row beyond M repeats the request of the batch's first row and is not looked at
+          const int mrow = my_row(rbase + r) < M ? my_row(rbase + r) : my_row(rbase);
+#pragma unroll
+          for (int k = 0; k < JW; ++k) {
+            const uint32_t* pp = slot_of(min(k, S - 2), mrow);
+            u0[r][k] = __hip_atomic_load(pp + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            u1[r][k] = __hip_atomic_load(pp + lane + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+        bool missing = false;
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          a0[r] = 0.f; a1[r] = 0.f;
+          const bool real = my_row(rbase + r) < M;
+#pragma unroll
+          for (int k = 0; k < JW; ++k)
+            if (real && k < S - 1) {
+              missing |= (u0[r][k] == 0u) | (u1[r][k] == 0u);
+              a0[r] += __uint_as_float(u0[r][k]); a1[r] += __uint_as_float(u1[r][k]);
+            }
+        }
+        if (!__any(missing)) break;
+        if (++tries >= t.spin_limit) { failed = true; break; }
+        __builtin_amdgcn_s_sleep(2);
+      }
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+        if (my_row(rbase + r) < M) finish_row(my_row(rbase + r), a0[r], a1[r], failed);
+    }
+  };
+  if (my_row(0) >= M) return;
+  if (S > 1 && S - 1 <= 8 && my_row(1) < M) {
+    if (S - 1 <= 1) finish_rows_together(std::integral_constant<int, 1>{});
+    else if (S - 1 <= 2) finish_rows_together(std::integral_constant<int, 2>{});
+    else if (S - 1 <= 4) finish_rows_together(std::integral_constant<int, 4>{});
+    else finish_rows_together(std::integral_constant<int, 8>{});
+    return;
+  }
+  for (int i = 0; my_row(i) < M; ++i) {
+    float v0s = 0.f, v1s = 0.f;
+    const bool failed = S > 1 ? wait_for_row(my_row(i), v0s, v1s) : false;
+    finish_row(my_row(i), v0s, v1s, failed);
+  }
+}
+
+
 // ------------------------------------------------------------------------------------------------ batched linear
 // Variant for 9 .. 128 activation rows.  With that many rows the rotated activations of a whole chunk no longer fit in
 // LDS next to useful chunk lengths, and short chunks mean that every workgroup copies a large activation slice and
@@ -127,23 +308,9 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
 
   // row constants of the output side (scale, sign, bias of rows lane and lane + 64), requested ahead of the weight stream by
   // the workgroups that finish rows of the row block, so that they have long arrived when they are needed
-  const int RG = (M + 7) >> 3;               // groups of eight activation rows
-  // the splits share the output side (below), unless the host found that the grid does not fit the chip at once: splits
-  // that wait for each other must all be resident, a last split that waits for the earlier ones need not be
-  const bool spread = (M > 16 || (M > 8 && S > 2)) && !(flags & FLAG_LAST_FINISHES);
-  const bool finisher = spread ? s_idx < RG : s_idx == S - 1;
-  const int r0 = rb * 128 + lane, r1 = r0 + 64;
-  uint32_t raw_sc0 = 0u, raw_sc1 = 0u, raw_sv0 = 0u, raw_sv1 = 0u, raw_b0 = 0u, raw_b1 = 0u;   // bits only: converted at the end
-  if (finisher) {
-    raw_sc0 = ((const HTR_GLOBAL uint16_t*)t.scales)[r0];
-    raw_sc1 = ((const HTR_GLOBAL uint16_t*)t.scales)[r1];
-    raw_sv0 = ((const HTR_GLOBAL uint8_t*)t.sv)[r0 >> 3];
-    raw_sv1 = ((const HTR_GLOBAL uint8_t*)t.sv)[r1 >> 3];
-    if (t.bias != nullptr) {
-      if (y_dtype == HTR_F32) { raw_b0 = ((const HTR_GLOBAL uint32_t*)t.bias)[r0]; raw_b1 = ((const HTR_GLOBAL uint32_t*)t.bias)[r1]; }
-      else { raw_b0 = ((const HTR_GLOBAL uint16_t*)t.bias)[r0]; raw_b1 = ((const HTR_GLOBAL uint16_t*)t.bias)[r1]; }
-    }
-  }
+  const SplitRole role = split_role(M, S, s_idx, flags);
+  RowBits raw = {0u, 0u, 0u, 0u, 0u, 0u};
+  if (role.finisher) raw = load_row_bits(t, y_dtype, rb * 128 + lane);
 
   // ---- the weight stream of this wave: per step, tiles 4 ch .. 4 ch + 3 of strips 2 sp and 2 sp + 1.  One descriptor
   // from the first strip's first byte of the split to the second strip's last: lanes of the second strip that run past
@@ -355,150 +522,6 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
     }
   }
   __syncthreads();
-  const int pos0 = batch_fin_pos(lane), pos1 = batch_fin_pos(lane + 64);
-  // ---- exchange between the splits of the row block.  The activation rows are dealt to the splits in groups of eight
-  // (group rg = rows 8 rg .. 8 rg + 7, one row per wave): split rg mod S finishes group rg, every other split leaves
-  // its partial of those rows in its slot.  So the output side of many rows is spread over the splits instead of
-  // falling to one workgroup (32 rows on 4096x14336, 8 splits: 23.0 -> 19.7 us; 128 rows: 56.6 -> 38.5).  The
-  // workgroups of one row block are neighbours in dispatch order and the grid fits the chip (the host checks it against
-  // the device's CU count and otherwise sets FLAG_LAST_FINISHES), so they run together; the wait is bounded all the same.  Up to 8 rows (one group), and up to 16 rows with two splits, the last split
-  // finishes everything, as in k_linear: two workgroups that wait for each other cost 0.3 us more than one that waits.
-  for (int rg = 0, owner = spread ? 0 : S - 1; rg < RG; ++rg, owner = !spread ? owner : (owner + 1 == S ? 0 : owner + 1)) {
-    const int mrow = 8 * rg + w;
-    if (owner != s_idx && mrow < M) {
-      const float* own = s_fin + mrow * BATCH_FIN_STRIDE;
-      const float* oth = own + M * BATCH_FIN_STRIDE;
-      uint32_t* dst = (uint32_t*)(part + (((size_t)rb * S + s_idx) * M + mrow) * 128);
-      __hip_atomic_store(dst + lane, __float_as_uint(own[pos0] + oth[pos0]) | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(dst + lane + 64, __float_as_uint(own[pos1] + oth[pos1]) | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  if (!finisher) return;
-  const uint32_t stale = load_status(t.status);     // non-zero: an earlier launch on this workspace gave up
-
-  // ---- output side of this split's row groups: add the other splits' partials (fixed order), finish
-  const float rs0 = f16_bits_to_float((uint16_t)raw_sc0) * t.cbscale * INV_SQRT128;
-  const float rs1 = f16_bits_to_float((uint16_t)raw_sc1) * t.cbscale * INV_SQRT128;
-  const float sg0 = ((raw_sv0 >> (lane & 7)) & 1u) ? -1.f : 1.f, sg1 = ((raw_sv1 >> (lane & 7)) & 1u) ? -1.f : 1.f;
-  auto cvt_bias = [&](uint32_t b) {
-    return y_dtype == HTR_F32 ? __uint_as_float(b) : y_dtype == HTR_BF16 ? bf16_bits_to_float((uint16_t)b) : f16_bits_to_float((uint16_t)b);
-  };
-  const float b0v = cvt_bias(raw_b0), b1v = cvt_bias(raw_b1);
-  // slot of the k-th other split (k = 0 .. S - 2, own split skipped) for activation row mrow
-  auto slot_of = [&](int k, int mrow) { return (uint32_t*)(part + (((size_t)rb * S + (k + (k >= s_idx ? 1 : 0))) * M + mrow) * 128); };
-  // waits (bounded) until every other split's partial of activation row mrow is there; their sum in fixed order
-  auto wait_for_row = [&](int mrow, float& v0s, float& v1s) {
-    int tries = 0;
-    for (;;) {
-      bool missing = false;
-      v0s = 0.f; v1s = 0.f;
-      for (int jb = 0; jb < S - 1; jb += 8) {
-        uint32_t u0[8], u1[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const uint32_t* pp = slot_of(min(jb + k, S - 2), mrow);
-          u0[k] = __hip_atomic_load(pp + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          u1[k] = __hip_atomic_load(pp + lane + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (jb + k < S - 1) {
-            missing |= (u0[k] == 0u) | (u1[k] == 0u);
-            v0s += __uint_as_float(u0[k]); v1s += __uint_as_float(u1[k]);
-          }
-      }
-      if (!__any(missing)) return false;
-      if (++tries >= t.spin_limit) return true;
-      __builtin_amdgcn_s_sleep(2);
-    }
-  };
-  // the rest of a row: slots back to zero for the next call (or the failure noted), own partial, output side
-  auto finish_row = [&](int mrow, float v0s, float v1s, bool failed) {
-    if (S > 1) {
-      if (!failed) {
-        for (int k = 0; k < S - 1; ++k) {
-          uint32_t* pp = slot_of(k, mrow);
-          __hip_atomic_store(pp + lane, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(pp + lane + 64, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      } else if (lane == 0) {
-        report_give_up(t.status);
-      }
-    }
-    failed |= stale != 0u;
-    const float* own = s_fin + mrow * BATCH_FIN_STRIDE;
-    const float* oth = own + M * BATCH_FIN_STRIDE;
-    v0s += own[pos0] + oth[pos0]; v1s += own[pos1] + oth[pos1];
-    v0s *= rs0; v1s *= rs1;
-    fwht128_wave(v0s, v1s, lane);
-    v0s = __builtin_fmaf(v0s, sg0, b0v);
-    v1s = __builtin_fmaf(v1s, sg1, b1v);
-    if (failed) { v0s = __builtin_nanf(""); v1s = v0s; }
-    store_elem_g(t.y, y_dtype, (size_t)mrow * m + r0, v0s);
-    store_elem_g(t.y, y_dtype, (size_t)mrow * m + r1, v1s);
-  };
-  // Wave w finishes row w of this split's groups s_idx, s_idx + S, ...: its i-th row is 8 (s_idx + i S) + w (all groups
-  // if the last split finishes everything).
-  constexpr int RPW = MG * 2;                    // rows per wave at most (a single split finishes all groups)
-  auto my_row = [&](int i) { return spread ? 8 * (s_idx + i * S) + w : 8 * i + w; };
-  // With up to eight other splits the slots of several of the wave's rows are requested together (at most 2 x 32
-  // registers of them), so that the rows behind the first cost no memory round trip of their own.  JW = slots
-  // requested per row (the next power of two from S - 1; the surplus repeats the last slot).
-  auto finish_rows_together = [&](auto jw) {
-    constexpr int JW = decltype(jw)::value;
-    constexpr int RB = RPW * JW <= 32 ? RPW : 32 / JW;      // rows per request
-#pragma unroll
-    for (int rbase = 0; rbase < RPW; rbase += RB) {
-      if (my_row(rbase) >= M) break;
-      float a0[RB], a1[RB];
-      int tries = 0;
-      bool failed = false;
-      for (;;) {
-        uint32_t u0[RB][JW], u1[RB][JW];
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-          // a row beyond M repeats the request of the batch's first row and is not looked at
-          const int mrow = my_row(rbase + r) < M ? my_row(rbase + r) : my_row(rbase);
-#pragma unroll
-          for (int k = 0; k < JW; ++k) {
-            const uint32_t* pp = slot_of(min(k, S - 2), mrow);
-            u0[r][k] = __hip_atomic_load(pp + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            u1[r][k] = __hip_atomic_load(pp + lane + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-        }
-        bool missing = false;
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-          a0[r] = 0.f; a1[r] = 0.f;
-          const bool real = my_row(rbase + r) < M;
-#pragma unroll
-          for (int k = 0; k < JW; ++k)
-            if (real && k < S - 1) {
-              missing |= (u0[r][k] == 0u) | (u1[r][k] == 0u);
-              a0[r] += __uint_as_float(u0[r][k]); a1[r] += __uint_as_float(u1[r][k]);
-            }
-        }
-        if (!__any(missing)) break;
-        if (++tries >= t.spin_limit) { failed = true; break; }
-        __builtin_amdgcn_s_sleep(2);
-      }
-#pragma unroll
-      for (int r = 0; r < RB; ++r)
-        if (my_row(rbase + r) < M) finish_row(my_row(rbase + r), a0[r], a1[r], failed);
-    }
-  };
-  if (my_row(0) >= M) return;
-  if (S > 1 && S - 1 <= 8 && my_row(1) < M) {
-    if (S - 1 <= 1) finish_rows_together(std::integral_constant<int, 1>{});
-    else if (S - 1 <= 2) finish_rows_together(std::integral_constant<int, 2>{});
-    else if (S - 1 <= 4) finish_rows_together(std::integral_constant<int, 4>{});
-    else finish_rows_together(std::integral_constant<int, 8>{});
-    return;
-  }
-  for (int i = 0; my_row(i) < M; ++i) {
-    float v0s = 0.f, v1s = 0.f;
-    const bool failed = S > 1 ? wait_for_row(my_row(i), v0s, v1s) : false;
-    finish_row(my_row(i), v0s, v1s, failed);
-  }
+  finish_row_block<MG * 2>(t, part, rb, m, M, role, raw, s_fin, BATCH_FIN_STRIDE, M * BATCH_FIN_STRIDE, batch_fin_pos(lane),
+                           batch_fin_pos(lane + 64), w, lane, y_dtype);
 }
-

@@ -30,7 +30,7 @@ constexpr size_t gemm_lds_bytes(int jb) {
   const size_t xb = GEMM_XBUFS * rows * GEMM_LD * 2 + GEMM_XBUFS * rows * 4;
   return (fin > xb ? fin : xb) + 16;
 }
-typedef float f16v __attribute__((ext_vector_type(16)));
+
 
 template <int K, int P, int JB>
 __global__ __launch_bounds__(GEMM_THREADS) void k_linear_gemm(const uint32_t* __restrict__ qw, float* __restrict__ part,

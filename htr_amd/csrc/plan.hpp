@@ -27,7 +27,12 @@ inline size_t ws_need(size_t slot_bytes, size_t scratch_bytes) {
 }
 inline size_t ws_half(size_t workspace_bytes) { return workspace_bytes / 2 / 256 * 256; }
 // bytes of the pre-rotated activations, their block sums and the row scales
-inline size_t prerot_bytes(int n, int M) { return align256((size_t)M * n * 2) + align256((size_t)M * (n / 128) * 16) + align256((size_t)M * 4); }
+inline size_t prerot_bytes(int n, size_t M) { return align256(M * n * 2) + align256(M * (n / 128) * 16) + align256(M * 4); }
+inline void place_prerot(LinearTail& t, unsigned char* at, int n, size_t M) {
+  t.xt_g = (const _Float16*)at;
+  t.xs_g = (const float*)(at + align256(M * n * 2));
+  t.sc_g = (const float*)(at + align256(M * n * 2) + align256(M * (n / 128) * 16));
+}
 
 // ---- facts of the device the plans are made for: compute units and LDS bytes per compute unit, read once per device
 // (the current one) from the runtime; an unpartitioned MI355X (256 CUs, 160 KB) where no device can be asked (plans
@@ -251,7 +256,15 @@ struct BatchPlan { int S, cb, wgs, mb, rot, last_finishes; size_t lds; };
 inline bool batch_rot_fits(int M, int cb) { return (M <= 16 && cb <= 16) || (M <= 32 && cb <= 8); }
 constexpr int BATCH_MIN_M = 9;      // rows from which the library policy takes the batched kernel on every shape
 inline int batch_groups(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : 8)); }   // groups of 16 activation rows
+// Activations that were rotated ahead go to k_linear_tile from 17 to 64 rows (one or two tiles of 32).  Measured on MI355X, K4,
+// us of the kernel, k_linear_batch / k_linear_tile: 32 rows on 28672x4096 26.9 / 22.1, 14336x4096 14.5 / 13.9, 4096x14336
+// 14.7 / 14.5; 64 rows 31.5 / 28.8, 19.4 / 18.2, 18.5 / 19.1.  Beyond 64 rows its loads of the activations bound it (64 KB
+// per step and compute unit at 128 rows, 70 GB/s; 97 rows of 14336x4096 at K5 32.6 / 33.9); up to 16 rows half of its
+// matrix instructions would be empty.
+inline bool tile_rows(int M) { return M >= 17 && M <= 64; }
+inline size_t batch_prerot_rows(int M) { return tile_rows(M) ? (size_t)(M + 31) / 32 * 32 : (size_t)M; }   // rows the layout holds
 inline size_t batch_lds_bytes(int M) {
+  if (tile_rows(M)) return tile_lds_bytes((M + 31) / 32);
   const int rows = 16 * batch_groups(M);
   const size_t blocks = (size_t)2 * rows * BATCH_ROWH * 2, small = (size_t)5 * rows * 4, fin = (size_t)2 * M * BATCH_FIN_STRIDE * 4;
   return M > 64 ? (blocks + small > fin ? blocks + small : fin) : blocks + small + fin;
@@ -352,14 +365,18 @@ template <int K, int MB, bool ROT> int launch_batch_v(const BatchArgs& a, const 
                               a.m, a.n, a.M, bp.S, a.flags, t));
   return HTR_OK;
 }
+template <int K, int JB> int launch_tile_v(const BatchArgs& a, const LinearTail& t, int S, int problems, hipStream_t st) {
+  constexpr int P = K <= 4 ? 4 : 2;
+  const size_t lds = problems == 1 ? balanced_lds_request(tile_lds_bytes(JB), S * (a.m / 128)) : tile_lds_bytes(JB);
+  HTR_CHECK_HIP((allow_full_lds<k_linear_tile<K, JB, P, 2>>()));
+  HTR_CHECK_HIP(launch_kernel(k_linear_tile<K, JB, P, 2>, dim3(S, a.m / 128, problems), dim3(WG_THREADS), lds, st, a.qw, a.part, a.m, a.n, a.M, S,
+                              a.flags, t));
+  return HTR_OK;
+}
 template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
   if (rot) return bp.mb == 1 ? launch_batch_v<K, 1, true>(a, t, bp, st) : launch_batch_v<K, 2, true>(a, t, bp, st);
-  switch (bp.mb) {
-    case 1: return launch_batch_v<K, 1, false>(a, t, bp, st);
-    case 2: return launch_batch_v<K, 2, false>(a, t, bp, st);
-    case 4: return launch_batch_v<K, 4, false>(a, t, bp, st);
-    default: return launch_batch_v<K, 8, false>(a, t, bp, st);
-  }
+  if (tile_rows(a.M)) return a.M <= 32 ? launch_tile_v<K, 1>(a, t, bp.S, 1, st) : launch_tile_v<K, 2>(a, t, bp.S, 1, st);
+  return bp.mb == 1 ? launch_batch_v<K, 1, false>(a, t, bp, st) : launch_batch_v<K, 8, false>(a, t, bp, st);
 }
 // nsplit bit 29: batched kernel with the split in the low bits (0 = policy); otherwise the policy decides by M
 // Tall matrices (192 row blocks and more) fill the chip without column splits, so the batched kernel needs no exchange
@@ -379,13 +396,14 @@ inline bool wants_batch(int M, int nsplit, int m, int n) {
 
 // Rotation of all rows of x ahead of a linear launch: on the matrix unit for 16-bit rows on 16-byte boundaries, else the
 // butterfly kernel (float32, odd alignments)
-inline hipError_t launch_rotation(const void* x, const uint8_t* su, int n, int M, int x_dtype, const LinearTail& t, hipStream_t st) {
+// (frag: in the order k_linear_tile reads)
+inline hipError_t launch_rotation(const void* x, const uint8_t* su, int n, int M, int x_dtype, const LinearTail& t, hipStream_t st, bool frag = false) {
   static const bool mfma_on = getenv("HTR_ROTATE_MFMA") == nullptr || atoi(getenv("HTR_ROTATE_MFMA")) != 0;
   if (mfma_on && x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0)
     return launch_kernel(k_rotate_mfma, dim3((n / 128 + 4 * WG_WAVES - 1) / (4 * WG_WAVES), M), dim3(WG_THREADS), 0, st, x, su, n,
-                         x_dtype == HTR_BF16 ? 1 : 0, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g);
+                         x_dtype == HTR_BF16 ? 1 : 0, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, frag ? 1 : 0);
   return launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, M), dim3(WG_THREADS), 0, st, x, su, n, x_dtype,
-                       (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, (const htr_group_entry*)nullptr, 0ull);
+                       (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, (const htr_group_entry*)nullptr, 0ull, frag ? 1 : 0);
 }
 
 #define HTR_FOR_K_OR(K, EXPR, OTHERWISE)   \

@@ -736,3 +736,33 @@ def test_batched_kernel_when_the_grid_exceeds_the_compute_units(dev, oracle, M, 
     assert _rel(y_small, ref) <= REL_TOL and _rel(y_full, ref) <= REL_TOL
     # the same products either way (the rotation may come from the launch of its own in one and from the workgroups in the other)
     assert np.abs(y_small - y_full).max() <= 2e-4 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("K,m,n,M", [(2, 256, 128, 17), (3, 128, 640, 31), (4, 384, 1152, 32), (4, 256, 256, 33), (5, 128, 896, 48),
+                                     (6, 256, 384, 63), (7, 128, 1024, 64), (8, 256, 1280, 50), (4, 1024, 2048, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_tiles_of_32_rows(dev, oracle, K, m, n, M, dtype):
+    """17 to 64 rows: both tile counts and their edges, block counts around the depth of the stream, every K, rotation on the
+    matrix unit (bf16) and by butterflies (float32).  1e-3 as for every float32 result: float16 activations."""
+    from htr_amd import ops
+    print(f"tiles K={K} {m}x{n} M={M} {dtype}", flush=True)
+    qw, sc, su, sv, x = _case(m, n, K, M, 900 + M + K, dtype)
+    w = [t.to(dev) for t in (qw, sc, su, sv)]
+    ref = _ref(oracle, qw, sc, su, sv, x)
+    for _ in range(2):                                                       # the second call finds the slots as the first left them
+        assert _rel(ops.linear_f32out(x.to(dev), *w).cpu().numpy(), ref) <= REL_TOL
+    odd = torch.empty(M * n + 1, dtype=dtype, device=dev)[1:].view(M, n)     # rows that start off a 16-byte boundary
+    odd.copy_(x)
+    assert _rel(ops.linear_f32out(odd, *w).cpu().numpy(), ref) <= REL_TOL
+
+
+def test_grouped_launch_of_9_to_32_rows(dev, oracle):
+    from htr_amd import ops, wire
+    print("grouped launch, tiles", flush=True)
+    rows = [9, 0, 32, 17]
+    ws = [wire.synth_linear(384, 640, 3, 9100 + i) for i in range(4)]
+    xs = [wire.synth_activation(r, 640, 9200 + i) for i, r in enumerate(rows)]
+    got = ops.linear_grouped([x.to(dev) for x in xs], [tuple(t.to(dev) for t in w) for w in ws], out_dtype=torch.float32)
+    for w, x, y in zip(ws, xs, got):
+        if x.shape[0]:
+            assert _rel(y.cpu().numpy(), _ref(oracle, *w, x)) <= REL_TOL
