@@ -36,6 +36,8 @@ SIGNATURES = {
     "htr_anchor_decode": (_i, [_i, _i, _i, _i, _vp, _vp]),
     "htr_grouped_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "htr_linear_grouped": (_i, [_vp, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
+    "htr_moe_scratch_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "htr_moe_experts": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _vp, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp, ctypes.c_uint, _vp]),
     "htr_set_spin_limit": (None, [_i]),
     "htr_workspace_init": (_i, [_vp, _sz, _vp, _vp]),
     "htr_stream_capture_id": (ctypes.c_ulonglong, [_vp]),
@@ -64,6 +66,24 @@ def lib():
             fn.restype, fn.argtypes = res, args
         _lib = L
     return _lib
+
+
+_fast = None
+
+
+def fast():
+    """The C++ host path (htr_amd._fast), bound to the library's entry points."""
+    global _fast
+    if _fast is None:
+        L = lib()
+        try:
+            from . import _fast as module
+        except ImportError as e:
+            raise NativeLibraryMissing(f"htr_amd/_fast.so cannot be loaded ({e}); run `python -m htr_amd.build`.") from e
+        address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
+        module.bind(address(L.htr_linear), address(L.htr_stream_capture_id), address(L.htr_moe_scratch_bytes), address(L.htr_moe_experts))
+        _fast = module
+    return _fast
 
 
 def check(status):

@@ -11,8 +11,10 @@ import sys
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB = os.path.join(CSRC, "libhtr_gfx950.so")
 SOURCES = [os.path.join(CSRC, "htr_gfx950.hip")]          # one translation unit; the kernels live in the parts it includes
-PARTS = [os.path.join(CSRC, f) for f in ("decode.hpp", "linear.hpp", "linear_batch.hpp", "linear_tile.hpp", "linear_gemm.hpp", "dequant.hpp",
+PARTS = [os.path.join(CSRC, f) for f in ("decode.hpp", "linear.hpp", "linear_batch.hpp", "linear_tile.hpp", "linear_gemm.hpp", "moe.hpp", "dequant.hpp",
                                          "viterbi.hpp", "anchors.hpp", "plan.hpp")]
+BINDING_SOURCE = os.path.join(CSRC, "torch_binding.cpp")
+BINDING = os.path.join(os.path.dirname(CSRC), "_fast.so")
 HEADER = os.path.join(os.path.dirname(CSRC), os.pardir, "include", "htr_gfx950.h")
 
 HIPCC_FLAGS = [
@@ -27,24 +29,38 @@ def hipcc():
     return os.environ.get("HIPCC") or os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
 
 
+def binding_command():
+    """The host-only extension htr_amd._fast: torch's headers, g++; no kernel in it."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    lib = os.path.join(root, "lib")
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            "-I" + os.path.join(root, "include"), "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"),
+            "-I" + sysconfig.get_paths()["include"], BINDING_SOURCE, "-o", BINDING, "-L" + lib, "-lc10", "-ltorch_cpu", "-ltorch_python"]
+
+
 def build(verbose=False, extra=()):
-    cmd = [hipcc()] + HIPCC_FLAGS + list(extra) + ["-o", LIB] + SOURCES
+    cmds = [[hipcc()] + HIPCC_FLAGS + list(extra) + ["-o", LIB] + SOURCES, binding_command()]
     if verbose:
-        print(" ".join(cmd), flush=True)
-    p = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    out = "\n".join(l for l in p.stdout.splitlines() if "not a recognized feature" not in l)
-    if p.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + out)
-    if verbose and out.strip():
-        print(out)
+        for cmd in cmds:
+            print(" ".join(cmd), flush=True)
+    procs = [subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for cmd in cmds]
+    outs = [p.communicate()[0] for p in procs]
+    for cmd, p, text in zip(cmds, procs, outs):
+        out = "\n".join(l for l in text.splitlines() if "not a recognized feature" not in l)
+        if p.returncode != 0:
+            raise RuntimeError(os.path.basename(cmd[0]) + " failed:\n" + out)
+        if verbose and out.strip():
+            print(out)
     return LIB
 
 
 def is_stale():
-    if not os.path.exists(LIB):
-        return True
-    t = os.path.getmtime(LIB)
-    return any(os.path.getmtime(s) > t for s in SOURCES + PARTS + [HEADER])
+    def older(built, sources):
+        return not os.path.exists(built) or any(os.path.getmtime(s) > os.path.getmtime(built) for s in sources)
+    return older(LIB, SOURCES + PARTS + [HEADER]) or older(BINDING, [BINDING_SOURCE])
 
 
 if __name__ == "__main__":

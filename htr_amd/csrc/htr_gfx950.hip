@@ -40,6 +40,7 @@ namespace {
 #include "linear_batch.hpp"
 #include "linear_tile.hpp"
 #include "linear_gemm.hpp"
+#include "moe.hpp"
 #include "dequant.hpp"
 #include "viterbi.hpp"
 #include "anchors.hpp"
@@ -386,6 +387,102 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
                               (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries,
                               (unsigned long long)pre, 0));
   HTR_FOR_K(K, return launch_linear_k<KK>(a, true, pl.mb, pl.wgs, pl.lds, st));
+  return HTR_OK;
+}
+
+// ---- routed experts: one MoE layer in a few launches (moe.hpp)
+namespace {
+struct MoePlan { int pairs, entries, tiles, rows; size_t table, e1, e2, pos, info, xt1, xs1, sc1, xt2, xs2, sc2, h, out, total; };
+// Rows per table entry.  An entry decodes its expert's weights once, so few tall entries decode least; but a step of a tall tile
+// takes longer also where it is half empty.
+inline int moe_rows_per_entry(int pairs, int experts) {
+  const int active = experts < pairs ? experts : pairs;
+  const int mean = pairs / active;
+  return mean <= 16 ? 32 : 64;
+}
+inline bool moe_plan(int tokens, int top, int experts, int hidden, int inter, MoePlan& p) {
+  if (tokens < 1 || top < 1 || experts < 1 || experts > MOE_MAX_EXPERTS || (long)tokens * top > (1L << 24)) return false;
+  if (!shape_ok(2 * inter, hidden) || !shape_ok(hidden, inter)) return false;
+  p.pairs = tokens * top;
+  p.rows = moe_rows_per_entry(p.pairs, experts);
+  const int active = experts < p.pairs ? experts : p.pairs;
+  p.entries = active + p.pairs / p.rows;
+  p.tiles = active + p.pairs / 32;
+  if (p.entries > 65535 || hidden / 128 > 65535) return false;
+  size_t o = 0;
+  auto take = [&](size_t bytes) { const size_t at = o; o += align256(bytes); return at; };
+  p.table = take((size_t)experts * 64);
+  p.e1 = take((size_t)p.entries * sizeof(htr_group_entry));
+  p.e2 = take((size_t)p.entries * sizeof(htr_group_entry));
+  p.pos = take((size_t)p.pairs * 4);
+  p.info = take((size_t)p.pairs * 16);
+  const size_t rows = (size_t)p.tiles * 32;
+  p.xt1 = take(rows * hidden * 2); p.xs1 = take(rows * (hidden / 128) * 16); p.sc1 = take(rows * 4);
+  p.xt2 = take(rows * inter * 2); p.xs2 = take(rows * (inter / 128) * 16); p.sc2 = take(rows * 4);
+  p.h = take((size_t)p.pairs * 2 * inter * 4);
+  p.out = take((size_t)p.pairs * hidden * 4);
+  p.total = o;
+  return true;
+}
+}
+
+size_t htr_moe_scratch_bytes(int tokens, int top, int experts, int hidden, int inter) {
+  MoePlan p;
+  return moe_plan(tokens, top, experts, hidden, inter, p) ? p.total : 0;
+}
+
+int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, const float* weights, int tokens, int top,
+                    const void* const* tensors, int experts, int hidden, int inter, int K_gate_up, int K_down, float* y,
+                    void* scratch, size_t scratch_bytes, unsigned int* host_word, unsigned int ticket, void* stream) {
+  if (!x || !ids || !weights || !tensors || !y) return HTR_ERR_NULL;
+  if (K_gate_up < 2 || K_gate_up > 8 || K_down < 2 || K_down > 8) return HTR_ERR_K;
+  if (!dtype_ok(x_dtype)) return HTR_ERR_DTYPE;
+  MoePlan p;
+  if (!moe_plan(tokens, top, experts, hidden, inter, p)) return HTR_ERR_SHAPE;
+  if (((uintptr_t)x & 15) || ((uintptr_t)y & 15) || ((uintptr_t)ids & (ids_int64 ? 7 : 3)) || ((uintptr_t)weights & 3)) return HTR_ERR_ALIGN;
+  for (int i = 0; i < experts * 8; ++i) {
+    if (!tensors[i]) return HTR_ERR_NULL;
+    if ((uintptr_t)tensors[i] & ((i & 3) == 0 ? 15 : ((i & 3) == 1 ? 1 : 0))) return HTR_ERR_ALIGN;
+  }
+  if (!scratch || scratch_bytes < p.total || ((uintptr_t)scratch & 255)) return HTR_ERR_WORKSPACE;
+  unsigned char* base = (unsigned char*)scratch;
+  hipStream_t st = (hipStream_t)stream;
+  const void** table = (const void**)(base + p.table);
+  for (int e0 = 0; e0 < experts; e0 += MOE_PTR_CHUNK) {
+    MoePtrs ptrs;
+    const int count = experts - e0 < MOE_PTR_CHUNK ? experts - e0 : MOE_PTR_CHUNK;
+    memcpy(&ptrs, tensors + (size_t)e0 * 8, (size_t)count * 64);
+    memset((unsigned char*)&ptrs + (size_t)count * 64, 0, sizeof(ptrs) - (size_t)count * 64);
+    HTR_CHECK_HIP(launch_kernel(k_moe_experts, dim3(1), dim3(256), 0, st, ptrs, table, e0, count));
+  }
+  MoeRoute r;
+  r.ids = ids; r.ids64 = ids_int64; r.pairs = p.pairs; r.top = top; r.experts = experts; r.entries = p.entries; r.rows_per_entry = p.rows;
+  r.table = table; r.m1 = 2 * inter; r.n1 = hidden; r.m2 = hidden; r.n2 = inter;
+  r.e1 = (htr_group_entry*)(base + p.e1); r.e2 = (htr_group_entry*)(base + p.e2);
+  r.h = (float*)(base + p.h); r.out = (float*)(base + p.out);
+  r.pos_of = (int*)(base + p.pos); r.info = (int4*)(base + p.info);
+  r.host_word = host_word; r.ticket = ticket;
+  HTR_CHECK_HIP(launch_kernel(k_moe_route, dim3(1), dim3(MOE_ROUTE_THREADS), 0, st, r));
+  LinearTail t1 = {}, t2 = {};
+  t1.xt_g = (const _Float16*)(base + p.xt1); t1.xs_g = (const float*)(base + p.xs1); t1.sc_g = (const float*)(base + p.sc1);
+  t2.xt_g = (const _Float16*)(base + p.xt2); t2.xs_g = (const float*)(base + p.xs2); t2.sc_g = (const float*)(base + p.sc2);
+  t1.cbscale = t2.cbscale = htr_cbscale();
+  t1.group = r.e1; t2.group = r.e2;
+  HTR_CHECK_HIP(launch_kernel(k_moe_rotate, dim3(p.pairs), dim3(256), 0, st, x, x_dtype, (const int4*)r.info, (const void* const*)table, hidden,
+                              (_Float16*)t1.xt_g, (float*)t1.xs_g, (float*)t1.sc_g));
+  const int flags = HTR_F32 << 2 | FLAG_ENTRY_TILES;
+  BatchArgs b1 = {nullptr, nullptr, nullptr, nullptr, 2 * inter, hidden, 0, flags}, b2 = {nullptr, nullptr, nullptr, nullptr, hidden, inter, 0, flags};
+  int rc = HTR_OK;
+  if (p.rows == 32) { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 1>(b1, t1, 1, p.entries, st))); }
+  else { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 2>(b1, t1, 1, p.entries, st))); }
+  if (rc != HTR_OK) return rc;
+  HTR_CHECK_HIP(launch_kernel(k_moe_act, dim3(p.pairs), dim3(256), 0, st, (const float*)r.h, x_dtype, (const int4*)r.info,
+                              (const void* const*)table, inter, (_Float16*)t2.xt_g, (float*)t2.xs_g, (float*)t2.sc_g));
+  if (p.rows == 32) { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 1>(b2, t2, 1, p.entries, st))); }
+  else { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 2>(b2, t2, 1, p.entries, st))); }
+  if (rc != HTR_OK) return rc;
+  HTR_CHECK_HIP(launch_kernel(k_moe_combine, dim3((hidden / 4 + 255) / 256, tokens), dim3(256), 0, st, (const float*)r.out, (const int*)r.pos_of,
+                              weights, top, hidden, y));
   return HTR_OK;
 }
 

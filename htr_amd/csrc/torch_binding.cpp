@@ -1,0 +1,199 @@
+// htr_amd._fast: the host side of a packed linear and of a routed-expert layer on torch tensors, in C++.
+//
+// A decode launch takes the GPU 6 microseconds and took the interpreter 16 (a dozen attribute reads, shape checks, two
+// dictionary look-ups, a 19-argument foreign call), so small calls ran at the interpreter's pace; collecting the 512
+// tensors of a 64-expert layer took it half a millisecond.  Here the same checks read the tensors' fields directly.  Every
+// function returns None where something is not as expected: the caller's Python path then handles the call, or says
+// what is wrong with it.  Only torch's C++ interface is used; the kernels stay behind the C ABI of libhtr_gfx950.so, whose
+// entry points bind() takes as addresses.
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <chrono>
+#include <cstdint>
+#include <vector>
+
+namespace {
+
+typedef int (*linear_fn)(const void*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int, int, int,
+                         int, void*, size_t, void*);
+typedef size_t (*moe_bytes_fn)(int, int, int, int, int);
+typedef int (*moe_fn)(const void*, int, const void*, int, const float*, int, int, const void* const*, int, int, int, int, int, float*, void*,
+                      size_t, unsigned int*, unsigned int, void*);
+typedef unsigned long long (*capture_fn)(void*);
+linear_fn f_linear = nullptr;
+capture_fn f_capture = nullptr;
+moe_bytes_fn f_moe_bytes = nullptr;
+moe_fn f_moe = nullptr;
+
+constexpr int OK = 0;
+constexpr int MAX_ROWS = 128;      // rows of one decode launch
+
+int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kBFloat16: return 0;
+    case at::kHalf: return 1;
+    case at::kFloat: return 2;
+    default: return -1;
+  }
+}
+
+struct Owned {      // one reference, given back at the end of the scope
+  PyObject* p;
+  ~Owned() { Py_XDECREF(p); }
+};
+
+const at::Tensor* tensor_of(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+struct Shape { int64_t m = 0, n = 0, K = 0; };
+
+// One HTR-W1 tensor set (qweight int32 [m/16, n/16, 8K], scales float16 [m], su uint8 [n/8], sv uint8 [m/8], all contiguous on
+// device `dev`): its shape, or false.
+bool weight_ok(const at::Tensor& qw, const at::Tensor& sc, const at::Tensor& su, const at::Tensor& sv, c10::Device dev, Shape& s) {
+  if (qw.dim() != 3 || qw.scalar_type() != at::kInt || sc.scalar_type() != at::kHalf || su.scalar_type() != at::kByte || sv.scalar_type() != at::kByte)
+    return false;
+  const int64_t W = qw.size(2);
+  s.m = qw.size(0) * 16; s.n = qw.size(1) * 16; s.K = W / 8;
+  if (W % 8 || s.K < 2 || s.K > 8 || s.m % 128 || s.n % 128 || s.m == 0 || s.n == 0) return false;
+  if (sc.numel() != s.m || su.numel() * 8 != s.n || sv.numel() * 8 != s.m) return false;
+  for (const at::Tensor* t : {&qw, &sc, &su, &sv})
+    if (t->device() != dev || !t->is_contiguous()) return false;
+  return true;
+}
+
+// linear(x, qweight, scales, su, sv, bias, workspace address, its bytes, address of its failure word (0: none), stream)
+// -> tensor or None; None also while the stream is being captured (a capture has workspaces of its own) and after a launch
+// on the workspace gave up
+PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 10 || f_linear == nullptr || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
+  const at::Tensor* t[6];
+  for (int i = 0; i < 6; ++i) t[i] = args[i] == Py_None ? nullptr : tensor_of(args[i]);
+  for (int i = 0; i < 5; ++i) if (t[i] == nullptr) Py_RETURN_NONE;
+  if (args[5] != Py_None && t[5] == nullptr) Py_RETURN_NONE;
+  const at::Tensor& x = *t[0];
+  Shape s;
+  const int code = dtype_code(x.scalar_type());
+  if (code < 0 || !x.is_cuda() || x.dim() < 1 || !x.is_contiguous() || !weight_ok(*t[1], *t[2], *t[3], *t[4], x.device(), s)) Py_RETURN_NONE;
+  if (x.size(-1) != s.n) Py_RETURN_NONE;
+  const int64_t M = x.numel() / s.n;
+  if (M < 1 || M > MAX_ROWS) Py_RETURN_NONE;
+  if (t[5] != nullptr && (t[5]->scalar_type() != x.scalar_type() || t[5]->numel() != s.m || t[5]->device() != x.device() || !t[5]->is_contiguous()))
+    Py_RETURN_NONE;
+  void* ws = PyLong_AsVoidPtr(args[6]);
+  const size_t bytes = PyLong_AsSize_t(args[7]);
+  const volatile int* failed = (const volatile int*)PyLong_AsVoidPtr(args[8]);
+  void* stream = PyLong_AsVoidPtr(args[9]);
+  if (PyErr_Occurred()) return nullptr;
+  if ((failed != nullptr && *failed != 0) || f_capture(stream) != 0) Py_RETURN_NONE;
+  c10::DeviceGuard guard(x.device());
+  at::DimVector shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = s.m;
+  at::Tensor y = at::empty(shape, x.options());
+  const int rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
+                          t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, 0,
+                          ws, bytes, stream);
+  if (rc != OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// The tensor addresses of one list of HTR-W1 tuples into every eighth slot group of `ptrs`; false where one is not like the first
+bool collect(PyObject* seq, int offset, c10::Device dev, Shape& shape, std::vector<const void*>& ptrs) {
+  const Py_ssize_t E = PySequence_Fast_GET_SIZE(seq);
+  PyObject** items = PySequence_Fast_ITEMS(seq);
+  for (Py_ssize_t e = 0; e < E; ++e) {
+    PyObject* tup = items[e];
+    if (!(PyTuple_Check(tup) || PyList_Check(tup)) || PySequence_Fast_GET_SIZE(tup) != 4) return false;
+    const at::Tensor* t[4];
+    for (int k = 0; k < 4; ++k) { t[k] = tensor_of(PySequence_Fast_GET_ITEM(tup, k)); if (t[k] == nullptr) return false; }
+    Shape s;
+    if (!weight_ok(*t[0], *t[1], *t[2], *t[3], dev, s)) return false;
+    if (e == 0) shape = s;
+    else if (s.m != shape.m || s.n != shape.n || s.K != shape.K) return false;
+    for (int k = 0; k < 4; ++k) ptrs[8 * e + offset + k] = t[k]->const_data_ptr();
+  }
+  return true;
+}
+
+// moe(x, ids, weights, gate_up, down, host word address (0: none), ticket, stream) -> float32 [tokens, hidden] or None
+PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 8 || f_moe == nullptr) Py_RETURN_NONE;
+  const at::Tensor *xt = tensor_of(args[0]), *it = tensor_of(args[1]), *wt = tensor_of(args[2]);
+  if (xt == nullptr || it == nullptr || wt == nullptr || !xt->is_cuda() || xt->dim() != 2 || it->dim() != 2 || wt->dim() != 2) Py_RETURN_NONE;
+  const int64_t T = xt->size(0), H = xt->size(1), top = it->size(1);
+  const int code = dtype_code(xt->scalar_type());
+  if (code < 0 || it->size(0) != T || wt->size(0) != T || wt->size(1) != top || it->device() != xt->device() || wt->device() != xt->device()) Py_RETURN_NONE;
+  if ((it->scalar_type() != at::kLong && it->scalar_type() != at::kInt) || !wt->is_floating_point()) Py_RETURN_NONE;
+  Owned gu{PySequence_Fast(args[3], "gate_up is not a sequence")}, dn{PySequence_Fast(args[4], "down is not a sequence")};
+  if (gu.p == nullptr || dn.p == nullptr) { PyErr_Clear(); Py_RETURN_NONE; }
+  const Py_ssize_t E = PySequence_Fast_GET_SIZE(gu.p);
+  if (E < 1 || PySequence_Fast_GET_SIZE(dn.p) != E) Py_RETURN_NONE;
+  std::vector<const void*> ptrs((size_t)E * 8);
+  Shape s1, s2;
+  if (!collect(gu.p, 0, xt->device(), s1, ptrs) || !collect(dn.p, 4, xt->device(), s2, ptrs)) Py_RETURN_NONE;
+  const int64_t F = s1.m / 2;
+  if (s1.n != H || s2.m != H || s2.n != F || T < 1 || top < 1 || T > (1 << 24) || E > (1 << 20)) Py_RETURN_NONE;
+  unsigned int* word = (unsigned int*)PyLong_AsVoidPtr(args[5]);
+  const unsigned int ticket = (unsigned int)PyLong_AsUnsignedLong(args[6]);
+  void* stream = PyLong_AsVoidPtr(args[7]);
+  if (PyErr_Occurred()) return nullptr;
+  c10::DeviceGuard guard(xt->device());
+  at::Tensor x = xt->contiguous(), ids = it->contiguous(), w = wt->to(at::kFloat).contiguous();
+  if ((uintptr_t)x.const_data_ptr() & 15) x = x.clone();
+  const size_t need = f_moe_bytes((int)T, (int)top, (int)E, (int)H, (int)F);
+  if (need == 0) Py_RETURN_NONE;
+  at::Tensor scratch = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
+  at::Tensor y = at::empty({T, H}, x.options().dtype(at::kFloat));
+  const int rc = f_moe(x.const_data_ptr(), code, ids.const_data_ptr(), ids.scalar_type() == at::kLong ? 1 : 0, (const float*)w.const_data_ptr(), (int)T,
+                       (int)top, ptrs.data(), (int)E, (int)H, (int)F, (int)s1.K, (int)s2.K, (float*)y.mutable_data_ptr(), scratch.mutable_data_ptr(),
+                       need, word, ticket, stream);
+  if (rc != OK) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
+}
+
+// wait_word(address, ticket, seconds) -> the word's low bit once its upper bits are the ticket, or None after that time
+PyObject* wait_word(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 3) Py_RETURN_NONE;
+  const volatile unsigned int* word = (const volatile unsigned int*)PyLong_AsVoidPtr(args[0]);
+  const unsigned int ticket = (unsigned int)PyLong_AsUnsignedLong(args[1]) & 0x7FFFFFFFu;
+  const double seconds = PyFloat_AsDouble(args[2]);
+  if (PyErr_Occurred()) return nullptr;
+  unsigned int v = 0;
+  bool done = false;
+  Py_BEGIN_ALLOW_THREADS
+  const auto until = std::chrono::steady_clock::now() + std::chrono::duration<double>(seconds);
+  for (;;) {
+    for (int i = 0; i < 256 && !done; ++i) { v = *word; done = (v >> 1) == ticket; __builtin_ia32_pause(); }
+    if (done || std::chrono::steady_clock::now() > until) break;
+  }
+  Py_END_ALLOW_THREADS
+  if (!done) Py_RETURN_NONE;
+  return PyLong_FromLong((long)(v & 1u));
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(htr_linear, htr_stream_capture_id, htr_moe_scratch_bytes, htr_moe_experts): addresses of the library's entry points
+PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 4) { PyErr_SetString(PyExc_TypeError, "bind wants four addresses"); return nullptr; }
+  void* p[4];
+  for (int i = 0; i < 4; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+  if (PyErr_Occurred()) return nullptr;
+  f_linear = (linear_fn)p[0]; f_capture = (capture_fn)p[1]; f_moe_bytes = (moe_bytes_fn)p[2]; f_moe = (moe_fn)p[3];
+  Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {{"bind", (PyCFunction)(void*)bind, METH_FASTCALL, nullptr},
+                         {"linear", (PyCFunction)(void*)linear, METH_FASTCALL, nullptr},
+                         {"moe", (PyCFunction)(void*)moe, METH_FASTCALL, nullptr},
+                         {"wait_word", (PyCFunction)(void*)wait_word, METH_FASTCALL, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__fast(void) { return PyModule_Create(&module); }

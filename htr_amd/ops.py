@@ -5,6 +5,7 @@ M-based dispatch of _linear_impl, htr/ops.py:69-122), but the body calls the gfx
 through its C ABI: tensors are passed as raw device pointers together with the current
 torch stream; outputs and the workspace are allocated here with torch.
 """
+import itertools
 import os
 
 import torch
@@ -69,10 +70,11 @@ PREFILL = os.environ.get("HTR_PREFILL", "w")
 
 class _Workspace:
     """One device buffer for split partials and pre-rotated activations, with its failure flag in pinned host memory."""
-    __slots__ = ("buf", "flag", "stream")
+    __slots__ = ("buf", "flag", "stream", "ptr", "size", "flag_ptr")
 
     def __init__(self, buf, flag, stream):
         self.buf, self.flag, self.stream = buf, flag, stream
+        self.ptr, self.size, self.flag_ptr = buf.data_ptr(), buf.numel(), 0 if flag is None else flag[1]
 
 
 _WORKSPACES = {}      # (device index, stream), (device index, "capture", capture id) or (device index, "shared") -> _Workspace
@@ -326,10 +328,15 @@ def moe_experts(x, expert_ids, expert_weights, gate_up, down, activation=torch.n
     """Routed-expert MLP on packed weights: y_t = sum_j w_tj * Down_e( act(Gate_e x_t) * Up_e x_t ), e = ids[t, j].
 
     x [T, H]; expert_ids [T, top] integer; expert_weights [T, top]; gate_up[e] = HTR-W1 tuple of the fused [2F, H] matrix
-    (gate rows first), down[e] = HTR-W1 tuple of [H, F].  Two grouped launches cover all active experts; the result is
-    float32 [T, H].  The reference defines no such runtime (its experts are a composition of packed linears), so this
-    is that composition, batched.
+    (gate rows first), down[e] = HTR-W1 tuple of [H, F].  The result is float32 [T, H].  The reference defines no such
+    runtime (its experts are a composition of packed linears), so this is that composition, batched: with the default
+    activation the whole layer is queued by one library call (sorting by expert, rotations, both grouped products, activation
+    and weighted sum on the device); another activation runs between two grouped launches.
     """
+    if activation is torch.nn.functional.silu and type(x) is torch.Tensor and x.is_cuda:
+        y = _moe_silu(x, expert_ids, expert_weights, gate_up, down)
+        if y is not None:
+            return y
     T, H = x.shape
     flat_e = expert_ids.reshape(-1)
     order = torch.argsort(flat_e, stable=True)
@@ -349,6 +356,36 @@ def moe_experts(x, expert_ids, expert_weights, gate_up, down, activation=torch.n
     wflat = expert_weights.reshape(-1)[order].to(torch.float32)
     y = torch.zeros((T, H), dtype=torch.float32, device=x.device)
     y.index_add_(0, tok, torch.cat(out, 0) * wflat[:, None])
+    return y
+
+
+_TICKETS = itertools.count(1)
+_TICKET_WORDS = 256
+_TICKET_POOLS = {}       # device index -> pinned words in which the routing kernels report expert numbers out of range
+
+
+def _moe_silu(x, expert_ids, expert_weights, gate_up, down):
+    """moe_experts with the default activation in one library call; None where the arguments are not as the library wants them."""
+    index = x.get_device()
+    stream = _raw_stream(index)
+    fast = _native.fast()
+    if torch.cuda.is_current_stream_capturing():
+        return fast.moe(x, expert_ids, expert_weights, gate_up, down, 0, 0, stream)
+    pool = _TICKET_POOLS.get(index)
+    if pool is None:
+        pool = _TICKET_POOLS.setdefault(index, torch.zeros(_TICKET_WORDS, dtype=torch.int32, pin_memory=True))
+    ticket = next(_TICKETS) & 0x7FFFFFFF
+    word = pool.data_ptr() + 4 * (ticket % _TICKET_WORDS)
+    y = fast.moe(x, expert_ids, expert_weights, gate_up, down, word, ticket, stream)
+    if y is None:
+        return None
+    # the layer is queued; its first kernel says whether every expert number was valid, while the others still run
+    bad = fast.wait_word(word, ticket, 2.0)
+    if bad is None:
+        torch.cuda.current_stream(x.device).synchronize()          # a long queue, or a failed launch, which raises here
+        bad = int(pool[ticket % _TICKET_WORDS].item()) & 1
+    if bad:
+        raise IndexError(f"moe_experts: an expert number is outside 0 .. {len(gate_up) - 1}")
     return y
 
 

@@ -201,6 +201,26 @@ int htr_linear_grouped(const htr_group_entry* entries_device, int count, int m, 
                        int x_dtype, int y_dtype, void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * One routed-expert layer on packed weights, without a copy or a synchronisation:
+ *   y_t = sum_j w[t, j] Down_e( round(silu(Gate_e x_t) * Up_e x_t) ),  e = ids[t, j],
+ * the rounding to x_dtype, sums and products in float32, slots added in ascending order.
+ *   x        [tokens, hidden] row-major in x_dtype, 16-byte aligned
+ *   ids      [tokens, top] int32 or int64 expert numbers; weights [tokens, top] float32; both on the device
+ *   tensors  HOST array of 8 device addresses per expert: qweight, scales, su, sv of the fused [2 inter, hidden] gate/up
+ *            matrix (gate rows first), then of the [hidden, inter] down matrix; read before the call returns
+ *   y        [tokens, hidden] float32, 16-byte aligned
+ *   scratch  htr_moe_scratch_bytes() bytes, 256-byte aligned, no zero requirement, used until the launches are done
+ *   host_word  NULL or a 4-byte word in pinned, device-visible host memory: the first of the launches that looks at the ids
+ *            stores (ticket << 1) | (some id is outside 0 .. experts - 1) there; tokens with such an id get NaN
+ * hidden and inter are multiples of 128; at most 4096 experts and 2^24 pairs.
+ * No counterpart in the reference, which composes routed experts from per-expert linears (docs/ADAPTERS.md:19).
+ */
+size_t htr_moe_scratch_bytes(int tokens, int top, int experts, int hidden, int inter);
+int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, const float* weights, int tokens, int top,
+                    const void* const* tensors, int experts, int hidden, int inter, int K_gate_up, int K_down, float* y,
+                    void* scratch, size_t scratch_bytes, unsigned int* host_word, unsigned int ticket, void* stream);
+
+/*
  * Polls (about a microsecond each) a finishing workgroup waits for the partials of earlier workgroups before it gives
  * up, stores NaN for its rows and sets bit 0 of the first workspace word.  Default 2^20.  No counterpart in the
  * reference; exists so that the bounded wait can be exercised.

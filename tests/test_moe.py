@@ -1,0 +1,101 @@
+"""ops.moe_experts with the default activation: the whole layer in one library call, against the per-expert composition on the
+CPU oracle with the same rounding between the two linears."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from htr_amd import _native
+    _native.lib()
+    return torch.device("cuda:0")
+
+
+def _layer(E, H, F, K1, K2, seed):
+    from htr_amd import wire
+    return [wire.synth_linear(2 * F, H, K1, seed + e) for e in range(E)], [wire.synth_linear(H, F, K2, seed + 500 + e) for e in range(E)]
+
+
+def _composition(oracle, x, ids, w, gate_up, down, F):
+    y = np.zeros((x.shape[0], x.shape[1]))
+    for e in range(len(gate_up)):
+        tok, slot = torch.nonzero(ids == e, as_tuple=True)
+        if tok.numel() == 0:
+            continue
+        h = torch.from_numpy(oracle.c_linear(x[tok].float().numpy(), *[t.numpy() for t in gate_up[e]])).float()
+        h = (torch.nn.functional.silu(h[:, :F]) * h[:, F:]).to(x.dtype).float().numpy()
+        np.add.at(y, tok.numpy(), oracle.c_linear(h, *[t.numpy() for t in down[e]]) * w[tok, slot].double().numpy()[:, None])
+    return y
+
+
+def _to(dev, ws):
+    return [tuple(t.to(dev) for t in w) for w in ws]
+
+
+# tokens per expert on both sides of a 32-row tile and of a 64-row entry, experts without tokens, one token, one expert
+@pytest.mark.parametrize("dtype,counts,top,K1,K2,H,F", [(torch.bfloat16, (1, 0, 32, 33), 1, 4, 4, 256, 128), (torch.float16, (64, 65, 0, 3), 1, 3, 5, 128, 384),
+                                                        (torch.bfloat16, (130,), 1, 4, 4, 256, 256), (torch.float32, (7, 40, 2), 1, 2, 4, 384, 128),
+                                                        (torch.bfloat16, (1,), 1, 4, 4, 128, 128), (torch.float16, None, 3, 4, 4, 2176, 256)])
+@pytest.mark.parametrize("id_type", [torch.int64, torch.int32])
+def test_whole_layer_matches_the_composition(dev, oracle, dtype, counts, top, K1, K2, H, F, id_type):
+    """Bound: two chained linears of 1e-3 each with a rounding to `dtype` between them (bf16: 2^-9 per element of the hidden
+    vector, averaged over F products), 4e-3 as for the 64-expert configuration; float16 and float32 stay within 2e-3."""
+    from htr_amd import ops
+    print(f"moe {dtype} {counts} top {top} K {K1}/{K2} H {H} F {F} {id_type}", flush=True)
+    g = torch.Generator().manual_seed(31)
+    if counts is None:
+        E, T = 5, 37
+        ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)])
+    else:
+        E, T = len(counts), sum(counts)
+        ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)][:, None]
+    gate_up, down = _layer(E, H, F, K1, K2, 600)
+    x = torch.randn(T, H, generator=g).to(dtype)
+    w = torch.rand(T, top, generator=g)
+    y = ops.moe_experts(x.to(dev), ids.to(id_type).to(dev), w.to(dev), _to(dev, gate_up), _to(dev, down)).cpu().numpy()
+    ref = _composition(oracle, x, ids, w, gate_up, down, F)
+    rel = float(np.abs(y - ref).max() / np.abs(ref).max())
+    assert y.dtype == np.float32 and rel <= (4e-3 if dtype == torch.bfloat16 else 2e-3), rel
+
+
+def test_expert_numbers_out_of_range_and_graph_capture(dev):
+    from htr_amd import ops
+    print("moe: bad ids, capture", flush=True)
+    gate_up, down = (_to(dev, ws) for ws in _layer(3, 128, 128, 4, 4, 700))
+    x = torch.randn(6, 128, device=dev).bfloat16()
+    ids = torch.tensor([[0], [2], [1], [1], [0], [2]], device=dev)
+    w = torch.ones(6, 1, device=dev)
+    good = ops.moe_experts(x, ids, w, gate_up, down)
+    for bad in (3, -1):
+        with pytest.raises(IndexError):
+            ops.moe_experts(x, torch.where(ids == 2, bad, ids), w, gate_up, down)
+    assert torch.equal(ops.moe_experts(x, ids, w, gate_up, down), good)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.moe_experts(x, ids, w, gate_up, down)
+    for _ in range(3):
+        x.copy_(torch.randn(6, 128, device=dev))
+        ids.copy_(ids.roll(1, 0))
+        want = ops.moe_experts(x, ids, w, gate_up, down)
+        graph.replay()
+        assert torch.equal(y, want)
+
+
+def test_another_activation_takes_the_two_grouped_launches(dev, oracle):
+    from htr_amd import ops
+    print("moe: relu", flush=True)
+    gate_up, down = _layer(3, 256, 128, 4, 4, 800)
+    g = torch.Generator().manual_seed(9)
+    x, ids, w = torch.randn(20, 256, generator=g).bfloat16(), torch.randint(0, 3, (20, 1), generator=g), torch.rand(20, 1, generator=g)
+    args = (x.to(dev), ids.to(dev), w.to(dev), _to(dev, gate_up), _to(dev, down))
+    relu = ops.moe_experts(*args, activation=torch.relu)
+    silu_by_hand = ops.moe_experts(*args, activation=lambda t: torch.nn.functional.silu(t))
+    whole = ops.moe_experts(*args)
+    assert not torch.allclose(relu, whole)
+    # the same products, rounded alike; only the order of the float32 sums over the slots could differ
+    assert float((silu_by_hand - whole).norm() / whole.norm()) <= 1e-3
