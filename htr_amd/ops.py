@@ -400,18 +400,39 @@ def _(x2, qweight, scales, su, sv, bias):
     return x2.new_empty((x2.shape[0], qweight.shape[0] * 16))
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _linear_decode(x, qweight, scales, su, sv, bias):
+    """The common case of linear() in C++: up to 128 contiguous rows on a stream that has a workspace already.  None where
+    something else is asked for, or is wrong: the general path then runs, or raises."""
+    if NSPLIT != 0 or GEMV_LOOP_MAX is not None or LAUNCH_MAX_M < _native.MAX_ROWS_PER_TILE or SHARE_CAPTURE_WORKSPACE:
+        return None
+    index = x.get_device()
+    if index < 0:
+        return None
+    stream = _raw_stream(index)
+    ws = _WORKSPACES.get((index, stream))
+    if ws is None:
+        return None
+    return _native.fast().linear(x, qweight, scales, su, sv, bias, ws.ptr, ws.size, ws.flag_ptr, stream)
+
+
 def linear(x, qweight, scales, su, sv, bias=None):
     """y = x @ W^T (+bias) for an HTR-W1 weight. x [..., n] -> [..., m] in x.dtype.
 
     Under tracing (torch.compile) the call goes through the registered op `htr::linear`, as in the reference
     (htr/ops.py:107-122), and so do tensor subclasses (fake and functional tensors of other tracers); eager calls on
     plain tensors skip the dispatcher, which costs more host time than the launch itself."""
+    if torch.compiler.is_compiling() or type(x) is not torch.Tensor or type(qweight) not in _PLAIN:
+        shp = x.shape
+        y = htr_linear_op(x.reshape(-1, shp[-1]), qweight, scales, su, sv, bias)      # tracing, fake or functional tensors: the registered op
+        return y.reshape(*shp[:-1], qweight.shape[0] * 16)
+    y = _linear_decode(x, qweight, scales, su, sv, bias)
+    if y is not None:
+        return y
     shp = x.shape
-    x2 = x.reshape(-1, shp[-1])
-    if torch.compiler.is_compiling() or type(x2) is not torch.Tensor or type(qweight) not in (torch.Tensor, torch.nn.Parameter):
-        y = htr_linear_op(x2, qweight, scales, su, sv, bias)      # tracing, fake or functional tensors: the registered op
-    else:
-        y = _linear_impl(x2.contiguous(), qweight, scales, su, sv, bias)
+    y = _linear_impl(x.reshape(-1, shp[-1]).contiguous(), qweight, scales, su, sv, bias)
     return y.reshape(*shp[:-1], qweight.shape[0] * 16)
 
 
