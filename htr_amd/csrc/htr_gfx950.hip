@@ -610,7 +610,7 @@ int htr_dequant_w(const void* qweight, const void* scales, const void* su, const
   if (((uintptr_t)qweight & 15) || ((uintptr_t)out_bf16 & 3) || ((uintptr_t)scales & 1) || ((uintptr_t)sv & 3)) return HTR_ERR_ALIGN;
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid(n / 128, m / 128);
-  const size_t lds = (size_t)128 * DQW_LD * sizeof(float);
+  const size_t lds = DQW_LDS;
   const float cb = htr_cbscale();
 #define HTR_LAUNCH_DQW(KK_)                                                                                              \
   {                                                                                                                      \
