@@ -74,7 +74,7 @@ __global__ __launch_bounds__(WG_THREADS, JB <= 1 ? 4 : 2) void k_linear_tile(con
   };
   const SplitRole role = split_role(M, S, s_idx, flags);
   RowBits raw = {0u, 0u, 0u, 0u, 0u, 0u};
-  if (role.finisher) raw = load_row_bits(t, y_dtype, rb * 128 + lane);
+  if (role.finisher) load_row_bits(t, y_dtype, rb * 128 + lane, raw);
   constexpr int STEP_BYTES = 256 * K;
   const uint32_t strip_bytes = (uint32_t)nblk * STEP_BYTES;
   const uint32_t* base = qw + ((size_t)(rb * 8) * nblk + (size_t)c_begin) * (STEP_BYTES / 4);
