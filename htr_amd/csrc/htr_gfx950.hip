@@ -361,7 +361,7 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
     HTR_CHECK_HIP(launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, max_M, count), dim3(WG_THREADS), 0, st, (const void*)nullptr,
                                 (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries, 0ull, 1));
     BatchArgs ba = {nullptr, nullptr, nullptr, nullptr, m, n, 0, x_dtype | (y_dtype << 2)};
-    HTR_FOR_K(K, return (launch_tile_v<KK, 1>(ba, t, 1, count, st)));
+    HTR_FOR_K(K, return (launch_tile_v<KK, 1, true>(ba, t, 1, count, st)));
   }
   Plan pl;
   if (!make_group_plan(count, m, n, max_M, pl)) return HTR_ERR_SPLIT;
@@ -473,13 +473,13 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   const int flags = HTR_F32 << 2 | FLAG_ENTRY_TILES;
   BatchArgs b1 = {nullptr, nullptr, nullptr, nullptr, 2 * inter, hidden, 0, flags}, b2 = {nullptr, nullptr, nullptr, nullptr, hidden, inter, 0, flags};
   int rc = HTR_OK;
-  if (p.rows == 32) { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 1>(b1, t1, 1, p.entries, st))); }
-  else { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 2>(b1, t1, 1, p.entries, st))); }
+  if (p.rows == 32) { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 1, true>(b1, t1, 1, p.entries, st))); }
+  else { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 2, true>(b1, t1, 1, p.entries, st))); }
   if (rc != HTR_OK) return rc;
   HTR_CHECK_HIP(launch_kernel(k_moe_act, dim3(p.pairs), dim3(256), 0, st, (const float*)r.h, x_dtype, (const int4*)r.info,
                               (const void* const*)table, inter, (_Float16*)t2.xt_g, (float*)t2.xs_g, (float*)t2.sc_g));
-  if (p.rows == 32) { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 1>(b2, t2, 1, p.entries, st))); }
-  else { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 2>(b2, t2, 1, p.entries, st))); }
+  if (p.rows == 32) { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 1, true>(b2, t2, 1, p.entries, st))); }
+  else { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 2, true>(b2, t2, 1, p.entries, st))); }
   if (rc != HTR_OK) return rc;
   HTR_CHECK_HIP(launch_kernel(k_moe_combine, dim3((hidden / 4 + 255) / 256, tokens), dim3(256), 0, st, (const float*)r.out, (const int*)r.pos_of,
                               weights, top, hidden, y));

@@ -365,17 +365,27 @@ template <int K, int MB, bool ROT> int launch_batch_v(const BatchArgs& a, const 
                               a.m, a.n, a.M, bp.S, a.flags, t));
   return HTR_OK;
 }
-template <int K, int JB> int launch_tile_v(const BatchArgs& a, const LinearTail& t, int S, int problems, hipStream_t st) {
-  constexpr int P = K <= 4 ? 4 : 2;
+// ONE: one split, an instantiation without the exchange between splits: few enough registers (128) for two workgroups per
+// compute unit also with two row tiles, where one workgroup's decode covers the other's first loads and output side.  The
+// second workgroup replaces the deeper rings: two stream buffers and one set of fragments instead of four and two.
+template <int K, int JB, bool ONE> int launch_tile_v(const BatchArgs& a, const LinearTail& t, int S, int problems, hipStream_t st) {
+  constexpr int P = K > 4 || (ONE && JB > 1) ? 2 : 4, DB = ONE && JB > 1 ? 1 : 2;
   const size_t lds = problems == 1 ? balanced_lds_request(tile_lds_bytes(JB), S * (a.m / 128)) : tile_lds_bytes(JB);
-  HTR_CHECK_HIP((allow_full_lds<k_linear_tile<K, JB, P, 2>>()));
-  HTR_CHECK_HIP(launch_kernel(k_linear_tile<K, JB, P, 2>, dim3(S, a.m / 128, problems), dim3(WG_THREADS), lds, st, a.qw, a.part, a.m, a.n, a.M, S,
-                              a.flags, t));
+  HTR_CHECK_HIP((allow_full_lds<k_linear_tile<K, JB, P, DB, ONE>>()));
+  HTR_CHECK_HIP(launch_kernel(k_linear_tile<K, JB, P, DB, ONE>, dim3(S, a.m / 128, problems), dim3(WG_THREADS), lds, st, a.qw, a.part, a.m, a.n,
+                              a.M, S, a.flags, t));
   return HTR_OK;
 }
 template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
   if (rot) return bp.mb == 1 ? launch_batch_v<K, 1, true>(a, t, bp, st) : launch_batch_v<K, 2, true>(a, t, bp, st);
-  if (tile_rows(a.M)) return a.M <= 32 ? launch_tile_v<K, 1>(a, t, bp.S, 1, st) : launch_tile_v<K, 2>(a, t, bp.S, 1, st);
+  if (tile_rows(a.M)) {
+    // Grids beyond one workgroup per compute unit, us without / with ONE: K4, 64 rows 65536x4096 67.0 / 59.4, 40960x1024 28.7 /
+    // 22.4, 33 rows 152064x4096 137.6 / 115.9; 32 rows 65536x4096 49.0 / 49.5.  Up to one per unit there is no second workgroup
+    // to gain from: eight decoder layers of 32 rows at K3, whose gate/up takes 224 workgroups, 558 to 562 / 565 to 571.
+    const bool one = bp.S == 1 && bp.wgs > num_cu();
+    if (a.M <= 32) return one ? launch_tile_v<K, 1, true>(a, t, 1, 1, st) : launch_tile_v<K, 1, false>(a, t, bp.S, 1, st);
+    return one ? launch_tile_v<K, 2, true>(a, t, 1, 1, st) : launch_tile_v<K, 2, false>(a, t, bp.S, 1, st);
+  }
   return bp.mb == 1 ? launch_batch_v<K, 1, false>(a, t, bp, st) : launch_batch_v<K, 8, false>(a, t, bp, st);
 }
 // nsplit bit 29: batched kernel with the split in the low bits (0 = policy); otherwise the policy decides by M

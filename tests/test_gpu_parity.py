@@ -756,6 +756,18 @@ def test_tiles_of_32_rows(dev, oracle, K, m, n, M, dtype):
     assert _rel(ops.linear_f32out(odd, *w).cpu().numpy(), ref) <= REL_TOL
 
 
+@pytest.mark.parametrize("K,n,M", [(3, 128, 17), (4, 640, 32), (4, 384, 33), (5, 256, 64), (8, 128, 41)])
+def test_tiles_on_more_row_blocks_than_compute_units(dev, oracle, K, n, M):
+    """17 to 64 rows on 258 row blocks: the instantiation without column splits, with one and two row tiles, block counts on
+    both sides of its stream's depth, K with different depths.  1e-3: float16 activations."""
+    from htr_amd import ops
+    m = 258 * 128
+    print(f"tall tiles K={K} n={n} M={M}", flush=True)
+    qw, sc, su, sv, x = _case(m, n, K, M, 1700 + M, torch.bfloat16)
+    ref = _ref(oracle, qw, sc, su, sv, x)
+    assert _rel(ops.linear_f32out(x.to(dev), *[t.to(dev) for t in (qw, sc, su, sv)]).cpu().numpy(), ref) <= REL_TOL
+
+
 def test_grouped_launch_of_9_to_32_rows(dev, oracle):
     from htr_amd import ops, wire
     print("grouped launch, tiles", flush=True)
