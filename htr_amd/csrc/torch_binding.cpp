@@ -10,6 +10,7 @@
 #include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
 #include <chrono>
 #include <cstdint>
 #include <vector>
@@ -45,6 +46,11 @@ struct Owned {      // one reference, given back at the end of the scope
 };
 
 const at::Tensor* tensor_of(PyObject* o) { return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr; }
+
+// Memory of its own (not the wrapper of a function transform such as torch.func.grad)
+bool raw_ok(const at::Tensor& t) { return t.has_storage(); }
+// Whether torch follows derivatives through t now, backward or forward
+bool differentiable(const at::Tensor& t) { return (c10::GradMode::is_enabled() && t.requires_grad()) || t._fw_grad(0).defined(); }
 
 struct Shape { int64_t m = 0, n = 0, K = 0; };
 
@@ -127,6 +133,8 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int code = dtype_code(xt->scalar_type());
   if (code < 0 || it->size(0) != T || wt->size(0) != T || wt->size(1) != top || it->device() != xt->device() || wt->device() != xt->device()) Py_RETURN_NONE;
   if ((it->scalar_type() != at::kLong && it->scalar_type() != at::kInt) || !wt->is_floating_point()) Py_RETURN_NONE;
+  // the result is differentiable in the routing weights only where torch adds it up: not behind a raw pointer
+  if (!raw_ok(*xt) || !raw_ok(*it) || !raw_ok(*wt) || differentiable(*wt)) Py_RETURN_NONE;
   Owned gu{PySequence_Fast(args[3], "gate_up is not a sequence")}, dn{PySequence_Fast(args[4], "down is not a sequence")};
   if (gu.p == nullptr || dn.p == nullptr) { PyErr_Clear(); Py_RETURN_NONE; }
   const Py_ssize_t E = PySequence_Fast_GET_SIZE(gu.p);

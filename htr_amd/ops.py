@@ -331,7 +331,8 @@ def moe_experts(x, expert_ids, expert_weights, gate_up, down, activation=torch.n
     (gate rows first), down[e] = HTR-W1 tuple of [H, F].  The result is float32 [T, H].  The reference defines no such
     runtime (its experts are a composition of packed linears), so this is that composition, batched: with the default
     activation the whole layer is queued by one library call (sorting by expert, rotations, both grouped products, activation
-    and weighted sum on the device); another activation runs between two grouped launches.
+    and weighted sum on the device); another activation runs between two grouped launches, and so does a call whose
+    expert_weights take part in differentiation: the result is differentiable in them (not in x, as for every packed linear).
     """
     if activation is torch.nn.functional.silu and type(x) is torch.Tensor and x.is_cuda:
         y = _moe_silu(x, expert_ids, expert_weights, gate_up, down)

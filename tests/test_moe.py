@@ -99,3 +99,33 @@ def test_another_activation_takes_the_two_grouped_launches(dev, oracle):
     assert not torch.allclose(relu, whole)
     # the same products, rounded alike; only the order of the float32 sums over the slots could differ
     assert float((silu_by_hand - whole).norm() / whole.norm()) <= 1e-3
+
+
+def test_gradient_of_the_routing_weights(dev, oracle):
+    """The default activation keeps y differentiable in the routing weights, backward and forward, as any other one does."""
+    from htr_amd import ops
+    print("moe: gradient of the routing weights", flush=True)
+    gate_up, down = _layer(4, 256, 128, 4, 4, 820)
+    g = torch.Generator().manual_seed(10)
+    x, w = torch.randn(9, 256, generator=g).bfloat16(), torch.rand(9, 2, generator=g)
+    ids = torch.stack([torch.randperm(4, generator=g)[:2] for _ in range(9)])
+    gy = torch.randn(9, 256, generator=g)
+    args = [x.to(dev), ids.to(dev), _to(dev, gate_up), _to(dev, down)]
+    # d sum(gy y) / d w[t, j] is the product of gy[t] with what slot j alone gives
+    want = torch.zeros(9, 2, dtype=torch.float64)
+    for j in range(2):
+        only = torch.zeros(9, 2)
+        only[:, j] = 1.0
+        want[:, j] = (torch.from_numpy(_composition(oracle, x, ids, only, gate_up, down, 128)) * gy.double()).sum(1)
+    wd = w.to(dev).requires_grad_()
+    y = ops.moe_experts(args[0], args[1], wd, *args[2:])
+    assert y.requires_grad
+    (y * gy.to(dev)).sum().backward()
+    assert float((wd.grad.cpu().double() - want).norm() / want.norm()) <= 4e-3      # as for the layer's result in bfloat16
+    with torch.no_grad():
+        assert not ops.moe_experts(args[0], args[1], wd, *args[2:]).requires_grad
+    with torch.autograd.forward_ad.dual_level():
+        y, t = torch.autograd.forward_ad.unpack_dual(
+            ops.moe_experts(args[0], args[1], torch.autograd.forward_ad.make_dual(w.to(dev), torch.ones(9, 2, device=dev)), *args[2:]))
+        alone = ops.moe_experts(args[0], args[1], torch.ones(9, 2, device=dev), *args[2:])
+        assert t is not None and float((t - alone).norm() / alone.norm()) <= 1e-3      # the result is linear in the weights
