@@ -330,7 +330,10 @@ static bool make_group_plan(int count, int m, int n, int max_M, Plan& pl) {
 
 size_t htr_grouped_workspace_bytes(int count, int m, int n, int K, int max_M) {
   if (K < 2 || K > 8 || !shape_ok(m, n) || max_M < 1 || max_M > HTR_MAX_GROUP_ROWS || count < 1 || count > HTR_MAX_GROUP) return 0;
-  if (max_M > 8) return ws_need(0, prerot_bytes(n, (size_t)32 * count));      // k_linear_tile: no partials, one row tile per problem
+  if (group_takes_tiles(count, m, n, K, max_M)) {                 // one row tile per problem, partials only with column splits
+    const int S = group_tile_splits(count, m, n);
+    return ws_need(S > 1 ? (size_t)count * (m / 128) * S * max_M * 128 * sizeof(float) : 0, prerot_bytes(n, (size_t)32 * count));
+  }
   Plan pl;
   if (!make_group_plan(count, m, n, max_M, pl)) return 0;
   return ws_need((size_t)count * pl.wgs * max_M * 128 * sizeof(float), (size_t)count * prerot_bytes(n, max_M));
@@ -350,18 +353,20 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
 
   unsigned char* wsp = (unsigned char*)workspace + ws_half(workspace_bytes);      // scratch half
-  if (max_M > 8) {
-    // 9 to 32 rows per problem: one tile of 32 rows each
+  if (group_takes_tiles(count, m, n, K, max_M)) {
+    // one tile of 32 rows per problem
     LinearTail t = {};
     place_prerot(t, wsp, n, (size_t)32 * count);
     t.status = (uint32_t*)workspace;
     t.cbscale = htr_cbscale();
+    t.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
     t.group = entries;
     hipStream_t st = (hipStream_t)stream;
+    const int S = group_tile_splits(count, m, n);
     HTR_CHECK_HIP(launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, max_M, count), dim3(WG_THREADS), 0, st, (const void*)nullptr,
                                 (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries, 0ull, 1));
-    BatchArgs ba = {nullptr, nullptr, nullptr, nullptr, m, n, 0, x_dtype | (y_dtype << 2)};
-    HTR_FOR_K(K, return (launch_tile_v<KK, 1, true>(ba, t, 1, count, st)));
+    BatchArgs ba = {nullptr, (float*)((unsigned char*)workspace + WS_HEADER), nullptr, nullptr, m, n, max_M, x_dtype | (y_dtype << 2)};
+    HTR_FOR_K(K, return (S > 1 ? launch_tile_v<KK, 1, false>(ba, t, S, count, st) : launch_tile_v<KK, 1, true>(ba, t, 1, count, st)));
   }
   Plan pl;
   if (!make_group_plan(count, m, n, max_M, pl)) return HTR_ERR_SPLIT;

@@ -14,7 +14,7 @@
 // of 32 rows, 0.53 with two, where k_linear_batch with its staging and barrier takes 0.49 and 0.69), then 6.7 to 8.6 us per
 // launch for launch, first loads, reduction and output side.  32x32x16 instead of 16x16x32 instructions because one of
 // them takes about 6 cycles of vector issue from the other waves for 16 K products, and the smaller one 12 for 8 K.
-// ONE (a single column split: grouped launches, tall matrices): two workgroups per compute unit.  A workgroup of 16 steps spends
+// ONE (a single column split: tall matrices, groups that fill the chip, routed experts): two workgroups per compute unit.  A workgroup of 16 steps spends
 // as long on its first loads and its output side as on a third of its steps; 500 tokens over 64 experts, 47 rows each on
 // average, two row tiles: gate/up 130 -> 95 us, down 80 -> 57 us.
 constexpr int FLAG_ENTRY_TILES = 1 << 6;                                    // grouped: an entry's `reserved` is its first row tile
@@ -40,6 +40,7 @@ __global__ __launch_bounds__(WG_THREADS, JB <= 1 || ONE ? 4 : 2) void k_linear_t
     t.xt_g = t_a.xt_g + tile0 * 32 * n;
     t.xs_g = t_a.xs_g + tile0 * 32 * (n >> 7) * 4;
     t.sc_g = t_a.sc_g + tile0 * 32;
+    if (!ONE) part += (size_t)blockIdx.z * gridDim.y * S * M_a * 128;      // M_a: the largest M of the group
   }
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));

@@ -370,11 +370,36 @@ template <int K, int MB, bool ROT> int launch_batch_v(const BatchArgs& a, const 
 // second workgroup replaces the deeper rings: two stream buffers and one set of fragments instead of four and two.
 template <int K, int JB, bool ONE> int launch_tile_v(const BatchArgs& a, const LinearTail& t, int S, int problems, hipStream_t st) {
   constexpr int P = K > 4 || (ONE && JB > 1) ? 2 : 4, DB = ONE && JB > 1 ? 1 : 2;
-  const size_t lds = problems == 1 ? balanced_lds_request(tile_lds_bytes(JB), S * (a.m / 128)) : tile_lds_bytes(JB);
+  const size_t lds = problems == 1 || !ONE ? balanced_lds_request(tile_lds_bytes(JB), S * (a.m / 128) * problems) : tile_lds_bytes(JB);
   HTR_CHECK_HIP((allow_full_lds<k_linear_tile<K, JB, P, DB, ONE>>()));
   HTR_CHECK_HIP(launch_kernel(k_linear_tile<K, JB, P, DB, ONE>, dim3(S, a.m / 128, problems), dim3(WG_THREADS), lds, st, a.qw, a.part, a.m, a.n,
                               a.M, S, a.flags, t));
   return HTR_OK;
+}
+// Grouped launches of 9 to 32 rows per problem: column splits while every workgroup of the grid has a compute unit to itself, as
+// for one linear (make_batch_plan); the splits of a row block wait for each other.  Measured on MI355X, K4, us, chunked kernel /
+// k_linear_tile without splits / with, rotation included: one problem of 4096x14336 with 9 rows 32.3 / 55.8 / 17.9, with 32 rows
+// 72.2 / 60.0 / 20.6; two of 256x4096 with 9 rows 16.2 / 21.1 / 11.6; two of 1024x1024 with 9 rows 10.9 / 11.3 / 10.3.
+inline int group_tile_splits(int count, int m, int n) {
+  const int nblk = n / 128, limit = num_cu() / count / (m / 128);
+  int best = 1;
+  for (int S = 2; S <= nblk && S <= limit && S <= 8; ++S) {
+    const int cb = (nblk + S - 1) / S;
+    if ((nblk + cb - 1) / cb == S) best = S;                       // no split is empty
+  }
+  return best;
+}
+// Whether k_linear_tile takes the group.  The chunked kernel keeps up to 8 rows (not compared) and, at five bits and more, up to
+// 12 rows of problems with long rows whose row blocks leave a quarter of the last round over the compute units empty, which its
+// chunks fill.  us, chunked / k_linear_tile: twelve problems of 4096x4096 with 9 rows K4 41.5 / 40.3, K5 44.0 / 50.3, K8 54.6 / 57.7,
+// with 16 rows K5 65.1 / 51.3; twelve of 4096x14336 with 9 rows K4 124 / 120, K5 137 / 158; six of them K5 77.9 / 84.4, eight
+// 99.2 / 91.1; six of 4096x4096 K5 31.9 / 28.3; twelve of 2816x2048 K5 34.4 / 26.8.  (Left as they are: ten of 4096x14336 or
+// 4096x8192 with 9 rows at K4, 7 % behind the chunked kernel.)
+inline bool group_takes_tiles(int count, int m, int n, int K, int max_M) {
+  if (max_M <= 8) return false;
+  if (K <= 4 || max_M > 12 || group_tile_splits(count, m, n) > 1) return true;
+  const int nblk = n / 128, cus = num_cu(), grid = count * (m / 128), rounds = (grid + cus - 1) / cus;
+  return rounds > 2 || nblk < (rounds == 1 ? 64 : 32) || 4 * grid > 3 * rounds * cus;
 }
 template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
   if (rot) return bp.mb == 1 ? launch_batch_v<K, 1, true>(a, t, bp, st) : launch_batch_v<K, 2, true>(a, t, bp, st);

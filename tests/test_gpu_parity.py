@@ -778,3 +778,23 @@ def test_grouped_launch_of_9_to_32_rows(dev, oracle):
     for w, x, y in zip(ws, xs, got):
         if x.shape[0]:
             assert _rel(y.cpu().numpy(), _ref(oracle, *w, x)) <= REL_TOL
+
+
+@pytest.mark.parametrize("K,m,n,rows", [(4, 128, 1024, [9]), (3, 384, 1408, [9, 0, 32, 17]), (5, 256, 2176, [8, 31]), (2, 1024, 640, [16, 1, 33]),
+                                        (8, 2048, 256, [12, 12, 12, 12, 12, 12, 12, 12, 12]), (4, 128, 128, [32])])
+def test_grouped_launch_with_column_splits(dev, oracle, K, m, n, rows):
+    """Groups too small to fill the chip: up to eight column splits, fewer blocks than splits, splits of unequal length, every
+    way the splits share their rows (up to 8, 16 and 32 rows), problems without rows, an entry cut off a long problem.  1e-3: float16 activations."""
+    from htr_amd import ops, wire
+    print(f"grouped splits K={K} {m}x{n} {rows}", flush=True)
+    ws = [wire.synth_linear(m, n, K, 9300 + i) for i in range(len(rows))]
+    xs = [wire.synth_activation(r, n, 9400 + i) for i, r in enumerate(rows)]
+    bias = [torch.randn(m, generator=torch.Generator().manual_seed(i)) if i % 2 else None for i in range(len(rows))]
+    wd = [tuple(t.to(dev) for t in w) for w in ws]
+    bd = [None if b is None else b.to(dev) for b in bias]
+    for _ in range(2):                                                       # the second call finds the slots as the first left them
+        got = ops.linear_grouped([x.to(dev) for x in xs], wd, bd, out_dtype=torch.float32)
+        for w, x, b, y in zip(ws, xs, bias, got):
+            if x.shape[0]:
+                ref = _ref(oracle, *w, x) + (0 if b is None else b.numpy())
+                assert _rel(y.cpu().numpy(), ref) <= REL_TOL

@@ -268,3 +268,17 @@ def test_fake_tensors_and_make_fx_go_through_the_registered_op():
         assert tuple(y.shape) == (3, 5, 256) and y.dtype == torch.bfloat16
     g = make_fx(lambda x, qw, sc, su, sv: ops.linear(x, qw, sc, su, sv), tracing_mode="fake")(torch.empty(2, 384, dtype=torch.bfloat16), *w)
     assert any("htr.linear" in str(n.target) for n in g.graph.nodes)
+
+
+def test_small_groups_of_9_to_32_rows_get_column_splits(L):
+    """The workspace of a group that does not fill the chip has a slot for every split's partials (256 compute units: 32 row
+    blocks of two problems leave room for four splits), that of a group that does has none."""
+    L.htr_plan_device_override(256, 160 * 1024)
+    try:
+        slots = lambda count, m, S, rows: count * (m // 128) * S * rows * 512
+        for count, m, n, S in [(1, 4096, 14336, 8), (2, 4096, 14336, 4), (4, 4096, 14336, 2), (1, 128, 16384, 8), (3, 4096, 14336, 2)]:
+            assert L.htr_grouped_workspace_bytes(count, m, n, 4, 32) >= 2 * slots(count, m, S, 32)
+        rows = 32 * 8
+        assert L.htr_grouped_workspace_bytes(8, 4096, 14336, 4, 32) <= 2 * (rows * 14336 * 2 + rows * 112 * 16 + rows * 4 + 4096)
+    finally:
+        L.htr_plan_device_override(0, 0)
