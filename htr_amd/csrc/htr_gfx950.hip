@@ -79,10 +79,10 @@ size_t htr_workspace_bytes(int m, int n, int K, int M, int nsplit) {
     return ws_need((size_t)gp.wgs * sizeof(uint32_t), gemm_scratch_bytes(n, M, gp));
   }
   if (M > HTR_MAX_ROWS_PER_TILE) return 0;       // the other kernels take up to 128 rows
-  if (wants_batch(M, nsplit, m, n)) {
+  if (wants_batch(M, nsplit, m, n, K)) {
     BatchPlan bp;
-    if (!make_batch_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return 0;
-    return ws_need((size_t)bp.wgs * M * 128 * sizeof(float), prerot_bytes(n, batch_prerot_rows(M)));
+    if (!make_batch_plan(m, n, K, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return 0;
+    return ws_need((size_t)bp.wgs * M * 128 * sizeof(float), prerot_bytes(n, batch_prerot_rows(M, bp.tile)));
   }
   if (M > HTR_MAX_GROUP_ROWS) return 0;          // the chunked kernel takes up to 32 rows
   Plan pl;
@@ -102,9 +102,9 @@ int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
     return HTR_OK;
   }
   if (M > HTR_MAX_ROWS_PER_TILE) return HTR_ERR_BATCH;
-  if (wants_batch(M, nsplit, m, n)) {
+  if (wants_batch(M, nsplit, m, n, K)) {
     BatchPlan bp;
-    if (!make_batch_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return HTR_ERR_SPLIT;
+    if (!make_batch_plan(m, n, K, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return HTR_ERR_SPLIT;
     out6[0] = bp.cb; out6[1] = bp.wgs; out6[2] = bp.last_finishes ? 0 : 1; out6[3] = bp.S; out6[4] = bp.rot ? 0 : 1; out6[5] = (int)bp.lds;
     return HTR_OK;
   }
@@ -201,15 +201,15 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     return HTR_OK;
   }
   if (M > HTR_MAX_ROWS_PER_TILE) return HTR_ERR_BATCH;        // explicit plans of the other kernels take up to 128 rows
-  if (wants_batch(M, nsplit, m, n)) {
+  if (wants_batch(M, nsplit, m, n, K)) {
     BatchPlan bp;
-    if (!make_batch_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return HTR_ERR_SPLIT;
+    if (!make_batch_plan(m, n, K, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp)) return HTR_ERR_SPLIT;
     const size_t need = htr_workspace_bytes(m, n, K, M, nsplit);
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
     unsigned char* wsp = (unsigned char*)workspace + ws_half(workspace_bytes);
     LinearTail t;
     t.scales = (const uint16_t*)scales; t.sv = (const uint8_t*)sv; t.bias = bias; t.y = y;
-    place_prerot(t, wsp, n, batch_prerot_rows(M));
+    place_prerot(t, wsp, n, batch_prerot_rows(M, bp.tile));
     t.status = (uint32_t*)workspace;
     t.cbscale = htr_cbscale();
     t.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
@@ -218,11 +218,11 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     hipStream_t st = (hipStream_t)stream;
     // the workgroups rotate their own activations where the plan allows it (16-bit rows on 16-byte boundaries)
     const bool rot = bp.rot && x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0;
-    if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, tile_rows(M)));
+    if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, bp.tile));
     BatchArgs ba;
     ba.qw = (const uint32_t*)qweight; ba.part = (float*)((unsigned char*)workspace + WS_HEADER); ba.x = x; ba.su = (const uint8_t*)su;
     ba.m = m; ba.n = n; ba.M = M; ba.flags = x_dtype | (y_dtype << 2) | (bp.last_finishes ? FLAG_LAST_FINISHES : 0);
-    if (bp.rot && !rot) bp.lds = batch_lds_bytes(M);            // the layout of the kernel for pre-rotated activations
+    if (bp.rot && !rot) bp.lds = batch_lds_bytes(M, bp.tile);            // the layout of the kernel for pre-rotated activations
     HTR_FOR_K(K, return launch_batch_k<KK>(ba, rot, t, bp, st));
     return HTR_OK;
   }

@@ -250,30 +250,42 @@ template <int K> int launch_linear_k(const LinearLaunch& a, bool prerot, int mb,
 }
 
 // ---- batched kernel: split S of the column blocks per row block
-struct BatchPlan { int S, cb, wgs, mb, rot, last_finishes; size_t lds; };
+struct BatchPlan { int S, cb, wgs, mb, rot, last_finishes; bool tile; size_t lds; };      // tile: k_linear_tile, unless rot
 // rows x column blocks per split up to which a workgroup of the batched kernel rotates its own activations (256 pairs,
 // eight passes per wave) instead of a rotation launch: 16 x 16 or 32 x 8
 inline bool batch_rot_fits(int M, int cb) { return (M <= 16 && cb <= 16) || (M <= 32 && cb <= 8); }
 constexpr int BATCH_MIN_M = 9;      // rows from which the library policy takes the batched kernel on every shape
 inline int batch_groups(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : 8)); }   // groups of 16 activation rows
-// Activations that were rotated ahead go to k_linear_tile from 17 to 64 rows (one or two tiles of 32).  Measured on MI355X, K4,
-// us of the kernel, k_linear_batch / k_linear_tile: 32 rows on 28672x4096 26.9 / 22.1, 14336x4096 14.5 / 13.9, 4096x14336
-// 14.7 / 14.5; 64 rows 31.5 / 28.8, 19.4 / 18.2, 18.5 / 19.1.  Beyond 64 rows its loads of the activations bound it (64 KB
-// per step and compute unit at 128 rows, 70 GB/s; 97 rows of 14336x4096 at K5 32.6 / 33.9); up to 16 rows half of its
-// matrix instructions would be empty.
-inline bool tile_rows(int M) { return M >= 17 && M <= 64; }
-inline size_t batch_prerot_rows(int M) { return tile_rows(M) ? (size_t)(M + 31) / 32 * 32 : (size_t)M; }   // rows the layout holds
-inline size_t batch_lds_bytes(int M) {
-  if (tile_rows(M)) return tile_lds_bytes((M + 31) / 32);
+// k_linear_tile instead of k_linear_batch for 17 to 64 activation rows that were rotated ahead.  Measured on MI355X, us of the call
+// with its rotation, k_linear_batch / k_linear_tile:
+//   more row blocks than compute units, one split: 33..64 rows, two workgroups per compute unit, always (65536x4096, 33 rows K4
+//     66.8 / 50.5, K5 64.0 / 61.8, K8 76.8 / 74.0; 40960x1024, 64 rows K4 29.5 / 22.0); 17..32 rows up to K4 (65536x4096, 32 rows
+//     47.8 / 45.5) and, at more bits, whose decode the two workgroups cannot hide behind each other, up to 16 column blocks
+//     (65536x4096, 32 rows K5 52.2 / 56.9, 40960x2048 K5 29.8 / 29.8, 65536x1024 K5 22.5 / 20.5)
+//   up to a quarter of the compute units: its loop without barriers wins from 8 column blocks per split (256x14336, 33 rows K4
+//     19.3 / 18.4, K5 19.7 / 18.7; 512x8192, 64 rows K4 16.1 / 15.8, K8 16.8 / 16.0; 4 blocks: 256x4096, 33 rows K4 12.0 / 12.6)
+//   else up to K4 from 14 column blocks per split (14336x4096, 33 rows K4 21.8 / 20.9; 4096x14336, 33 rows K3 22.1 / 20.8; 11 blocks:
+//     4096x11008, 48 rows K4 19.8 / 21.8; 4 blocks: 4096x4096, 33 rows K4 12.5 / 13.2; 14336x4096, 33 rows K5 22.0 / 22.9)
+// Beyond 64 rows its loads of the activations bound it (64 KB per step and compute unit at 128 rows, 70 GB/s; 97 rows of
+// 14336x4096 at K5 32.6 / 33.9); up to 16 rows half of its matrix instructions would be empty.
+inline bool tile_takes(int K, int M, int S, int cb, int wgs) {
+  if (M < 17 || M > 64) return false;
+  const int cus = num_cu();
+  if (S == 1 && wgs > cus) return M > 32 || K <= 4 || cb <= 16;
+  if (4 * wgs <= cus) return cb >= 8;
+  return K <= 4 && cb >= 14;
+}
+inline size_t batch_prerot_rows(int M, bool tile) { return tile ? (size_t)(M + 31) / 32 * 32 : (size_t)M; }   // rows the layout holds
+inline size_t batch_lds_bytes(int M, bool tile) {
+  if (tile) return tile_lds_bytes((M + 31) / 32);
   const int rows = 16 * batch_groups(M);
   const size_t blocks = (size_t)2 * rows * BATCH_ROWH * 2, small = (size_t)5 * rows * 4, fin = (size_t)2 * M * BATCH_FIN_STRIDE * 4;
   return M > 64 ? (blocks + small > fin ? blocks + small : fin) : blocks + small + fin;
 }
-inline bool make_batch_plan(int m, int n, int M, int want_S, BatchPlan& bp) {
+inline bool make_batch_plan(int m, int n, int K, int M, int want_S, BatchPlan& bp) {
   const int nblk = n / 128, rbs = m / 128;
   if ((long)M * n * 2 >= (1L << 31)) return false;          // the kernels address the rotated activations with 32-bit byte offsets
   bp.mb = batch_groups(M);
-  bp.lds = batch_lds_bytes(M);
   bp.rot = 0;
   // Measured on MI355X (K4, 6..128 rows, 1024..28672 output rows): one workgroup per CU is the best fill; every further
   // split adds partial traffic that grows with the rows (14336x4096, 32 rows: 2 splits 19.9 us, 4 splits 24.5; 128
@@ -290,19 +302,22 @@ inline bool make_batch_plan(int m, int n, int M, int want_S, BatchPlan& bp) {
     if (want_S > 0 && S != want_S) continue;
     bp.S = S; bp.cb = cb; bp.wgs = rbs * S; found = true;
   }
+  if (!found) return false;
+  bp.tile = tile_takes(K, M, bp.S, bp.cb, bp.wgs);
+  bp.lds = batch_lds_bytes(M, bp.tile);
   // Splits that finish rows for each other wait for each other, which is only safe while every workgroup of the grid is
   // resident at once: one workgroup per CU at most.  A larger grid (an explicit split, a device with fewer CUs than the
   // policy assumed) falls back to the last split finishing everything: it waits only for workgroups dispatched before it.
-  bp.last_finishes = found && bp.wgs > cus ? 1 : 0;
+  bp.last_finishes = bp.wgs > cus ? 1 : 0;
   // Few rows over few column blocks per split, one workgroup per CU: every workgroup rotates its own slice.
   // HTR_BATCH_ROT=0 switches it off.
   static const bool rot_on = getenv("HTR_BATCH_ROT") == nullptr || atoi(getenv("HTR_BATCH_ROT")) != 0;
-  if (found && rot_on && batch_rot_fits(M, bp.cb) && bp.wgs <= cus) {
+  if (rot_on && batch_rot_fits(M, bp.cb) && bp.wgs <= cus) {
     const int rows = 16 * bp.mb;
     bp.rot = 1;
     bp.lds = (size_t)bp.cb * rows * BATCH_ROWH * 2 + (size_t)bp.cb * 2 * rows * 4 + rows * 4 + (size_t)2 * M * BATCH_FIN_STRIDE * 4;
   }
-  return found;
+  return true;
 }
 
 // ---- GEMM kernel (more than 128 rows): tiles of GEMM_ROWS activation rows in the grid's z, split S of the column blocks
@@ -403,28 +418,34 @@ inline bool group_takes_tiles(int count, int m, int n, int K, int max_M) {
 }
 template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
   if (rot) return bp.mb == 1 ? launch_batch_v<K, 1, true>(a, t, bp, st) : launch_batch_v<K, 2, true>(a, t, bp, st);
-  if (tile_rows(a.M)) {
+  if (bp.tile) {
     // Grids beyond one workgroup per compute unit, us without / with ONE: K4, 64 rows 65536x4096 67.0 / 59.4, 40960x1024 28.7 /
-    // 22.4, 33 rows 152064x4096 137.6 / 115.9; 32 rows 65536x4096 49.0 / 49.5.  Up to one per unit there is no second workgroup
+    // 22.4, 33 rows 152064x4096 137.6 / 115.9; 17 rows 40960x2048 24.0 / 23.6, 32 rows 25.5 /
+    // 24.7, 65536x4096 45.4 / 44.9.  Up to one per unit there is no second workgroup
     // to gain from: eight decoder layers of 32 rows at K3, whose gate/up takes 224 workgroups, 558 to 562 / 565 to 571.
     const bool one = bp.S == 1 && bp.wgs > num_cu();
     if (a.M <= 32) return one ? launch_tile_v<K, 1, true>(a, t, 1, 1, st) : launch_tile_v<K, 1, false>(a, t, bp.S, 1, st);
     return one ? launch_tile_v<K, 2, true>(a, t, 1, 1, st) : launch_tile_v<K, 2, false>(a, t, bp.S, 1, st);
   }
-  return bp.mb == 1 ? launch_batch_v<K, 1, false>(a, t, bp, st) : launch_batch_v<K, 8, false>(a, t, bp, st);
+  switch (bp.mb) {
+    case 1: return launch_batch_v<K, 1, false>(a, t, bp, st);
+    case 2: return launch_batch_v<K, 2, false>(a, t, bp, st);
+    case 4: return launch_batch_v<K, 4, false>(a, t, bp, st);
+    default: return launch_batch_v<K, 8, false>(a, t, bp, st);
+  }
 }
 // nsplit bit 29: batched kernel with the split in the low bits (0 = policy); otherwise the policy decides by M
 // Tall matrices (192 row blocks and more) fill the chip without column splits, so the batched kernel needs no exchange
 // there and wins from 6 rows (65536x4096, 8 rows: 41 against 50 us; 152064x4096: 91 against 95).
 // A matrix whose splits are four column blocks or fewer on a full grid (4096x4096: 8 splits of 4 blocks) is also ahead
 // with the batched kernel at 7 and 8 rows, when its workgroups rotate their own slices (8 rows: 9.2 against 10.4 us).
-inline bool wants_batch(int M, int nsplit, int m, int n) {
+inline bool wants_batch(int M, int nsplit, int m, int n, int K) {
   if (wants_gemm(M, nsplit)) return false;
   if (nsplit > 0) return (nsplit & (1 << 29)) != 0;
   if (M >= BATCH_MIN_M || (M >= 6 && m / 128 >= 192)) return true;
   if (M >= 7) {
     BatchPlan bp;
-    return make_batch_plan(m, n, M, 0, bp) && bp.rot && bp.cb <= 4 && bp.wgs >= num_cu();
+    return make_batch_plan(m, n, K, M, 0, bp) && bp.rot && bp.cb <= 4 && bp.wgs >= num_cu();
   }
   return false;
 }

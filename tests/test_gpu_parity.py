@@ -798,3 +798,22 @@ def test_grouped_launch_with_column_splits(dev, oracle, K, m, n, rows):
             if x.shape[0]:
                 ref = _ref(oracle, *w, x) + (0 if b is None else b.numpy())
                 assert _rel(y.cpu().numpy(), ref) <= REL_TOL
+
+
+@pytest.mark.parametrize("K,m,n,M,S", [(2, 256, 1024, 17, 1), (3, 128, 1152, 31, 1), (4, 384, 1280, 32, 1), (4, 256, 2176, 33, 2), (5, 128, 1408, 48, 1),
+                                       (6, 256, 3328, 63, 3), (7, 128, 1024, 64, 1), (8, 256, 2048, 50, 2), (4, 1024, 8192, 40, 8), (3, 384, 2304, 20, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_tiles_of_32_rows_over_8_and_more_blocks(dev, oracle, K, m, n, M, S, dtype):
+    """17 to 64 rows where the kernel with tiles of 32 rows takes them (8 column blocks per split and more on a small grid): both tile
+    counts and their edges, block counts around the depth of the stream, one to eight splits, every K.  1e-3: float16 activations."""
+    from htr_amd import ops
+    print(f"tiles, long rows K={K} {m}x{n} M={M} S={S} {dtype}", flush=True)
+    qw, sc, su, sv, x = _case(m, n, K, M, 2900 + M + K, dtype)
+    w = [t.to(dev) for t in (qw, sc, su, sv)]
+    ref = _ref(oracle, qw, sc, su, sv, x)
+    ops.NSPLIT = (1 << 29) | S
+    try:
+        for _ in range(2):                                                   # the second call finds the slots as the first left them
+            assert _rel(ops.linear_f32out(x.to(dev), *w).cpu().numpy(), ref) <= REL_TOL
+    finally:
+        ops.NSPLIT = 0

@@ -282,3 +282,24 @@ def test_small_groups_of_9_to_32_rows_get_column_splits(L):
         assert L.htr_grouped_workspace_bytes(8, 4096, 14336, 4, 32) <= 2 * (rows * 14336 * 2 + rows * 112 * 16 + rows * 4 + 4096)
     finally:
         L.htr_plan_device_override(0, 0)
+
+
+_TILE_LDS = {1: 2 * 32 * 132 * 4 + 2 * 32 * 4, 2: 2 * 64 * 132 * 4 + 2 * 64 * 4}      # k_linear_tile with one and two row tiles
+
+
+@pytest.mark.parametrize("m,n,K,M,tile", [
+    (28672, 4096, 5, 32, False), (28672, 4096, 5, 64, False), (14336, 4096, 6, 48, False), (65536, 4096, 5, 24, False),   # decode-heavy
+    (4096, 4096, 4, 33, False), (2048, 2048, 3, 64, False), (1024, 4096, 4, 48, False), (6144, 4096, 2, 64, False),       # few column blocks
+    (4096, 11008, 4, 48, False), (10240, 4096, 3, 33, False),
+    (65536, 4096, 5, 33, True), (65536, 4096, 4, 32, True), (40960, 1024, 8, 24, True), (14336, 4096, 4, 33, True),
+    (28672, 4096, 3, 32, True), (4096, 14336, 3, 32, True), (256, 14336, 8, 64, True), (512, 8192, 4, 64, True)])
+def test_tile_kernel_only_where_it_is_ahead(L, m, n, K, M, tile):
+    """17 to 64 rows that are rotated ahead go to the kernel with tiles of 32 rows only where that one measured faster than the
+    staged one (256 compute units): seen by the LDS that the plan asks for."""
+    out = (ctypes.c_int * 6)()
+    L.htr_plan_device_override(256, 160 * 1024)
+    try:
+        assert L.htr_linear_plan(m, n, K, M, 0, out) == 0
+    finally:
+        L.htr_plan_device_override(0, 0)
+    assert out[4] == 1 and (out[5] == _TILE_LDS[(M + 31) // 32]) == tile, list(out)
