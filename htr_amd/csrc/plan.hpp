@@ -304,6 +304,14 @@ inline bool make_batch_plan(int m, int n, int K, int M, int want_S, BatchPlan& b
   }
   if (!found) return false;
   bp.tile = tile_takes(K, M, bp.S, bp.cb, bp.wgs);
+  if (bp.tile) {
+    // The order for k_linear_tile has room for whole tiles of 32 rows, up to twice what the rows take.  What fits the library's
+    // own workspace (htr_linear_static) as rows goes on fitting it, with k_linear_batch; and 32-bit offsets bound it as well.
+    // (An order without gaps, offsets from the rows of the last tile, costs every call 0.2 to 0.4 us: 256x14336, 64 rows K4 19.4 / 19.8.)
+    const size_t slots = (size_t)bp.wgs * M * 128 * sizeof(float), padded = batch_prerot_rows(M, true);
+    if ((padded * n * 2 >> 31) != 0 || (ws_need(slots, prerot_bytes(n, padded)) > HTR_STATIC_SCRATCH_BYTES &&
+                                        ws_need(slots, prerot_bytes(n, M)) <= HTR_STATIC_SCRATCH_BYTES)) bp.tile = false;
+  }
   bp.lds = batch_lds_bytes(M, bp.tile);
   // Splits that finish rows for each other wait for each other, which is only safe while every workgroup of the grid is
   // resident at once: one workgroup per CU at most.  A larger grid (an explicit split, a device with fewer CUs than the
@@ -420,9 +428,8 @@ template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTa
   if (rot) return bp.mb == 1 ? launch_batch_v<K, 1, true>(a, t, bp, st) : launch_batch_v<K, 2, true>(a, t, bp, st);
   if (bp.tile) {
     // Grids beyond one workgroup per compute unit, us without / with ONE: K4, 64 rows 65536x4096 67.0 / 59.4, 40960x1024 28.7 /
-    // 22.4, 33 rows 152064x4096 137.6 / 115.9; 17 rows 40960x2048 24.0 / 23.6, 32 rows 25.5 /
-    // 24.7, 65536x4096 45.4 / 44.9.  Up to one per unit there is no second workgroup
-    // to gain from: eight decoder layers of 32 rows at K3, whose gate/up takes 224 workgroups, 558 to 562 / 565 to 571.
+    // 22.4, 33 rows 152064x4096 137.6 / 115.9; 17 rows 40960x2048 24.0 / 23.6, 32 rows 25.5 / 24.7, 65536x4096 45.4 / 44.9.  Up to one
+    // per unit there is no second workgroup to gain from: eight decoder layers of 32 rows at K3, whose gate/up takes 224 workgroups, 558 to 562 / 565 to 571.
     const bool one = bp.S == 1 && bp.wgs > num_cu();
     if (a.M <= 32) return one ? launch_tile_v<K, 1, true>(a, t, 1, 1, st) : launch_tile_v<K, 1, false>(a, t, bp.S, 1, st);
     return one ? launch_tile_v<K, 2, true>(a, t, 1, 1, st) : launch_tile_v<K, 2, false>(a, t, bp.S, 1, st);

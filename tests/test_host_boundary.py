@@ -303,3 +303,22 @@ def test_tile_kernel_only_where_it_is_ahead(L, m, n, K, M, tile):
     finally:
         L.htr_plan_device_override(0, 0)
     assert out[4] == 1 and (out[5] == _TILE_LDS[(M + 31) // 32]) == tile, list(out)
+
+
+@pytest.mark.parametrize("m,n", [(128, 30848), (1024, 38016), (128, 49152), (256, 14336), (4096, 14336), (128, 122880)])
+@pytest.mark.parametrize("K,M", [(4, 17), (4, 31), (3, 32), (4, 33), (8, 40), (2, 47), (4, 64)])
+def test_static_workspace_takes_what_fits_it_as_rows(L, m, n, K, M):
+    """The tile kernel's order of the activations rounds the rows up to 32; a call whose M rows of f16, block sums and scales (each
+    rounded up to 256 bytes) fit htr_linear_static's built-in workspace must not be refused for that."""
+    from htr_amd import _native
+    up = lambda b: (b + 255) // 256 * 256
+    L.htr_plan_device_override(256, 160 * 1024)
+    try:
+        out = (ctypes.c_int * 6)()
+        assert L.htr_linear_plan(m, n, K, M, 0, out) == 0
+        need = L.htr_workspace_bytes(m, n, K, M, 0)
+    finally:
+        L.htr_plan_device_override(0, 0)
+    scratch, slots = up(M * n * 2) + up(M * (n // 128) * 16) + up(M * 4), out[1] * M * 512
+    if 2 * max(scratch, slots) + 2048 <= _native.STATIC_SCRATCH_BYTES:
+        assert 0 < need <= _native.STATIC_SCRATCH_BYTES

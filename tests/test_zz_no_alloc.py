@@ -109,3 +109,21 @@ def test_static_entry_recovers_with_reset_after_a_give_up():
     torch.cuda.synchronize()
     assert np.array_equal(y.cpu().numpy(), y_ref.cpu().numpy())
     print(f"static entry: {gave_up} of 16 launches gave up under a one-poll bound", flush=True)
+
+
+def test_static_entry_takes_long_rows(oracle):
+    """33 rows of 30848 columns fit the built-in workspace as rows, not rounded up to tiles of 32."""
+    from htr_amd import _native, wire
+    L = _native.lib()
+    dev = torch.device("cuda:0")
+    m, n, K, M = 128, 30848, 4, 33
+    print(f"static entry {m}x{n} M={M}", flush=True)
+    assert L.htr_workspace_bytes(m, n, K, M, 0) <= _native.STATIC_SCRATCH_BYTES
+    host = wire.synth_linear(m, n, K, 20261125 + 31)
+    tensors = [t.to(dev) for t in host]
+    x = wire.synth_activation(M, n, 32, torch.bfloat16, dev)
+    y = torch.full((M, m), float("nan"), dtype=torch.float32, device=dev)
+    _call(L, _native, L.htr_linear_static, tensors, x, y, m, n, K, M, (1,))
+    torch.cuda.synchronize()
+    ref = oracle.c_linear(x.float().cpu().numpy(), *[t.numpy() for t in host])
+    assert float(np.abs(y.cpu().numpy() - ref).max() / np.abs(ref).max()) <= 1e-3        # float16 activations
