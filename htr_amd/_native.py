@@ -5,7 +5,9 @@ Loading never compiles: the library is built ahead of time by `python -m htr_amd
 PyTorch fallback for the packed-linear path.
 """
 import ctypes
+import importlib
 import os
+import warnings
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 # HTR_GFX950_LIB names another build of the same library (e.g. a tuning build); it must exist, there is no fallback
@@ -72,18 +74,22 @@ _fast = None
 
 
 def fast():
-    """The C++ host path (htr_amd._fast), bound to the library's entry points."""
+    """The C++ host path (htr_amd._fast), bound to the library's entry points; None where it cannot be loaded (not built, built
+    for another Python or torch): calls then prepare their launches in Python, with the same kernels and more host time."""
     global _fast
     if _fast is None:
         L = lib()
         try:
-            from . import _fast as module
+            module = importlib.import_module("._fast", __package__)
         except ImportError as e:
-            raise NativeLibraryMissing(f"htr_amd/_fast.so cannot be loaded ({e}); run `python -m htr_amd.build`.") from e
+            warnings.warn(f"htr_amd/_fast.so cannot be loaded ({e}): launches are prepared in Python; `python -m htr_amd.build` builds it",
+                          RuntimeWarning, stacklevel=2)
+            _fast = False
+            return None
         address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
         module.bind(address(L.htr_linear), address(L.htr_stream_capture_id), address(L.htr_moe_scratch_bytes), address(L.htr_moe_experts))
         _fast = module
-    return _fast
+    return _fast or None
 
 
 def check(status):

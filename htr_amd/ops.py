@@ -367,9 +367,11 @@ _TICKET_POOLS = {}       # device index -> pinned words in which the routing ker
 
 def _moe_silu(x, expert_ids, expert_weights, gate_up, down):
     """moe_experts with the default activation in one library call; None where the arguments are not as the library wants them."""
+    fast = _native.fast()
+    if fast is None:
+        return None
     index = x.get_device()
     stream = _raw_stream(index)
-    fast = _native.fast()
     if torch.cuda.is_current_stream_capturing():
         return fast.moe(x, expert_ids, expert_weights, gate_up, down, 0, 0, stream)
     pool = _TICKET_POOLS.get(index)
@@ -414,9 +416,10 @@ def _linear_decode(x, qweight, scales, su, sv, bias):
         return None
     stream = _raw_stream(index)
     ws = _WORKSPACES.get((index, stream))
-    if ws is None:
+    fast = _native.fast()
+    if ws is None or fast is None:
         return None
-    return _native.fast().linear(x, qweight, scales, su, sv, bias, ws.ptr, ws.size, ws.flag_ptr, stream)
+    return fast.linear(x, qweight, scales, su, sv, bias, ws.ptr, ws.size, ws.flag_ptr, stream)
 
 
 def linear(x, qweight, scales, su, sv, bias=None):

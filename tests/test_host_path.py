@@ -1,0 +1,69 @@
+"""The C++ host path (htr_amd._fast) and the ways around it: without it, with arguments it does not take, with failures behind it."""
+import os
+import sys
+
+import pytest
+import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def dev():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from htr_amd import _native
+    _native.lib()
+    return torch.device("cuda:0")
+
+
+@pytest.fixture
+def without_fast(monkeypatch):
+    from htr_amd import _native
+    monkeypatch.setattr(_native, "_fast", None)
+    monkeypatch.setitem(sys.modules, "htr_amd._fast", None)          # importing it fails
+
+
+def _linear(m, n, K, seed, dev):
+    from htr_amd import wire
+    return tuple(t.to(dev) for t in wire.synth_linear(m, n, K, seed))
+
+
+def test_missing_extension_is_said_once(without_fast):
+    from htr_amd import _native
+    with pytest.warns(RuntimeWarning, match="_fast.so"):
+        assert _native.fast() is None
+    import warnings
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _native.fast() is None
+
+
+def test_package_ships_every_built_file():
+    import fnmatch
+    import re
+    from htr_amd import build
+    patterns = re.findall(r'"([^"]+)"', re.search(r"^htr_amd = \[(.*)\]$", open(os.path.join(ROOT, "pyproject.toml")).read(), re.M).group(1))
+    for built in (build.LIB, build.BINDING):
+        path = os.path.relpath(built, os.path.join(ROOT, "htr_amd"))
+        assert any(fnmatch.fnmatch(path, p) and os.path.dirname(path) == os.path.dirname(p) for p in patterns), path
+
+
+@pytest.mark.gpu
+def test_calls_without_the_extension(dev, without_fast):
+    """Every call of a stream, not only the first one, which has no workspace yet."""
+    from htr_amd import ops
+    print("linear and experts without the extension", flush=True)
+    w, x = _linear(256, 384, 4, 51, dev), torch.randn(3, 384, device=dev).bfloat16()
+    with pytest.warns(RuntimeWarning):
+        first = [ops.linear(x, *w) for _ in range(3)]
+    gate_up, down = [_linear(256, 128, 4, 60 + e, dev) for e in range(2)], [_linear(128, 128, 4, 70 + e, dev) for e in range(2)]
+    xe, ids, we = torch.randn(5, 128, device=dev).bfloat16(), torch.tensor([[0], [1], [1], [0], [1]], device=dev), torch.rand(5, 1, device=dev)
+    layer = ops.moe_experts(xe, ids, we, gate_up, down)
+    from htr_amd import _native
+    _native._fast = None
+    sys.modules.pop("htr_amd._fast")
+    assert _native.fast() is not None
+    assert all(torch.equal(y, ops.linear(x, *w)) for y in first)
+    whole = ops.moe_experts(xe, ids, we, gate_up, down)
+    assert float((whole - layer).norm() / layer.norm()) <= 1e-3          # the same products, rounded alike
