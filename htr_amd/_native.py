@@ -78,16 +78,18 @@ def fast():
     for another Python or torch): calls then prepare their launches in Python, with the same kernels and more host time."""
     global _fast
     if _fast is None:
+        import torch
         L = lib()
+        address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
         try:
             module = importlib.import_module("._fast", __package__)
+            module.bind(L.htr_abi_version(), str(torch.__version__), address(L.htr_linear), address(L.htr_stream_capture_id),
+                        address(L.htr_moe_scratch_bytes), address(L.htr_moe_experts))
         except ImportError as e:
-            warnings.warn(f"htr_amd/_fast.so cannot be loaded ({e}): launches are prepared in Python; `python -m htr_amd.build` builds it",
+            warnings.warn(f"htr_amd/_fast.so cannot be used ({e}): launches are prepared in Python; `python -m htr_amd.build` builds it",
                           RuntimeWarning, stacklevel=2)
             _fast = False
             return None
-        address = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
-        module.bind(address(L.htr_linear), address(L.htr_stream_capture_id), address(L.htr_moe_scratch_bytes), address(L.htr_moe_experts))
         _fast = module
     return _fast or None
 

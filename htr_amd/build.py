@@ -36,7 +36,7 @@ def binding_command():
     root = os.path.dirname(torch.__file__)
     lib = os.path.join(root, "lib")
     return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-Wall",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DHTR_BUILD_TORCH="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
             "-I" + os.path.join(root, "include"), "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"),
             "-I" + sysconfig.get_paths()["include"], BINDING_SOURCE, "-o", BINDING, "-L" + lib, "-lc10", "-ltorch_cpu", "-ltorch_python"]
 
@@ -60,7 +60,7 @@ def build(verbose=False, extra=()):
 def is_stale():
     def older(built, sources):
         return not os.path.exists(built) or any(os.path.getmtime(s) > os.path.getmtime(built) for s in sources)
-    return older(LIB, SOURCES + PARTS + [HEADER]) or older(BINDING, [BINDING_SOURCE])
+    return older(LIB, SOURCES + PARTS + [HEADER]) or older(BINDING, [BINDING_SOURCE, HEADER])
 
 
 if __name__ == "__main__":

@@ -68,7 +68,7 @@ const char* htr_strerror(int status) {
 }
 
 int htr_last_hip_error(void) { return g_last_hip_error; }
-int htr_abi_version(void) { return 1; }
+int htr_abi_version(void) { return HTR_ABI_VERSION; }
 float htr_cbscale(void) { return (float)(1.0 / __builtin_sqrt(MEAN_SQ)); }
 
 size_t htr_workspace_bytes(int m, int n, int K, int M, int nsplit) {

@@ -13,23 +13,19 @@
 #include <c10/core/GradMode.h>
 #include <chrono>
 #include <cstdint>
+#include <cstring>
 #include <vector>
+#include "../../include/htr_gfx950.h"
 
 namespace {
 
-typedef int (*linear_fn)(const void*, const void*, const void*, const void*, const void*, const void*, void*, int, int, int, int, int, int,
-                         int, void*, size_t, void*);
-typedef size_t (*moe_bytes_fn)(int, int, int, int, int);
-typedef int (*moe_fn)(const void*, int, const void*, int, const float*, int, int, const void* const*, int, int, int, int, int, float*, void*,
-                      size_t, unsigned int*, unsigned int, void*);
-typedef unsigned long long (*capture_fn)(void*);
-linear_fn f_linear = nullptr;
-capture_fn f_capture = nullptr;
-moe_bytes_fn f_moe_bytes = nullptr;
-moe_fn f_moe = nullptr;
+// the library's entry points, with the types that its header declares
+decltype(&htr_linear) f_linear = nullptr;
+decltype(&htr_stream_capture_id) f_capture = nullptr;
+decltype(&htr_moe_scratch_bytes) f_moe_bytes = nullptr;
+decltype(&htr_moe_experts) f_moe = nullptr;
 
-constexpr int OK = 0;
-constexpr int MAX_ROWS = 128;      // rows of one decode launch
+constexpr int MAX_ROWS = HTR_MAX_ROWS_PER_TILE;      // rows of one decode launch
 
 int dtype_code(at::ScalarType t) {
   switch (t) {
@@ -100,7 +96,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
                           t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, 0,
                           ws, bytes, stream);
-  if (rc != OK) Py_RETURN_NONE;
+  if (rc != HTR_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -158,7 +154,7 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int rc = f_moe(x.const_data_ptr(), code, ids.const_data_ptr(), ids.scalar_type() == at::kLong ? 1 : 0, (const float*)w.const_data_ptr(), (int)T,
                        (int)top, ptrs.data(), (int)E, (int)H, (int)F, (int)s1.K, (int)s2.K, (float*)y.mutable_data_ptr(), scratch.mutable_data_ptr(),
                        need, word, ticket, stream);
-  if (rc != OK) Py_RETURN_NONE;
+  if (rc != HTR_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
@@ -185,13 +181,19 @@ PyObject* wait_word(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(htr_linear, htr_stream_capture_id, htr_moe_scratch_bytes, htr_moe_experts): addresses of the library's entry points
+// bind(version of the library's C ABI, version of the running torch, addresses of htr_linear, htr_stream_capture_id,
+// htr_moe_scratch_bytes and htr_moe_experts); ImportError where either version is not the one that this file was compiled with
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  if (nargs != 4) { PyErr_SetString(PyExc_TypeError, "bind wants four addresses"); return nullptr; }
+  if (nargs != 6) { PyErr_SetString(PyExc_TypeError, "bind wants two versions and four addresses"); return nullptr; }
+  const long abi = PyLong_AsLong(args[0]);
+  const char* torch_version = PyUnicode_AsUTF8(args[1]);
   void* p[4];
-  for (int i = 0; i < 4; ++i) p[i] = PyLong_AsVoidPtr(args[i]);
+  for (int i = 0; i < 4; ++i) p[i] = PyLong_AsVoidPtr(args[2 + i]);
   if (PyErr_Occurred()) return nullptr;
-  f_linear = (linear_fn)p[0]; f_capture = (capture_fn)p[1]; f_moe_bytes = (moe_bytes_fn)p[2]; f_moe = (moe_fn)p[3];
+  if (abi != HTR_ABI_VERSION) return PyErr_Format(PyExc_ImportError, "compiled for version %d of the library's C ABI, not %ld", HTR_ABI_VERSION, abi);
+  if (strcmp(torch_version, HTR_BUILD_TORCH) != 0) return PyErr_Format(PyExc_ImportError, "compiled for torch %s, not %s", HTR_BUILD_TORCH, torch_version);
+  f_linear = (decltype(f_linear))p[0]; f_capture = (decltype(f_capture))p[1];
+  f_moe_bytes = (decltype(f_moe_bytes))p[2]; f_moe = (decltype(f_moe))p[3];
   Py_RETURN_NONE;
 }
 

@@ -49,6 +49,34 @@ def test_package_ships_every_built_file():
         assert any(fnmatch.fnmatch(path, p) and os.path.dirname(path) == os.path.dirname(p) for p in patterns), path
 
 
+def test_extension_of_another_build_is_not_used(monkeypatch):
+    """Another C ABI or another torch than it was compiled with: launches are prepared in Python."""
+    from htr_amd import _native
+    module = _native.fast()
+    assert module is not None
+    abi = _native.lib().htr_abi_version()
+    with pytest.raises(ImportError, match="ABI"):
+        module.bind(abi + 1, torch.__version__, 0, 0, 0, 0)
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    monkeypatch.setattr(_native, "_fast", None)
+    with pytest.warns(RuntimeWarning, match="torch 0.0.1|not 0.0.1"):
+        assert _native.fast() is None
+
+
+def test_a_newer_header_makes_the_extension_stale(monkeypatch, tmp_path):
+    from htr_amd import build
+    now = os.path.getmtime(build.BINDING)
+    for name, age in (("HEADER", 100), ("LIB", 200)):
+        f = tmp_path / name
+        f.write_text("")
+        os.utime(f, (now + age, now + age))
+        monkeypatch.setattr(build, name, str(f))
+    monkeypatch.setattr(build, "SOURCES", [])
+    monkeypatch.setattr(build, "PARTS", [])
+    monkeypatch.setattr(build, "BINDING_SOURCE", build.BINDING)
+    assert build.is_stale()
+
+
 @pytest.mark.gpu
 def test_calls_without_the_extension(dev, without_fast):
     """Every call of a stream, not only the first one, which has no workspace yet."""
