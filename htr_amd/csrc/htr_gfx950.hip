@@ -30,6 +30,7 @@
 #include <string.h>
 #include <stdlib.h>
 #include <atomic>
+#include <mutex>
 #include <type_traits>
 
 #include "../../include/htr_gfx950.h"
@@ -136,6 +137,22 @@ int htr_workspace_init(void* workspace, size_t workspace_bytes, void* host_statu
   return HTR_OK;
 }
 
+namespace {
+// The launches of one call on a workspace stay together in their stream: two host threads that share a stream, and with it a
+// workspace, would otherwise rotate into the scratch half that the other one's product is about to read.  One of 64 locks by
+// address, held while the launches are queued.
+struct Together {
+  std::mutex& m;
+  static std::mutex& of(const void* workspace) {
+    static std::mutex locks[64];
+    return locks[((uint64_t)(uintptr_t)workspace >> 8) * 0x9E3779B97F4A7C15ull >> 58];
+  }
+  explicit Together(const void* workspace) : m(of(workspace)) { m.lock(); }
+  ~Together() { m.unlock(); }
+  Together(const Together&) = delete;
+};
+}
+
 unsigned long long htr_stream_capture_id(void* stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   unsigned long long id = 0;
@@ -154,6 +171,7 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
   if (((uintptr_t)qweight & 15) || ((uintptr_t)scales & 1) || ((uintptr_t)x & (x_dtype == HTR_F32 ? 3 : 1)) ||
       ((uintptr_t)y & (y_dtype == HTR_F32 ? 3 : 1)) || (bias && ((uintptr_t)bias & (y_dtype == HTR_F32 ? 3 : 1))))
     return HTR_ERR_ALIGN;
+  const Together together(workspace);
   if (wants_gemm(M, nsplit)) {
     GemmPlan gp;
     if (!make_gemm_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, gemm_want_jb(nsplit), gp)) return HTR_ERR_SPLIT;
@@ -352,6 +370,7 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
   if (need == 0) return HTR_ERR_SPLIT;
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
 
+  const Together together(workspace);
   unsigned char* wsp = (unsigned char*)workspace + ws_half(workspace_bytes);      // scratch half
   if (group_takes_tiles(count, m, n, K, max_M)) {
     // one tile of 32 rows per problem

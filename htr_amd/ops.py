@@ -149,8 +149,9 @@ def check_status(device=None):
 def _new_workspace(key, device, stream_id, size):
     buf = torch.empty(size, dtype=torch.uint8, device=device)
     flag = _flag_word(device)
-    ws = _WORKSPACES[key] = _Workspace(buf, flag, stream_id)
+    ws = _Workspace(buf, flag, stream_id)
     _native.check(_native.lib().htr_workspace_init(buf.data_ptr(), size, None if flag is None else flag[1], stream_id))
+    _WORKSPACES[key] = ws        # only now: another thread on this stream launches on what it finds here
     return ws
 
 

@@ -95,3 +95,30 @@ def test_calls_without_the_extension(dev, without_fast):
     assert all(torch.equal(y, ops.linear(x, *w)) for y in first)
     whole = ops.moe_experts(xe, ids, we, gate_up, down)
     assert float((whole - layer).norm() / layer.norm()) <= 1e-3          # the same products, rounded alike
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [20, 200])
+def test_two_threads_on_one_stream(dev, M):
+    """Calls of two launches each (rotation, product) from two threads on one stream, which share its workspace: each one's
+    launches stay together, in the C++ host path (20 rows, float32) and in the Python one (200 rows)."""
+    import threading
+    from htr_amd import ops
+    print(f"two threads on one stream M={M}", flush=True)
+    w = _linear(4096, 4096, 4, 52, dev)
+    xs = [torch.randn(M, 4096, device=dev, generator=torch.Generator(device=dev).manual_seed(i)) for i in range(2)]
+    want = [ops.linear(x, *w) for x in xs]
+    torch.cuda.synchronize()
+    wrong = [0, 0]
+
+    def work(i):
+        ys = [ops.linear(xs[i], *w) for _ in range(100)]
+        torch.cuda.synchronize()
+        wrong[i] = sum(not torch.equal(y, want[i]) for y in ys)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == [0, 0]
