@@ -89,24 +89,30 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   void* stream = PyLong_AsVoidPtr(args[9]);
   if (PyErr_Occurred()) return nullptr;
   if ((failed != nullptr && *failed != 0) || f_capture(stream) != 0) Py_RETURN_NONE;
-  c10::DeviceGuard guard(x.device());
-  at::DimVector shape(x.sizes().begin(), x.sizes().end());
-  shape.back() = s.m;
-  at::Tensor y = at::empty(shape, x.options());
-  const int rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
-                          t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, 0,
-                          ws, bytes, stream);
+  at::Tensor y;
+  int rc;
+  {
+    // other threads run meanwhile: a launch waits where the stream's queue is full.  The caller's frame holds the tensors.
+    pybind11::gil_scoped_release no_lock;
+    c10::DeviceGuard guard(x.device());
+    at::DimVector shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = s.m;
+    y = at::empty(shape, x.options());
+    rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
+                  t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, 0,
+                  ws, bytes, stream);
+  }
   if (rc != HTR_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS
 }
 
-// The tensor addresses of one list of HTR-W1 tuples into every eighth slot group of `ptrs`; false where one is not like the first
-bool collect(PyObject* seq, int offset, c10::Device dev, Shape& shape, std::vector<const void*>& ptrs) {
-  const Py_ssize_t E = PySequence_Fast_GET_SIZE(seq);
-  PyObject** items = PySequence_Fast_ITEMS(seq);
+// The tensor addresses of one tuple of HTR-W1 tuples into every eighth slot group of `ptrs`; false where one is not like the first.
+// The tensors of an expert given as a list, which another thread may change, go to `keep`.
+bool collect(PyObject* experts, int offset, c10::Device dev, Shape& shape, std::vector<const void*>& ptrs, std::vector<at::Tensor>& keep) {
+  const Py_ssize_t E = PyTuple_GET_SIZE(experts);
   for (Py_ssize_t e = 0; e < E; ++e) {
-    PyObject* tup = items[e];
+    PyObject* tup = PyTuple_GET_ITEM(experts, e);
     if (!(PyTuple_Check(tup) || PyList_Check(tup)) || PySequence_Fast_GET_SIZE(tup) != 4) return false;
     const at::Tensor* t[4];
     for (int k = 0; k < 4; ++k) { t[k] = tensor_of(PySequence_Fast_GET_ITEM(tup, k)); if (t[k] == nullptr) return false; }
@@ -115,6 +121,7 @@ bool collect(PyObject* seq, int offset, c10::Device dev, Shape& shape, std::vect
     if (e == 0) shape = s;
     else if (s.m != shape.m || s.n != shape.n || s.K != shape.K) return false;
     for (int k = 0; k < 4; ++k) ptrs[8 * e + offset + k] = t[k]->const_data_ptr();
+    if (PyList_Check(tup)) for (int k = 0; k < 4; ++k) keep.push_back(*t[k]);
   }
   return true;
 }
@@ -131,29 +138,38 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if ((it->scalar_type() != at::kLong && it->scalar_type() != at::kInt) || !wt->is_floating_point()) Py_RETURN_NONE;
   // the result is differentiable in the routing weights only where torch adds it up: not behind a raw pointer
   if (!raw_ok(*xt) || !raw_ok(*it) || !raw_ok(*wt) || differentiable(*wt)) Py_RETURN_NONE;
-  Owned gu{PySequence_Fast(args[3], "gate_up is not a sequence")}, dn{PySequence_Fast(args[4], "down is not a sequence")};
+  Owned gu{PySequence_Tuple(args[3])}, dn{PySequence_Tuple(args[4])};      // own references to the experts: no other thread can drop one
   if (gu.p == nullptr || dn.p == nullptr) { PyErr_Clear(); Py_RETURN_NONE; }
-  const Py_ssize_t E = PySequence_Fast_GET_SIZE(gu.p);
-  if (E < 1 || PySequence_Fast_GET_SIZE(dn.p) != E) Py_RETURN_NONE;
+  const Py_ssize_t E = PyTuple_GET_SIZE(gu.p);
+  if (E < 1 || PyTuple_GET_SIZE(dn.p) != E) Py_RETURN_NONE;
   std::vector<const void*> ptrs((size_t)E * 8);
+  std::vector<at::Tensor> keep;
   Shape s1, s2;
-  if (!collect(gu.p, 0, xt->device(), s1, ptrs) || !collect(dn.p, 4, xt->device(), s2, ptrs)) Py_RETURN_NONE;
+  if (!collect(gu.p, 0, xt->device(), s1, ptrs, keep) || !collect(dn.p, 4, xt->device(), s2, ptrs, keep)) Py_RETURN_NONE;
   const int64_t F = s1.m / 2;
   if (s1.n != H || s2.m != H || s2.n != F || T < 1 || top < 1 || T > (1 << 24) || E > (1 << 20)) Py_RETURN_NONE;
   unsigned int* word = (unsigned int*)PyLong_AsVoidPtr(args[5]);
   const unsigned int ticket = (unsigned int)PyLong_AsUnsignedLong(args[6]);
   void* stream = PyLong_AsVoidPtr(args[7]);
   if (PyErr_Occurred()) return nullptr;
-  c10::DeviceGuard guard(xt->device());
-  at::Tensor x = xt->contiguous(), ids = it->contiguous(), w = wt->to(at::kFloat).contiguous();
-  if ((uintptr_t)x.const_data_ptr() & 15) x = x.clone();
-  const size_t need = f_moe_bytes((int)T, (int)top, (int)E, (int)H, (int)F);
-  if (need == 0) Py_RETURN_NONE;
-  at::Tensor scratch = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
-  at::Tensor y = at::empty({T, H}, x.options().dtype(at::kFloat));
-  const int rc = f_moe(x.const_data_ptr(), code, ids.const_data_ptr(), ids.scalar_type() == at::kLong ? 1 : 0, (const float*)w.const_data_ptr(), (int)T,
-                       (int)top, ptrs.data(), (int)E, (int)H, (int)F, (int)s1.K, (int)s2.K, (float*)y.mutable_data_ptr(), scratch.mutable_data_ptr(),
-                       need, word, ticket, stream);
+  at::Tensor y;
+  int rc;
+  {
+    pybind11::gil_scoped_release no_lock;      // as in linear()
+    c10::DeviceGuard guard(xt->device());
+    at::Tensor x = xt->contiguous(), ids = it->contiguous(), w = wt->to(at::kFloat).contiguous();
+    if ((uintptr_t)x.const_data_ptr() & 15) x = x.clone();
+    const size_t need = f_moe_bytes((int)T, (int)top, (int)E, (int)H, (int)F);
+    if (need == 0) {
+      rc = HTR_ERR_SHAPE;
+    } else {
+      at::Tensor scratch = at::empty({(int64_t)need}, x.options().dtype(at::kByte));
+      y = at::empty({T, H}, x.options().dtype(at::kFloat));
+      rc = f_moe(x.const_data_ptr(), code, ids.const_data_ptr(), ids.scalar_type() == at::kLong ? 1 : 0, (const float*)w.const_data_ptr(), (int)T,
+                 (int)top, ptrs.data(), (int)E, (int)H, (int)F, (int)s1.K, (int)s2.K, (float*)y.mutable_data_ptr(), scratch.mutable_data_ptr(),
+                 need, word, ticket, stream);
+    }
+  }
   if (rc != HTR_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS

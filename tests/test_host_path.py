@@ -122,3 +122,26 @@ def test_two_threads_on_one_stream(dev, M):
     for t in threads:
         t.join()
     assert wrong == [0, 0]
+
+
+@pytest.mark.gpu
+def test_interpreter_lock_is_free_during_launches(dev):
+    """In the place of the library's launches, the interpreter's own PyGILState_Check: it returns 0, which is success, only while
+    this thread does not hold the lock.  No kernel runs."""
+    import ctypes
+    from htr_amd import _native, ops
+    print("interpreter lock", flush=True)
+    module, L = _native.fast(), _native.lib()
+    at = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
+    check = at(ctypes.pythonapi.PyGILState_Check)
+    w, x = _linear(256, 384, 4, 51, dev), torch.randn(3, 384, device=dev).bfloat16()
+    gate_up, down = [_linear(256, 128, 4, 60, dev)], [list(_linear(128, 128, 4, 70, dev))]
+    xe, ids, we = torch.randn(5, 128, device=dev).bfloat16(), torch.zeros(5, 1, dtype=torch.int64, device=dev), torch.rand(5, 1, device=dev)
+    stream = ops._raw_stream(0)
+    module.bind(L.htr_abi_version(), str(torch.__version__), check, at(L.htr_stream_capture_id), at(L.htr_moe_scratch_bytes), check)
+    try:
+        assert module.linear(x, *w, None, 0, 0, 0, stream) is not None
+        assert module.moe(xe, ids, we, gate_up, down, 0, 0, stream) is not None
+    finally:
+        _native._fast = None
+        _native.fast()
