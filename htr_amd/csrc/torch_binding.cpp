@@ -138,8 +138,10 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if ((it->scalar_type() != at::kLong && it->scalar_type() != at::kInt) || !wt->is_floating_point()) Py_RETURN_NONE;
   // the result is differentiable in the routing weights only where torch adds it up: not behind a raw pointer
   if (!raw_ok(*xt) || !raw_ok(*it) || !raw_ok(*wt) || differentiable(*wt)) Py_RETURN_NONE;
+  // plain lists and tuples only: another kind of collection may load an expert when it is asked for, and is asked for the chosen ones
+  for (int i = 3; i < 5; ++i) if (!PyTuple_CheckExact(args[i]) && !PyList_CheckExact(args[i])) Py_RETURN_NONE;
   Owned gu{PySequence_Tuple(args[3])}, dn{PySequence_Tuple(args[4])};      // own references to the experts: no other thread can drop one
-  if (gu.p == nullptr || dn.p == nullptr) { PyErr_Clear(); Py_RETURN_NONE; }
+  if (gu.p == nullptr || dn.p == nullptr) return nullptr;
   const Py_ssize_t E = PyTuple_GET_SIZE(gu.p);
   if (E < 1 || PyTuple_GET_SIZE(dn.p) != E) Py_RETURN_NONE;
   std::vector<const void*> ptrs((size_t)E * 8);

@@ -129,3 +129,33 @@ def test_gradient_of_the_routing_weights(dev, oracle):
             ops.moe_experts(args[0], args[1], torch.autograd.forward_ad.make_dual(w.to(dev), torch.ones(9, 2, device=dev)), *args[2:]))
         alone = ops.moe_experts(args[0], args[1], torch.ones(9, 2, device=dev), *args[2:])
         assert t is not None and float((t - alone).norm() / alone.norm()) <= 1e-3      # the result is linear in the weights
+
+
+def test_collections_that_load_experts_on_demand(dev):
+    """Anything but a plain list or tuple is asked for the experts that some token chose, and for no other."""
+    from htr_amd import ops
+    print("moe: experts on demand", flush=True)
+    gate_up, down = (_to(dev, ws) for ws in _layer(4, 128, 128, 4, 4, 840))
+
+    class OnDemand:
+        def __init__(self, experts):
+            self.experts, self.asked = experts, set()
+
+        def __len__(self):
+            return len(self.experts)
+
+        def __getitem__(self, e):
+            if not 0 <= e < len(self.experts):
+                raise IndexError(e)
+            self.asked.add(e)
+            return self.experts[e]
+
+    x = torch.randn(6, 128, device=dev).bfloat16()
+    ids, w = torch.tensor([[0], [2], [2], [0], [2], [2]], device=dev), torch.rand(6, 1, device=dev)
+    lazy = [OnDemand(gate_up), OnDemand(down)]
+    y = ops.moe_experts(x, ids, w, *lazy)
+    assert all(c.asked == {0, 2} for c in lazy)
+    whole = ops.moe_experts(x, ids, w, gate_up, tuple(down))
+    assert float((whole - y).norm() / y.norm()) <= 1e-3          # the same products, rounded alike
+    with pytest.raises(TypeError):
+        ops.moe_experts(x, ids, w, (t for t in gate_up), (t for t in down))
