@@ -425,14 +425,15 @@ inline int moe_rows_per_entry(int pairs, int experts) {
   return mean <= 16 ? 32 : 64;
 }
 inline bool moe_plan(int tokens, int top, int experts, int hidden, int inter, MoePlan& p) {
-  if (tokens < 1 || top < 1 || experts < 1 || experts > MOE_MAX_EXPERTS || (long)tokens * top > (1L << 24)) return false;
+  if (tokens < 1 || top < 1 || experts < 1 || experts > MOE_MAX_EXPERTS || (long)tokens * top >= (1L << 24)) return false;
   if (!shape_ok(2 * inter, hidden) || !shape_ok(hidden, inter)) return false;
   p.pairs = tokens * top;
   p.rows = moe_rows_per_entry(p.pairs, experts);
   const int active = experts < p.pairs ? experts : p.pairs;
   p.entries = active + p.pairs / p.rows;
   p.tiles = active + p.pairs / 32;
-  if (p.entries > 65535 || hidden / 128 > 65535) return false;
+  // with shape_ok and the pairs, every launch of the layer is within the grid's limits (65535 in y and z, 2^32 threads in x)
+  if (p.entries > 65535) return false;
   size_t o = 0;
   auto take = [&](size_t bytes) { const size_t at = o; o += align256(bytes); return at; };
   p.table = take((size_t)experts * 64);
@@ -505,7 +506,7 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   if (p.rows == 32) { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 1, true>(b2, t2, 1, p.entries, st))); }
   else { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 2, true>(b2, t2, 1, p.entries, st))); }
   if (rc != HTR_OK) return rc;
-  HTR_CHECK_HIP(launch_kernel(k_moe_combine, dim3((hidden / 4 + 255) / 256, tokens), dim3(256), 0, st, (const float*)r.out, (const int*)r.pos_of,
+  HTR_CHECK_HIP(launch_kernel(k_moe_combine, dim3(tokens, (hidden / 4 + 255) / 256), dim3(256), 0, st, (const float*)r.out, (const int*)r.pos_of,
                               weights, top, hidden, y));
   return HTR_OK;
 }

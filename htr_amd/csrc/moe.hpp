@@ -271,7 +271,7 @@ __global__ __launch_bounds__(256) void k_moe_act(const float* __restrict__ h, in
 // y[token] = sum over its slots, ascending; a slot without a valid expert gives NaN
 __global__ __launch_bounds__(256) void k_moe_combine(const float* __restrict__ out, const int* __restrict__ pos_of, const float* __restrict__ wt,
                                                      int top, int H, float* __restrict__ y) {
-  const int token = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
+  const int token = blockIdx.x, c = (blockIdx.y * 256 + threadIdx.x) * 4;      // tokens in x, the grid's only dimension beyond 65535
   if (c >= H) return;
   f4 s = {0.f, 0.f, 0.f, 0.f};
   for (int j = 0; j < top; ++j) {

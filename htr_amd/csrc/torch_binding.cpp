@@ -126,7 +126,8 @@ bool collect(PyObject* experts, int offset, c10::Device dev, Shape& shape, std::
   return true;
 }
 
-// moe(x, ids, weights, gate_up, down, host word address (0: none), ticket, stream) -> float32 [tokens, hidden] or None
+// moe(x, ids, weights, gate_up, down, host word address (0: none), ticket, stream) -> float32 [tokens, hidden], None, or the status of
+// a launch that the runtime refused
 PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs != 8 || f_moe == nullptr) Py_RETURN_NONE;
@@ -172,6 +173,7 @@ PyObject* moe(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                  need, word, ticket, stream);
     }
   }
+  if (rc == HTR_ERR_LAUNCH) return PyLong_FromLong(rc);      // part of the layer may be queued: an error, not another way to run it
   if (rc != HTR_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
   END_HANDLE_TH_ERRORS

@@ -366,6 +366,12 @@ _TICKET_WORDS = 256
 _TICKET_POOLS = {}       # device index -> pinned words in which the routing kernels report expert numbers out of range
 
 
+def _queued(y):
+    if type(y) is int:
+        _native.check(y)
+    return y
+
+
 def _moe_silu(x, expert_ids, expert_weights, gate_up, down):
     """moe_experts with the default activation in one library call; None where the arguments are not as the library wants them."""
     fast = _native.fast()
@@ -374,13 +380,13 @@ def _moe_silu(x, expert_ids, expert_weights, gate_up, down):
     index = x.get_device()
     stream = _raw_stream(index)
     if torch.cuda.is_current_stream_capturing():
-        return fast.moe(x, expert_ids, expert_weights, gate_up, down, 0, 0, stream)
+        return _queued(fast.moe(x, expert_ids, expert_weights, gate_up, down, 0, 0, stream))
     pool = _TICKET_POOLS.get(index)
     if pool is None:
         pool = _TICKET_POOLS.setdefault(index, torch.zeros(_TICKET_WORDS, dtype=torch.int32, pin_memory=True))
     ticket = next(_TICKETS) & 0x7FFFFFFF
     word = pool.data_ptr() + 4 * (ticket % _TICKET_WORDS)
-    y = fast.moe(x, expert_ids, expert_weights, gate_up, down, word, ticket, stream)
+    y = _queued(fast.moe(x, expert_ids, expert_weights, gate_up, down, word, ticket, stream))
     if y is None:
         return None
     # the layer is queued; its first kernel says whether every expert number was valid, while the others still run

@@ -322,3 +322,12 @@ def test_static_workspace_takes_what_fits_it_as_rows(L, m, n, K, M):
     scratch, slots = up(M * n * 2) + up(M * (n // 128) * 16) + up(M * 4), out[1] * M * 512
     if 2 * max(scratch, slots) + 2048 <= _native.STATIC_SCRATCH_BYTES:
         assert 0 < need <= _native.STATIC_SCRATCH_BYTES
+
+
+def test_limits_of_the_routed_expert_layer(L):
+    """Sizes that some launch of the layer could not have as its grid are refused before anything is queued."""
+    need = lambda tokens, top=1, experts=8, hidden=128, inter=128: L.htr_moe_scratch_bytes(tokens, top, experts, hidden, inter)
+    assert need(70000) > 0 and need(70000, top=8) > 0
+    assert need(1, inter=1 << 22) == 0 and need(1, hidden=1 << 23) == 0
+    assert need(4000000) > 0 and need(4 << 20) == 0 and need(1 << 23, experts=4096) == 0 and need(1 << 24) == 0
+    assert need(1, experts=4096) > 0 and need(1, experts=4097) == 0 and need(0) == 0 and need(1, top=0) == 0

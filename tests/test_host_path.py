@@ -145,3 +145,24 @@ def test_interpreter_lock_is_free_during_launches(dev):
     finally:
         _native._fast = None
         _native.fast()
+
+
+@pytest.mark.gpu
+def test_a_refused_launch_of_the_layer_is_an_error(dev):
+    """A status of the runtime from the library's call (here from a function in its place) is raised, and the layer is not run again."""
+    import ctypes
+    from htr_amd import _native, ops
+    print("refused launch", flush=True)
+    module, L = _native.fast(), _native.lib()
+    at = lambda fn: ctypes.cast(fn, ctypes.c_void_p).value
+    res, args = _native.SIGNATURES["htr_moe_experts"]
+    refuse = ctypes.CFUNCTYPE(res, *args)(lambda *a: 8)
+    gate_up, down = [_linear(256, 128, 4, 60, dev)], [_linear(128, 128, 4, 70, dev)]
+    xe, ids, we = torch.randn(5, 128, device=dev).bfloat16(), torch.zeros(5, 1, dtype=torch.int64, device=dev), torch.rand(5, 1, device=dev)
+    module.bind(L.htr_abi_version(), str(torch.__version__), at(L.htr_linear), at(L.htr_stream_capture_id), at(L.htr_moe_scratch_bytes), at(refuse))
+    try:
+        with pytest.raises(RuntimeError, match="status 8"):
+            ops.moe_experts(xe, ids, we, gate_up, down)
+    finally:
+        _native._fast = None
+        _native.fast()

@@ -159,3 +159,13 @@ def test_collections_that_load_experts_on_demand(dev):
     assert float((whole - y).norm() / y.norm()) <= 1e-3          # the same products, rounded alike
     with pytest.raises(TypeError):
         ops.moe_experts(x, ids, w, (t for t in gate_up), (t for t in down))
+
+
+def test_more_than_65535_tokens(dev):
+    """Each token's result is its own: the same bits as in calls of 30000."""
+    from htr_amd import ops
+    print("moe: 70000 tokens", flush=True)
+    gate_up, down = (_to(dev, ws) for ws in _layer(2, 128, 128, 4, 4, 860))
+    x, ids, w = torch.randn(70000, 128, device=dev).bfloat16(), torch.randint(0, 2, (70000, 1), device=dev), torch.rand(70000, 1, device=dev)
+    parts = [ops.moe_experts(x[i:i + 30000], ids[i:i + 30000], w[i:i + 30000], gate_up, down) for i in range(0, 70000, 30000)]
+    assert torch.equal(ops.moe_experts(x, ids, w, gate_up, down), torch.cat(parts))
