@@ -5,6 +5,7 @@ M-based dispatch of _linear_impl, htr/ops.py:69-122), but the body calls the gfx
 through its C ABI: tensors are passed as raw device pointers together with the current
 torch stream; outputs and the workspace are allocated here with torch.
 """
+import collections
 import itertools
 import os
 
@@ -334,6 +335,7 @@ def moe_experts(x, expert_ids, expert_weights, gate_up, down, activation=torch.n
     activation the whole layer is queued by one library call (sorting by expert, rotations, both grouped products, activation
     and weighted sum on the device); another activation runs between two grouped launches, and so does a call whose
     expert_weights take part in differentiation: the result is differentiable in them (not in x, as for every packed linear).
+    An expert number out of range raises IndexError; under graph capture, where nothing can be reported, its token becomes NaN.
     """
     if activation is torch.nn.functional.silu and type(x) is torch.Tensor and x.is_cuda:
         y = _moe_silu(x, expert_ids, expert_weights, gate_up, down)
@@ -361,9 +363,26 @@ def moe_experts(x, expert_ids, expert_weights, gate_up, down, activation=torch.n
     return y
 
 
-_TICKETS = itertools.count(1)
+_TICKETS = itertools.count()
 _TICKET_WORDS = 256
-_TICKET_POOLS = {}       # device index -> pinned words in which the routing kernels report expert numbers out of range
+_FREE_WORDS = {}         # device index -> addresses of pinned words in which a routing kernel may report to the call that took one
+_TICKET_PAGES = []       # what they lie in; kept for good, as many as calls have waited at once
+
+
+def _ticket_page():
+    return torch.zeros(_TICKET_WORDS, dtype=torch.int32, pin_memory=True)
+
+
+def _take_word(index):
+    """A word for one call: no other call uses it until it is given back (append and pop of a deque are atomic)."""
+    free = _FREE_WORDS.setdefault(index, collections.deque())
+    try:
+        return free.pop()
+    except IndexError:
+        page = _ticket_page()
+        _TICKET_PAGES.append(page)
+        free.extend(page.data_ptr() + 4 * i for i in range(1, _TICKET_WORDS))
+        return page.data_ptr()
 
 
 def _queued(y):
@@ -381,20 +400,19 @@ def _moe_silu(x, expert_ids, expert_weights, gate_up, down):
     stream = _raw_stream(index)
     if torch.cuda.is_current_stream_capturing():
         return _queued(fast.moe(x, expert_ids, expert_weights, gate_up, down, 0, 0, stream))
-    pool = _TICKET_POOLS.get(index)
-    if pool is None:
-        pool = _TICKET_POOLS.setdefault(index, torch.zeros(_TICKET_WORDS, dtype=torch.int32, pin_memory=True))
-    ticket = next(_TICKETS) & 0x7FFFFFFF
-    word = pool.data_ptr() + 4 * (ticket % _TICKET_WORDS)
+    word, ticket = _take_word(index), next(_TICKETS) % 0x7FFFFFFF + 1
     y = _queued(fast.moe(x, expert_ids, expert_weights, gate_up, down, word, ticket, stream))
-    if y is None:
-        return None
-    # the layer is queued; its first kernel says whether every expert number was valid, while the others still run
-    bad = fast.wait_word(word, ticket, 2.0)
-    if bad is None:
-        torch.cuda.current_stream(x.device).synchronize()          # a long queue, or a failed launch, which raises here
-        bad = int(pool[ticket % _TICKET_WORDS].item()) & 1
-    if bad:
+    if y is not None:
+        # the layer is queued; its first kernel says whether every expert number was valid, while the others still run
+        bad = fast.wait_word(word, ticket, 2.0)
+        if bad is None:
+            torch.cuda.current_stream(x.device).synchronize()          # a long queue, or a failed launch, which raises here
+            bad = fast.wait_word(word, ticket, 0.0)
+            if bad is None:
+                raise RuntimeError("libhtr_gfx950: the routing kernel has not reported")
+    # given back only where nothing writes to it any more: nothing was queued, or the kernel has reported
+    _FREE_WORDS[index].append(word)
+    if y is not None and bad:
         raise IndexError(f"moe_experts: an expert number is outside 0 .. {len(gate_up) - 1}")
     return y
 

@@ -77,6 +77,61 @@ def test_a_newer_header_makes_the_extension_stale(monkeypatch, tmp_path):
     assert build.is_stale()
 
 
+def _expert_call(monkeypatch, report, waited=None):
+    """ops._moe_silu with a stand-in for the device: `report(word address, ticket)` is what its routing kernel does."""
+    from htr_amd import _native, ops
+    real = _native.fast()
+
+    class Fast:
+        wait_word = staticmethod(lambda word, ticket, seconds: real.wait_word(word, ticket, min(seconds, 0.01)))
+
+        @staticmethod
+        def moe(x, ids, weights, gate_up, down, word, ticket, stream):
+            report(word, ticket)
+            return "queued"
+
+    class Stream:
+        synchronize = staticmethod(lambda: waited.append(1) if waited is not None else None)
+
+    monkeypatch.setattr(_native, "fast", lambda: Fast)
+    monkeypatch.setattr(ops, "_raw_stream", lambda index: 0)
+    monkeypatch.setattr(ops, "_ticket_page", lambda: torch.zeros(ops._TICKET_WORDS, dtype=torch.int32))
+    monkeypatch.setattr(ops, "_FREE_WORDS", {})
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream)
+    return ops._moe_silu(torch.zeros(1, 128), None, None, [1, 2, 3], [1, 2, 3])
+
+
+def _store(word, value):
+    import ctypes
+    ctypes.c_uint32.from_address(word).value = value
+
+
+def test_report_of_the_routing_kernel(monkeypatch):
+    assert _expert_call(monkeypatch, lambda word, ticket: _store(word, ticket << 1)) == "queued"
+    with pytest.raises(IndexError, match="0 .. 2"):
+        _expert_call(monkeypatch, lambda word, ticket: _store(word, ticket << 1 | 1))
+
+
+def test_report_of_another_call_is_not_taken_for_this_one(monkeypatch):
+    """After the wait ran out and the stream was drained, the word has to hold this call's ticket: another one's is an error."""
+    waited = []
+    for low in (0, 1):
+        with pytest.raises(RuntimeError, match="not reported"):
+            _expert_call(monkeypatch, lambda word, ticket: _store(word, (ticket + 256) << 1 | low), waited)
+    assert len(waited) == 2
+
+
+def test_words_of_calls_in_flight_differ(monkeypatch):
+    from htr_amd import ops
+    monkeypatch.setattr(ops, "_ticket_page", lambda: torch.zeros(ops._TICKET_WORDS, dtype=torch.int32))
+    monkeypatch.setattr(ops, "_FREE_WORDS", {})
+    words = [ops._take_word(0) for _ in range(3 * ops._TICKET_WORDS + 5)]
+    assert len(set(words)) == len(words)
+    ops._FREE_WORDS[0].append(words[7])
+    assert ops._take_word(0) == words[7]          # given back, used again: no new page per call
+
+
 @pytest.mark.gpu
 def test_calls_without_the_extension(dev, without_fast):
     """Every call of a stream, not only the first one, which has no workspace yet."""
