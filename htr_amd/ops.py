@@ -398,7 +398,7 @@ def _moe_silu(x, expert_ids, expert_weights, gate_up, down):
         return None
     index = x.get_device()
     stream = _raw_stream(index)
-    if torch.cuda.is_current_stream_capturing():
+    if _native.lib().htr_stream_capture_id(stream) != 0:           # of x's device, which need not be the current one
         return _queued(fast.moe(x, expert_ids, expert_weights, gate_up, down, 0, 0, stream))
     word, ticket = _take_word(index), next(_TICKETS) % 0x7FFFFFFF + 1
     y = _queued(fast.moe(x, expert_ids, expert_weights, gate_up, down, word, ticket, stream))

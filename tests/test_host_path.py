@@ -79,8 +79,8 @@ def test_a_newer_header_makes_the_extension_stale(monkeypatch, tmp_path):
 
 def _expert_call(monkeypatch, report, waited=None):
     """ops._moe_silu with a stand-in for the device: `report(word address, ticket)` is what its routing kernel does."""
+    import htr_amd._fast as real
     from htr_amd import _native, ops
-    real = _native.fast()
 
     class Fast:
         wait_word = staticmethod(lambda word, ticket, seconds: real.wait_word(word, ticket, min(seconds, 0.01)))
@@ -97,7 +97,6 @@ def _expert_call(monkeypatch, report, waited=None):
     monkeypatch.setattr(ops, "_raw_stream", lambda index: 0)
     monkeypatch.setattr(ops, "_ticket_page", lambda: torch.zeros(ops._TICKET_WORDS, dtype=torch.int32))
     monkeypatch.setattr(ops, "_FREE_WORDS", {})
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream)
     return ops._moe_silu(torch.zeros(1, 128), None, None, [1, 2, 3], [1, 2, 3])
 
@@ -120,6 +119,20 @@ def test_report_of_another_call_is_not_taken_for_this_one(monkeypatch):
         with pytest.raises(RuntimeError, match="not reported"):
             _expert_call(monkeypatch, lambda word, ticket: _store(word, (ticket + 256) << 1 | low), waited)
     assert len(waited) == 2
+
+
+def test_capture_is_that_of_the_stream_the_layer_goes_to(monkeypatch):
+    """Not the current device's: a layer on another device than the current one is captured, or not, on its own stream."""
+    from htr_amd import _native
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    asked, given = [], []
+
+    class Lib:
+        htr_stream_capture_id = staticmethod(lambda stream: asked.append(stream) or 7)
+
+    monkeypatch.setattr(_native, "lib", lambda real=_native.lib(): Lib)
+    assert _expert_call(monkeypatch, lambda word, ticket: given.append((word, ticket))) == "queued"
+    assert asked == [0] and given == [(0, 0)]
 
 
 def test_words_of_calls_in_flight_differ(monkeypatch):
