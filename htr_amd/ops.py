@@ -453,15 +453,17 @@ def linear(x, qweight, scales, su, sv, bias=None):
     Under tracing (torch.compile) the call goes through the registered op `htr::linear`, as in the reference
     (htr/ops.py:107-122), and so do tensor subclasses (fake and functional tensors of other tracers); eager calls on
     plain tensors skip the dispatcher, which costs more host time than the launch itself."""
-    if torch.compiler.is_compiling() or type(x) is not torch.Tensor or type(qweight) not in _PLAIN:
-        shp = x.shape
-        y = htr_linear_op(x.reshape(-1, shp[-1]), qweight, scales, su, sv, bias)      # tracing, fake or functional tensors: the registered op
-        return y.reshape(*shp[:-1], qweight.shape[0] * 16)
-    y = _linear_decode(x, qweight, scales, su, sv, bias)
-    if y is not None:
-        return y
+    plain = type(qweight) in _PLAIN and not torch.compiler.is_compiling()
+    if plain and type(x) in _PLAIN:
+        y = _linear_decode(x, qweight, scales, su, sv, bias)
+        if y is not None:
+            return y
     shp = x.shape
-    y = _linear_impl(x.reshape(-1, shp[-1]).contiguous(), qweight, scales, su, sv, bias)
+    x2 = x.reshape(-1, shp[-1])
+    if plain and type(x2) is torch.Tensor:        # also what a parameter or a subclass with plain views gives
+        y = _linear_impl(x2.contiguous(), qweight, scales, su, sv, bias)
+    else:
+        y = htr_linear_op(x2, qweight, scales, su, sv, bias)      # tracing, fake or functional tensors: the registered op
     return y.reshape(*shp[:-1], qweight.shape[0] * 16)
 
 

@@ -77,6 +77,19 @@ def test_a_newer_header_makes_the_extension_stale(monkeypatch, tmp_path):
     assert build.is_stale()
 
 
+@pytest.mark.parametrize("kind", ["tensor", "parameter", "buffer"])
+def test_plain_activations_skip_the_dispatcher(monkeypatch, kind):
+    """A parameter's rows are a plain tensor: the call does not go through the registered op, whose result would ask for a gradient
+    that it cannot give."""
+    from htr_amd import ops, wire
+    w = wire.synth_linear(256, 384, 4, 51)
+    x = torch.randn(2, 3, 384)
+    x = {"tensor": lambda: x, "parameter": lambda: torch.nn.Parameter(x), "buffer": lambda: torch.nn.Buffer(x)}[kind]()
+    monkeypatch.setattr(ops, "htr_linear_op", lambda *a: pytest.fail("through the dispatcher"))
+    monkeypatch.setattr(ops, "_linear_impl", lambda x2, *a: torch.zeros(x2.shape[0], 256))
+    assert ops.linear(x, *w).shape == (2, 3, 256)
+
+
 def _expert_call(monkeypatch, report, waited=None):
     """ops._moe_silu with a stand-in for the device: `report(word address, ticket)` is what its routing kernel does."""
     import htr_amd._fast as real
