@@ -13,6 +13,9 @@ from . import _native, wire
 
 # callable(x[B, 256], w[B, 256], cb[65536], K) -> int64 states [B, 256]; None = the library's search on the GPU
 VITERBI = None
+# bytes of device scratch that one search may take ((T - 2) / C stored arrays per workgroup, C = 4, 3, 2, 1 at K = 2, 3, 4, 5 and more,
+# of (65536 >> K) floats); a smaller limit means more launches of fewer tiles
+MAX_SCRATCH_BYTES = 1 << 30
 _SCRATCH = {}
 _CHECKED_CB = set()          # data pointers of codebook tensors already compared with the procedural codebook
 
@@ -37,21 +40,25 @@ def viterbi(x, w, cb=None, K=4, tailbite=True):
     if w.shape != x.shape or not 1 <= T <= 256:
         raise RuntimeError("viterbi wants x and w of one shape [B, T <= 256]")
     L = _native.lib()
-    if B == 0:
-        return torch.empty((0, T), dtype=torch.int64, device=x.device)
     with torch.cuda.device(x.device):
-        need = L.htr_viterbi_workspace_bytes(B, T, K)
-        if need == 0:
+        per_tile = L.htr_viterbi_workspace_bytes(1, T, K)
+        if per_tile == 0:
             raise RuntimeError(f"viterbi: unsupported K {K} (2..8)")
         out = torch.empty((B, T), dtype=torch.int16, device=x.device)
+        batch = max(1, B)
+        need = L.htr_viterbi_workspace_bytes(batch, T, K)
+        if need > MAX_SCRATCH_BYTES:
+            batch = min(batch, max(1, MAX_SCRATCH_BYTES // per_tile))
+            need = L.htr_viterbi_workspace_bytes(batch, T, K)
         stream = torch.cuda.current_stream(x.device)
         key = (x.device.index, stream.cuda_stream)
         ws = _SCRATCH.get(key)
         if ws is None or ws.numel() < need:
             ws = torch.empty(need, dtype=torch.uint8, device=x.device)
             _SCRATCH[key] = ws
-        _native.check(L.htr_viterbi(x.data_ptr(), w.data_ptr(), B, T, K, 1 if tailbite else 0, out.data_ptr(), ws.data_ptr(),
-                                    ws.numel(), stream.cuda_stream))
+        for b0 in range(0, B, batch):
+            _native.check(L.htr_viterbi(x[b0:].data_ptr(), w[b0:].data_ptr(), min(batch, B - b0), T, K, 1 if tailbite else 0,
+                                        out[b0:].data_ptr(), ws.data_ptr(), ws.numel(), stream.cuda_stream))
     return out.long() & 0xFFFF
 
 

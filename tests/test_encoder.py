@@ -179,6 +179,26 @@ def test_gpu_search_at_the_edges_of_its_trace_back(dev, oracle, K, B, lengths, t
 
 
 @pytest.mark.gpu
+def test_gpu_search_within_a_scratch_limit(dev, oracle, monkeypatch):
+    """MAX_SCRATCH_BYTES bounds the scratch also where it does not hold one workgroup per compute unit; no tiles at all, and a number
+    of bits that is refused whatever the number of tiles."""
+    from htr_amd import _native, encode
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(11, 19, generator=g).to(dev), (torch.rand(11, 19, generator=g) + 0.25).to(dev)
+    want = encode.viterbi(x, w, None, 4)
+    monkeypatch.setattr(encode, "_SCRATCH", {})
+    for tiles in (3, 0):                                              # 3: four launches; 0: less than one tile, one at a time
+        monkeypatch.setattr(encode, "MAX_SCRATCH_BYTES", max(1, tiles * _native.lib().htr_viterbi_workspace_bytes(1, 19, 4)))
+        print(f"viterbi, scratch for {tiles} tiles", flush=True)
+        assert torch.equal(encode.viterbi(x, w, None, 4), want)
+        if tiles:
+            assert max(t.numel() for t in encode._SCRATCH.values()) <= encode.MAX_SCRATCH_BYTES
+    assert encode.viterbi(x[:0], w[:0], None, 4).shape == (0, 19)
+    with pytest.raises(RuntimeError, match="K 9"):
+        encode.viterbi(x[:0], w[:0], None, 9)
+
+
+@pytest.mark.gpu
 def test_gpu_search_refuses_another_codebook(dev):
     from htr_amd import encode, wire
     print("viterbi: codebook check", flush=True)
