@@ -590,7 +590,7 @@ size_t htr_viterbi_workspace_bytes(int64_t tiles, int T, int K) {
   if (tiles <= 0 || T < 1 || T > 256 || K < 2 || K > 8) return 0;
   size_t rows = 0;
   HTR_FOR_K_OR(K, rows = (size_t)vit_rows(T, VitCfg<KK>::C), return 0);
-  return align256(viterbi_grid(tiles) * (rows > 0 ? rows : 1) * (65536u >> K) * sizeof(float));
+  return align256(viterbi_grid(tiles) * (rows > 0 ? rows : 1) * (65536u >> K) * sizeof(float)) + 16;      // 16: any start will do
 }
 
 int htr_viterbi(const void* x, const void* w, int64_t tiles, int T, int K, int tailbite, void* states_u16, void* workspace,
@@ -600,7 +600,8 @@ int htr_viterbi(const void* x, const void* w, int64_t tiles, int T, int K, int t
   if (tiles <= 0 || tiles > 0x7FFFFFFF || T < 1 || T > 256) return HTR_ERR_SHAPE;
   if (((uintptr_t)x & 3) || ((uintptr_t)w & 3) || ((uintptr_t)states_u16 & 1)) return HTR_ERR_ALIGN;
   const size_t need = htr_viterbi_workspace_bytes(tiles, T, K);
-  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15)) return HTR_ERR_WORKSPACE;
+  if (!workspace || workspace_bytes < need) return HTR_ERR_WORKSPACE;
+  workspace = (void*)(((uintptr_t)workspace + 15) & ~(uintptr_t)15);
   hipStream_t st = (hipStream_t)stream;
   const double rms = __builtin_sqrt(MEAN_SQ);
 #define HTR_LAUNCH_VIT(KK_)                                                                                              \

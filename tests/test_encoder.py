@@ -199,6 +199,24 @@ def test_gpu_search_within_a_scratch_limit(dev, oracle, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K", [2, 4, 8])
+def test_gpu_search_with_scratch_at_any_address(dev, K):
+    """The C entry takes the scratch where it is, as it always did; the stored arrays find their own 16-byte boundary in it."""
+    from htr_amd import _native, encode
+    L = _native.lib()
+    g = torch.Generator().manual_seed(6)
+    x, w = torch.randn(5, 21, generator=g).to(dev), (torch.rand(5, 21, generator=g) + 0.25).to(dev)
+    want = encode.viterbi(x, w, None, K)
+    need = L.htr_viterbi_workspace_bytes(5, 21, K)
+    for offset in (1, 8, 15):
+        print(f"viterbi K={K}, scratch {offset} bytes off", flush=True)
+        buf, out = torch.empty(need + offset, dtype=torch.uint8, device=dev), torch.empty(5, 21, dtype=torch.int16, device=dev)
+        _native.check(L.htr_viterbi(x.data_ptr(), w.data_ptr(), 5, 21, K, 1, out.data_ptr(), buf.data_ptr() + offset, need,
+                                    torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(out.long() & 0xFFFF, want)
+
+
+@pytest.mark.gpu
 def test_gpu_search_refuses_another_codebook(dev):
     from htr_amd import encode, wire
     print("viterbi: codebook check", flush=True)
