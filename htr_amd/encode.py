@@ -17,7 +17,22 @@ VITERBI = None
 # of (65536 >> K) floats); a smaller limit means more launches of fewer tiles
 MAX_SCRATCH_BYTES = 1 << 30
 _SCRATCH = {}
-_CHECKED_CB = set()          # data pointers of codebook tensors already compared with the procedural codebook
+# codebook tensors already compared with the procedural codebook: (address, type, shape, strides) -> the tensor and its version.
+# Held, so that no other tensor can come to lie at the address; the last 16 of them.
+_CHECKED_CB = {}
+
+
+def _check_codebook(cb):
+    key = (cb.data_ptr(), cb.dtype, cb.shape, cb.stride())
+    version = None if cb.is_inference() else cb._version
+    known = _CHECKED_CB.get(key)
+    if known is not None and known[1] == version:
+        return
+    if cb.numel() != wire.S or not torch.equal(cb.detach().float().cpu().reshape(-1), wire.codebook_f32("cpu")):
+        raise RuntimeError("viterbi: cb is not the HTR-W1 codebook; the GPU search evaluates that codebook only")
+    for old in list(_CHECKED_CB)[:-15]:
+        _CHECKED_CB.pop(old, None)
+    _CHECKED_CB[key] = (cb, version)
 
 
 def viterbi(x, w, cb=None, K=4, tailbite=True):
@@ -30,10 +45,8 @@ def viterbi(x, w, cb=None, K=4, tailbite=True):
     """
     if not x.is_cuda:
         return viterbi_cpu(x, w, K, tailbite)                       # the reference falls back to its torch search too
-    if cb is not None and cb.data_ptr() not in _CHECKED_CB:
-        if cb.numel() != wire.S or not torch.equal(cb.detach().float().cpu().reshape(-1), wire.codebook_f32("cpu")):
-            raise RuntimeError("viterbi: cb is not the HTR-W1 codebook; the GPU search evaluates that codebook only")
-        _CHECKED_CB.add(cb.data_ptr())
+    if cb is not None:
+        _check_codebook(cb)
     x = x.float().contiguous()
     w = w.float().contiguous()
     B, T = x.shape

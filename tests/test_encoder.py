@@ -179,6 +179,28 @@ def test_gpu_search_at_the_edges_of_its_trace_back(dev, oracle, K, B, lengths, t
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K", range(2, 9))
+@pytest.mark.parametrize("tailbite", [True, False])
+def test_gpu_search_takes_the_first_of_equal_costs(dev, oracle, K, tailbite):
+    """Equal costs in every step (no weight, no target, targets and weights of a few values) and infinite ones, where the trace back's
+    masks decide: the first index, as in the oracle.  Exact."""
+    from htr_amd import encode
+    g = torch.Generator().manual_seed(90 + K)
+    for T in (2, 3, 5, 8, 14):
+        x, w = torch.randn(8, T, generator=g), torch.rand(8, T, generator=g) + 0.25
+        x[0], w[1] = 0.0, 0.0
+        w[2] *= torch.arange(T) % 2
+        x[3], w[3] = x[3].round(), (4 * w[3]).round()
+        x[4], w[4] = 0.0, 1.0
+        x[5, T // 2] = float("inf")
+        w[6, T // 2] = float("inf")
+        x[7] *= 1e20                                                  # every cost overflows
+        print(f"viterbi ties K={K} T={T} tailbite={tailbite}", flush=True)
+        st = encode.viterbi(x.to(dev), w.to(dev), None, K, tailbite=tailbite).cpu().numpy()
+        assert np.array_equal(st.astype(np.uint32), oracle.c_viterbi(x.numpy(), w.numpy(), K, tailbite=tailbite))
+
+
+@pytest.mark.gpu
 def test_gpu_search_within_a_scratch_limit(dev, oracle, monkeypatch):
     """MAX_SCRATCH_BYTES bounds the scratch also where it does not hold one workgroup per compute unit; no tiles at all, and a number
     of bits that is refused whatever the number of tiles."""
@@ -249,3 +271,27 @@ def test_gpu_encoder_round_trip(dev, enc_gold):
     y = ops.linear_f32out(x, *d)
     ref = x @ actual.T
     assert float((y - ref).abs().max() / ref.abs().max()) <= 1e-3
+
+
+def test_codebook_check_is_not_fooled_by_a_reused_address(monkeypatch):
+    """A table that was checked once is known by its memory only while that memory is its own and unchanged."""
+    from htr_amd import encode, wire
+    monkeypatch.setattr(encode, "_CHECKED_CB", {})
+    good = wire.codebook_f32("cpu").clone()
+    encode._check_codebook(good)
+    encode._check_codebook(good)
+    assert len(encode._CHECKED_CB) == 1
+    with pytest.raises(RuntimeError, match="codebook"):
+        encode._check_codebook(good.flip(0).contiguous())
+    good[3] += 1.0                                                    # changed in place
+    with pytest.raises(RuntimeError, match="codebook"):
+        encode._check_codebook(good)
+    address = wire.codebook_f32("cpu").clone()
+    encode._check_codebook(address)
+    held, at = address.untyped_storage().data_ptr(), address.data_ptr()
+    del address
+    others = [torch.zeros(wire.S) for _ in range(8)]                  # would take freed memory of the same size
+    assert all(t.data_ptr() != at for t in others) and held == at
+    for _ in range(40):
+        encode._check_codebook(wire.codebook_f32("cpu").clone())
+    assert len(encode._CHECKED_CB) <= 16
