@@ -55,21 +55,21 @@ __global__ __launch_bounds__(WG_THREADS, JB <= 1 || ONE ? 4 : 2) void k_linear_t
   float* s_fin = (float*)lds;                      // [2][ROWS][TILE_FIN_LD]
   float* s_off = s_fin + 2 * ROWS * TILE_FIN_LD;   // [ROWS] 1534 x sum of the rotated activations over the split
   float* s_sc = s_off + ROWS;                      // [ROWS] activation scale
-  constexpr int OUT_OF_RANGE = 0x7FFFF000;
+  constexpr uint32_t OUT_OF_RANGE = 0x7FFFF000u;     // beyond every descriptor, with all the steps that are added to it
 
   // ---- requests: the first fragments and weights
   const int jbs = (M + 31) >> 5;                   // row tiles that hold rows
   const __amdgpu_buffer_rsrc_t brsrc = __builtin_amdgcn_make_buffer_rsrc((void*)t.xt_g, 0, jbs * 32 * n * 2, 0x00020000);
-  int boff[JB];
+  uint32_t boff[JB];
 #pragma unroll
-  for (int jb = 0; jb < JB; ++jb) boff[jb] = 32 * jb + l32 < M ? ((jb * (n >> 5) + c_begin * 4 + cq) * 2048 + lane * 16) : OUT_OF_RANGE;
+  for (int jb = 0; jb < JB; ++jb) boff[jb] = 32 * jb + l32 < M ? (uint32_t)((jb * (n >> 5) + c_begin * 4 + cq) * 2048 + lane * 16) : OUT_OF_RANGE;
   h8 B[DB][JB][2];
   int b_left = nsteps;
   auto load_b = [&](int set) {                     // fragments of the next step not yet requested
     HTR_PIN();
 #pragma unroll
     for (int jb = 0; jb < JB; ++jb) {
-      const int o = b_left > 0 ? boff[jb] : OUT_OF_RANGE;          // rows beyond M, steps beyond the split: zeros, no traffic
+      const uint32_t o = b_left > 0 ? boff[jb] : OUT_OF_RANGE;          // rows beyond M, steps beyond the split: zeros, no traffic
       B[set][jb][0] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(brsrc, o, 0, 0));
       B[set][jb][1] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(brsrc, o + 1024, 0, 0));
       boff[jb] += 4 * 2048;
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(WG_THREADS, JB <= 1 || ONE ? 4 : 2) void k_linear_t
   const uint32_t* base = qw + ((size_t)(rb * 8) * nblk + (size_t)c_begin) * (STEP_BYTES / 4);
   const __amdgpu_buffer_rsrc_t rsrc =
       __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)(7u * strip_bytes + (uint32_t)nsteps * STEP_BYTES), 0x00020000);
-  int pf_off = (4 * rh + (l32 >> 3)) * (int)strip_bytes + ((2 * cq + kg) * 8 + (lane & 7)) * 4 * K;
+  uint32_t pf_off = (4 * rh + (l32 >> 3)) * strip_bytes + ((2 * cq + kg) * 8 + (lane & 7)) * 4 * K;
   int pf_left = nsteps;
   StreamRegs<K> buf[P];
   auto prefetch = [&](StreamRegs<K>& dst) {
