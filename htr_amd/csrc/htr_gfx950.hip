@@ -482,7 +482,7 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   }
   MoeRoute r;
   r.ids = ids; r.ids64 = ids_int64; r.pairs = p.pairs; r.top = top; r.experts = experts; r.entries = p.entries; r.rows_per_entry = p.rows;
-  r.table = table; r.m1 = 2 * inter; r.n1 = hidden; r.m2 = hidden; r.n2 = inter;
+  r.table = table; r.m1 = 2 * inter; r.m2 = hidden;
   r.e1 = (htr_group_entry*)(base + p.e1); r.e2 = (htr_group_entry*)(base + p.e2);
   r.h = (float*)(base + p.h); r.out = (float*)(base + p.out);
   r.pos_of = (int*)(base + p.pos); r.info = (int4*)(base + p.info);

@@ -14,16 +14,16 @@
 // of 32 rows, 0.53 with two, where k_linear_batch with its staging and barrier takes 0.49 and 0.69), then 6.7 to 8.6 us per
 // launch for launch, first loads, reduction and output side.  32x32x16 instead of 16x16x32 instructions because one of
 // them takes about 6 cycles of vector issue from the other waves for 16 K products, and the smaller one 12 for 8 K.
-// ONE (a single column split: tall matrices, groups that fill the chip, routed experts): two workgroups per compute unit.  A workgroup of 16 steps spends
-// as long on its first loads and its output side as on a third of its steps; 500 tokens over 64 experts, 47 rows each on
-// average, two row tiles: gate/up 130 -> 95 us, down 80 -> 57 us.
+// ONE (a single column split: tall matrices, groups that fill the chip, routed experts): two workgroups per compute unit.  A
+// workgroup of 16 steps spends as long on its first loads and its output side as on a third of its steps; 500 tokens over 64
+// experts, 47 rows each on average, two row tiles: gate/up 130 -> 95 us, down 80 -> 57 us.
 constexpr int FLAG_ENTRY_TILES = 1 << 6;                                    // grouped: an entry's `reserved` is its first row tile
 constexpr int TILE_FIN_LD = 128 + 4;                                        // floats per activation row of the output in LDS
 constexpr size_t tile_lds_bytes(int jb) { return (size_t)2 * 32 * jb * TILE_FIN_LD * 4 + 2 * 32 * jb * 4; }
 
 template <int K, int JB, int P, int DB, bool ONE>
-__global__ __launch_bounds__(WG_THREADS, JB <= 1 || ONE ? 4 : 2) void k_linear_tile(const uint32_t* __restrict__ qw_a, float* __restrict__ part,
-                                                                                    int m, int n, int M_a, int S_a, int flags, const LinearTail t_a) {
+__global__ __launch_bounds__(WG_THREADS, ONE ? 4 : 2) void k_linear_tile(const uint32_t* __restrict__ qw_a, float* __restrict__ part,
+                                                                         int m, int n, int M_a, int S_a, int flags, const LinearTail t_a) {
   extern __shared__ __align__(16) unsigned char lds[];
   const uint32_t* __restrict__ qw = qw_a;
   LinearTail t = t_a;
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(WG_THREADS, JB <= 1 || ONE ? 4 : 2) void k_linear_t
 
   // sums of the rotated activations over the split's columns: 512 / ROWS (a power of two) lanes per row
   {
-    constexpr int LPR = JB == 3 ? 4 : WG_THREADS / ROWS;
+    constexpr int LPR = WG_THREADS / ROWS;
     const int row = (int)threadIdx.x / LPR, sub = (int)threadIdx.x % LPR;
     float v = 0.f;
     if (row < M)

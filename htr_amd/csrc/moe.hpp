@@ -1,7 +1,7 @@
 // Part of htr_gfx950.hip, included inside its anonymous namespace: routing, rotation, activation and combination around the
 // two grouped launches (k_linear_tile) of a routed-expert layer.
 // ------------------------------------------------------------------------------------------------ routed experts
-// One layer is six launches and no copy or synchronisation between them:
+// One layer is seven launches, of which the first comes once per 32 experts, and no copy or synchronisation between them:
 //   k_moe_experts   the experts' tensor addresses, from the kernel arguments to a device table (one launch per 32 experts)
 //   k_moe_route     one workgroup: tokens sorted by expert, the problem tables of both grouped launches
 //   k_moe_rotate    one workgroup per (token, expert) pair: gather, sign, H128, f16, in fragment order
@@ -9,7 +9,7 @@
 //   k_moe_act       one workgroup per pair: silu(gate) * up, rounded to the activations' type, then as k_moe_rotate
 //   k_linear_tile   down, float32
 //   k_moe_combine   y_t = sum_j w_tj out(t, j), j ascending
-// Every entry of the problem tables is one expert and up to ENTRY_ROWS of its pairs; the number of entries is known to the
+// Every entry of the problem tables is one expert and up to rows_per_entry of its pairs; the number of entries is known to the
 // host only as a bound (experts + pairs / rows per entry), entries beyond the used ones have no rows and their workgroups
 // return at once.
 constexpr int MOE_PTR_CHUNK = 32;                 // experts per k_moe_experts launch: 2 KB of kernel arguments
@@ -24,7 +24,7 @@ struct MoeRoute {
   const void* ids;               // [pairs] int32 or int64
   int ids64, pairs, top, experts, entries, rows_per_entry;
   const void* const* table;      // [experts][8]
-  int m1, n1, m2, n2;            // gate_up: [m1, n1], down: [m2, n2]
+  int m1, m2;                    // rows of gate_up and of down
   htr_group_entry* e1;           // [entries]
   htr_group_entry* e2;
   float* h;                      // [pairs][m1]
