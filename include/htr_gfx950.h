@@ -214,7 +214,7 @@ int htr_linear_grouped(const htr_group_entry* entries_device, int count, int m, 
  *   host_word  NULL or a 4-byte word in pinned, device-visible host memory: the first of the launches that looks at the ids
  *            stores (ticket << 1) | (some id is outside 0 .. experts - 1) there; tokens with such an id get NaN
  * [2 inter, hidden] and [hidden, inter] are shapes that htr_linear takes; at most 4096 experts, and 65535 entries of up to 32 rows (64
- * where the experts get more than 16 rows on average): chosen experts + tokens top / rows, about four million pairs.
+ * where the experts get more than 25 rows on average): chosen experts + tokens top / rows, about four million pairs.
  * No counterpart in the reference, which composes routed experts from per-expert linears (docs/ADAPTERS.md:19).
  */
 size_t htr_moe_scratch_bytes(int tokens, int top, int experts, int hidden, int inter);
