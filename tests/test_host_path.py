@@ -247,3 +247,84 @@ def test_a_refused_launch_of_the_layer_is_an_error(dev):
     finally:
         _native._fast = None
         _native.fast()
+
+
+@pytest.mark.gpu
+def test_what_the_extension_leaves_to_the_general_path(dev):
+    """linear(): None, and nothing launched, for every form that is not the plain decode call; the general path then runs it or says
+    what is wrong."""
+    from htr_amd import _native, ops
+    print("ways out of the extension's linear", flush=True)
+    fast = _native.fast()
+    m, n = 256, 384
+    w, x = _linear(m, n, 4, 51, dev), torch.randn(3, n, device=dev).bfloat16()
+    want, bias = ops.linear(x, *w), torch.randn(m, device=dev).bfloat16()
+    stream = ops._raw_stream(0)
+    ws = ops._WORKSPACES[(0, stream)]
+    call = lambda x=x, w=w, bias=None, ptr=ws.ptr, size=ws.size, failed=0: fast.linear(x, *w, bias, ptr, size, failed, stream)
+    assert torch.equal(call(), want) and call(bias=bias) is not None
+    flag = torch.ones(1, dtype=torch.int32)
+    assert call(failed=flag.data_ptr()) is None                                   # an earlier launch gave up
+    assert call(size=256) is None and call(ptr=ws.ptr + 8) is None                # too small, misaligned
+    assert call(bias=bias.float()) is None and call(bias=bias[:-1]) is None and call(bias=bias.cpu()) is None
+    wide = torch.randn(3, 2 * n, device=dev).bfloat16()
+    assert call(x=wide[:, ::2]) is None and call(x=wide) is None and call(x=x.double()) is None and call(x=x.cpu()) is None
+    assert call(x=x[:0]) is None and call(x=x.repeat(43, 1)) is None              # no rows, 129 rows
+    for k, t in enumerate((w[0][:, :, ::2], w[1].float(), w[2][:-1], w[3].cpu())):
+        assert call(w=tuple(t if i == k else o for i, o in enumerate(w))) is None
+    assert torch.equal(ops.linear(x[1], *w), want[1]) and torch.equal(call(x=x[1]), want[1])      # one dimension
+    assert torch.equal(ops.linear(x.reshape(1, 3, 1, n), *w), want.reshape(1, 3, 1, m))
+    strided = torch.stack([x, x], dim=-1)[..., 0]
+    assert not strided.is_contiguous() and torch.equal(ops.linear(strided, *w), want)
+    for wrong in (bias.float(), bias[:-1]):
+        with pytest.raises(RuntimeError, match="bias"):
+            ops.linear(x, *w, wrong)
+
+
+@pytest.mark.gpu
+def test_what_the_extension_leaves_to_the_two_grouped_launches(dev):
+    """moe(): None for more than 4096 experts, experts of several shapes or bits, other index types; the general path runs what it ran."""
+    from htr_amd import _native, ops
+    print("ways out of the extension's expert layer", flush=True)
+    fast, stream = _native.fast(), ops._raw_stream(0)
+    gate_up, down = [_linear(256, 128, 4, 60 + e, dev) for e in range(3)], [_linear(128, 128, 4, 70 + e, dev) for e in range(3)]
+    x, w = torch.randn(6, 128, device=dev).bfloat16(), torch.rand(6, 1, device=dev)
+    ids = torch.tensor([[0], [1], [1], [0], [1], [0]], device=dev)
+    want = ops.moe_experts(x, ids, w, gate_up, down)
+    near = lambda y: float((y - want).norm() / want.norm()) <= 1e-3               # the same products, rounded alike
+    call = lambda ids=ids, w=w, gate_up=gate_up, down=down: fast.moe(x, ids, w, gate_up, down, 0, 0, stream)
+    assert torch.equal(call(), want)
+    many = [gate_up + [gate_up[2]] * 4094, down + [down[2]] * 4094]
+    assert call(gate_up=many[0], down=many[1]) is None and near(ops.moe_experts(x, ids, w, *many))
+    for other in (_linear(512, 128, 4, 80, dev), _linear(256, 128, 3, 80, dev), None):      # an expert that no token chose
+        mixed = [gate_up[0], gate_up[1], other]
+        assert call(gate_up=mixed) is None and near(ops.moe_experts(x, ids, w, mixed, down))
+    with pytest.raises(RuntimeError, match="same m, n and K"):
+        ops.moe_experts(x, ids.clamp(max=1) + 1, w, [gate_up[0], gate_up[1], _linear(256, 128, 3, 80, dev)], down)
+    assert call(ids=ids.short()) is None and near(ops.moe_experts(x, ids.short(), w, gate_up, down))
+    assert call(ids=ids[:5]) is None and call(w=w.long()) is None and call(down=down[:2]) is None
+
+
+@pytest.mark.gpu
+def test_expert_numbers_out_of_range_under_capture(dev):
+    """Nothing can be raised from a replay: such a token is not a number, the others are as without it."""
+    from htr_amd import ops
+    print("bad expert numbers under capture", flush=True)
+    gate_up, down = [_linear(256, 128, 4, 60 + e, dev) for e in range(3)], [_linear(128, 128, 4, 70 + e, dev) for e in range(3)]
+    x, w = torch.randn(6, 128, device=dev).bfloat16(), torch.rand(6, 2, device=dev)
+    good = torch.tensor([[0, 1], [1, 2], [2, 0], [0, 2], [1, 0], [2, 1]], device=dev)
+    want = ops.moe_experts(x, good, w, gate_up, down)
+    ids = good.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.moe_experts(x, ids, w, gate_up, down)
+    for token, bad in ((1, 3), (4, -1), (1, 1 << 40)):
+        ids.copy_(good)
+        ids[token, 1] = bad
+        graph.replay()
+        torch.cuda.synchronize()
+        others = [t for t in range(6) if t != token]
+        assert bool(torch.isnan(y[token]).all()) and torch.equal(y[others], want[others])
+        ids.copy_(good)
+        graph.replay()
+        assert torch.equal(y, want)
