@@ -262,18 +262,20 @@ inline int batch_groups(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 
 //     66.8 / 50.5, K5 64.0 / 61.8, K8 76.8 / 74.0; 40960x1024, 64 rows K4 29.5 / 22.0); 17..32 rows up to K4 (65536x4096, 32 rows
 //     47.8 / 45.5) and, at more bits, whose decode the two workgroups cannot hide behind each other, up to 16 column blocks
 //     (65536x4096, 32 rows K5 52.2 / 56.9, 40960x2048 K5 29.8 / 29.8, 65536x1024 K5 22.5 / 20.5)
-//   up to a quarter of the compute units: its loop without barriers wins from 8 column blocks per split (256x14336, 33 rows K4
-//     19.3 / 18.4, K5 19.7 / 18.7; 512x8192, 64 rows K4 16.1 / 15.8, K8 16.8 / 16.0; 4 blocks: 256x4096, 33 rows K4 12.0 / 12.6)
-//   else up to K4 from 14 column blocks per split (14336x4096, 33 rows K4 21.8 / 20.9; 4096x14336, 33 rows K3 22.1 / 20.8; 11 blocks:
-//     4096x11008, 48 rows K4 19.8 / 21.8; 4 blocks: 4096x4096, 33 rows K4 12.5 / 13.2; 14336x4096, 33 rows K5 22.0 / 22.9)
+//   else up to K4 from 14 column blocks per split (28672x4096, 33 rows K4 33.6 / 30.5; 14336x4096 21.8 / 20.9; 10240x4096 with 11
+//     blocks, 48 rows 19.5 / 20.1, 4096x4096 with 4, 33 rows 12.5 / 13.2; 28672x4096, 64 rows K5 36.5 / 41.5)
+//   and up to two splits: with more, single calls are ahead (4096x14336, eight splits, 33 rows K3 22.1 / 20.8), but whole layers
+//     are not, where the launch follows a larger one.  Graphs of six layers, us, k_linear_batch throughout / k_linear_tile for any
+//     number of splits / for up to two: hidden 4096, inter 14336, 32 rows K3 417.5 / 419.8 / 411.3, K4 422.7 / 429.2 / 417.4, 48
+//     rows K4 538.9 / 534.1 / 525.4; inter 7168, 48 rows K4 431.2 / 428.0 / 428.1; hidden 5120, inter 13824, 32 rows K4 482.5 /
+//     492.9 / 483.9; hidden 1024, inter 14336, 64 rows K5 385.8 / 394.9 (small grids at any K) / 387.4.
 // Beyond 64 rows its loads of the activations bound it (64 KB per step and compute unit at 128 rows, 70 GB/s; 97 rows of
 // 14336x4096 at K5 32.6 / 33.9); up to 16 rows half of its matrix instructions would be empty.
 inline bool tile_takes(int K, int M, int S, int cb, int wgs) {
   if (M < 17 || M > 64) return false;
   const int cus = num_cu();
   if (S == 1 && wgs > cus) return M > 32 || K <= 4 || cb <= 16;
-  if (4 * wgs <= cus) return cb >= 8;
-  return K <= 4 && cb >= 14;
+  return K <= 4 && cb >= 14 && S <= 2;
 }
 inline size_t batch_prerot_rows(int M, bool tile) { return tile ? (size_t)(M + 31) / 32 * 32 : (size_t)M; }   // rows the layout holds
 inline size_t batch_lds_bytes(int M, bool tile) {
@@ -307,7 +309,7 @@ inline bool make_batch_plan(int m, int n, int K, int M, int want_S, BatchPlan& b
   if (bp.tile) {
     // The order for k_linear_tile has room for whole tiles of 32 rows, up to twice what the rows take.  What fits the library's
     // own workspace (htr_linear_static) as rows goes on fitting it, with k_linear_batch; and 32-bit offsets bound it as well.
-    // (An order without gaps, offsets from the rows of the last tile, costs every call 0.2 to 0.4 us: 256x14336, 64 rows K4 19.4 / 19.8.)
+    // (An order without gaps, offsets from the rows of the last tile, costs every call 0.2 to 0.4 us: 28672x4096, 64 rows K4 35.1 / 35.6.)
     const size_t slots = (size_t)bp.wgs * M * 128 * sizeof(float), padded = batch_prerot_rows(M, true);
     if ((padded * n * 2 >> 31) != 0 || (ws_need(slots, prerot_bytes(n, padded)) > HTR_STATIC_SCRATCH_BYTES &&
                                         ws_need(slots, prerot_bytes(n, M)) <= HTR_STATIC_SCRATCH_BYTES)) bp.tile = false;
@@ -431,8 +433,8 @@ template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTa
     // 22.4, 33 rows 152064x4096 137.6 / 115.9; 17 rows 40960x2048 24.0 / 23.6, 32 rows 25.5 / 24.7, 65536x4096 45.4 / 44.9.  Up to one
     // per unit there is no second workgroup to gain from: eight decoder layers of 32 rows at K3, whose gate/up takes 224 workgroups, 558 to 562 / 565 to 571.
     const bool one = bp.S == 1 && bp.wgs > num_cu();
-    if (a.M <= 32) return one ? launch_tile_v<K, 1, true>(a, t, 1, 1, st) : launch_tile_v<K, 1, false>(a, t, bp.S, 1, st);
-    return one ? launch_tile_v<K, 2, true>(a, t, 1, 1, st) : launch_tile_v<K, 2, false>(a, t, bp.S, 1, st);
+    if (one) return a.M <= 32 ? launch_tile_v<K, 1, true>(a, t, 1, 1, st) : launch_tile_v<K, 2, true>(a, t, 1, 1, st);
+    if constexpr (K <= 4) return a.M <= 32 ? launch_tile_v<K, 1, false>(a, t, bp.S, 1, st) : launch_tile_v<K, 2, false>(a, t, bp.S, 1, st);
   }
   switch (bp.mb) {
     case 1: return launch_batch_v<K, 1, false>(a, t, bp, st);

@@ -291,8 +291,9 @@ _TILE_LDS = {1: 2 * 32 * 132 * 4 + 2 * 32 * 4, 2: 2 * 64 * 132 * 4 + 2 * 64 * 4}
     (28672, 4096, 5, 32, False), (28672, 4096, 5, 64, False), (14336, 4096, 6, 48, False), (65536, 4096, 5, 24, False),   # decode-heavy
     (4096, 4096, 4, 33, False), (2048, 2048, 3, 64, False), (1024, 4096, 4, 48, False), (6144, 4096, 2, 64, False),       # few column blocks
     (4096, 11008, 4, 48, False), (10240, 4096, 3, 33, False),
+    (4096, 14336, 3, 32, False), (5120, 13824, 4, 48, False), (256, 14336, 8, 64, False), (8192, 14336, 4, 32, False),   # more than two splits
     (65536, 4096, 5, 33, True), (65536, 4096, 4, 32, True), (40960, 1024, 8, 24, True), (14336, 4096, 4, 33, True),
-    (28672, 4096, 3, 32, True), (4096, 14336, 3, 32, True), (256, 14336, 8, 64, True), (512, 8192, 4, 64, True)])
+    (28672, 4096, 3, 32, True), (28672, 8192, 4, 64, True), (152064, 4096, 6, 64, True), (28672, 2048, 4, 33, True)])
 def test_tile_kernel_only_where_it_is_ahead(L, m, n, K, M, tile):
     """17 to 64 rows that are rotated ahead go to the kernel with tiles of 32 rows only where that one measured faster than the
     staged one (256 compute units): seen by the LDS that the plan asks for."""
@@ -305,10 +306,10 @@ def test_tile_kernel_only_where_it_is_ahead(L, m, n, K, M, tile):
     assert out[4] == 1 and (out[5] == _TILE_LDS[(M + 31) // 32]) == tile, list(out)
 
 
-@pytest.mark.parametrize("m,n", [(128, 30848), (1024, 38016), (128, 49152), (256, 14336), (4096, 14336), (128, 122880)])
+@pytest.mark.parametrize("m,n", [(128, 30848), (1024, 38016), (14336, 30848), (14336, 38016), (28672, 49152), (4096, 14336), (128, 122880)])
 @pytest.mark.parametrize("K,M", [(4, 17), (4, 31), (3, 32), (4, 33), (8, 40), (2, 47), (4, 64)])
 def test_static_workspace_takes_what_fits_it_as_rows(L, m, n, K, M):
-    """The tile kernel's order of the activations rounds the rows up to 32; a call whose M rows of f16, block sums and scales (each
+    """The tile kernel's order of the activations rounds the rows up to 32 (here where its plan takes it, and beside it); a call whose M rows of f16, block sums and scales (each
     rounded up to 256 bytes) fit htr_linear_static's built-in workspace must not be refused for that."""
     from htr_amd import _native
     up = lambda b: (b + 255) // 256 * 256
