@@ -18,6 +18,8 @@
 // Bound: vector issue in the forward passes (K4: 2890 cycles a step, 2944 by the rates above; 0.74 M cycles a pass), then
 // the trace back, 13 % of a tile: with every CU at it, the stored arrays (2 MB a tile) arrive at 5 TB/s.  C: a larger one
 // stores less and recomputes more (K3: C = 2 439 k cycles, C = 3 281 k; K5: C = 1 290 k, C = 2 327 k).
+// Registers: the trace back needs more than the 64 that the codebook values leave, so 8 (K6) to 111 (K7) of a lane's registers, 20
+// at K4, live in scratch, from K3 on outside the forward loop; at K2 (82) the trace back loads about 20 of them every turn.
 // 1024 tiles at K4: 7.46 ms with the table and one byte of backpointer per entry and step, 3.25 ms now; 176 tiles at K3,
 // one per CU: 2.60 -> 0.87 ms.
 // Arithmetic and tie-breaking are the reference's: float32, d = (x - cb)^2, m + w * d without fusing, the first index
