@@ -327,7 +327,7 @@ int htr_linear_static(const void* qweight, const void* scales, const void* su, c
 static bool make_group_plan(int count, int m, int n, int max_M, Plan& pl) {
   const int nblk = n / 128, rbs = m / 128;
   const long vtotal = (long)rbs * nblk;
-  pl.mb = max_M <= 8 ? 1 : (max_M <= 16 ? 2 : 4);
+  pl.mb = max_M <= 8 ? 1 : 2;      // up to 12 rows come here (group_takes_tiles)
   // aim at a few workgroups per CU over all problems; chunks are whole rows of column blocks or divide one, so that
   // no chunk straddles a row block; of those the one nearest the target (in ratio) that fits LDS
   static const int per_cu = getenv("HTR_GROUP_WGS_PER_CU") ? atoi(getenv("HTR_GROUP_WGS_PER_CU")) : 4;

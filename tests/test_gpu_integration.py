@@ -217,6 +217,48 @@ def test_bounded_wait_gives_up_cleanly(dev, oracle, M):
     assert np.array_equal(again, good)
 
 
+def test_bounded_wait_of_a_grouped_launch(dev, oracle):
+    """The same for a group whose problems have column splits: one poll instead of a wait, every kernel runs to its end, what could
+    not be finished is NaN and flagged, the next call clears the workspace and raises, the one after that is right."""
+    from htr_amd import _native, ops
+    print("bounded wait, grouped", flush=True)
+    L = _native.lib()
+    cases = [_case(1024, 4096, 4, M, 4600 + M) for M in (32, 9, 17)]
+    ws = [tuple(t.to(dev) for t in c[:4]) for c in cases]
+    xs = [c[4].to(dev) for c in cases]
+    refs = [_ref(oracle, *c) for c in cases]
+    call = lambda: ops.linear_grouped(xs, ws, out_dtype=torch.float32)
+    good = [y.cpu().numpy() for y in call()]
+    assert all(float(np.abs(y - r).max() / np.abs(r).max()) <= REL_TOL for y, r in zip(good, refs))
+    pending = False
+    try:
+        L.htr_set_spin_limit(1)
+        for _ in range(12):
+            try:
+                ys = call()
+            except RuntimeError as e:
+                assert pending and "gave up" in str(e)
+                pending = False
+                continue
+            assert not pending
+            torch.cuda.synchronize()
+            buf = ops._WORKSPACES[(dev.index, torch.cuda.current_stream(dev).cuda_stream)]
+            bad = [~np.isfinite(y.cpu().numpy()) for y in ys]
+            pending = any(b.any() for b in bad)
+            assert pending == bool(buf.flag[0][0])
+            for y, r, b in zip(ys, refs, bad):
+                blocks = b.reshape(b.shape[0], -1, 128)
+                assert np.all(blocks.all(axis=2) | ~blocks.any(axis=2))         # whole 128-row blocks, never single values
+                if (~b).any():
+                    assert float(np.abs(y.cpu().numpy()[~b] - r[~b]).max() / np.abs(r).max()) <= REL_TOL
+    finally:
+        L.htr_set_spin_limit(1 << 20)
+    if pending:
+        with pytest.raises(RuntimeError):
+            call()
+    assert all(np.array_equal(y.cpu().numpy(), g) for y, g in zip(call(), good))
+
+
 def test_stale_workspace_poisons_later_launches(dev):
     """A workspace whose status word is set (an earlier launch gave up) must not be trusted: a launch on it returns NaN
     everywhere instead of summing whatever the slots hold; htr_workspace_init makes it usable again."""
