@@ -21,6 +21,175 @@ constexpr int FLAG_ENTRY_TILES = 1 << 6;                                    // g
 constexpr int TILE_FIN_LD = 128 + 4;                                        // floats per activation row of the output in LDS
 constexpr size_t tile_lds_bytes(int jb) { return (size_t)2 * 32 * jb * TILE_FIN_LD * 4 + 2 * 32 * jb * 4; }
 
+// ---- output side of a row block for tiles.  What finish_row_block does (same slots, same owners of the activation rows), with
+// four activation rows to a wave, 16 lanes each: lane i holds output rows i, 16 + i, .. 112 + i, so bits 4 to 6 of H128 are
+// additions between its registers; through the row's place in LDS it gets rows 8 i .. 8 i + 7, so bits 0 to 2 are again, bit 3 is
+// a DPP exchange, and the eight results leave in one or two 16-byte stores.  About 28 vector instructions per activation row where
+// one row to a wave, two output rows to a lane, takes 75: there every butterfly stage is an exchange.  Bound: latency of the LDS
+// trips, then vector issue.  500 tokens over 64 experts (2048x1408, K4, two row tiles): gate/up 98 -> 93 us, down 58 -> 54.
+// Row constants come through LDS: 64 groups of four words (scales in the order in which a lane takes them, then biases) and 16
+// sign bytes, a word each.
+struct RowConsts { float* groups; int stride; uint32_t* signs; };           // stride: floats from one group to the next
+__device__ __forceinline__ void place_row_consts(const LinearTail& t, const RowBits& raw, int y_dtype, int lane, const RowConsts& c) {
+  auto cvt_bias = [&](uint32_t b) {
+    return y_dtype == HTR_F32 ? __uint_as_float(b) : y_dtype == HTR_BF16 ? bf16_bits_to_float((uint16_t)b) : f16_bits_to_float((uint16_t)b);
+  };
+  float* rs = c.groups + (lane & 15) * 2 * c.stride + (lane >> 4);          // output row 16 j + i is word 8 i + j
+  rs[0] = f16_bits_to_float((uint16_t)raw.sc0) * t.cbscale * INV_SQRT128;
+  rs[c.stride] = f16_bits_to_float((uint16_t)raw.sc1) * t.cbscale * INV_SQRT128;
+  float* bs = c.groups + (32 + (lane >> 2)) * c.stride + (lane & 3);
+  bs[0] = cvt_bias(raw.b0);
+  bs[16 * c.stride] = cvt_bias(raw.b1);
+}
+__device__ __forceinline__ void place_row_signs(const RowBits& raw, int lane, const RowConsts& c) {
+  if ((lane & 7) == 0) { c.signs[lane >> 3] = raw.sv0; c.signs[8 + (lane >> 3)] = raw.sv1; }
+}
+__device__ __forceinline__ void butterflies8(float (&v)[8]) {               // H8 over the index
+#pragma unroll
+  for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (!(k & h)) { const float a = v[k], b = v[k | h]; v[k] = a + b; v[k | h] = a - b; }
+}
+// eight consecutive values of an output row; 16-byte stores where the output starts on such a boundary
+__device__ __forceinline__ void store8(void* y, int y_dtype, size_t idx, const float (&v)[8]) {
+  if (((uintptr_t)y & 15) == 0) {
+    if (y_dtype == HTR_F32) {
+      HTR_GLOBAL f4* p = (HTR_GLOBAL f4*)((HTR_GLOBAL float*)y + idx);
+      p[0] = f4{v[0], v[1], v[2], v[3]};
+      p[1] = f4{v[4], v[5], v[6], v[7]};
+    } else {
+      typedef float f8 __attribute__((ext_vector_type(8)));
+      const f8 q = {v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+      *(HTR_GLOBAL u4*)((HTR_GLOBAL uint16_t*)y + idx) =
+          y_dtype == HTR_BF16 ? __builtin_bit_cast(u4, __builtin_convertvector(q, b8)) : __builtin_bit_cast(u4, __builtin_convertvector(q, h8));
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) store_elem_g(y, y_dtype, idx + k, v[k]);
+  }
+}
+// s_fin: [activation row][TILE_FIN_LD], with TWO two copies to be added, the second `copy` floats behind the first.  ONE: a single split.
+template <bool ONE, bool TWO>
+__device__ __forceinline__ void finish_tile(const LinearTail& t, void* y, float* __restrict__ part, int rb, int m, int M, const SplitRole& role,
+                                            float* s_fin, int copy, const RowConsts& consts, uint32_t stale, int w, int lane, int y_dtype) {
+  const int S = ONE ? 1 : role.S, s_idx = ONE ? 0 : role.s_idx, RG = (M + 7) >> 3;
+  const bool spread = ONE ? false : role.spread;
+  if (!ONE) {
+    for (int rg = 0, owner = spread ? 0 : S - 1; rg < RG; ++rg, owner = !spread ? owner : (owner + 1 == S ? 0 : owner + 1)) {
+      const int mrow = 8 * rg + w;
+      if (owner != s_idx && mrow < M) {
+        const float* own = s_fin + mrow * TILE_FIN_LD;
+        const float* oth = own + copy;
+        uint32_t* dst = (uint32_t*)(part + (((size_t)rb * S + s_idx) * M + mrow) * 128);
+        __hip_atomic_store(dst + lane, __float_as_uint(TWO ? own[lane] + oth[lane] : own[lane]) | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(dst + lane + 64, __float_as_uint(TWO ? own[lane + 64] + oth[lane + 64] : own[lane + 64]) | 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    if (!role.finisher) return;
+  }
+  const int i = lane & 15;
+  float rs[8], bias[8];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const f4 r = *(const f4*)(consts.groups + (2 * i + h) * consts.stride), b = *(const f4*)(consts.groups + (32 + 2 * i + h) * consts.stride);
+    rs[4 * h] = r.x; rs[4 * h + 1] = r.y; rs[4 * h + 2] = r.z; rs[4 * h + 3] = r.w;
+    bias[4 * h] = b.x; bias[4 * h + 1] = b.y; bias[4 * h + 2] = b.z; bias[4 * h + 3] = b.w;
+  }
+  const uint32_t signs = consts.signs[i];
+  const float s1 = (i & 1) ? -1.f : 1.f;
+  // the o-th activation row that this split finishes; a wave takes rows o, o + 4, o + 8, o + 12 at once, whose places in LDS
+  // are 16 banks apart
+  const int mine = 8 * (spread ? (RG - s_idx + S - 1) / S : RG), o0 = 16 * (w >> 2) + (w & 3) + 4 * (lane >> 4);
+  auto row_of = [&](int o) { return o < mine ? 8 * (spread ? s_idx + (o >> 3) * S : o >> 3) + (o & 7) : M; };
+  // slot of the k-th other split for an activation row
+  auto slot_of = [&](int k, int mrow) { return (uint32_t*)(part + (((size_t)rb * S + k + (k >= s_idx ? 1 : 0)) * M + mrow) * 128) + i; };
+  // the output side of one row; v = the other splits' sum
+  auto finish_row = [&](int mrow, float (&v)[8], bool failed) {
+    float* own = s_fin + mrow * TILE_FIN_LD;
+    const float* oth = own + copy;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (v[j] + (TWO ? own[16 * j + i] + oth[16 * j + i] : own[16 * j + i])) * rs[j];
+    butterflies8(v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) own[16 * j + i] = v[j];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");                    // the row's 16 lanes are in one wave
+    __builtin_amdgcn_wave_barrier();
+    const f4 lo = *(const f4*)(own + 8 * i), hi = *(const f4*)(own + 8 * i + 4);
+    v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
+    butterflies8(v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      butterfly_dpp<1>(v[k], s1);
+      v[k] = __uint_as_float(__float_as_uint(v[k]) ^ ((signs << (31 - k)) & 0x80000000u)) + bias[k];
+      if (failed) v[k] = __builtin_nanf("");
+    }
+    store8(y, y_dtype, (size_t)mrow * m + rb * 128 + 8 * i, v);
+  };
+  if (ONE || S == 1) {
+    for (int o = o0; row_of(o) < M; o += 32) {
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      finish_row(row_of(o), v, stale != 0u);
+    }
+    return;
+  }
+  // With other splits: the slots of up to RB of the wave's rows (JW splits each) are requested together, so that the rows behind
+  // the first cost no memory round trip of their own; repeated (bounded) until every partial is there, summed in fixed order.
+  auto finish_rows = [&](auto jw_c, auto rb_c) {
+    constexpr int JW = decltype(jw_c)::value, RB = decltype(rb_c)::value;
+    for (int o = o0; row_of(o) < M; o += 32 * RB) {
+      float sum[RB][8];
+      bool failed = false;
+      int tries = 0;
+      for (;;) {
+        uint32_t u[RB][JW][8];
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          const int mrow = row_of(o + 32 * r) < M ? row_of(o + 32 * r) : row_of(o);       // beyond the last row: the first again, not looked at
+#pragma unroll
+          for (int k = 0; k < JW; ++k) {
+            const uint32_t* pp = slot_of(min(k, S - 2), mrow);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) u[r][k][j] = __hip_atomic_load(pp + 16 * j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+        bool missing = false;
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          const bool real = row_of(o + 32 * r) < M;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) sum[r][j] = 0.f;
+#pragma unroll
+          for (int k = 0; k < JW; ++k)
+            if (real && k < S - 1)
+#pragma unroll
+              for (int j = 0; j < 8; ++j) { missing |= u[r][k][j] == 0u; sum[r][j] += __uint_as_float(u[r][k][j]); }
+        }
+        if (!__any(missing)) break;
+        if (++tries >= t.spin_limit) { failed = true; break; }
+        __builtin_amdgcn_s_sleep(2);
+      }
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        const int mrow = row_of(o + 32 * r);
+        if (mrow >= M) continue;
+        if (!failed) {                                                        // slots back to zero for the next call
+          for (int k = 0; k < S - 1; ++k) {
+            uint32_t* pp = slot_of(k, mrow);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) __hip_atomic_store(pp + 16 * j, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        } else if (i == 0) {
+          report_give_up(t.status);
+        }
+        finish_row(mrow, sum[r], failed || stale != 0u);
+      }
+    }
+  };
+  if (S == 2) finish_rows(std::integral_constant<int, 1>{}, std::integral_constant<int, 4>{});
+  else if (S <= 4) finish_rows(std::integral_constant<int, 3>{}, std::integral_constant<int, 2>{});
+  else finish_rows(std::integral_constant<int, 7>{}, std::integral_constant<int, 1>{});
+}
 template <int K, int JB, int P, int DB, bool ONE>
 __global__ __launch_bounds__(WG_THREADS, ONE ? 4 : 2) void k_linear_tile(const uint32_t* __restrict__ qw_a, float* __restrict__ part,
                                                                          int m, int n, int M_a, int S_a, int flags, const LinearTail t_a) {
@@ -55,6 +224,8 @@ __global__ __launch_bounds__(WG_THREADS, ONE ? 4 : 2) void k_linear_tile(const u
   float* s_fin = (float*)lds;                      // [2][ROWS][TILE_FIN_LD]
   float* s_off = s_fin + 2 * ROWS * TILE_FIN_LD;   // [ROWS] 1534 x sum of the rotated activations over the split
   float* s_sc = s_off + ROWS;                      // [ROWS] activation scale
+  // row constants of the output side: in the four floats behind each of the 64 JB rows, signs later in the place of s_off
+  const RowConsts consts = {s_fin + 128, TILE_FIN_LD, (uint32_t*)s_off};
   constexpr uint32_t OUT_OF_RANGE = 0x7FFFF000u;     // beyond every descriptor, with all the steps that are added to it
 
   // ---- requests: the first fragments and weights
@@ -79,7 +250,11 @@ __global__ __launch_bounds__(WG_THREADS, ONE ? 4 : 2) void k_linear_tile(const u
   };
   const SplitRole role = ONE ? SplitRole{1, 0, false, true} : split_role(M, S, s_idx, flags);
   RowBits raw = {0u, 0u, 0u, 0u, 0u, 0u};
-  if (role.finisher) load_row_bits(t, y_dtype, rb * 128 + lane, raw);
+  // ONE, one row tile: few rows of many experts.  Up to 8 rows a wave finishes one row by itself, with no trip through LDS: half a
+  // microsecond of the 45 us that both products of 16 tokens over 64 experts take.
+  constexpr bool FEW = ONE && JB == 1;
+  const bool few = FEW && M <= 8;
+  if (role.finisher && (w == 0 || few)) load_row_bits(t, y_dtype, rb * 128 + lane, raw);
   constexpr int STEP_BYTES = 256 * K;
   const uint32_t strip_bytes = (uint32_t)nblk * STEP_BYTES;
   const uint32_t* base = qw + ((size_t)(rb * 8) * nblk + (size_t)c_begin) * (STEP_BYTES / 4);
@@ -166,6 +341,7 @@ __global__ __launch_bounds__(WG_THREADS, ONE ? 4 : 2) void k_linear_tile(const u
   // ---- the four column quarters meet in LDS, in two copies: D[i][j]: lane holds column j = lane % 32 (activation row), register
   // r row i = 8 (r / 4) + 4 kg + r % 4; row i of an A operand is strip 4 rh + i / 8, row pair i % 8, so a lane's values for
   // r = 4 rq .. 4 rq + 3, both parities interleaved, are the 8 consecutive weight rows 64 rh + 16 rq + 8 kg ..
+  if (role.finisher && w == 0 && !few) place_row_consts(t, raw, y_dtype, lane, consts);
   __syncthreads();                                  // s_off, s_sc
   float scl[JB], off[JB];
 #pragma unroll
@@ -189,7 +365,15 @@ __global__ __launch_bounds__(WG_THREADS, ONE ? 4 : 2) void k_linear_tile(const u
         }
       }
     }
+    if (phase == 1 && role.finisher && w == 0 && !few) place_row_signs(raw, lane, consts);      // every wave has its offsets
     __syncthreads();
   }
-  finish_row_block<JB * 4>(t, part, rb, m, M, role, raw, s_fin, TILE_FIN_LD, ROWS * TILE_FIN_LD, lane, lane + 64, w, lane, y_dtype);
+  if constexpr (FEW) {
+    if (few) {
+      finish_row_block<1>(t, part, rb, m, M, role, raw, s_fin, TILE_FIN_LD, ROWS * TILE_FIN_LD, lane, lane + 64, w, lane, y_dtype);
+      return;
+    }
+  }
+  const uint32_t stale = t.status != nullptr ? load_status(t.status) : 0u;     // non-zero: an earlier launch on this workspace gave up
+  finish_tile<ONE, true>(t, t.y, part, rb, m, M, role, s_fin, ROWS * TILE_FIN_LD, consts, stale, w, lane, y_dtype);
 }
