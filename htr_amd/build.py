@@ -11,7 +11,7 @@ import sys
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB = os.path.join(CSRC, "libhtr_gfx950.so")
 SOURCES = [os.path.join(CSRC, "htr_gfx950.hip")]          # one translation unit; the kernels live in the parts it includes
-PARTS = [os.path.join(CSRC, f) for f in ("decode.hpp", "linear.hpp", "linear_batch.hpp", "linear_tile.hpp", "linear_gemm.hpp", "moe.hpp", "dequant.hpp",
+PARTS = [os.path.join(CSRC, f) for f in ("decode.hpp", "linear.hpp", "linear_batch.hpp", "linear_tile.hpp", "linear_gemm.hpp", "linear_wide.hpp", "moe.hpp", "dequant.hpp",
                                          "viterbi.hpp", "anchors.hpp", "plan.hpp")]
 BINDING_SOURCE = os.path.join(CSRC, "torch_binding.cpp")
 BINDING = os.path.join(os.path.dirname(CSRC), "_fast.so")

@@ -41,6 +41,7 @@ namespace {
 #include "linear_batch.hpp"
 #include "linear_tile.hpp"
 #include "linear_gemm.hpp"
+#include "linear_wide.hpp"
 #include "moe.hpp"
 #include "dequant.hpp"
 #include "viterbi.hpp"
@@ -74,6 +75,13 @@ float htr_cbscale(void) { return (float)(1.0 / __builtin_sqrt(MEAN_SQ)); }
 
 size_t htr_workspace_bytes(int m, int n, int K, int M, int nsplit) {
   if (K < 2 || K > 8 || !shape_ok(m, n) || M < 1 || M > HTR_MAX_BATCH) return 0;
+  if (wants_wide(M, nsplit)) {
+    WidePlan wp;
+    if (!make_wide_plan(m, n, M, wide_want_S(nsplit), wp)) return 0;
+    // up to 128 rows a slot per workgroup whatever the plan, as the batched kernel's plans: a workspace for one serves the other
+    const size_t slots = nsplit > 0 ? wide_slot_bytes(m, M, wp) : (size_t)wp.wgs * M * 128 * sizeof(float);
+    return ws_need(slots, prerot_bytes(n, M));
+  }
   if (wants_gemm(M, nsplit)) {
     GemmPlan gp;
     if (!make_gemm_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, gemm_want_jb(nsplit), gp)) return 0;
@@ -96,6 +104,12 @@ int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
   if (K < 2 || K > 8) return HTR_ERR_K;
   if (!shape_ok(m, n)) return HTR_ERR_SHAPE;
   if (M < 1 || M > HTR_MAX_BATCH) return HTR_ERR_BATCH;
+  if (wants_wide(M, nsplit)) {
+    WidePlan wp;
+    if (!make_wide_plan(m, n, M, wide_want_S(nsplit), wp)) return HTR_ERR_SPLIT;
+    out6[0] = wp.cb; out6[1] = wp.wgs; out6[2] = nsplit > 0 ? wp.mtiles : (wp.wgs > num_cu() ? 0 : 1); out6[3] = wp.S; out6[4] = 1; out6[5] = (int)WIDE_LDS;
+    return HTR_OK;
+  }
   if (wants_gemm(M, nsplit)) {
     GemmPlan gp;
     if (!make_gemm_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, gemm_want_jb(nsplit), gp)) return HTR_ERR_SPLIT;
@@ -114,6 +128,13 @@ int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
   if (!make_plan(m, n, M, nsplit, pl)) return HTR_ERR_SPLIT;
   out6[0] = pl.chunk; out6[1] = pl.wgs; out6[2] = pl.segfin; out6[3] = pl.nbl; out6[4] = pl.prerot; out6[5] = (int)pl.lds;
   return HTR_OK;
+}
+
+int htr_linear_route(int m, int n, int K, int M, int x_dtype) {
+  if (K < 2 || K > 8 || !shape_ok(m, n) || M < 1 || M > HTR_MAX_BATCH || !dtype_ok(x_dtype)) return -1;
+  if (M <= HTR_MAX_ROWS_PER_TILE) return 0;
+  WidePlan wp;
+  return make_wide_plan(m, n, M, 0, wp) && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype) ? 1 << 27 : -1;
 }
 
 void htr_set_spin_limit(int polls) { g_spin_limit.store(polls < 1 ? 1 : polls, std::memory_order_relaxed); }
@@ -172,6 +193,24 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
       ((uintptr_t)y & (y_dtype == HTR_F32 ? 3 : 1)) || (bias && ((uintptr_t)bias & (y_dtype == HTR_F32 ? 3 : 1))))
     return HTR_ERR_ALIGN;
   const Together together(workspace);
+  if (wants_wide(M, nsplit)) {
+    WidePlan wp;
+    if (!make_wide_plan(m, n, M, wide_want_S(nsplit), wp)) return HTR_ERR_SPLIT;
+    const size_t need = htr_workspace_bytes(m, n, K, M, nsplit);
+    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
+    LinearTail t = {};
+    t.scales = (const uint16_t*)scales; t.sv = (const uint8_t*)sv; t.bias = bias; t.y = y;
+    place_prerot(t, (unsigned char*)workspace + ws_half(workspace_bytes), n, M);
+    t.status = (uint32_t*)workspace;
+    t.cbscale = htr_cbscale();
+    t.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
+    hipStream_t st = (hipStream_t)stream;
+    HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, (size_t)M));
+    const BatchArgs a = {(const uint32_t*)qweight, (float*)((unsigned char*)workspace + WS_HEADER), nullptr, nullptr, m, n, M,
+                         x_dtype | (y_dtype << 2) | (wp.wgs > num_cu() ? FLAG_LAST_FINISHES : 0)};
+    HTR_FOR_K(K, return launch_wide_k<KK>(a, t, wp, st));
+    return HTR_OK;
+  }
   if (wants_gemm(M, nsplit)) {
     GemmPlan gp;
     if (!make_gemm_plan(m, n, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, gemm_want_jb(nsplit), gp)) return HTR_ERR_SPLIT;
@@ -236,7 +275,7 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     hipStream_t st = (hipStream_t)stream;
     // the workgroups rotate their own activations where the plan allows it (16-bit rows on 16-byte boundaries)
     const bool rot = bp.rot && x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0;
-    if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, bp.tile));
+    if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, bp.tile ? FRAG_FULL : 0));
     BatchArgs ba;
     ba.qw = (const uint32_t*)qweight; ba.part = (float*)((unsigned char*)workspace + WS_HEADER); ba.x = x; ba.su = (const uint8_t*)su;
     ba.m = m; ba.n = n; ba.M = M; ba.flags = x_dtype | (y_dtype << 2) | (bp.last_finishes ? FLAG_LAST_FINISHES : 0);
@@ -383,7 +422,7 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
     hipStream_t st = (hipStream_t)stream;
     const int S = group_tile_splits(count, m, n);
     HTR_CHECK_HIP(launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, max_M, count), dim3(WG_THREADS), 0, st, (const void*)nullptr,
-                                (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries, 0ull, 1));
+                                (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries, 0ull, FRAG_FULL));
     BatchArgs ba = {nullptr, (float*)((unsigned char*)workspace + WS_HEADER), nullptr, nullptr, m, n, max_M, x_dtype | (y_dtype << 2)};
     HTR_FOR_K(K, return (S > 1 ? launch_tile_v<KK, 1, false>(ba, t, S, count, st) : launch_tile_v<KK, 1, true>(ba, t, 1, count, st)));
   }
@@ -409,7 +448,7 @@ int htr_linear_grouped(const htr_group_entry* entries, int count, int m, int n, 
   hipStream_t st = (hipStream_t)stream;
   HTR_CHECK_HIP(launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, max_M, count), dim3(WG_THREADS), 0, st, (const void*)nullptr,
                               (const uint8_t*)nullptr, n, x_dtype, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, entries,
-                              (unsigned long long)pre, 0));
+                              (unsigned long long)pre, (size_t)0));
   HTR_FOR_K(K, return launch_linear_k<KK>(a, true, pl.mb, pl.wgs, pl.lds, st));
   return HTR_OK;
 }

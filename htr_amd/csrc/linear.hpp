@@ -51,9 +51,15 @@ __host__ __device__ inline size_t lds_bytes(int M, int nbl, int segfin) {
 // Order of the rotated activations for k_linear_tile: fragments of 32 rows x 16 columns, 1 KB each, as the lanes of a matrix
 // instruction want them.  Fragment (row tile jt, 32-column unit u, half hf): lane (kg = lane / 32, l32) holds row 32 jt + l32, columns
 // 32 u + 16 kg + 8 hf .. + 7.
-__host__ __device__ inline size_t frag_half(int n, size_t row, int col) {      // half-index of an element in the fragment order
-  const size_t unit = (row >> 5) * (size_t)(n >> 5) + (col >> 5);
-  return ((unit * 2 + ((col >> 3) & 1)) * 64 + ((col >> 4) & 1) * 32 + (row & 31)) * 8 + (col & 7);
+// `rows` = rows of the order: the last tile may hold fewer than 32, and its fragments are that much shorter (no gaps).
+__host__ __device__ inline int frag_tile_rows(size_t row, size_t rows) {       // rows in the tile of `row`
+  const size_t left = rows - (row & ~(size_t)31);
+  return left < 32 ? (int)left : 32;
+}
+constexpr size_t FRAG_FULL = ~(size_t)0;                                       // whole tiles only
+__host__ __device__ inline size_t frag_half(int n, size_t row, int col, size_t rows = FRAG_FULL) {      // half-index of an element in the fragment order
+  const int r = frag_tile_rows(row, rows);
+  return (row >> 5) * 32 * (size_t)n + ((size_t)((col >> 5) * 2 + ((col >> 3) & 1)) * 2 * r + (size_t)(((col >> 4) & 1) * r) + (row & 31)) * 8 + (col & 7);
 }
 
 // power-of-two activation scale 2^e with sqrt(128) * amax / 2^e in (8192, 16384]: |H128 x| / sqrt(128) <= sqrt(128) * max|x|,
@@ -121,7 +127,7 @@ __device__ __forceinline__ void rotate4_mfma(const u4& xr, uint32_t sb, bool is_
 // (n / 512 loads per thread), which is cheaper than a second launch or an exchange between workgroups.
 __global__ __launch_bounds__(WG_THREADS) void k_rotate(const void* __restrict__ x, const uint8_t* __restrict__ su, int n, int x_dtype,
                                                        _Float16* __restrict__ xt_g, float* __restrict__ xs_g, float* __restrict__ sc_g,
-                                                       const htr_group_entry* __restrict__ group, unsigned long long group_stride, int frag) {
+                                                       const htr_group_entry* __restrict__ group, unsigned long long group_stride, size_t frag) {
   __shared__ float s_max[WG_WAVES];
   if (group != nullptr) {                  // grouped: blockIdx.z = problem, outputs shifted by the problem's stride
     const htr_group_entry& ge = group[blockIdx.z];
@@ -201,8 +207,8 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate(const void* __restrict__ 
     va *= inv_sc; vb *= inv_sc;
     fwht128_wave(va, vb, lane);
     const _Float16 ha = (_Float16)(va * INV_SQRT128), hb = (_Float16)(vb * INV_SQRT128);
-    xt_g[frag ? frag_half(n, orow, col + lane) : row + col + lane] = ha;
-    xt_g[frag ? frag_half(n, orow, col + lane + 64) : row + col + lane + 64] = hb;
+    xt_g[frag ? frag_half(n, orow, col + lane, frag) : row + col + lane] = ha;
+    xt_g[frag ? frag_half(n, orow, col + lane + 64, frag) : row + col + lane + 64] = hb;
     // sums of the rounded values: the lane's first element lies in tile lane / 16, its second in tile 4 + lane / 16, so the
     // 16-lane row parity is the tile parity of both, and the two elements are the two halves of the block
     float ea, oa, eb, ob;
@@ -217,7 +223,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate(const void* __restrict__ 
 // seventh of the vector instructions of the butterfly version per block, which shows where the rotation is not just
 // latency: 128 rows of 14336 columns take 8.6 us there.
 __global__ __launch_bounds__(WG_THREADS) void k_rotate_mfma(const void* __restrict__ x, const uint8_t* __restrict__ su, int n, int is_bf16,
-                                                            _Float16* __restrict__ xt_g, float* __restrict__ xs_g, float* __restrict__ sc_g, int frag) {
+                                                            _Float16* __restrict__ xt_g, float* __restrict__ xs_g, float* __restrict__ sc_g, size_t frag) {
   __shared__ uint32_t s_amax[WG_WAVES];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int mrow = blockIdx.y, nblk = n >> 7;
@@ -261,8 +267,8 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate_mfma(const void* __restri
   const int b_o = b0 + gk;                                 // lane (p = lane / 16, j) holds elements 32 a' + 16 h + j of block b0 + p
   const bool live_o = b_o < nblk;
   // element 32 a + 16 h of the lane: row-major, or in fragment order (unit 4 b_o + a, half j / 8, lane 32 h + row % 32, j % 8)
-  HTR_GLOBAL _Float16* dst = (HTR_GLOBAL _Float16*)xt_g + (frag ? frag_half(n, mrow, b_o * 128 + j) : (size_t)mrow * n + b_o * 128 + j);
-  const int step_a = frag ? 1024 : 32, step_h = frag ? 256 : 16;
+  HTR_GLOBAL _Float16* dst = (HTR_GLOBAL _Float16*)xt_g + (frag ? frag_half(n, mrow, b_o * 128 + j, frag) : (size_t)mrow * n + b_o * 128 + j);
+  const int tr = frag ? frag_tile_rows(mrow, frag) : 0, step_a = frag ? 32 * tr : 32, step_h = frag ? 8 * tr : 16;
   float r[2][4];
 #pragma unroll
   for (int h = 0; h < 2; ++h)

@@ -382,6 +382,76 @@ inline int gemm_want_jb(int nsplit) { return nsplit > 0 ? ((nsplit >> 20) & 1 ? 
 // nsplit bit 28: the GEMM kernel with the split in the low bits (0 = its own policy); otherwise from GEMM_MIN_M rows
 inline bool wants_gemm(int M, int nsplit) { return nsplit > 0 ? (nsplit & (1 << 28)) != 0 : M >= GEMM_MIN_M; }
 
+// ---- wide kernel: tiles of 256 activation rows, every tile's column blocks in S splits, the last tile's, which may hold fewer rows,
+// in S_last, while the grid stays within one workgroup per compute unit
+struct WidePlan { int S, S_last, cb, mtiles, wgs; };
+constexpr int WIDE_MAX_SPLITS = 8;
+inline bool split_fits(int nblk, int S) { const int cb = (nblk + S - 1) / S; return S >= 1 && S <= nblk && (nblk + cb - 1) / cb == S; }      // none empty
+// us per column block of a workgroup whose tile holds `rows` rows.  K4, 48 workgroups on the chip: 96 rows 0.76, 128 rows 0.78, 256
+// rows 1.2 (from 129 rows on two waves of a SIMD multiply); exchange between S splits at 128 / 256 rows: 2 / 4.7 for two, 3 / 6.2
+// for four.
+inline double wide_step_us(int rows) { return rows <= 128 ? 0.65 + 0.001 * rows : 0.96 + 0.001 * rows; }
+inline double wide_exchange_us(int rows, int S) { return S == 1 ? 0.0 : (1.0 + 0.25 * S) * (rows <= 128 ? 1.0 : 2.0); }
+inline bool make_wide_plan(int m, int n, int M, int want_S, WidePlan& wp) {
+  const int nblk = n / 128, rbs = m / 128, cus = num_cu();
+  if ((long)M * n * 2 >= (1L << 31) - (1L << 20)) return false;          // 32-bit byte offsets into the rotated activations
+  wp.mtiles = (M + WIDE_ROWS - 1) / WIDE_ROWS;
+  const int rest = M - (wp.mtiles - 1) * WIDE_ROWS;
+  if ((long)rbs * wp.mtiles * WIDE_MAX_SPLITS >= (1L << 31)) return false;
+  double best = 1e30;
+  for (int S = 1; S <= WIDE_MAX_SPLITS; ++S) {
+    if (!split_fits(nblk, S) || (want_S > 0 ? S != want_S : S == 5 || S == 7)) continue;
+    for (int L = 1; L <= WIDE_MAX_SPLITS; ++L) {
+      if (!split_fits(nblk, L) || (want_S > 0 ? L != want_S : L == 5 || L == 7) || (wp.mtiles == 1 && L != S)) continue;
+      const long wgs = (long)rbs * (S * (long)(wp.mtiles - 1) + L);
+      const long rounds = (wgs + cus - 1) / cus;
+      if (want_S == 0 && rounds > 1 && S + L > 2) continue;
+      const double full = wp.mtiles > 1 ? ((nblk + S - 1) / S) * wide_step_us(WIDE_ROWS) + wide_exchange_us(WIDE_ROWS, S) : 0.0;
+      const double part = ((nblk + L - 1) / L) * wide_step_us(rest) + wide_exchange_us(rest, L);
+      const double cost = rounds * (full > part ? full : part) + (S != L ? 2.0 : 0.0);
+      if (cost < best) { best = cost; wp.S = S; wp.S_last = L; wp.cb = (nblk + S - 1) / S; wp.wgs = (int)wgs; }
+    }
+  }
+  return best < 1e30;
+}
+// partial slots of all splits: [workgroup][rows of its tile][128] floats (the last tile's workgroups come last)
+inline size_t wide_slot_bytes(int m, int M, const WidePlan& wp) {
+  if (wp.S == 1 && wp.S_last == 1) return 0;
+  const size_t full = (size_t)(wp.mtiles - 1) * (m / 128) * wp.S * WIDE_ROWS, rest = (size_t)(m / 128) * wp.S_last * (M - (wp.mtiles - 1) * WIDE_ROWS);
+  return (full + rest) * 128 * sizeof(float);
+}
+// The wide kernel: nsplit bit 27, with the split of all tiles in the low bits (0 = its own policy), and by policy from 65 rows to 128.
+// us of the call with its rotation, k_linear_batch / k_linear_wide: 14336x4096 K4 65 rows 32.5 / 26.3, 97 rows 33.7 / 28.4, 128 rows
+// 35.3 / 29.8, K8 38.0 / 31.4 at 97 rows; 4096x14336 K4 65 rows 30.0 / 26.3; 2048x2048 K4 128 rows 16.4 / 16.0; 152064x4096 K4 128 rows
+// 249 / 205; 128x128 65 rows 11.2 / 8.9; the worst are 1024x1024 K5 65 rows 12.5 / 13.1 and K2 to K8 128 rows level.  At 64 rows it is
+// behind (14336x4096 K4 23.9 / 25.7, 2048x2048 11.9 / 13.1).  From 129 rows against k_linear_gemm: 6144x4096 K4 129 rows 32.2 / 24.3, 256
+// rows 40.1 / 29.7, 333 rows 39.8 / 37.1; 14336x4096 256 rows 50.6 / 44.3, 333 rows 76.3 / 60.4, 512 rows 94.9 / 72.4; 4096x14336 256 rows
+// 60.6 / 52.2 (htr_linear_route says who takes it there).
+constexpr int WIDE_MIN_M = 65;
+inline bool wants_wide(int M, int nsplit) {
+  return nsplit > 0 ? (nsplit & (1 << 27)) != 0 : M >= WIDE_MIN_M && M <= HTR_MAX_ROWS_PER_TILE;
+}
+inline int wide_want_S(int nsplit) { return nsplit > 0 ? nsplit & 0xFFFFF : 0; }
+
+// More than 128 rows: the wide kernel, or the weight dequantized and the library's product?  Both in us.  The wide kernel: its plan's
+// steps, or what the matrix units of the whole chip sustain (1.1 PFLOP/s with everything around them, where the grid fills it), and
+// launches, rotation and output.  Dequantization and product: 0.66 us per million weights, the product at 1.45 PFLOP/s, launches;
+// float16 converts the weight once more, and the library's float32 product reaches about a tenth.  Measured / these, K4, bfloat16:
+// wide 6144x4096 129 rows 24.3 / 26, 512 rows 42.9 / 42, 14336x4096 512 rows 72.4 / 73, 4096x4096 512 rows 35.5 / 32; dequantization and
+// product 2048x2048 512 rows 21.6 / 22, 6144x4096 512 rows 52 / 50, 14336x4096 1024 rows 131 / 137, 2048 rows 216 / 221.
+inline double wide_us(int m, int n, int M, const WidePlan& wp) {
+  const int cus = num_cu(), nblk = n / 128, rest = M - (wp.mtiles - 1) * WIDE_ROWS, cb_last = (nblk + wp.S_last - 1) / wp.S_last;
+  const long rounds = (wp.wgs + cus - 1) / cus;
+  const double full = wp.mtiles > 1 ? wp.cb * wide_step_us(WIDE_ROWS) + wide_exchange_us(WIDE_ROWS, wp.S) : 0.0;
+  const double last = cb_last * wide_step_us(rest) + wide_exchange_us(rest, wp.S_last);
+  const double steps = rounds * (full > last ? full : last), units = 2.0 * M * m * n / 1.1e9;
+  return 11.0 + 0.015 * M + (steps > units ? steps : units);
+}
+inline double dequant_us(int m, int n, int M, int x_dtype) {
+  const double weights = (double)m * n;
+  return 16.0 + weights * (x_dtype == HTR_BF16 ? 0.66e-6 : 1.6e-6) + 2.0 * M * weights / (x_dtype == HTR_F32 ? 0.12e9 : 1.45e9);
+}
+
 struct BatchArgs { const uint32_t* qw; float* part; const void* x; const uint8_t* su; int m, n, M, flags; };
 template <int K, int MB, bool ROT> int launch_batch_v(const BatchArgs& a, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
   const size_t lds = balanced_lds_request(bp.lds, bp.wgs);
@@ -399,6 +469,11 @@ template <int K, int JB, bool ONE> int launch_tile_v(const BatchArgs& a, const L
   HTR_CHECK_HIP((allow_full_lds<k_linear_tile<K, JB, P, DB, ONE>>()));
   HTR_CHECK_HIP(launch_kernel(k_linear_tile<K, JB, P, DB, ONE>, dim3(S, a.m / 128, problems), dim3(WG_THREADS), lds, st, a.qw, a.part, a.m, a.n,
                               a.M, S, a.flags, t));
+  return HTR_OK;
+}
+template <int K> int launch_wide_k(const BatchArgs& a, const LinearTail& t, const WidePlan& wp, hipStream_t st) {
+  HTR_CHECK_HIP((allow_full_lds<k_linear_wide<K>>()));
+  HTR_CHECK_HIP(launch_kernel(k_linear_wide<K>, dim3(wp.wgs), dim3(WG_THREADS), WIDE_LDS, st, a.qw, a.part, a.m, a.n, a.M, wp.S, wp.S_last, a.flags, t));
   return HTR_OK;
 }
 // Grouped launches of 9 to 32 rows per problem: column splits while every workgroup of the grid has a compute unit to itself, as
@@ -461,14 +536,14 @@ inline bool wants_batch(int M, int nsplit, int m, int n, int K) {
 
 // Rotation of all rows of x ahead of a linear launch: on the matrix unit for 16-bit rows on 16-byte boundaries, else the
 // butterfly kernel (float32, odd alignments)
-// (frag: in the order k_linear_tile reads)
-inline hipError_t launch_rotation(const void* x, const uint8_t* su, int n, int M, int x_dtype, const LinearTail& t, hipStream_t st, bool frag = false) {
+// (frag: not 0 = in fragment order for that many rows, FRAG_FULL = in whole tiles)
+inline hipError_t launch_rotation(const void* x, const uint8_t* su, int n, int M, int x_dtype, const LinearTail& t, hipStream_t st, size_t frag = 0) {
   static const bool mfma_on = getenv("HTR_ROTATE_MFMA") == nullptr || atoi(getenv("HTR_ROTATE_MFMA")) != 0;
   if (mfma_on && x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0)
     return launch_kernel(k_rotate_mfma, dim3((n / 128 + 4 * WG_WAVES - 1) / (4 * WG_WAVES), M), dim3(WG_THREADS), 0, st, x, su, n,
-                         x_dtype == HTR_BF16 ? 1 : 0, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, frag ? 1 : 0);
+                         x_dtype == HTR_BF16 ? 1 : 0, (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, frag);
   return launch_kernel(k_rotate, dim3((n / 128 + WG_WAVES - 1) / WG_WAVES, M), dim3(WG_THREADS), 0, st, x, su, n, x_dtype,
-                       (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, (const htr_group_entry*)nullptr, 0ull, frag ? 1 : 0);
+                       (_Float16*)t.xt_g, (float*)t.xs_g, (float*)t.sc_g, (const htr_group_entry*)nullptr, 0ull, frag);
 }
 
 #define HTR_FOR_K_OR(K, EXPR, OTHERWISE)   \

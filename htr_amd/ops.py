@@ -25,17 +25,18 @@ GROUP_MAX_M = _native.MAX_GROUP_ROWS      # rows per entry of a grouped launch
 NSPLIT = int(os.environ.get("HTR_NSPLIT", "0"))
 # Above a number of activation rows the weight is dequantized once to the original basis (bf16) and a library GEMM does
 # the product, as the reference does for prefill (HTR_PREFILL="w", htr/ops.py:52-54,89-93); up to it, fused launches
-# run (the reference's HTR_GEMV_LOOP_MAX, htr/ops.py:59-61): up to 128 rows the batched decode kernel; beyond, the
-# fused decode -> matrix-unit kernel in ONE launch (it re-decodes the weight once per 96 activation rows, so it pays while
-# few such tiles cover the input).
-# Measured on MI355X (K4, eager, us; one fused launch incl. its rotation launch / launches of 128 rows / dequantize + GEMM):
-#   14336x4096: 160 rows 44 / 64 / 77, 192 rows 45 / 68 / 81, 256 rows 55 / 81 / 89, 384 rows 93 / 126 / 95, 512 rows 119 / 167 / 102
-#   4096x14336: 160 rows 49 / 60 / 116, 192 rows 52 / 68 / 127, 256 rows 74 / 96 / 95, 384 rows 90 / 139 / 113, 512 rows 113 / 175 / 130
-#   6144x4096:  160 rows 34 / 43 / 48, 192 rows 35 / 49 / 51, 256 rows 42 / 57 / 59, 384 rows 46 / 88 / 54, 512 rows 56 / 113 / 56
-#   4096x4096:  160 rows 31 / 37 / 41, 192 rows 32 / 39 / 44, 256 rows 37 / 47 / 36, 384 rows 41 / 74 / 40, 512 rows 48 / 93 / 44
-# So: one fused launch up to 384 rows on matrices from 4096x4096 up (512 rows where the rows are long, n >= 8192),
-# dequantize beyond (and from 129 rows on smaller matrices, whose dequantization is cheap and which were not measured).
-# HTR_GEMV_LOOP_MAX overrides the row limit for every shape (launches of LAUNCH_MAX_M rows up to it).
+# run (the reference's HTR_GEMV_LOOP_MAX, htr/ops.py:59-61): up to 128 rows the decode kernels; beyond, ONE launch of a kernel that
+# decodes the weight once per tile of activation rows.
+# Which of the two is ahead beyond 128 rows says htr_linear_route, by a model of both (the wide kernel, tiles of 256 rows, against
+# dequantization and product).  The limits below are those of the kernel with tiles of 96 or 128 rows (htr_linear's own policy),
+# which still takes what the wide kernel may not: calls whose derivatives or transforms torch follows go on as they went before it.
+# HTR_GEMV_LOOP_MAX overrides the row limit for every shape (launches of LAUNCH_MAX_M rows up to it) and leaves the wide kernel out.
+# Measured on MI355X (K4, us; one launch with tiles of 96 or 128 rows / wide kernel / dequantize + GEMM, GPU time):
+#   14336x4096: 192 rows 43 / 37 / 85, 256 rows 51 / 44 / 80, 333 rows 76 / 60 / 86, 512 rows 95 / 72 / 94, 1024 rows 186 / 130 / 131
+#   4096x14336: 129 rows 45 / 37 / 79, 256 rows 61 / 52 / 90, 333 rows 75 / 65 / 102, 512 rows 95 / 83 / 118
+#   6144x4096:  129 rows 32 / 24 / 57, 256 rows 40 / 30 / 57, 333 rows 40 / 37 / 51, 512 rows 49 / 43 / 52
+#   4096x4096:  129 rows 29 / 21 / 37, 288 rows 35 / 28 / 38, 512 rows 44 / 36 / 41
+#   2048x2048:  129 rows 23 / 17 / 17, 256 rows 26 / 20 / 20, 512 rows 28 / 24 / 22
 _LOOP_MAX_ENV = os.environ.get("HTR_GEMV_LOOP_MAX")
 GEMV_LOOP_MAX = None if _LOOP_MAX_ENV is None else int(_LOOP_MAX_ENV)
 ONE_LAUNCH = _native.MAX_BATCH
@@ -209,20 +210,51 @@ _NEED = {}       # workspace bytes per (m, n, K, M, nsplit)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
-def _launch(x2, qweight, scales, su, sv, bias, y, m, n, K, out_code):
-    L = _native.lib()
-    M = x2.shape[0]
-    key = (m, n, K, M, NSPLIT)
+def _workspace_need(m, n, K, M, nsplit):
+    key = (m, n, K, M, nsplit)
     need = _NEED.get(key)
     if need is None:
-        need = _NEED[key] = L.htr_workspace_bytes(m, n, K, M, NSPLIT)
+        need = _NEED[key] = _native.lib().htr_workspace_bytes(m, n, K, M, nsplit)
+    return need
+
+
+def _followed(*tensors):
+    """Whether torch follows derivatives or a function transform through one of these: a launch on raw pointers would drop them."""
+    for t in tensors:
+        if t is not None and ((t.requires_grad and torch.is_grad_enabled()) or torch._C._functorch.is_functorch_wrapped_tensor(t)
+                              or torch.autograd.forward_ad._current_level >= 0):
+            return True
+    return False
+
+
+def _wide_route(x2, bias, m, n, K, M, per_launch):
+    """nsplit of one launch of the wide kernel where that is ahead beyond 128 rows, else None."""
+    if M <= _native.MAX_ROWS_PER_TILE or M > LAUNCH_MAX_M or GEMV_LOOP_MAX is not None or NSPLIT != 0 or PREFILL != "w":
+        return None
+    if per_launch == 0 and _followed(x2, bias):
+        return None
+    nsplit = _native.lib().htr_linear_route(m, n, K, M, _DTYPE_CODE[x2.dtype])
+    if nsplit < 0:
+        return None
+    if SHARE_CAPTURE_WORKSPACE and torch.cuda.is_current_stream_capturing():
+        # the shared buffer cannot grow now, and may have been sized for what ran before
+        ws = _WORKSPACES.get((x2.device.index, "shared"))
+        if ws is None or ws.buf.numel() < _workspace_need(m, n, K, M, nsplit):
+            return None
+    return nsplit
+
+
+def _launch(x2, qweight, scales, su, sv, bias, y, m, n, K, out_code, nsplit):
+    L = _native.lib()
+    M = x2.shape[0]
+    need = _workspace_need(m, n, K, M, nsplit)
     if need == 0:
         raise RuntimeError("libhtr_gfx950: no launch plan for this shape / split")
     stream = _raw_stream(x2.device.index)
     ws = workspace(x2.device, stream, need)
     _native.check(L.htr_linear(qweight.data_ptr(), scales.data_ptr(), su.data_ptr(), sv.data_ptr(), x2.data_ptr(),
                                None if bias is None else bias.data_ptr(), y.data_ptr(), m, n, K, M,
-                               _DTYPE_CODE[x2.dtype], out_code, NSPLIT, ws.data_ptr(), ws.numel(), stream))
+                               _DTYPE_CODE[x2.dtype], out_code, nsplit, ws.data_ptr(), ws.numel(), stream))
 
 
 def _linear_impl(x2, qweight, scales, su, sv, bias, out_dtype=None):
@@ -242,7 +274,10 @@ def _linear_impl(x2, qweight, scales, su, sv, bias, out_dtype=None):
             raise RuntimeError("HTR-W1 tensors must be contiguous and on the device of x")
     if bias is not None and (bias.dtype != out_dtype or bias.numel() != m or bias.device != x2.device):
         raise RuntimeError("bias must be [m] in the output dtype on the device of x")
-    per_launch = fused_rows_per_launch(m, n, M)
+    per_launch, nsplit = fused_rows_per_launch(m, n, M), NSPLIT
+    wide = _wide_route(x2, bias, m, n, K, M, per_launch)
+    if wide is not None:
+        per_launch, nsplit = M, wide
     if per_launch == 0 and PREFILL == "rot":
         xr = wire.blk_had_cols_T(x2.float() * wire.unpack_signs(su, n).to(x2.device))
         yr = wire.blk_had_cols_T(xr @ dequant_q(qweight, scales).T) * wire.unpack_signs(sv, m).to(x2.device)
@@ -262,7 +297,7 @@ def _linear_impl(x2, qweight, scales, su, sv, bias, out_dtype=None):
     with torch.cuda.device(x2.device):
         for r0 in range(0, M, per_launch):
             r1 = min(M, r0 + per_launch)
-            _launch(x2[r0:r1], qweight, scales, su, sv, bias, y[r0:r1], m, n, K, code)
+            _launch(x2[r0:r1], qweight, scales, su, sv, bias, y[r0:r1], m, n, K, code, nsplit)
     return y
 
 

@@ -43,9 +43,9 @@ typedef enum {
 /* element type codes; same numbering as the reference's out-dtype map (htr/ops.py:79,94) */
 enum { HTR_BF16 = 0, HTR_F16 = 1, HTR_F32 = 2 };
 
-#define HTR_ABI_VERSION 1      /* what htr_abi_version returns */
+#define HTR_ABI_VERSION 2      /* what htr_abi_version returns */
 #define HTR_MAX_BATCH 2048      /* activation rows one htr_linear launch accepts */
-#define HTR_MAX_ROWS_PER_TILE 128   /* up to here one workgroup holds all rows; beyond, the GEMM kernel works in tiles of 96 or 128 rows */
+#define HTR_MAX_ROWS_PER_TILE 128   /* up to here one workgroup holds all rows; beyond, the GEMM kernel works in tiles of 96 or 128 rows, the wide one of 256 */
 #define HTR_MAX_GROUP_ROWS 32   /* rows per problem of htr_linear_grouped (and of an explicit chunked plan, see nsplit) */
 #define HTR_MAX_GROUP 4096 /* problems one htr_linear_grouped launch accepts */
 
@@ -111,6 +111,8 @@ unsigned long long htr_stream_capture_id(void* stream);
  * own (0: the workgroups rotate their own slices: up to 16 rows over at most 16 column blocks per split, or up to 32 rows
  * over at most 8), dynamic LDS bytes}.  Entries 4 and 5 assume bf16 / f16 activations on a 16-byte boundary; float32 or
  * otherwise aligned activations always take the rotation launch and the staged kernel's LDS layout.
+ * From 65 rows to HTR_MAX_ROWS_PER_TILE the wide kernel runs (tiles of up to 256 activation rows, which share what a workgroup
+ * decodes), out6 as for the batched kernel; with bit 27 of nsplit it takes any row count, and out6[2] is the number of row tiles.
  * With more than HTR_MAX_ROWS_PER_TILE rows the fused decode -> matrix-unit (GEMM) kernel runs: the activations are
  * always rotated by a launch of their own, a workgroup owns one 128-row block of the weight, one tile of 96 or of 128
  * activation rows (the planner takes the height that saves a round of workgroups or allows more splits) and one of S
@@ -124,9 +126,18 @@ unsigned long long htr_stream_capture_id(void* stream);
  * bit 30 set: force the separate rotation launch), or, with bit 29 set, the batched kernel with that many column
  * splits in the low bits (0 = its own policy; up to HTR_MAX_ROWS_PER_TILE rows), or, with bit 28 set, the GEMM kernel
  * with that many column splits in the low bits (0 = its own policy; at most 8; any row count up to HTR_MAX_BATCH) and
- * tiles of 96 (bit 20) or 128 (bit 21) activation rows (neither: its own policy).
+ * tiles of 96 (bit 20) or 128 (bit 21) activation rows (neither: its own policy), or, with bit 27 set, the wide kernel with
+ * that many column splits of every tile in the low bits (0 = its own policy; at most 8; any row count up to HTR_MAX_BATCH).
  */
 int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6);
+
+/*
+ * What is fastest for this call: a value for htr_linear's nsplit (0, or 2^27, the wide kernel, beyond HTR_MAX_ROWS_PER_TILE
+ * rows), or -1: dequantize the weight (htr_dequant_w) and multiply with a library GEMM, which is ahead from a few hundred
+ * rows on small matrices and from about a thousand on large ones; also -1 for arguments that htr_linear refuses.
+ * Reference: the row limit of its fused launches, HTR_GEMV_LOOP_MAX (htr/ops.py:59-61).
+ */
+int htr_linear_route(int m, int n, int K, int M, int x_dtype);
 
 /*
  * Makes every later plan assume a device of `compute_units` compute units with `lds_bytes_per_cu` bytes of LDS each,

@@ -1,0 +1,129 @@
+"""k_linear_wide (65 rows and more) against the oracle: edges of its 32- and 256-row tiles, every K, splits, types and alignments; and who takes a call."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+REL_TOL = 1e-3          # float32 results against decode-then-matmul in float64, max norm; activations are rounded to float16 (2e-4)
+WIDE = 1 << 27
+
+
+def _plan(L, m, n, K, M, nsplit):
+    out = (ctypes.c_int * 6)()
+    return list(out) if L.htr_linear_plan(m, n, K, M, nsplit, out) == 0 else None
+
+
+@pytest.fixture(scope="module")
+def L():
+    from htr_amd import _native
+    return _native.lib()
+
+
+@pytest.mark.parametrize("m,n", [(128, 128), (1024, 4096), (6144, 4096), (14336, 4096), (4096, 14336), (152064, 4096)])
+def test_wide_plan(L, m, n):
+    nblk, rbs = n // 128, m // 128
+    for M in (65, 128, 129, 256, 257, 512, 513, 2048):
+        cb, wgs, tiles, S, prerot, lds = _plan(L, m, n, 4, M, WIDE)
+        assert tiles == -(-M // 256) and prerot == 1 and lds <= 160 * 1024 and 1 <= S <= 8 and cb == -(-nblk // S)
+        last = wgs // rbs - S * (tiles - 1)                                       # splits of the last tile
+        assert wgs == rbs * (S * (tiles - 1) + last) and 1 <= last <= 8 and (wgs <= 256 or S == last == 1)
+        need = L.htr_workspace_bytes(m, n, 4, M, WIDE)
+        assert need >= 256 + M * n * 2 and (S == last == 1 or need >= 2 * rbs * last * (M - 256 * (tiles - 1)) * 512)
+    assert _plan(L, m, n, 4, 128, 0)[3] == _plan(L, m, n, 4, 128, WIDE)[3]         # the policy from 65 rows to 128
+    for want in (1, 2, 3, 8):
+        p = _plan(L, m, n, 4, 300, WIDE | want)
+        assert (p is None) == (want > nblk or -(-nblk // -(-nblk // want)) != want) and (p is None or p[3] == want)
+
+
+def test_route(L):
+    wide = lambda m, n, M, x=0: L.htr_linear_route(m, n, 4, M, x)
+    assert wide(4096, 4096, 128) == 0 and wide(4096, 4096, 129) == WIDE and wide(14336, 4096, 512) == WIDE
+    assert wide(14336, 4096, 2048) == -1 and wide(1024, 1024, 1024) == -1          # dequantize and multiply
+    assert wide(14336, 4096, 2048, 2) == WIDE                                     # float32: the library's product is slow
+    assert wide(4096, 4096, 2049) == -1 and wide(100, 128, 200) == -1 and L.htr_linear_route(128, 128, 9, 200, 0) == -1
+
+
+def _case(m, n, K, M, seed, dtype=torch.bfloat16):
+    from htr_amd import wire
+    qw, sc, su, sv = wire.synth_linear(m, n, K, seed)
+    return (qw, sc, su, sv), torch.randn(M, n, generator=torch.Generator().manual_seed(seed)).to(dtype)
+
+
+def _ref(oracle, w, x, bias=None):
+    qw, sc, su, sv = w
+    y = oracle.c_linear(x.float().numpy(), qw.numpy(), sc.numpy(), su.numpy(), sv.numpy())
+    return y if bias is None else y + bias.double().numpy()
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+@pytest.fixture(scope="module")
+def oracle():
+    from oracle import oracle as o
+    return o
+
+
+# K, rows, m, n, splits of every tile (0: policy), activation type, elements by which x and y are off a 16-byte boundary
+_CASES = [(4, 65, 256, 512, 0, "bf16", 0), (4, 96, 256, 128, 1, "bf16", 0), (4, 127, 256, 384, 3, "f16", 0), (4, 129, 256, 512, 2, "bf16", 0),
+          (4, 255, 128, 1024, 8, "bf16", 0), (4, 256, 256, 256, 2, "bf16", 0), (4, 257, 256, 512, 4, "bf16", 0), (4, 333, 384, 1408, 0, "f16", 0),
+          (4, 513, 128, 640, 5, "bf16", 0), (4, 40, 128, 256, 2, "bf16", 0), (4, 300, 128, 384, 0, "f32", 0), (4, 70, 128, 256, 1, "bf16", 1),
+          (2, 97, 128, 384, 1, "bf16", 0), (3, 160, 128, 256, 2, "bf16", 0), (5, 97, 256, 512, 0, "f16", 0), (6, 200, 128, 384, 3, "bf16", 0),
+          (7, 66, 128, 256, 1, "bf16", 0), (8, 288, 128, 512, 4, "bf16", 0), (4, 2048, 128, 128, 1, "bf16", 0)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,M,m,n,S,xt,off", _CASES)
+def test_wide_kernel(dev, oracle, L, K, M, m, n, S, xt, off):
+    from htr_amd import _native
+    print(f"wide kernel K={K} M={M} {m}x{n} S={S} {xt} off={off}", flush=True)
+    dtype = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[xt]
+    w, x = _case(m, n, K, M, 500 + 7 * K + M, dtype)
+    d = [t.to(dev) for t in w]
+    room = torch.zeros(M * n + off, dtype=dtype, device=dev)
+    xd = room[off:].view(M, n).copy_(x)
+    bias = torch.randn(m, generator=torch.Generator().manual_seed(M))
+    ns = WIDE | S
+    need = L.htr_workspace_bytes(m, n, K, M, ns)
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    ref = _ref(oracle, w, x, bias)
+    code = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+    # float32 results; then those of the activations' type, from an address that allows no wide stores
+    for yt, o, tol in ((torch.float32, 0, REL_TOL), (dtype, off, REL_TOL + (0 if xt == "f32" else 2.0 ** -8 if xt == "bf16" else 2.0 ** -11))):
+        outs = []
+        b = bias.to(yt).to(dev)
+        for _ in range(2):                                                        # again on the same workspace: the slots are clean
+            y = torch.full((M * m + o,), float("nan"), dtype=yt, device=dev)
+            _native.check(L.htr_linear(*[t.data_ptr() for t in d], xd.data_ptr(), b.data_ptr(), y[o:].data_ptr(), m, n, K, M, code[dtype], code[yt], ns,
+                                       ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream))
+            torch.cuda.synchronize()
+            outs.append(y[o:].view(M, m))
+        assert torch.equal(outs[0], outs[1])
+        want = ref if yt == torch.float32 else ref - bias.double().numpy() + b.double().cpu().numpy()
+        err = np.abs(outs[0].double().cpu().numpy() - want).max() / np.abs(want).max()
+        assert err <= tol, (yt, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,M", [(4096, 4096, 65), (4096, 4096, 200), (2048, 2048, 700)])
+def test_rows_beyond_64_through_ops(dev, oracle, m, n, M, monkeypatch):
+    """Both host paths take the same route and give the same result; what torch differentiates goes on being differentiated."""
+    from htr_amd import _native, ops
+    print(f"through ops {m}x{n} M={M}", flush=True)
+    w, x = _case(m, n, 4, M, 77)
+    d, xd = [t.to(dev) for t in w], x.to(dev)
+    ref = _ref(oracle, w, x)
+    first = ops.linear(xd, *d)
+    again = ops.linear(xd, *d)                                                    # with the workspace of the first: in C++
+    monkeypatch.setattr(_native, "_fast", False)
+    assert torch.equal(first, again) and torch.equal(first, ops.linear(xd, *d))
+    wide = _native.lib().htr_linear_route(m, n, 4, M, 0) >= 0
+    # bfloat16 results, and bfloat16 weights where the weight is dequantized
+    assert np.abs(first.double().cpu().numpy() - ref).max() / np.abs(ref).max() <= (REL_TOL + 2.0 ** -8 if wide else 2.0 ** -6)
+    monkeypatch.setattr(_native, "_fast", None)
+    leaf = xd.clone().requires_grad_()
+    y = ops.linear(leaf, *d)
+    assert y.requires_grad == (M > 128 and ops.fused_rows_per_launch(m, n, M) == 0)
