@@ -31,7 +31,7 @@ SIGNATURES = {
     "htr_cbscale": (ctypes.c_float, []),
     "htr_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "htr_linear_plan": (_i, [_i, _i, _i, _i, _i, ctypes.POINTER(ctypes.c_int)]),
-    "htr_linear_route": (_i, [_i, _i, _i, _i, _i]),
+    "htr_linear_route": (_i, [_i, _i, _i, _i, _i, _i]),
     "htr_plan_device_override": (_i, [_i, ctypes.c_long]),
     "htr_linear": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "htr_linear_static": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp]),
@@ -85,7 +85,8 @@ def fast():
         try:
             module = importlib.import_module("._fast", __package__)
             module.bind(L.htr_abi_version(), str(torch.__version__), address(L.htr_linear), address(L.htr_stream_capture_id),
-                        address(L.htr_moe_scratch_bytes), address(L.htr_moe_experts))
+                        address(L.htr_moe_scratch_bytes), address(L.htr_moe_experts),
+                        address(L.htr_linear_route), address(L.htr_dequant_w))
         except ImportError as e:
             warnings.warn(f"htr_amd/_fast.so cannot be used ({e}): launches are prepared in Python; `python -m htr_amd.build` builds it",
                           RuntimeWarning, stacklevel=2)

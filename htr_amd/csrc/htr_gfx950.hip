@@ -130,11 +130,11 @@ int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
   return HTR_OK;
 }
 
-int htr_linear_route(int m, int n, int K, int M, int x_dtype) {
+int htr_linear_route(int m, int n, int K, int M, int x_dtype, int eager) {
   if (K < 2 || K > 8 || !shape_ok(m, n) || M < 1 || M > HTR_MAX_BATCH || !dtype_ok(x_dtype)) return -1;
   if (M <= HTR_MAX_ROWS_PER_TILE) return 0;
   WidePlan wp;
-  return make_wide_plan(m, n, M, 0, wp) && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype) ? 1 << 27 : -1;
+  return make_wide_plan(m, n, M, 0, wp) && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype, eager != 0) ? 1 << 27 : -1;
 }
 
 void htr_set_spin_limit(int polls) { g_spin_limit.store(polls < 1 ? 1 : polls, std::memory_order_relaxed); }

@@ -447,9 +447,13 @@ inline double wide_us(int m, int n, int M, const WidePlan& wp) {
   const double steps = rounds * (full > last ? full : last), units = 2.0 * M * m * n / 1.1e9;
   return 11.0 + 0.015 * M + (steps > units ? steps : units);
 }
-inline double dequant_us(int m, int n, int M, int x_dtype) {
+// eager: not from a graph; the host then takes 25 us to queue a dequantization and torch's product (1024x1024 and 4096x1024, 129 to 1024
+// rows, 25.4 to 26.1), and 8 for a wide launch, and where the GPU takes longer the call is still 3 us behind the graph (3072x3072 512
+// rows 32.3 / 34.9).
+inline double dequant_us(int m, int n, int M, int x_dtype, bool eager) {
   const double weights = (double)m * n;
-  return 16.0 + weights * (x_dtype == HTR_BF16 ? 0.66e-6 : 1.6e-6) + 2.0 * M * weights / (x_dtype == HTR_F32 ? 0.12e9 : 1.45e9);
+  const double gpu = 16.0 + weights * (x_dtype == HTR_BF16 ? 0.66e-6 : 1.6e-6) + 2.0 * M * weights / (x_dtype == HTR_F32 ? 0.12e9 : 1.45e9);
+  return !eager ? gpu : gpu < 22.0 ? 25.0 : gpu + 3.0;
 }
 
 struct BatchArgs { const uint32_t* qw; float* part; const void* x; const uint8_t* su; int m, n, M, flags; };

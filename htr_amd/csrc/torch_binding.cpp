@@ -24,8 +24,9 @@ decltype(&htr_linear) f_linear = nullptr;
 decltype(&htr_stream_capture_id) f_capture = nullptr;
 decltype(&htr_moe_scratch_bytes) f_moe_bytes = nullptr;
 decltype(&htr_moe_experts) f_moe = nullptr;
+decltype(&htr_linear_route) f_route = nullptr;
+decltype(&htr_dequant_w) f_dequant = nullptr;
 
-constexpr int MAX_ROWS = HTR_MAX_ROWS_PER_TILE;      // rows of one decode launch
 
 int dtype_code(at::ScalarType t) {
   switch (t) {
@@ -64,12 +65,14 @@ bool weight_ok(const at::Tensor& qw, const at::Tensor& sc, const at::Tensor& su,
   return true;
 }
 
-// linear(x, qweight, scales, su, sv, bias, workspace address, its bytes, address of its failure word (0: none), stream)
-// -> tensor or None; None also while the stream is being captured (a capture has workspaces of its own) and after a launch
-// on the workspace gave up
+// linear(x, qweight, scales, su, sv, bias, workspace address, its bytes, address of its failure word (0: none), stream, rows)
+// -> tensor or None; None also while the stream is being captured (a capture has workspaces of its own), after a launch
+// on the workspace gave up, and for more activation rows than `rows` (if not
+// given 128).  Beyond 128 rows the call goes where the library says:
+// one launch, or the weight dequantized and multiplied by torch, as ops._linear_impl does it.
 PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
-  if (nargs != 10 || f_linear == nullptr || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
+  if (nargs < 10 || nargs > 11 || f_linear == nullptr || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
   const at::Tensor* t[6];
   for (int i = 0; i < 6; ++i) t[i] = args[i] == Py_None ? nullptr : tensor_of(args[i]);
   for (int i = 0; i < 5; ++i) if (t[i] == nullptr) Py_RETURN_NONE;
@@ -80,14 +83,21 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (code < 0 || !x.is_cuda() || x.dim() < 1 || !x.is_contiguous() || !weight_ok(*t[1], *t[2], *t[3], *t[4], x.device(), s)) Py_RETURN_NONE;
   if (x.size(-1) != s.n) Py_RETURN_NONE;
   const int64_t M = x.numel() / s.n;
-  if (M < 1 || M > MAX_ROWS) Py_RETURN_NONE;
   if (t[5] != nullptr && (t[5]->scalar_type() != x.scalar_type() || t[5]->numel() != s.m || t[5]->device() != x.device() || !t[5]->is_contiguous()))
     Py_RETURN_NONE;
   void* ws = PyLong_AsVoidPtr(args[6]);
   const size_t bytes = PyLong_AsSize_t(args[7]);
   const volatile int* failed = (const volatile int*)PyLong_AsVoidPtr(args[8]);
   void* stream = PyLong_AsVoidPtr(args[9]);
+  const long rows = nargs > 10 && f_route != nullptr && f_dequant != nullptr ? PyLong_AsLong(args[10]) : HTR_MAX_ROWS_PER_TILE;
   if (PyErr_Occurred()) return nullptr;
+  if (M < 1 || M > rows) Py_RETURN_NONE;
+  int route = 0;
+  if (M > HTR_MAX_ROWS_PER_TILE) {
+    // torch's product can be differentiated and transformed, a launch on raw pointers cannot: the general path tells them apart
+    if (M > HTR_MAX_BATCH || !raw_ok(x) || differentiable(x) || (t[5] != nullptr && (!raw_ok(*t[5]) || differentiable(*t[5])))) Py_RETURN_NONE;
+    route = f_route((int)s.m, (int)s.n, (int)s.K, (int)M, code, 1);
+  }
   if ((failed != nullptr && *failed != 0) || f_capture(stream) != 0) Py_RETURN_NONE;
   at::Tensor y;
   int rc;
@@ -95,12 +105,22 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // other threads run meanwhile: a launch waits where the stream's queue is full.  The caller's frame holds the tensors.
     pybind11::gil_scoped_release no_lock;
     c10::DeviceGuard guard(x.device());
-    at::DimVector shape(x.sizes().begin(), x.sizes().end());
-    shape.back() = s.m;
-    y = at::empty(shape, x.options());
-    rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
-                  t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, 0,
+    if (route < 0) {
+      at::Tensor w = at::empty({s.m, s.n}, x.options().dtype(at::kBFloat16));
+      rc = f_dequant(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), w.mutable_data_ptr(),
+                     (int)s.m, (int)s.n, (int)s.K, stream);
+      if (rc == HTR_OK) {
+        y = at::linear(x, code == 0 ? w : w.to(x.scalar_type()), t[5] == nullptr ? std::optional<at::Tensor>() : std::optional<at::Tensor>(*t[5]));
+        if (y.scalar_type() != x.scalar_type()) y = y.to(x.scalar_type());      // autocast
+      }
+    } else {
+      at::DimVector shape(x.sizes().begin(), x.sizes().end());
+      shape.back() = s.m;
+      y = at::empty(shape, x.options());
+      rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
+                  t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, route,
                   ws, bytes, stream);
+    }
   }
   if (rc != HTR_OK) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(y));
@@ -202,18 +222,19 @@ PyObject* wait_word(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // bind(version of the library's C ABI, version of the running torch, addresses of htr_linear, htr_stream_capture_id,
-// htr_moe_scratch_bytes and htr_moe_experts); ImportError where either version is not the one that this file was compiled with
+// htr_moe_scratch_bytes, htr_moe_experts and, for linear() beyond 128 rows, htr_linear_route and htr_dequant_w); ImportError where either version is not the one that this file was compiled with
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  if (nargs != 6) { PyErr_SetString(PyExc_TypeError, "bind wants two versions and four addresses"); return nullptr; }
+  if (nargs != 6 && nargs != 8) { PyErr_SetString(PyExc_TypeError, "bind wants two versions and four or six addresses"); return nullptr; }
   const long abi = PyLong_AsLong(args[0]);
   const char* torch_version = PyUnicode_AsUTF8(args[1]);
-  void* p[4];
-  for (int i = 0; i < 4; ++i) p[i] = PyLong_AsVoidPtr(args[2 + i]);
+  void* p[6] = {};
+  for (int i = 0; i < nargs - 2; ++i) p[i] = PyLong_AsVoidPtr(args[2 + i]);
   if (PyErr_Occurred()) return nullptr;
   if (abi != HTR_ABI_VERSION) return PyErr_Format(PyExc_ImportError, "compiled for version %d of the library's C ABI, not %ld", HTR_ABI_VERSION, abi);
   if (strcmp(torch_version, HTR_BUILD_TORCH) != 0) return PyErr_Format(PyExc_ImportError, "compiled for torch %s, not %s", HTR_BUILD_TORCH, torch_version);
   f_linear = (decltype(f_linear))p[0]; f_capture = (decltype(f_capture))p[1];
   f_moe_bytes = (decltype(f_moe_bytes))p[2]; f_moe = (decltype(f_moe))p[3];
+  f_route = (decltype(f_route))p[4]; f_dequant = (decltype(f_dequant))p[5];
   Py_RETURN_NONE;
 }
 

@@ -233,10 +233,11 @@ def _wide_route(x2, bias, m, n, K, M, per_launch):
         return None
     if per_launch == 0 and _followed(x2, bias):
         return None
-    nsplit = _native.lib().htr_linear_route(m, n, K, M, _DTYPE_CODE[x2.dtype])
+    capturing = torch.cuda.is_current_stream_capturing()
+    nsplit = _native.lib().htr_linear_route(m, n, K, M, _DTYPE_CODE[x2.dtype], 0 if capturing else 1)
     if nsplit < 0:
         return None
-    if SHARE_CAPTURE_WORKSPACE and torch.cuda.is_current_stream_capturing():
+    if SHARE_CAPTURE_WORKSPACE and capturing:
         # the shared buffer cannot grow now, and may have been sized for what ran before
         ws = _WORKSPACES.get((x2.device.index, "shared"))
         if ws is None or ws.buf.numel() < _workspace_need(m, n, K, M, nsplit):
@@ -467,8 +468,8 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _linear_decode(x, qweight, scales, su, sv, bias):
-    """The common case of linear() in C++: up to 128 contiguous rows on a stream that has a workspace already.  None where
-    something else is asked for, or is wrong: the general path then runs, or raises."""
+    """The common case of linear() in C++: contiguous rows on a stream that has a workspace already, if one is needed.  None where something
+    else is asked for, or is wrong: the general path then runs, or raises."""
     if NSPLIT != 0 or GEMV_LOOP_MAX is not None or LAUNCH_MAX_M < _native.MAX_ROWS_PER_TILE or SHARE_CAPTURE_WORKSPACE:
         return None
     index = x.get_device()
@@ -477,9 +478,12 @@ def _linear_decode(x, qweight, scales, su, sv, bias):
     stream = _raw_stream(index)
     ws = _WORKSPACES.get((index, stream))
     fast = _native.fast()
-    if ws is None or fast is None:
+    if fast is None:
         return None
-    return fast.linear(x, qweight, scales, su, sv, bias, ws.ptr, ws.size, ws.flag_ptr, stream)
+    rows = LAUNCH_MAX_M if PREFILL == "w" else _native.MAX_ROWS_PER_TILE
+    if ws is None:         # dequantization and product need none
+        return fast.linear(x, qweight, scales, su, sv, bias, 0, 0, 0, stream, rows) if rows > _native.MAX_ROWS_PER_TILE else None
+    return fast.linear(x, qweight, scales, su, sv, bias, ws.ptr, ws.size, ws.flag_ptr, stream, rows)
 
 
 def linear(x, qweight, scales, su, sv, bias=None):

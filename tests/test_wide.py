@@ -37,11 +37,12 @@ def test_wide_plan(L, m, n):
 
 
 def test_route(L):
-    wide = lambda m, n, M, x=0: L.htr_linear_route(m, n, 4, M, x)
+    wide = lambda m, n, M, x=0, eager=0: L.htr_linear_route(m, n, 4, M, x, eager)
     assert wide(4096, 4096, 128) == 0 and wide(4096, 4096, 129) == WIDE and wide(14336, 4096, 512) == WIDE
     assert wide(14336, 4096, 2048) == -1 and wide(1024, 1024, 1024) == -1          # dequantize and multiply
+    assert wide(512, 512, 512) == -1 and wide(512, 512, 512, eager=1) == WIDE      # where the host's time counts
     assert wide(14336, 4096, 2048, 2) == WIDE                                     # float32: the library's product is slow
-    assert wide(4096, 4096, 2049) == -1 and wide(100, 128, 200) == -1 and L.htr_linear_route(128, 128, 9, 200, 0) == -1
+    assert wide(4096, 4096, 2049) == -1 and wide(100, 128, 200) == -1 and L.htr_linear_route(128, 128, 9, 200, 0, 1) == -1
 
 
 def _case(m, n, K, M, seed, dtype=torch.bfloat16):
@@ -120,7 +121,7 @@ def test_rows_beyond_64_through_ops(dev, oracle, m, n, M, monkeypatch):
     again = ops.linear(xd, *d)                                                    # with the workspace of the first: in C++
     monkeypatch.setattr(_native, "_fast", False)
     assert torch.equal(first, again) and torch.equal(first, ops.linear(xd, *d))
-    wide = _native.lib().htr_linear_route(m, n, 4, M, 0) >= 0
+    wide = _native.lib().htr_linear_route(m, n, 4, M, 0, 1) >= 0
     # bfloat16 results, and bfloat16 weights where the weight is dequantized
     assert np.abs(first.double().cpu().numpy() - ref).max() / np.abs(ref).max() <= (REL_TOL + 2.0 ** -8 if wide else 2.0 ** -6)
     monkeypatch.setattr(_native, "_fast", None)
