@@ -515,13 +515,18 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   unsigned char* base = (unsigned char*)scratch;
   hipStream_t st = (hipStream_t)stream;
   const void** table = (const void**)(base + p.table);
-  for (int e0 = 0; e0 < experts; e0 += MOE_PTR_CHUNK) {
-    MoePtrs ptrs;
-    const int count = experts - e0 < MOE_PTR_CHUNK ? experts - e0 : MOE_PTR_CHUNK;
+  MoePtrs ptrs;
+  auto addresses = [&](int e0, int count) {
     memcpy(&ptrs, tensors + (size_t)e0 * 8, (size_t)count * 64);
     memset((unsigned char*)&ptrs + (size_t)count * 64, 0, sizeof(ptrs) - (size_t)count * 64);
-    HTR_CHECK_HIP(launch_kernel(k_moe_experts, dim3(1), dim3(256), 0, st, ptrs, table, e0, count));
+  };
+  const bool given = experts <= MOE_PTR_CHUNK;                    // the routing kernel takes the addresses itself
+  for (int e0 = 0; !given && e0 < experts; e0 += MOE_PTR_CHUNK) {
+    const int count = experts - e0 < MOE_PTR_CHUNK ? experts - e0 : MOE_PTR_CHUNK;
+    addresses(e0, count);
+    HTR_CHECK_HIP(launch_kernel(k_moe_experts, dim3(1), dim3(MOE_PTR_CHUNK * 8), 0, st, ptrs, table, e0, count));
   }
+  addresses(0, given ? experts : 0);
   MoeRoute r;
   r.ids = ids; r.ids64 = ids_int64; r.pairs = p.pairs; r.top = top; r.experts = experts; r.entries = p.entries; r.rows_per_entry = p.rows;
   r.table = table; r.m1 = 2 * inter; r.m2 = hidden;
@@ -529,7 +534,8 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   r.h = (float*)(base + p.h); r.out = (float*)(base + p.out);
   r.pos_of = (int*)(base + p.pos); r.info = (int4*)(base + p.info);
   r.host_word = host_word; r.ticket = ticket;
-  HTR_CHECK_HIP(launch_kernel(k_moe_route, dim3(1), dim3(MOE_ROUTE_THREADS), 0, st, r));
+  HTR_CHECK_HIP(given ? launch_kernel(k_moe_route<true>, dim3(1), dim3(MOE_ROUTE_THREADS), 0, st, r, ptrs)
+                      : launch_kernel(k_moe_route<false>, dim3(1), dim3(MOE_ROUTE_THREADS), 0, st, r, ptrs));
   LinearTail t1 = {}, t2 = {};
   t1.xt_g = (const _Float16*)(base + p.xt1); t1.xs_g = (const float*)(base + p.xs1); t1.sc_g = (const float*)(base + p.sc1);
   t2.xt_g = (const _Float16*)(base + p.xt2); t2.xs_g = (const float*)(base + p.xs2); t2.sc_g = (const float*)(base + p.sc2);

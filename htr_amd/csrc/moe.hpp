@@ -1,9 +1,10 @@
 // Part of htr_gfx950.hip, included inside its anonymous namespace: routing, rotation, activation and combination around the
 // two grouped launches (k_linear_tile) of a routed-expert layer.
 // ------------------------------------------------------------------------------------------------ routed experts
-// One layer is seven launches, of which the first comes once per 32 experts, and no copy or synchronisation between them:
-//   k_moe_experts   the experts' tensor addresses, from the kernel arguments to a device table (one launch per 32 experts)
-//   k_moe_route     one workgroup: tokens sorted by expert, the problem tables of both grouped launches
+// One layer is six launches, and no copy or synchronisation between them:
+//   k_moe_route     one workgroup: tokens sorted by expert, the problem tables of both grouped launches; up to 64 experts' tensor
+//                   addresses come as kernel arguments (16 tokens, 64 experts: two launches of k_moe_experts less, 4 of 76 us), more of
+//                   them through a device table that k_moe_experts fills (one launch per 64 experts)
 //   k_moe_rotate    one workgroup per (token, expert) pair: gather, sign, H128, f16, in fragment order
 //   k_linear_tile   gate and up of every active expert, float32
 //   k_moe_act       one workgroup per pair: silu(gate) * up, rounded to the activations' type, then as k_moe_rotate
@@ -12,10 +13,10 @@
 // Every entry of the problem tables is one expert and up to rows_per_entry of its pairs; the number of entries is known to the
 // host only as a bound (experts + pairs / rows per entry), entries beyond the used ones have no rows and their workgroups
 // return at once.
-constexpr int MOE_PTR_CHUNK = 32;                 // experts per k_moe_experts launch: 2 KB of kernel arguments
+constexpr int MOE_PTR_CHUNK = 64;                 // experts per launch that takes their addresses: 4 KB of kernel arguments
 struct MoePtrs { const void* p[MOE_PTR_CHUNK][8]; };      // gate_up: qweight, scales, su, sv; down: the same
 
-__global__ __launch_bounds__(256) void k_moe_experts(const MoePtrs src, const void** __restrict__ table, int first, int count) {
+__global__ __launch_bounds__(MOE_PTR_CHUNK * 8) void k_moe_experts(const MoePtrs src, const void** __restrict__ table, int first, int count) {
   const int i = threadIdx.x;
   if (i < count * 8) table[first * 8 + i] = src.p[i >> 3][i & 7];
 }
@@ -23,7 +24,7 @@ __global__ __launch_bounds__(256) void k_moe_experts(const MoePtrs src, const vo
 struct MoeRoute {
   const void* ids;               // [pairs] int32 or int64
   int ids64, pairs, top, experts, entries, rows_per_entry;
-  const void* const* table;      // [experts][8]
+  const void** table;            // [experts][8]
   int m1, m2;                    // rows of gate_up and of down
   htr_group_entry* e1;           // [entries]
   htr_group_entry* e2;
@@ -40,7 +41,9 @@ struct MoeRoute {
 // that for every pair).
 constexpr int MOE_ROUTE_THREADS = 1024;
 constexpr int MOE_MAX_EXPERTS = 4096;
-__global__ __launch_bounds__(MOE_ROUTE_THREADS) void k_moe_route(const MoeRoute a) {
+// GIVEN: the experts' addresses are in `ptrs` and go to the table here; otherwise they are in it
+template <bool GIVEN>
+__global__ __launch_bounds__(MOE_ROUTE_THREADS) void k_moe_route(const MoeRoute a, const MoePtrs ptrs) {
   __shared__ uint32_t cnt[MOE_MAX_EXPERTS];       // pairs of the expert, then its first position
   __shared__ uint32_t row0[MOE_MAX_EXPERTS];      // row of the fragment order of a pair = its position + this (mod 2^32)
   __shared__ uint32_t s_scan[3][16];
@@ -51,6 +54,7 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void k_moe_route(const MoeRoute 
     return v < 0 || v >= E ? -1 : (int)v;
   };
   for (int i = tid; i < E; i += MOE_ROUTE_THREADS) cnt[i] = 0u;
+  if (GIVEN && tid < E * 8) a.table[tid] = ptrs.p[tid >> 3][tid & 7];
   __syncthreads();
   bool bad = false;
   for (int q0 = w * 64; q0 < a.pairs; q0 += MOE_ROUTE_THREADS) {
@@ -93,7 +97,9 @@ __global__ __launch_bounds__(MOE_ROUTE_THREADS) void k_moe_route(const MoeRoute 
     if (e < E) {
       cnt[e] = pos;
       row0[e] = tile * 32u - pos;
-      const void* const* t = a.table + (size_t)e * 8;
+      const void* t[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) t[k] = GIVEN ? ptrs.p[e][k] : a.table[(size_t)e * 8 + k];
       for (uint32_t i = 0; i < ents; ++i) {
         const uint32_t r0 = i * R, rows = min((uint32_t)R, total - r0);
         htr_group_entry g;

@@ -63,6 +63,21 @@ def test_whole_layer_matches_the_composition(dev, oracle, dtype, counts, top, K1
     assert y.dtype == np.float32 and rel <= (4e-3 if dtype == torch.bfloat16 else 2e-3), rel
 
 
+@pytest.mark.parametrize("E", [63, 64, 65, 129])
+def test_number_of_experts_around_one_launch_of_addresses(dev, E):
+    """Up to 64 experts' addresses travel with the routing launch, more of them through a table: a pair's result does not depend on
+    how many experts stand beside its own, so every size must give, bit for bit, what the chosen experts alone give."""
+    from htr_amd import ops
+    print(f"moe: {E} experts", flush=True)
+    gate_up, down = (_to(dev, part) for part in _layer(E, 128, 128, 4, 4, 640))
+    g = torch.Generator().manual_seed(E)
+    few = torch.tensor([0, 1, E // 2, E - 2, E - 1])
+    pick = torch.stack([torch.randperm(5, generator=g)[:2] for _ in range(11)])
+    x, w = torch.randn(11, 128, generator=g).bfloat16().to(dev), torch.rand(11, 2, generator=g).to(dev)
+    y = ops.moe_experts(x, few[pick].to(dev), w, gate_up, down)
+    assert torch.equal(y, ops.moe_experts(x, pick.to(dev), w, [gate_up[e] for e in few], [down[e] for e in few]))
+
+
 def test_expert_numbers_out_of_range_and_graph_capture(dev):
     from htr_amd import ops
     print("moe: bad ids, capture", flush=True)
