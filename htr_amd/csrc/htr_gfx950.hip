@@ -541,7 +541,7 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   t2.xt_g = (const _Float16*)(base + p.xt2); t2.xs_g = (const float*)(base + p.xs2); t2.sc_g = (const float*)(base + p.sc2);
   t1.cbscale = t2.cbscale = htr_cbscale();
   t1.group = r.e1; t2.group = r.e2;
-  HTR_CHECK_HIP(launch_kernel(k_moe_rotate, dim3(p.pairs), dim3(256), 0, st, x, x_dtype, (const int4*)r.info, (const void* const*)table, hidden,
+  HTR_CHECK_HIP(launch_kernel(k_moe_rotate, dim3(moe_rotate_grid(p.pairs)), dim3(256), 0, st, x, x_dtype, p.pairs, (const int4*)r.info, (const void* const*)table, hidden,
                               (_Float16*)t1.xt_g, (float*)t1.xs_g, (float*)t1.sc_g));
   const int flags = HTR_F32 << 2 | FLAG_ENTRY_TILES;
   BatchArgs b1 = {nullptr, nullptr, nullptr, nullptr, 2 * inter, hidden, 0, flags}, b2 = {nullptr, nullptr, nullptr, nullptr, hidden, inter, 0, flags};
@@ -549,7 +549,7 @@ int htr_moe_experts(const void* x, int x_dtype, const void* ids, int ids_int64, 
   if (p.rows == 32) { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 1, true>(b1, t1, 1, p.entries, st))); }
   else { HTR_FOR_K(K_gate_up, rc = (launch_tile_v<KK, 2, true>(b1, t1, 1, p.entries, st))); }
   if (rc != HTR_OK) return rc;
-  HTR_CHECK_HIP(launch_kernel(k_moe_act, dim3(p.pairs), dim3(256), 0, st, (const float*)r.h, x_dtype, (const int4*)r.info,
+  HTR_CHECK_HIP(launch_kernel(k_moe_act, dim3(moe_rotate_grid(p.pairs)), dim3(256), 0, st, (const float*)r.h, x_dtype, p.pairs, (const int4*)r.info,
                               (const void* const*)table, inter, (_Float16*)t2.xt_g, (float*)t2.xs_g, (float*)t2.sc_g));
   if (p.rows == 32) { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 1, true>(b2, t2, 1, p.entries, st))); }
   else { HTR_FOR_K(K_down, rc = (launch_tile_v<KK, 2, true>(b2, t2, 1, p.entries, st))); }

@@ -230,11 +230,20 @@ __device__ __forceinline__ void rotate_row_frag32(Get&& get, const uint8_t* __re
   }
 }
 
-__global__ __launch_bounds__(256) void k_moe_rotate(const void* __restrict__ x, int x_dtype, const int4* __restrict__ info,
+// Sorted position of the pair that a workgroup rotates.  Eight rows of an expert share every 128-byte line of the fragment order, 16
+// bytes each, and workgroups go to the eight XCDs in turn, each with an L2 of its own: an eighth of the consecutive positions
+// to every XCD, so that its L2 puts the lines together.
+constexpr int MOE_XCDS = 8;
+__host__ __device__ inline int moe_rotate_grid(int pairs) { return (pairs + MOE_XCDS - 1) / MOE_XCDS * MOE_XCDS; }
+__device__ __forceinline__ int moe_pair_of(int block, int grid) { return (block % MOE_XCDS) * (grid / MOE_XCDS) + block / MOE_XCDS; }
+
+__global__ __launch_bounds__(256) void k_moe_rotate(const void* __restrict__ x, int x_dtype, int pairs, const int4* __restrict__ info,
                                                     const void* const* __restrict__ table, int n, _Float16* __restrict__ xt_g,
                                                     float* __restrict__ xs_g, float* __restrict__ sc_g) {
   __shared__ uint32_t s_amax[4];
-  const int4 q = info[blockIdx.x];                               // uniform
+  const int pos = moe_pair_of(blockIdx.x, moe_rotate_grid(pairs));
+  if (pos >= pairs) return;
+  const int4 q = info[pos];                                      // uniform
   if (q.y < 0) return;
   const uint8_t* su = (const uint8_t*)table[(size_t)q.y * 8 + 2];
   if (x_dtype == HTR_F32) {
@@ -247,14 +256,16 @@ __global__ __launch_bounds__(256) void k_moe_rotate(const void* __restrict__ x, 
 }
 
 // silu(gate) * up of one pair, rounded to the activations' type, rotated for the down projection
-__global__ __launch_bounds__(256) void k_moe_act(const float* __restrict__ h, int x_dtype, const int4* __restrict__ info,
+__global__ __launch_bounds__(256) void k_moe_act(const float* __restrict__ h, int x_dtype, int pairs, const int4* __restrict__ info,
                                                  const void* const* __restrict__ table, int F, _Float16* __restrict__ xt_g,
                                                  float* __restrict__ xs_g, float* __restrict__ sc_g) {
   __shared__ uint32_t s_amax[4];
-  const int4 q = info[blockIdx.x];
+  const int pos = moe_pair_of(blockIdx.x, moe_rotate_grid(pairs));
+  if (pos >= pairs) return;
+  const int4 q = info[pos];
   if (q.y < 0) return;
   const uint8_t* su = (const uint8_t*)table[(size_t)q.y * 8 + 6];
-  const float* gate = h + (size_t)blockIdx.x * 2 * F;
+  const float* gate = h + (size_t)pos * 2 * F;
   const float* up = gate + F;
   auto act = [](float g, float u) { return g / (1.f + expf(-g)) * u; };
   if (x_dtype == HTR_F32) {
