@@ -232,7 +232,8 @@ __device__ __forceinline__ void rotate_row_frag32(Get&& get, const uint8_t* __re
 
 // Sorted position of the pair that a workgroup rotates.  Eight rows of an expert share every 128-byte line of the fragment order, 16
 // bytes each, and workgroups go to the eight XCDs in turn, each with an L2 of its own: an eighth of the consecutive positions
-// to every XCD, so that its L2 puts the lines together.
+// to every XCD, so that its L2 puts the lines together.  Bound of both rotations: memory latency and these writes.  500 tokens over 64
+// experts (2048x1408), whole layer: 189.7 -> 185 us; 16 tokens level.
 constexpr int MOE_XCDS = 8;
 __host__ __device__ inline int moe_rotate_grid(int pairs) { return (pairs + MOE_XCDS - 1) / MOE_XCDS * MOE_XCDS; }
 __device__ __forceinline__ int moe_pair_of(int block, int grid) { return (block % MOE_XCDS) * (grid / MOE_XCDS) + block / MOE_XCDS; }
