@@ -134,6 +134,7 @@ int htr_linear_route(int m, int n, int K, int M, int x_dtype, int eager) {
   if (K < 2 || K > 8 || !shape_ok(m, n) || M < 1 || M > HTR_MAX_BATCH || !dtype_ok(x_dtype)) return -1;
   if (M <= HTR_MAX_ROWS_PER_TILE) return 0;
   WidePlan wp;
+  if (x_dtype == HTR_F32) return M <= fused_rows(m, n) && make_wide_plan(m, n, M, 0, wp) ? 1 << 27 : -1;
   return make_wide_plan(m, n, M, 0, wp) && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype, eager != 0) ? 1 << 27 : -1;
 }
 

@@ -433,10 +433,16 @@ inline bool wants_wide(int M, int nsplit) {
 }
 inline int wide_want_S(int nsplit) { return nsplit > 0 ? nsplit & 0xFFFFF : 0; }
 
+// Rows up to which a fused launch takes a matrix for activations of any type.  Beyond, float32 activations stay float32: the fused
+// kernels round the rotated activations to float16, which only the library's product on the dequantized weight does not.
+inline int fused_rows(int m, int n) {
+  return (long)m * n < 4096L * 4096 ? HTR_MAX_ROWS_PER_TILE : n >= 8192 ? 512 : 384;
+}
+
 // More than 128 rows: the wide kernel, or the weight dequantized and the library's product?  Both in us.  The wide kernel: its plan's
 // steps, or what the matrix units of the whole chip sustain (1.1 PFLOP/s with everything around them, where the grid fills it), and
 // launches, rotation and output.  Dequantization and product: 0.66 us per million weights, the product at 1.45 PFLOP/s, launches;
-// float16 converts the weight once more, and the library's float32 product reaches about a tenth.  Measured / these, K4, bfloat16:
+// float16 converts the weight once more.  Measured / these, K4, bfloat16:
 // wide 6144x4096 129 rows 24.3 / 26, 512 rows 42.9 / 42, 14336x4096 512 rows 72.4 / 73, 4096x4096 512 rows 35.5 / 32; dequantization and
 // product 2048x2048 512 rows 21.6 / 22, 6144x4096 512 rows 52 / 50, 14336x4096 1024 rows 131 / 137, 2048 rows 216 / 221.
 inline double wide_us(int m, int n, int M, const WidePlan& wp) {
@@ -452,7 +458,7 @@ inline double wide_us(int m, int n, int M, const WidePlan& wp) {
 // rows 32.3 / 34.9).
 inline double dequant_us(int m, int n, int M, int x_dtype, bool eager) {
   const double weights = (double)m * n;
-  const double gpu = 16.0 + weights * (x_dtype == HTR_BF16 ? 0.66e-6 : 1.6e-6) + 2.0 * M * weights / (x_dtype == HTR_F32 ? 0.12e9 : 1.45e9);
+  const double gpu = 16.0 + weights * (x_dtype == HTR_BF16 ? 0.66e-6 : 1.6e-6) + 2.0 * M * weights / 1.45e9;
   return !eager ? gpu : gpu < 22.0 ? 25.0 : gpu + 3.0;
 }
 

@@ -41,7 +41,10 @@ def test_route(L):
     assert wide(4096, 4096, 128) == 0 and wide(4096, 4096, 129) == WIDE and wide(14336, 4096, 512) == WIDE
     assert wide(14336, 4096, 2048) == -1 and wide(1024, 1024, 1024) == -1          # dequantize and multiply
     assert wide(512, 512, 512) == -1 and wide(512, 512, 512, eager=1) == WIDE      # where the host's time counts
-    assert wide(14336, 4096, 2048, 2) == WIDE                                     # float32: the library's product is slow
+    # float32 activations are rounded to float16 where a launch always took them, and nowhere else
+    for eager in (0, 1):
+        assert wide(4096, 4096, 384, 2, eager) == wide(4096, 14336, 512, 2, eager) == WIDE
+        assert wide(4096, 4096, 385, 2, eager) == wide(4096, 14336, 513, 2, eager) == wide(2048, 2048, 129, 2, eager) == wide(14336, 4096, 2048, 2, eager) == -1
     assert wide(4096, 4096, 2049) == -1 and wide(100, 128, 200) == -1 and L.htr_linear_route(128, 128, 9, 200, 0, 1) == -1
 
 
@@ -106,6 +109,21 @@ def test_wide_kernel(dev, oracle, L, K, M, m, n, S, xt, off):
         want = ref if yt == torch.float32 else ref - bias.double().numpy() + b.double().cpu().numpy()
         err = np.abs(outs[0].double().cpu().numpy() - want).max() / np.abs(want).max()
         assert err <= tol, (yt, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,M", [(512, 1024, 129), (2048, 2048, 700), (4096, 4096, 400)])
+def test_float32_activations_stay_float32(dev, m, n, M, monkeypatch):
+    """Beyond the rows that were always fused: the float32 product with the dequantized weight, bit for bit, on both host paths."""
+    from htr_amd import _native, ops
+    print(f"float32 {m}x{n} M={M}", flush=True)
+    w, x = _case(m, n, 4, M, 78, torch.float32)
+    d, xd = [t.to(dev) for t in w], x.to(dev)
+    want = torch.nn.functional.linear(xd, ops.dequant_w(*d).float())
+    for fast in (None, False):
+        monkeypatch.setattr(_native, "_fast", fast)
+        for _ in range(2):
+            assert torch.equal(ops.linear(xd, *d), want)
 
 
 @pytest.mark.gpu
