@@ -105,17 +105,20 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // other threads run meanwhile: a launch waits where the stream's queue is full.  The caller's frame holds the tensors.
     pybind11::gil_scoped_release no_lock;
     c10::DeviceGuard guard(x.device());
+    at::DimVector shape(x.sizes().begin(), x.sizes().end());
+    shape.back() = s.m;
     if (route < 0) {
       at::Tensor w = at::empty({s.m, s.n}, x.options().dtype(at::kBFloat16));
       rc = f_dequant(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), w.mutable_data_ptr(),
                      (int)s.m, (int)s.n, (int)s.K, stream);
       if (rc == HTR_OK) {
-        y = at::linear(x, code == 0 ? w : w.to(x.scalar_type()), t[5] == nullptr ? std::optional<at::Tensor>() : std::optional<at::Tensor>(*t[5]));
+        // rows and columns only: with more dimensions, and an outer one of size 1 whose stride is not the inner ones' product (a prompt cut
+        // from a longer buffer), torch takes a batched product with a transposed view of the weight
+        y = at::linear(x.view({M, s.n}), code == 0 ? w : w.to(x.scalar_type()),
+                       t[5] == nullptr ? std::optional<at::Tensor>() : std::optional<at::Tensor>(*t[5])).view(shape);
         if (y.scalar_type() != x.scalar_type()) y = y.to(x.scalar_type());      // autocast
       }
     } else {
-      at::DimVector shape(x.sizes().begin(), x.sizes().end());
-      shape.back() = s.m;
       y = at::empty(shape, x.options());
       rc = f_linear(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), x.const_data_ptr(),
                   t[5] == nullptr ? nullptr : t[5]->const_data_ptr(), y.mutable_data_ptr(), (int)s.m, (int)s.n, (int)s.K, (int)M, code, code, route,

@@ -146,3 +146,33 @@ def test_rows_beyond_64_through_ops(dev, oracle, m, n, M, monkeypatch):
     leaf = xd.clone().requires_grad_()
     y = ops.linear(leaf, *d)
     assert y.requires_grad == (M > 128 and ops.fused_rows_per_launch(m, n, M) == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lead", [(1,), (1, 1)])
+def test_a_prompt_cut_from_a_longer_buffer(dev, lead):
+    """Contiguous rows under outer dimensions of size 1 whose strides are the buffer's: one product of matrices, never a batched one
+    (torch's own linear takes one for this layout), with the result of the rows alone."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from htr_amd import _native, ops
+    m = n = 2048
+    M = 700
+    print(f"prompt cut from a longer buffer, {len(lead)} outer dimensions", flush=True)
+    assert _native.lib().htr_linear_route(m, n, 4, M, 0, 1) == -1 and _native.fast() is not None
+    w, x = _case(m, n, 4, M, 79)
+    d, rows = [t.to(dev) for t in w], x.to(dev)
+    buffer = torch.zeros(*lead, M + 100, n, dtype=torch.bfloat16, device=dev)
+    cut = buffer[..., :M, :]
+    cut.copy_(rows)
+    assert cut.is_contiguous() and cut.stride(0) != M * n
+    called = []
+
+    class Record(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            called.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    with Record():
+        y = ops.linear(cut, *d)
+    assert "mm" in called and not {"bmm", "baddbmm"} & set(called), called
+    assert y.shape == (*lead, M, m) and torch.equal(y.reshape(M, m), ops.linear(rows, *d))
