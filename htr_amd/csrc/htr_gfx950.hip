@@ -131,11 +131,13 @@ int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
 }
 
 int htr_linear_route(int m, int n, int K, int M, int x_dtype, int eager) {
-  if (K < 2 || K > 8 || !shape_ok(m, n) || M < 1 || M > HTR_MAX_BATCH || !dtype_ok(x_dtype)) return -1;
+  const int refused = K < 2 || K > 8 ? HTR_ERR_K : !shape_ok(m, n) ? HTR_ERR_SHAPE : M < 1 || M > HTR_MAX_BATCH ? HTR_ERR_BATCH : !dtype_ok(x_dtype) ? HTR_ERR_DTYPE : HTR_OK;
+  if (refused != HTR_OK) return HTR_ROUTE_DEQUANTIZE - refused;
   if (M <= HTR_MAX_ROWS_PER_TILE) return 0;
   WidePlan wp;
-  if (x_dtype == HTR_F32) return M <= fused_rows(m, n) && make_wide_plan(m, n, M, 0, wp) ? 1 << 27 : -1;
-  return make_wide_plan(m, n, M, 0, wp) && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype, eager != 0) ? 1 << 27 : -1;
+  const bool wide = make_wide_plan(m, n, M, 0, wp);
+  if (M <= fused_rows(m, n)) return wide ? NSPLIT_WIDE : 0;
+  return wide && x_dtype != HTR_F32 && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype, eager != 0) ? NSPLIT_WIDE : HTR_ROUTE_DEQUANTIZE;
 }
 
 void htr_set_spin_limit(int polls) { g_spin_limit.store(polls < 1 ? 1 : polls, std::memory_order_relaxed); }

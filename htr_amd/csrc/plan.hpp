@@ -427,14 +427,19 @@ inline size_t wide_slot_bytes(int m, int M, const WidePlan& wp) {
 // behind (14336x4096 K4 23.9 / 25.7, 2048x2048 11.9 / 13.1).  From 129 rows against k_linear_gemm: 6144x4096 K4 129 rows 32.2 / 24.3, 256
 // rows 40.1 / 29.7, 333 rows 39.8 / 37.1; 14336x4096 256 rows 50.6 / 44.3, 333 rows 76.3 / 60.4, 512 rows 94.9 / 72.4; 4096x14336 256 rows
 // 60.6 / 52.2 (htr_linear_route says who takes it there).
-constexpr int WIDE_MIN_M = 65;
+constexpr int WIDE_MIN_M = 65, NSPLIT_WIDE = 1 << 27;
 inline bool wants_wide(int M, int nsplit) {
-  return nsplit > 0 ? (nsplit & (1 << 27)) != 0 : M >= WIDE_MIN_M && M <= HTR_MAX_ROWS_PER_TILE;
+  return nsplit > 0 ? (nsplit & NSPLIT_WIDE) != 0 : M >= WIDE_MIN_M && M <= HTR_MAX_ROWS_PER_TILE;
 }
 inline int wide_want_S(int nsplit) { return nsplit > 0 ? nsplit & 0xFFFFF : 0; }
 
-// Rows up to which a fused launch takes a matrix for activations of any type.  Beyond, float32 activations stay float32: the fused
-// kernels round the rotated activations to float16, which only the library's product on the dequantized weight does not.
+// Rows up to which a matrix is always multiplied by a fused launch, the wide kernel's: the codes stay exact there (2e-4 against float64,
+// 2.4e-3 with a dequantized weight, whose entries are bfloat16).  The other kernel for these rows, k_linear_gemm, is no further choice:
+// of 476 shapes within them (K 2 to 8, 129 to 512 rows, GPU time) it was ahead in three, by 2 % at most (4096x4096 K8 192 and 256 rows
+// 33.5 / 34.0 us and 39.8 / 40.5, 10240x2560 K3 245 rows 33.2 / 33.9), and took 1.03 to 1.76 times the wide kernel's time in the others;
+// of 276 dequantization and product was ahead of the wide kernel in one (4096x4096 K8 256 rows 37.6).
+// Beyond these rows float32 activations stay float32: the fused kernels round the rotated activations to float16, which only the
+// library's product on the dequantized weight does not.
 inline int fused_rows(int m, int n) {
   return (long)m * n < 4096L * 4096 ? HTR_MAX_ROWS_PER_TILE : n >= 8192 ? 512 : 384;
 }

@@ -97,6 +97,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     // torch's product can be differentiated and transformed, a launch on raw pointers cannot: the general path tells them apart
     if (M > HTR_MAX_BATCH || !raw_ok(x) || differentiable(x) || (t[5] != nullptr && (!raw_ok(*t[5]) || differentiable(*t[5])))) Py_RETURN_NONE;
     route = f_route((int)s.m, (int)s.n, (int)s.K, (int)M, code, 1);
+    if (route < HTR_ROUTE_DEQUANTIZE) Py_RETURN_NONE;
   }
   if ((failed != nullptr && *failed != 0) || f_capture(stream) != 0) Py_RETURN_NONE;
   at::Tensor y;
@@ -107,7 +108,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     c10::DeviceGuard guard(x.device());
     at::DimVector shape(x.sizes().begin(), x.sizes().end());
     shape.back() = s.m;
-    if (route < 0) {
+    if (route == HTR_ROUTE_DEQUANTIZE) {
       at::Tensor w = at::empty({s.m, s.n}, x.options().dtype(at::kBFloat16));
       rc = f_dequant(t[1]->const_data_ptr(), t[2]->const_data_ptr(), t[3]->const_data_ptr(), t[4]->const_data_ptr(), w.mutable_data_ptr(),
                      (int)s.m, (int)s.n, (int)s.K, stream);

@@ -227,22 +227,27 @@ def _followed(*tensors):
     return False
 
 
-def _wide_route(x2, bias, m, n, K, M, per_launch):
-    """nsplit of one launch of the wide kernel where that is ahead beyond 128 rows, else None."""
+DEQUANTIZE = -1      # what htr_linear_route returns where the weight is to be dequantized and multiplied by the library
+
+
+def _route(x2, bias, m, n, K, M, per_launch):
+    """(rows per launch, nsplit) for more than 128 rows: what htr_linear_route says, as in the C++ host path; 0 rows = dequantize."""
     if M <= _native.MAX_ROWS_PER_TILE or M > LAUNCH_MAX_M or GEMV_LOOP_MAX is not None or NSPLIT != 0 or PREFILL != "w":
-        return None
+        return per_launch, NSPLIT
     if per_launch == 0 and _followed(x2, bias):
-        return None
+        return per_launch, NSPLIT
     capturing = torch.cuda.is_current_stream_capturing()
     nsplit = _native.lib().htr_linear_route(m, n, K, M, _DTYPE_CODE[x2.dtype], 0 if capturing else 1)
-    if nsplit < 0:
-        return None
+    if nsplit == DEQUANTIZE:
+        return 0, NSPLIT
+    if nsplit < 0:                    # more rows or columns than a launch takes: refused where a launch is asked for, not by dequant_w
+        return per_launch, NSPLIT
     if SHARE_CAPTURE_WORKSPACE and capturing:
-        # the shared buffer cannot grow now, and may have been sized for what ran before
+        # the shared buffer cannot grow now, and may have been sized for what htr_linear needs by its own policy
         ws = _WORKSPACES.get((x2.device.index, "shared"))
         if ws is None or ws.buf.numel() < _workspace_need(m, n, K, M, nsplit):
-            return None
-    return nsplit
+            return per_launch, NSPLIT
+    return M, nsplit
 
 
 def _launch(x2, qweight, scales, su, sv, bias, y, m, n, K, out_code, nsplit):
@@ -275,10 +280,7 @@ def _linear_impl(x2, qweight, scales, su, sv, bias, out_dtype=None):
             raise RuntimeError("HTR-W1 tensors must be contiguous and on the device of x")
     if bias is not None and (bias.dtype != out_dtype or bias.numel() != m or bias.device != x2.device):
         raise RuntimeError("bias must be [m] in the output dtype on the device of x")
-    per_launch, nsplit = fused_rows_per_launch(m, n, M), NSPLIT
-    wide = _wide_route(x2, bias, m, n, K, M, per_launch)
-    if wide is not None:
-        per_launch, nsplit = M, wide
+    per_launch, nsplit = _route(x2, bias, m, n, K, M, fused_rows_per_launch(m, n, M))
     if per_launch == 0 and PREFILL == "rot":
         xr = wire.blk_had_cols_T(x2.float() * wire.unpack_signs(su, n).to(x2.device))
         yr = wire.blk_had_cols_T(xr @ dequant_q(qweight, scales).T) * wire.unpack_signs(sv, m).to(x2.device)

@@ -132,14 +132,16 @@ unsigned long long htr_stream_capture_id(void* stream);
 int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6);
 
 /*
- * What is fastest for this call: a value for htr_linear's nsplit (0, or 2^27, the wide kernel, beyond HTR_MAX_ROWS_PER_TILE
- * rows), or -1: dequantize the weight (htr_dequant_w) and multiply with a library GEMM, which is ahead from a few hundred
- * rows on small matrices and from about a thousand on large ones; also -1 for arguments that htr_linear refuses.  Float32
- * activations, which the kernels round to float16 in the rotated basis, are fused up to 384 rows of matrices from 4096x4096
- * weights up (512 rows if n >= 8192) and multiplied in float32 beyond.  eager: 1 if
- * the call is queued by itself, where the host's time for two launches and a product counts, 0 if it is part of a graph.
+ * How this call is best made: a value for htr_linear's nsplit (0, or 2^27, the wide kernel, beyond HTR_MAX_ROWS_PER_TILE rows), or
+ * HTR_ROUTE_DEQUANTIZE: dequantize the weight (htr_dequant_w) and multiply with a library GEMM; for arguments that htr_linear
+ * refuses, HTR_ROUTE_DEQUANTIZE minus the status that it returns.  Up to 384 rows of matrices from 4096x4096 weights up (512 rows
+ * if n >= 8192) the call is always fused; beyond, bf16 and f16 activations go where they are faster (the GEMM from a few hundred
+ * rows on small matrices, from about a thousand on large ones), and float32 activations, which the kernels would round to
+ * float16 in the rotated basis, to the GEMM.  eager: 1 if the call is queued by itself, where the host's time for two launches
+ * and a product counts, 0 if it is part of a graph.
  * Reference: the row limit of its fused launches, HTR_GEMV_LOOP_MAX (htr/ops.py:59-61).
  */
+#define HTR_ROUTE_DEQUANTIZE (-1)
 int htr_linear_route(int m, int n, int K, int M, int x_dtype, int eager);
 
 /*

@@ -45,7 +45,37 @@ def test_route(L):
     for eager in (0, 1):
         assert wide(4096, 4096, 384, 2, eager) == wide(4096, 14336, 512, 2, eager) == WIDE
         assert wide(4096, 4096, 385, 2, eager) == wide(4096, 14336, 513, 2, eager) == wide(2048, 2048, 129, 2, eager) == wide(14336, 4096, 2048, 2, eager) == -1
-    assert wide(4096, 4096, 2049) == -1 and wide(100, 128, 200) == -1 and L.htr_linear_route(128, 128, 9, 200, 0, 1) == -1
+    # refused as htr_linear refuses it, and not to be mistaken for "dequantize"
+    assert [wide(4096, 4096, 2049), wide(100, 128, 200), wide(128, 128, 200, 3), L.htr_linear_route(128, 128, 9, 200, 0, 1)] == [-5, -4, -6, -3]
+
+
+def test_what_was_fused_is_never_dequantized(L):
+    """Rows and matrices that ops.fused_rows_per_launch names are fused for every type, width and mode: a dequantized weight is rounded
+    to bfloat16."""
+    from htr_amd import ops
+    shapes = [(m, n) for m in (1024, 4096, 6144, 10880, 14336, 17024, 17408, 17664, 28672) for n in (1408, 4096, 5120, 8192, 12544, 14336)]
+    for m, n in shapes:
+        limit = ops.fused_max_rows(m, n)
+        for M in {129, 160, 192, 256, 257, 264, 282, 288, 311, 320, 384, 385, 512, 513}:
+            fused = M <= limit
+            assert (ops.fused_rows_per_launch(m, n, M) > 0) == fused
+            routes = {L.htr_linear_route(m, n, K, M, x, eager) for K in (2, 4, 8) for x in (0, 1, 2) for eager in (0, 1)}
+            assert not fused or routes == {WIDE}, (m, n, M, routes)
+            assert routes <= {WIDE, -1} and (fused or L.htr_linear_route(m, n, 4, M, 2, 1) == -1)
+
+
+@pytest.mark.parametrize("m,n,M", [(17408, 5120, 264), (16640, 11264, 311), (17024, 13696, 282), (6144, 4096, 333), (4096, 4096, 400), (2048, 2048, 700)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_the_general_path_asks_the_library(L, monkeypatch, m, n, M, dtype):
+    """What the C++ host path does with these calls (htr_linear_route's answer) is what ops._linear_impl does, outside of a capture and in one."""
+    from htr_amd import ops
+    code = {torch.bfloat16: 0, torch.float32: 2}[dtype]
+    x = torch.empty(1, dtype=dtype).expand(M, n)
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        route = L.htr_linear_route(m, n, 4, M, code, 0 if capturing else 1)
+        want = (0, 0) if route == -1 else (M, route)
+        assert ops._route(x, None, m, n, 4, M, ops.fused_rows_per_launch(m, n, M)) == want
 
 
 def _case(m, n, K, M, seed, dtype=torch.bfloat16):
