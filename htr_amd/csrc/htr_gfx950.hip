@@ -137,7 +137,7 @@ int htr_linear_route(int m, int n, int K, int M, int x_dtype, int eager) {
   WidePlan wp;
   const bool wide = make_wide_plan(m, n, M, 0, wp);
   if (M <= fused_rows(m, n)) return wide ? NSPLIT_WIDE : 0;
-  return wide && x_dtype != HTR_F32 && wide_us(m, n, M, wp) < dequant_us(m, n, M, x_dtype, eager != 0) ? NSPLIT_WIDE : HTR_ROUTE_DEQUANTIZE;
+  return wide && x_dtype != HTR_F32 && wide_ahead(m, n, K, M, x_dtype, wp, eager != 0) ? NSPLIT_WIDE : HTR_ROUTE_DEQUANTIZE;
 }
 
 void htr_set_spin_limit(int polls) { g_spin_limit.store(polls < 1 ? 1 : polls, std::memory_order_relaxed); }

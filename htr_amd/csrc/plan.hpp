@@ -435,36 +435,66 @@ inline int wide_want_S(int nsplit) { return nsplit > 0 ? nsplit & 0xFFFFF : 0; }
 
 // Rows up to which a matrix is always multiplied by a fused launch, the wide kernel's: the codes stay exact there (2e-4 against float64,
 // 2.4e-3 with a dequantized weight, whose entries are bfloat16).  The other kernel for these rows, k_linear_gemm, is no further choice:
-// of 476 shapes within them (K 2 to 8, 129 to 512 rows, GPU time) it was ahead in three, by 2 % at most (4096x4096 K8 192 and 256 rows
-// 33.5 / 34.0 us and 39.8 / 40.5, 10240x2560 K3 245 rows 33.2 / 33.9), and took 1.03 to 1.76 times the wide kernel's time in the others;
-// of 276 dequantization and product was ahead of the wide kernel in one (4096x4096 K8 256 rows 37.6).
+// of 476 shapes within them (K 2 to 8, 129 to 512 rows, GPU time) it was ahead in three, and measured again in one (10240x2560 K3 245
+// rows, 33.5 / 34.6 us; 4096x4096 K8 192 and 256 rows 33.4 / 27.6, 39.3 / 35.5); it took 1.03 to 1.76 times the wide kernel's time in
+// the others.  Dequantization and product was ahead of the wide kernel in none of 276 (4096x4096 K8 256 rows 37.1).
 // Beyond these rows float32 activations stay float32: the fused kernels round the rotated activations to float16, which only the
 // library's product on the dequantized weight does not.
 inline int fused_rows(int m, int n) {
   return (long)m * n < 4096L * 4096 ? HTR_MAX_ROWS_PER_TILE : n >= 8192 ? 512 : 384;
 }
 
-// More than 128 rows: the wide kernel, or the weight dequantized and the library's product?  Both in us.  The wide kernel: its plan's
-// steps, or what the matrix units of the whole chip sustain (1.1 PFLOP/s with everything around them, where the grid fills it), and
-// launches, rotation and output.  Dequantization and product: 0.66 us per million weights, the product at 1.45 PFLOP/s, launches;
-// float16 converts the weight once more.  Measured / these, K4, bfloat16:
-// wide 6144x4096 129 rows 24.3 / 26, 512 rows 42.9 / 42, 14336x4096 512 rows 72.4 / 73, 4096x4096 512 rows 35.5 / 32; dequantization and
-// product 2048x2048 512 rows 21.6 / 22, 6144x4096 512 rows 52 / 50, 14336x4096 1024 rows 131 / 137, 2048 rows 216 / 221.
-inline double wide_us(int m, int n, int M, const WidePlan& wp) {
-  const int cus = num_cu(), nblk = n / 128, rest = M - (wp.mtiles - 1) * WIDE_ROWS, cb_last = (nblk + wp.S_last - 1) / wp.S_last;
-  const long rounds = (wp.wgs + cus - 1) / cus;
-  const double full = wp.mtiles > 1 ? wp.cb * wide_step_us(WIDE_ROWS) + wide_exchange_us(WIDE_ROWS, wp.S) : 0.0;
-  const double last = cb_last * wide_step_us(rest) + wide_exchange_us(rest, wp.S_last);
-  const double steps = rounds * (full > last ? full : last), units = 2.0 * M * m * n / 1.1e9;
-  return 11.0 + 0.015 * M + (steps > units ? steps : units);
+// Beyond fused_rows: the wide kernel, or the weight dequantized and the library's product?  Two models in us of GPU time, fitted to 1200
+// shapes (256x256 to 28672x14336, 129 to 2048 rows, K 2 to 8, bfloat16 and float16) and sweeps of splits.  The wide kernel's is within
+// 10 % for nine in ten of them.  The library's product varies by more from one size to the next, so dequantization's is fitted to the
+// faster ones of like size (30 % of all calls are faster), and the wide kernel is taken where it is a tenth ahead of that.  Of the 1200
+// it is then taken for 708 (321 in a graph) and more than 2 % behind in four (two); of 700 that were not fitted, for 390 (187) and in
+// four (three), 14 % at most.  Wide / dequantized, us in a graph, K4 and bfloat16 where nothing else is said: 14336x4096 512 rows 80 / 99, 1024 rows 149 / 144, K8 156 / 142; 3072x3072 333 rows 27 / 36;
+// 2048x2048 200 rows 19.7 / 18.1; 10624x8320 934 rows 235 / 200; 6400x512 K8 171 rows 18.3 / 16.3; 24448x3712 K8 584 rows float16 146 / 362.
+//
+// Time of a grid of `full` workgroups of t_full us and, behind them, `last` ones of t_last us: they start in order, each on the compute
+// unit that is free first, so short ones fill the places beside a round of full ones that does not take all units.
+inline double grid_us(long full, double t_full, long last, double t_last, int cus) {
+  const long early = cus - full % cus, late = full % cus;             // units that do one full workgroup less, and the others
+  double t_early = (double)(full / cus) * t_full, t_late = t_early + t_full, end = late > 0 ? t_late : t_early;
+  while (last > 0) {
+    const bool on_early = late == 0 || t_early <= t_late;
+    double& t = on_early ? t_early : t_late;
+    last -= on_early ? early : late;
+    t += t_last;
+    if (t > end) end = t;
+  }
+  return end;
 }
-// eager: not from a graph; the host then takes 25 us to queue a dequantization and torch's product (1024x1024 and 4096x1024, 129 to 1024
-// rows, 25.4 to 26.1), and 8 for a wide launch, and where the GPU takes longer the call is still 3 us behind the graph (3072x3072 512
-// rows 32.3 / 34.9).
-inline double dequant_us(int m, int n, int M, int x_dtype, bool eager) {
+// Launches; rotation; steps, which take longer with more bits to decode and on a chip that is full; the end of a workgroup by its
+// rows; partials of column splits by their bytes (written, read, cleared); output.
+inline double wide_us(int m, int n, int K, int M, const WidePlan& wp) {
+  const int cus = num_cu(), nblk = n / 128, rest = M - (wp.mtiles - 1) * WIDE_ROWS;
+  const long full = (long)(m / 128) * wp.S * (wp.mtiles - 1), last = (long)(m / 128) * wp.S_last;
+  const double clock = 0.73 + 0.27 * (full + last < cus ? (double)(full + last) / cus : 1.0);
+  auto workgroup = [&](int rows, int S) {
+    const double step = rows <= 128 ? 0.88 + 0.0024 * rows + 0.022 * (K - 4) : 1.44 + 0.0001 * rows + 0.03 * (K - 4);
+    return ((nblk + S - 1) / S) * step * clock + 0.0285 * rows;
+  };
+  const double partials = 512.0 * ((wp.S > 1 ? (double)full * WIDE_ROWS : 0.0) + (wp.S_last > 1 ? (double)last * rest : 0.0));
+  return 8.3 + 2.4e-6 * M * n + grid_us(full, workgroup(WIDE_ROWS, wp.S), last, workgroup(rest, wp.S_last), cus) + 0.14e-6 * partials + 0.5e-6 * M * m;
+}
+// Launches; dequantization; product, its output, and its serial part by columns; float16 converts the weight once more.
+inline double dequant_us(int m, int n, int M, int x_dtype) {
   const double weights = (double)m * n;
-  const double gpu = 16.0 + weights * (x_dtype == HTR_BF16 ? 0.66e-6 : 1.6e-6) + 2.0 * M * weights / 1.45e9;
-  return !eager ? gpu : gpu < 22.0 ? 25.0 : gpu + 3.0;
+  const bool converted = x_dtype != HTR_BF16;
+  return 9.6 + weights * 0.93e-6 + 2.0 * M * weights / 1.73e9 + 1.03e-6 * M * m + 0.00165 * n + (converted ? 3.7 + weights * 1.6e-6 : 0.0);
+}
+// eager: the call is queued by itself.  The host then takes 25 us for dequantization and product (30 with the conversion), and 9 for a
+// wide launch; longer calls take what the GPU takes.
+inline bool wide_ahead(int m, int n, int K, int M, int x_dtype, const WidePlan& wp, bool eager) {
+  double wide = wide_us(m, n, K, M, wp), dequant = dequant_us(m, n, M, x_dtype);
+  if (eager) {
+    const double host = x_dtype == HTR_BF16 ? 25.0 : 30.0;
+    if (wide < 9.0) wide = 9.0;
+    if (dequant < host) dequant = host;
+  }
+  return 1.1 * wide < dequant;
 }
 
 struct BatchArgs { const uint32_t* qw; float* part; const void* x; const uint8_t* su; int m, n, M, flags; };

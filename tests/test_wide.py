@@ -49,6 +49,37 @@ def test_route(L):
     assert [wide(4096, 4096, 2049), wide(100, 128, 200), wide(128, 128, 200, 3), L.htr_linear_route(128, 128, 9, 200, 0, 1)] == [-5, -4, -6, -3]
 
 
+# m, n, K, rows, type: us in a graph, wide kernel / dequantization and product, and eager, each with one of them at least 15 % ahead
+_MEASURED = [(256, 4352, 3, 1089, 1, (36.7, 26.0), (36.0, 29.6)),
+             (256, 7168, 3, 1112, 0, (40.4, 27.8), (41.0, 29.8)),
+             (384, 512, 6, 579, 1, (20.3, 15.3), (19.8, 30.0)),
+             (512, 384, 4, 810, 1, (19.0, 14.9), (18.6, 29.7)),
+             (512, 768, 4, 753, 0, (21.3, 12.4), (20.9, 24.7)),
+             (512, 8192, 2, 761, 0, (38.8, 30.9), (38.5, 32.3)),
+             (512, 12672, 5, 208, 1, (37.4, 49.5), (36.4, 49.7)),
+             (768, 384, 4, 1137, 0, (20.2, 11.6), (20.0, 25.0)),
+             (768, 5248, 2, 1833, 1, (52.9, 42.8), (52.7, 43.6)),
+             (768, 7168, 4, 934, 0, (41.5, 33.6), (41.9, 33.9)),
+             (1152, 8960, 3, 347, 1, (34.5, 56.7), (34.4, 54.9)),
+             (1408, 3456, 5, 746, 1, (34.5, 40.6), (33.9, 41.4)),
+             (2944, 256, 8, 1998, 1, (25.3, 21.2), (24.9, 29.5)),
+             (3200, 384, 8, 194, 0, (17.1, 12.4), (16.5, 25.8)),
+             (4736, 2304, 6, 1437, 1, (55.7, 68.9), (55.9, 68.8)),
+             (5760, 256, 5, 254, 0, (17.8, 13.2), (17.8, 25.4)),
+             (7168, 1408, 2, 174, 0, (20.3, 29.6), (19.8, 30.5)),
+             (9344, 256, 4, 269, 0, (18.0, 13.9), (17.6, 25.3)),
+             (13568, 1152, 4, 177, 0, (22.6, 36.2), (21.8, 35.6)),
+             (19328, 8832, 2, 733, 0, (266.3, 318.5), (264.6, 310.7)),
+             (20352, 384, 2, 187, 1, (18.1, 42.3), (17.6, 42.1))]
+
+
+@pytest.mark.parametrize("m,n,K,M,x,graph,eager", _MEASURED)
+def test_route_follows_what_was_measured(L, m, n, K, M, x, graph, eager):
+    for mode, (wide, dequantized) in enumerate((graph, eager)):
+        route = L.htr_linear_route(m, n, K, M, x, mode)
+        assert route == (-1 if dequantized < wide else WIDE), (mode, route)
+
+
 def test_what_was_fused_is_never_dequantized(L):
     """Rows and matrices that ops.fused_rows_per_launch names are fused for every type, width and mode: a dequantized weight is rounded
     to bfloat16."""
