@@ -394,7 +394,7 @@ inline double wide_step_us(int rows) { return rows <= 128 ? 0.65 + 0.001 * rows 
 inline double wide_exchange_us(int rows, int S) { return S == 1 ? 0.0 : (1.0 + 0.25 * S) * (rows <= 128 ? 1.0 : 2.0); }
 inline bool make_wide_plan(int m, int n, int M, int want_S, WidePlan& wp) {
   const int nblk = n / 128, rbs = m / 128, cus = num_cu();
-  if ((long)M * n * 2 >= (1L << 31) - (1L << 20)) return false;          // 32-bit byte offsets into the rotated activations
+  if ((long)M * n * 2 >= (1L << 31)) return false;          // 32-bit byte offsets into the rotated activations; none beyond M n 2
   wp.mtiles = (M + WIDE_ROWS - 1) / WIDE_ROWS;
   const int rest = M - (wp.mtiles - 1) * WIDE_ROWS;
   if ((long)rbs * wp.mtiles * WIDE_MAX_SPLITS >= (1L << 31)) return false;
@@ -449,8 +449,9 @@ inline int fused_rows(int m, int n) {
 // 10 % for nine in ten of them.  The library's product varies by more from one size to the next, so dequantization's is fitted to the
 // faster ones of like size (30 % of all calls are faster), and the wide kernel is taken where it is a tenth ahead of that.  Of the 1200
 // it is then taken for 708 (321 in a graph) and more than 2 % behind in four (two); of 700 that were not fitted, for 390 (187) and in
-// four (three), 14 % at most.  Wide / dequantized, us in a graph, K4 and bfloat16 where nothing else is said: 14336x4096 512 rows 80 / 99, 1024 rows 149 / 144, K8 156 / 142; 3072x3072 333 rows 27 / 36;
-// 2048x2048 200 rows 19.7 / 18.1; 10624x8320 934 rows 235 / 200; 6400x512 K8 171 rows 18.3 / 16.3; 24448x3712 K8 584 rows float16 146 / 362.
+// four (three), 14 % at most.  Wide / dequantized, us in a graph, K4 and bfloat16 where nothing else is said: 14336x4096 512 rows
+// 80 / 99, 1024 rows 149 / 144, K8 156 / 142; 3072x3072 333 rows 27 / 36; 2048x2048 200 rows 19.7 / 18.1; 10624x8320 934 rows 235 / 200;
+// 6400x512 K8 171 rows 18.3 / 16.3; 24448x3712 K8 584 rows float16 146 / 362.
 //
 // Time of a grid of `full` workgroups of t_full us and, behind them, `last` ones of t_last us: they start in order, each on the compute
 // unit that is free first, so short ones fill the places beside a round of full ones that does not take all units.

@@ -36,6 +36,14 @@ def test_wide_plan(L, m, n):
         assert (p is None) == (want > nblk or -(-nblk // -(-nblk // want)) != want) and (p is None or p[3] == want)
 
 
+def test_the_longest_rows_have_a_plan(L):
+    """Up to what a launch takes in columns (65535 blocks) 65 to 128 rows have one, as every other row count."""
+    for n in (8384512, 8388480):
+        for M in (64, 65, 127, 128):
+            assert _plan(L, 128, n, 4, M, 0) is not None and L.htr_workspace_bytes(128, n, 4, M, 0) >= 256 + M * n * 2
+    assert _plan(L, 128, 8388480, 4, 129, WIDE) is None and L.htr_workspace_bytes(128, 8388480, 4, 129, WIDE) == 0      # 2^31 bytes of activations
+
+
 def test_route(L):
     wide = lambda m, n, M, x=0, eager=0: L.htr_linear_route(m, n, 4, M, x, eager)
     assert wide(4096, 4096, 128) == 0 and wide(4096, 4096, 129) == WIDE and wide(14336, 4096, 512) == WIDE
