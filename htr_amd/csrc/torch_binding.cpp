@@ -27,7 +27,6 @@ decltype(&htr_moe_experts) f_moe = nullptr;
 decltype(&htr_linear_route) f_route = nullptr;
 decltype(&htr_dequant_w) f_dequant = nullptr;
 
-
 int dtype_code(at::ScalarType t) {
   switch (t) {
     case at::kBFloat16: return 0;
@@ -67,9 +66,9 @@ bool weight_ok(const at::Tensor& qw, const at::Tensor& sc, const at::Tensor& su,
 
 // linear(x, qweight, scales, su, sv, bias, workspace address, its bytes, address of its failure word (0: none), stream, rows)
 // -> tensor or None; None also while the stream is being captured (a capture has workspaces of its own), after a launch
-// on the workspace gave up, and for more activation rows than `rows` (if not
-// given 128).  Beyond 128 rows the call goes where the library says:
-// one launch, or the weight dequantized and multiplied by torch, as ops._linear_impl does it.
+// on the workspace gave up, and for more activation rows than `rows` (128 if not given).  Beyond 128 rows the call goes where
+// htr_linear_route says, as in ops._linear_impl: one launch, or the weight dequantized and multiplied by torch, for which the workspace may
+// be missing (address 0).
 PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs < 10 || nargs > 11 || f_linear == nullptr || !THPVariable_CheckExact(args[0])) Py_RETURN_NONE;
@@ -226,7 +225,8 @@ PyObject* wait_word(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 // bind(version of the library's C ABI, version of the running torch, addresses of htr_linear, htr_stream_capture_id,
-// htr_moe_scratch_bytes, htr_moe_experts and, for linear() beyond 128 rows, htr_linear_route and htr_dequant_w); ImportError where either version is not the one that this file was compiled with
+// htr_moe_scratch_bytes, htr_moe_experts and, for linear() beyond 128 rows, htr_linear_route and htr_dequant_w); ImportError where either
+// version is not the one that this file was compiled with
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 6 && nargs != 8) { PyErr_SetString(PyExc_TypeError, "bind wants two versions and four or six addresses"); return nullptr; }
   const long abi = PyLong_AsLong(args[0]);
