@@ -161,10 +161,10 @@ def test_two_streams_with_their_own_workspaces(dev, Ma, Mb):
     assert all(torch.equal(o, want_b) for o in outs_b)
 
 
-@pytest.mark.parametrize("M", [1, 32])
-def test_bounded_wait_gives_up_cleanly(dev, oracle, M):
+@pytest.mark.parametrize("M", [1, 32, 97, 333])
+def test_bounded_wait_gives_up_cleanly(dev, oracle, M, monkeypatch):
     """The finishing workgroup's wait for the other chunks' partials is bounded (chunked kernel at 1 row; batched kernel
-    at 32 rows, where the splits of a row block wait for each other).  With the bound forced down to a single
+    at 32 rows and wide kernel at 97 and, asked for, 333, where the splits of a row block wait for each other).  With the bound forced down to a single
     poll from the host, a launch either comes out right or marks what it could not finish: NaN for those rows, bit 0
     of the workspace's status word and the host-side flag; every kernel still runs to its end.  The call after a
     failure clears the workspace and raises; the one after that is right again.  Nothing here touches the operator's
@@ -172,6 +172,9 @@ def test_bounded_wait_gives_up_cleanly(dev, oracle, M):
     from htr_amd import _native, ops
     print(f"bounded wait M={M}", flush=True)
     L = _native.lib()
+    if M > 128:
+        monkeypatch.setattr(ops, "NSPLIT", 1 << 27)
+        monkeypatch.setattr(ops, "GEMV_LOOP_MAX", M)
     qw, sc, su, sv, x = _case(2048, 4096, 4, M, 4500 + M)
     d = [t.to(dev) for t in (qw, sc, su, sv)]
     ref = _ref(oracle, qw, sc, su, sv, x)

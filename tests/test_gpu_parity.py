@@ -104,6 +104,15 @@ def test_prefill_path_dequant_then_gemm(dev, oracle):
     ref = _ref(oracle, qw, sc, su, sv, x, bias)
     # bf16 weights and bf16 output: compare at bf16 resolution of the largest magnitudes
     assert _rel(y.float().cpu().numpy(), ref) <= 2.0 ** -6
+    # queued by itself that call is one launch; these are dequantized: float32 activations, and more rows of a larger matrix
+    from htr_amd import _native
+    route = lambda m, n, M, x_dtype: _native.lib().htr_linear_route(m, n, 4, M, x_dtype, 1)
+    assert (route(512, 384, 160, 0), route(512, 384, 160, 2), route(1024, 2048, 1024, 0)) == (1 << 27, -1, -1)
+    y = ops.linear(x.float().to(dev), *[t.to(dev) for t in (qw, sc, su, sv)], bias.float().to(dev))
+    assert y.dtype == torch.float32 and _rel(y.cpu().numpy(), ref) <= 2.0 ** -8                        # bf16 weights only
+    qw, sc, su, sv, x = _case(1024, 2048, 4, 1024, 809)
+    y = ops.linear(x.to(dev), *[t.to(dev) for t in (qw, sc, su, sv)])
+    assert _rel(y.float().cpu().numpy(), _ref(oracle, qw, sc, su, sv, x)) <= 2.0 ** -6
 
 
 def test_reference_env_knobs(dev, oracle, monkeypatch):
@@ -412,7 +421,7 @@ def test_more_than_128_rows_in_one_launch(dev, oracle, K, M, m, n, S, T):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_more_than_128_rows_through_ops_with_bias(dev, oracle, dtype, monkeypatch):
     from htr_amd import ops
-    print(f"gemm kernel through ops, {dtype}", flush=True)
+    print(f"gemm kernel through ops, {dtype}", flush=True)          # HTR_GEMV_LOOP_MAX leaves the wide kernel out
     monkeypatch.setattr(ops, "GEMV_LOOP_MAX", 1 << 30)
     qw, sc, su, sv, x = _case(384, 512, 4, 210, 9100, dtype)
     bias = torch.randn(384, generator=torch.Generator().manual_seed(9)).to(dtype)
@@ -424,30 +433,34 @@ def test_more_than_128_rows_through_ops_with_bias(dev, oracle, dtype, monkeypatc
 
 
 def test_fused_row_limit_follows_the_shape(dev, oracle, monkeypatch):
-    """ops.linear takes one launch of the fused GEMM kernel, launches of 128 rows or dequantize + GEMM depending on shape
+    """ops.linear takes one launch of the wide kernel, launches of 128 rows or dequantize + GEMM depending on shape
     and row count; all three give the same product."""
-    from htr_amd import ops
+    from htr_amd import _native, ops
+    route = lambda M: _native.lib().htr_linear_route(14336, 4096, 4, M, 0, 1)
+    assert (route(192), route(484), route(2048)) == (1 << 27, 1 << 27, -1)
     big = ops.ONE_LAUNCH
     assert ops.fused_max_rows(4096, 4096) == 384 and ops.fused_max_rows(14336, 4096) == 384 and ops.fused_max_rows(1024, 4096) == 128
     assert ops.fused_max_rows(4096, 14336) == 512 and ops.fused_rows_per_launch(4096, 14336, 512) == big
     assert [ops.fused_rows_per_launch(14336, 4096, M) for M in (1, 128, 129, 384, 385)] == [128, 128, big, big, 0]
     assert [ops.fused_rows_per_launch(4096, 4096, M) for M in (129, 384, 385)] == [big, big, 0]
     assert ops.fused_rows_per_launch(2048, 2048, 129) == 0
-    print("gemm kernel at the policy's shape", flush=True)
+    print("wide kernel at the policy's shape", flush=True)
     qw, sc, su, sv, x = _case(14336, 4096, 4, 192, 9200)
     d = [t.to(dev) for t in (qw, sc, su, sv)]
     ref = _ref(oracle, qw, sc, su, sv, x)
-    y = ops.linear_f32out(x.to(dev), *d).cpu().numpy()                                # one launch of the GEMM kernel
+    y = ops.linear_f32out(x.to(dev), *d).cpu().numpy()                                # one launch of the wide kernel
     assert _rel(y, ref) <= REL_TOL
     monkeypatch.setattr(ops, "GEMV_LOOP_MAX", 1 << 30)
     monkeypatch.setattr(ops, "LAUNCH_MAX_M", 128)
     x200 = torch.cat([x, x[:8]])
-    y2 = ops.linear_f32out(x200.to(dev), *d).cpu().numpy()                            # 128 + 72 rows, batched kernel
+    y2 = ops.linear_f32out(x200.to(dev), *d).cpu().numpy()                            # 128 + 72 rows, wide kernel
     assert _rel(y2[:192], ref) <= REL_TOL and _rel(y2[192:], ref[:8]) <= REL_TOL
     monkeypatch.setattr(ops, "GEMV_LOOP_MAX", None)
     monkeypatch.setattr(ops, "LAUNCH_MAX_M", ops.ONE_LAUNCH)
-    y3 = ops.linear(torch.cat([x, x, x[:100]]).to(dev), *d).float().cpu().numpy()     # 484 rows: dequantize + GEMM
+    y3 = ops.linear(torch.cat([x, x, x[:100]]).to(dev), *d).float().cpu().numpy()     # 484 rows: wide kernel
     assert _rel(y3[:192], ref) <= 2.0 ** -6
+    y4 = ops.linear(x.repeat(11, 1)[:2048].to(dev), *d).float().cpu().numpy()         # dequantize + GEMM
+    assert _rel(y4[:192], ref) <= 2.0 ** -6 and _rel(y4[1920:], ref[:128]) <= 2.0 ** -6
 
 
 def test_moe_expert_stack_top6_of_64(dev, oracle):

@@ -263,6 +263,10 @@ def test_what_the_extension_leaves_to_the_general_path(dev):
     ws = ops._WORKSPACES[(0, stream)]
     call = lambda x=x, w=w, bias=None, ptr=ws.ptr, size=ws.size, failed=0: fast.linear(x, *w, bias, ptr, size, failed, stream)
     assert torch.equal(call(), want) and call(bias=bias) is not None
+    upto = lambda rows, x=x: fast.linear(x, *w, None, ws.ptr, ws.size, 0, stream, rows)      # as ops calls it
+    assert torch.equal(upto(2048), want) and torch.equal(upto(3), want) and upto(2) is None
+    assert upto(128, x.repeat(43, 1)) is None and torch.equal(upto(2048, x.repeat(43, 1)), ops.linear(x.repeat(43, 1), *w))      # 129 rows
+    assert upto(4096, x.repeat(683, 1)) is None                                   # 2049 rows: more than one launch holds
     flag = torch.ones(1, dtype=torch.int32)
     assert call(failed=flag.data_ptr()) is None                                   # an earlier launch gave up
     assert call(size=256) is None and call(ptr=ws.ptr + 8) is None                # too small, misaligned

@@ -74,8 +74,15 @@ def test_number_of_experts_around_one_launch_of_addresses(dev, E):
     few = torch.tensor([0, 1, E // 2, E - 2, E - 1])
     pick = torch.stack([torch.randperm(5, generator=g)[:2] for _ in range(11)])
     x, w = torch.randn(11, 128, generator=g).bfloat16().to(dev), torch.rand(11, 2, generator=g).to(dev)
-    y = ops.moe_experts(x, few[pick].to(dev), w, gate_up, down)
+    chosen = few[pick].to(dev)
+    y = ops.moe_experts(x, chosen, w, gate_up, down)
     assert torch.equal(y, ops.moe_experts(x, pick.to(dev), w, [gate_up[e] for e in few], [down[e] for e in few]))
+    graph = torch.cuda.CUDAGraph()                                                # the addresses are recorded with the launch
+    with torch.cuda.graph(graph):
+        z = ops.moe_experts(x, chosen, w, gate_up, down)
+    for _ in range(3):
+        graph.replay()
+        assert torch.equal(z, y)
 
 
 def test_expert_numbers_out_of_range_and_graph_capture(dev):

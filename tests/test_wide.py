@@ -1,4 +1,5 @@
-"""k_linear_wide (65 rows and more) against the oracle: edges of its 32- and 256-row tiles, every K, splits, types and alignments; and who takes a call."""
+"""k_linear_wide (65 rows and more) against the oracle: edges of its 32- and 256-row tiles, every K, splits, types and alignments; and who
+takes a call beyond 128 rows: the rule, what was measured on both of its sides, and the two host paths that follow it."""
 import ctypes
 
 import numpy as np
@@ -117,6 +118,24 @@ def test_the_general_path_asks_the_library(L, monkeypatch, m, n, M, dtype):
         assert ops._route(x, None, m, n, 4, M, ops.fused_rows_per_launch(m, n, M)) == want
 
 
+def test_a_shared_capture_buffer_that_is_too_small(L, monkeypatch):
+    """It cannot grow while a capture is in progress: the call then goes where it went before the wide kernel was there."""
+    from types import SimpleNamespace
+    from htr_amd import ops
+    x = lambda M, n: SimpleNamespace(dtype=torch.bfloat16, device=torch.device("cuda", 0), requires_grad=False)
+    monkeypatch.setattr(ops, "_followed", lambda *a: False)
+    monkeypatch.setattr(ops, "SHARE_CAPTURE_WORKSPACE", True)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    for m, n, M in ((4096, 4096, 200), (14336, 4096, 484)):
+        assert L.htr_linear_route(m, n, 4, M, 0, 0) == WIDE
+        before = ops.fused_rows_per_launch(m, n, M)
+        need = L.htr_workspace_bytes(m, n, 4, M, WIDE)
+        for held, want in ((None, (before, 0)), (need - 1, (before, 0)), (need, (M, WIDE))):
+            table = {} if held is None else {(0, "shared"): SimpleNamespace(buf=SimpleNamespace(numel=lambda: held))}
+            monkeypatch.setattr(ops, "_WORKSPACES", table)
+            assert ops._route(x(M, n), None, m, n, 4, M, before) == want
+
+
 def _case(m, n, K, M, seed, dtype=torch.bfloat16):
     from htr_amd import wire
     qw, sc, su, sv = wire.synth_linear(m, n, K, seed)
@@ -181,6 +200,55 @@ def test_wide_kernel(dev, oracle, L, K, M, m, n, S, xt, off):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,M,splits", [(5504, 1408, 257, (4, 1)), (2816, 3712, 260, (8, 3)), (6144, 4096, 333, (3, 2)), (2176, 7040, 280, (8, 4)),
+                                          (5504, 1280, 513, (2, 1)), (1920, 3712, 530, (6, 3))])
+def test_last_tile_with_a_split_of_its_own(dev, oracle, L, m, n, M, splits):
+    """Plans of the policy whose last tile is split otherwise than the full ones: its workgroups and its slots start behind theirs."""
+    _, wgs, tiles, S, _, _ = _plan(L, m, n, 4, M, WIDE)
+    assert (S, wgs // (m // 128) - S * (tiles - 1)) == splits
+    test_wide_kernel(dev, oracle, L, 4, M, m, n, 0, "bf16", 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,S", [(97, 4), (128, 8), (300, 2), (513, 5)])
+def test_grid_beyond_the_compute_units(dev, oracle, L, M, S):
+    """On a device of fewer compute units than the grid has workgroups (the planner's override) the last split finishes every row."""
+    m, n = 1024, 2048
+    try:
+        assert L.htr_plan_device_override(8, 160 * 1024) == 0
+        if _plan(L, m, n, 4, M, WIDE | S) is None:                                # 16 column blocks in 5 splits: one would be empty
+            n = 1920
+        assert _plan(L, m, n, 4, M, WIDE | S)[1] > 8
+        test_wide_kernel(dev, oracle, L, 4, M, m, n, S, "bf16", 0)
+    finally:
+        assert L.htr_plan_device_override(0, 0) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [97, 200, 333])
+def test_captured_and_replayed(dev, L, M):
+    """A captured call of the wide kernel, replayed with new inputs and eager work in between, gives what the eager call gives."""
+    from htr_amd import ops
+    print(f"wide kernel in a graph M={M}", flush=True)
+    m = n = 4096
+    w, x = _case(m, n, 4, M, 80)
+    d, x_in = [t.to(dev) for t in w], x.to(dev)
+    other, x_other = [t.to(dev) for t in _case(384, 512, 3, 70, 81)[0]], torch.randn(70, 512, device=dev).bfloat16()
+    assert M <= 128 or {L.htr_linear_route(m, n, 4, M, 0, eager) for eager in (0, 1)} == {WIDE}
+    ops.linear(x_in, *d)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ops.linear(x_in, *d)
+    for i in range(3):
+        x_in.copy_(torch.randn(M, n, generator=torch.Generator().manual_seed(i)))
+        ops.linear(x_other, *other)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ops.linear(x_in, *d)), i
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,n,M", [(512, 1024, 129), (2048, 2048, 700), (4096, 4096, 400)])
 def test_float32_activations_stay_float32(dev, m, n, M, monkeypatch):
     """Beyond the rows that were always fused: the float32 product with the dequantized weight, bit for bit, on both host paths."""
@@ -196,7 +264,7 @@ def test_float32_activations_stay_float32(dev, m, n, M, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,M", [(4096, 4096, 65), (4096, 4096, 200), (2048, 2048, 700)])
+@pytest.mark.parametrize("m,n,M", [(4096, 4096, 65), (4096, 4096, 200), (2048, 2048, 700), (17408, 2048, 264)])
 def test_rows_beyond_64_through_ops(dev, oracle, m, n, M, monkeypatch):
     """Both host paths take the same route and give the same result; what torch differentiates goes on being differentiated."""
     from htr_amd import _native, ops
@@ -215,6 +283,66 @@ def test_rows_beyond_64_through_ops(dev, oracle, m, n, M, monkeypatch):
     leaf = xd.clone().requires_grad_()
     y = ops.linear(leaf, *d)
     assert y.requires_grad == (M > 128 and ops.fused_rows_per_launch(m, n, M) == 0)
+
+
+def _followed_by_dequantization(L, m, n, M):
+    assert {L.htr_linear_route(m, n, 4, M, x, eager) for x in (0, 1, 2) for eager in (0, 1)} == {-1}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("cast", [None, torch.bfloat16, torch.float16])
+def test_dequantization_and_product_on_both_host_paths(dev, oracle, L, dtype, cast, monkeypatch):
+    """Bias, more dimensions and autocast where the weight is dequantized: C++ and Python give the same, near the oracle's product."""
+    from htr_amd import _native, ops
+    m, n, M = 1024, 2048, 1024
+    print(f"dequantized {dtype}, autocast {cast}", flush=True)
+    _followed_by_dequantization(L, m, n, M)
+    w, x = _case(m, n, 4, M, 82, dtype)
+    d, xd, bias = [t.to(dev) for t in w], x.to(dev), torch.randn(m, generator=torch.Generator().manual_seed(3)).to(dtype).to(dev)
+    got = {}
+    for path in (None, False):                                                    # C++, Python
+        monkeypatch.setattr(_native, "_fast", path)
+        with torch.autocast("cuda", dtype=cast or torch.bfloat16, enabled=cast is not None):
+            got[path] = [ops.linear(xd, *d), ops.linear(xd, *d, bias), ops.linear(xd.view(4, M // 4, n), *d, bias)]
+        if path is None:
+            assert _native._fast not in (None, False)
+    assert all(torch.equal(a, b) for a, b in zip(got[None], got[False]))
+    plain, biased, three = got[None]
+    assert all(y.dtype == dtype for y in got[None]) and three.shape == (4, M // 4, m) and torch.equal(three.view(M, m), biased)
+    for y, ref in ((plain, _ref(oracle, w, x)), (biased, _ref(oracle, w, x, bias.cpu()))):
+        assert np.abs(y.double().cpu().numpy() - ref).max() / np.abs(ref).max() <= 2.0 ** -6      # bfloat16 weights, bfloat16 or cast results
+
+
+@pytest.mark.gpu
+def test_what_torch_follows_beyond_128_rows(dev, L):
+    """Derivatives where the weight is dequantized, of the activations and of the bias, forward and backward, and vmap (in float32, where
+    torch's products of batches are safe)."""
+    from torch.autograd import forward_ad
+    from htr_amd import ops
+    m, n, M = 1024, 2048, 1024
+    print("followed by torch", flush=True)
+    _followed_by_dequantization(L, m, n, M)
+    w, x = _case(m, n, 4, M, 83, torch.float32)
+    d, xd = [t.to(dev) for t in w], x.to(dev)
+    g = torch.Generator(device=dev).manual_seed(4)
+    t, bias, bt = (torch.randn(*shape, device=dev, generator=g) for shape in ((M, n), (m,), (m,)))
+    W = ops.dequant_w(*d).float()
+    near = lambda a, b: float((a - b).norm() / b.norm()) <= 1e-5                  # float32 sums in another order
+    want, moved = xd @ W.T + bias, t @ W.T
+    with forward_ad.dual_level():
+        for call, tangent in ((lambda: ops.linear(forward_ad.make_dual(xd, t), *d, bias), moved),
+                              (lambda: ops.linear(xd, *d, forward_ad.make_dual(bias, bt)), bt.expand(M, m))):
+            y = forward_ad.unpack_dual(call())
+            assert near(y.primal, want) and near(y.tangent, tangent)
+    both = torch.func.vmap(lambda a: ops.linear(a, *d, bias))(torch.stack([xd, t]))
+    assert near(both[0], want) and near(both[1], moved + bias)
+    leaf, lb = xd.clone().requires_grad_(), bias.clone().requires_grad_()
+    ops.linear(leaf, *d, lb).backward(moved)
+    assert near(leaf.grad, moved @ W) and near(lb.grad, moved.sum(0))
+    assert ops.linear(xd, *d, lb).requires_grad and not ops.linear(leaf.detach(), *d, lb.detach()).requires_grad
+    with torch.no_grad():
+        assert not ops.linear(leaf, *d, lb).requires_grad and near(ops.linear(leaf, *d, lb), want)
 
 
 @pytest.mark.gpu
