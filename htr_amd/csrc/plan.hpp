@@ -387,9 +387,11 @@ inline bool wants_gemm(int M, int nsplit) { return nsplit > 0 ? (nsplit & (1 << 
 struct WidePlan { int S, S_last, cb, mtiles, wgs; };
 constexpr int WIDE_MAX_SPLITS = 8;
 inline bool split_fits(int nblk, int S) { const int cb = (nblk + S - 1) / S; return S >= 1 && S <= nblk && (nblk + cb - 1) / cb == S; }      // none empty
-// us per column block of a workgroup whose tile holds `rows` rows.  K4, 48 workgroups on the chip: 96 rows 0.76, 128 rows 0.78, 256
-// rows 1.2 (from 129 rows on two waves of a SIMD multiply); exchange between S splits at 128 / 256 rows: 2 / 4.7 for two, 3 / 6.2
-// for four.
+// For the choice of splits alone (wide_us says what a call takes): us per column block of a workgroup whose tile holds `rows` rows.  K4, 48
+// workgroups on the chip: 96 rows 0.76, 128 rows 0.78, 256 rows 1.2 (from 129 rows on two waves of a SIMD multiply); exchange between S
+// splits at 128 / 256 rows: 2 / 4.7 for two, 3 / 6.2 for four.  On 405 sizes at K 2 to 8 the chosen split takes 1.3 % more than the best
+// one on average.  Five and seven splits are not among them: us at 4 / 5 / 6 / 7 of them, K4, 4096x4480 97 rows 21.9 / 21.6 / 20.9 / 23.6,
+// 256 rows 32.3 / 34.5 / 33.3 / 37.4, 6144x8960 200 rows 48.8 / 47.3 / - / -, 256 rows 53.6 / 53.0 / - / -.
 inline double wide_step_us(int rows) { return rows <= 128 ? 0.65 + 0.001 * rows : 0.96 + 0.001 * rows; }
 inline double wide_exchange_us(int rows, int S) { return S == 1 ? 0.0 : (1.0 + 0.25 * S) * (rows <= 128 ? 1.0 : 2.0); }
 inline bool make_wide_plan(int m, int n, int M, int want_S, WidePlan& wp) {
@@ -421,9 +423,10 @@ inline size_t wide_slot_bytes(int m, int M, const WidePlan& wp) {
   return (full + rest) * 128 * sizeof(float);
 }
 // The wide kernel: nsplit bit 27, with the split of all tiles in the low bits (0 = its own policy), and by policy from 65 rows to 128.
-// us of the call with its rotation, k_linear_batch / k_linear_wide: 14336x4096 K4 65 rows 32.5 / 26.3, 97 rows 33.7 / 28.4, 128 rows
-// 35.3 / 29.8, K8 38.0 / 31.4 at 97 rows; 4096x14336 K4 65 rows 30.0 / 26.3; 2048x2048 K4 128 rows 16.4 / 16.0; 152064x4096 K4 128 rows
-// 249 / 205; 128x128 65 rows 11.2 / 8.9; the worst are 1024x1024 K5 65 rows 12.5 / 13.1 and K2 to K8 128 rows level.  At 64 rows it is
+// us of the call with its rotation, in a graph over several weights, k_linear_batch / k_linear_wide: 14336x4096 K4 65 rows 32.6 / 26.9, 97
+// rows 35.2 / 32.1, 128 rows 38.0 / 33.7, K8 97 rows 39.3 / 33.1, K5 float16 97 rows 36.5 / 30.6; 4096x14336 K4 65 rows 32.8 / 28.9, K8
+// 128 rows 41.7 / 40.7; 2048x2048 K4 128 rows 17.1 / 15.5; 28672x4096 K4 128 rows 61.3 / 48.8.  Of 260 sizes (13 matrices, K 2 to 8, 65
+// to 128 rows) it was behind in none; the nearest, 1024x1024 K5 65 rows, 13.3 / 13.1 and, measured again, 12.6 / 12.8.  At 64 rows it is
 // behind (14336x4096 K4 23.9 / 25.7, 2048x2048 11.9 / 13.1).  From 129 rows against k_linear_gemm: 6144x4096 K4 129 rows 32.2 / 24.3, 256
 // rows 40.1 / 29.7, 333 rows 39.8 / 37.1; 14336x4096 256 rows 50.6 / 44.3, 333 rows 76.3 / 60.4, 512 rows 94.9 / 72.4; 4096x14336 256 rows
 // 60.6 / 52.2 (htr_linear_route says who takes it there).
@@ -444,14 +447,15 @@ inline int fused_rows(int m, int n) {
   return (long)m * n < 4096L * 4096 ? HTR_MAX_ROWS_PER_TILE : n >= 8192 ? 512 : 384;
 }
 
-// Beyond fused_rows: the wide kernel, or the weight dequantized and the library's product?  Two models in us of GPU time, fitted to 1200
-// shapes (256x256 to 28672x14336, 129 to 2048 rows, K 2 to 8, bfloat16 and float16) and sweeps of splits.  The wide kernel's is within
-// 10 % for nine in ten of them.  The library's product varies by more from one size to the next, so dequantization's is fitted to the
-// faster ones of like size (30 % of all calls are faster), and the wide kernel is taken where it is a tenth ahead of that.  Of the 1200
-// it is then taken for 708 (321 in a graph) and more than 2 % behind in four (two); of 700 that were not fitted, for 390 (187) and in
-// four (three), 14 % at most.  Wide / dequantized, us in a graph, K4 and bfloat16 where nothing else is said: 14336x4096 512 rows
-// 80 / 99, 1024 rows 149 / 144, K8 156 / 142; 3072x3072 333 rows 27 / 36; 2048x2048 200 rows 19.7 / 18.1; 10624x8320 934 rows 235 / 200;
-// 6400x512 K8 171 rows 18.3 / 16.3; 24448x3712 K8 584 rows float16 146 / 362.
+// Beyond fused_rows: the wide kernel, or the weight dequantized and the library's product?  Two models in us of GPU time, fitted to 2394
+// measurements (256x256 to 28672x14336 and the matrices of common models, 129 to 2048 rows, K 2 to 8, bfloat16 and float16) and sweeps of
+// splits.  The wide kernel's is within 8 % for nine in ten.  The library's product varies by more from one size to the next; its model is
+// fitted so that two calls in five are faster, and the wide kernel is taken where it is 4 % ahead of that.  Of 975 sizes that were not
+// fitted it is taken for 366 in a graph and more than 3 % behind in seven (of 800 queued eagerly for 526, and eight), 29 % at worst
+// (4352x384 K5 1913 rows float16 36 / 28); for 77 (66) that are dequantized it would be more than 3 % ahead.  Wide / dequantized, us
+// in a graph, K4 and bfloat16 where nothing else is said: 14336x4096 512 rows 80 / 99, 1024 rows 149 / 144, K8 156 / 142; 3072x3072 333
+// rows 27 / 36; 2048x2048 200 rows 19.7 / 18.1; 10624x8320 934 rows 235 / 200; 6400x512 K8 171 rows 18.3 / 16.3; 24448x3712 K8 584 rows
+// float16 146 / 362.
 //
 // Time of a grid of `full` workgroups of t_full us and, behind them, `last` ones of t_last us: they start in order, each on the compute
 // unit that is free first, so short ones fill the places beside a round of full ones that does not take all units.
@@ -467,35 +471,39 @@ inline double grid_us(long full, double t_full, long last, double t_last, int cu
   }
   return end;
 }
-// Launches; rotation; steps, which take longer with more bits to decode and on a chip that is full; the end of a workgroup by its
-// rows; partials of column splits by their bytes (written, read, cleared); output.
+// Launches; rotation; the workgroups, each with first loads and decode, steps that take longer with more bits, and an output side by
+// its rows; partials of column splits by their bytes (written, read, cleared); output; and the matrix work of the whole chip, which slows
+// all steps the more of it there is.
 inline double wide_us(int m, int n, int K, int M, const WidePlan& wp) {
-  const int cus = num_cu(), nblk = n / 128, rest = M - (wp.mtiles - 1) * WIDE_ROWS;
+  const int nblk = n / 128, rest = M - (wp.mtiles - 1) * WIDE_ROWS;
   const long full = (long)(m / 128) * wp.S * (wp.mtiles - 1), last = (long)(m / 128) * wp.S_last;
-  const double clock = 0.73 + 0.27 * (full + last < cus ? (double)(full + last) / cus : 1.0);
   auto workgroup = [&](int rows, int S) {
-    const double step = rows <= 128 ? 0.88 + 0.0024 * rows + 0.022 * (K - 4) : 1.44 + 0.0001 * rows + 0.03 * (K - 4);
-    return ((nblk + S - 1) / S) * step * clock + 0.0285 * rows;
+    const double step = rows <= 128 ? 0.68 + 0.0007 * rows + 0.02 * (K - 4) : 1.05 + 0.025 * (K - 4);
+    return 4.7 + ((nblk + S - 1) / S) * step + 0.025 * rows;
   };
   const double partials = 512.0 * ((wp.S > 1 ? (double)full * WIDE_ROWS : 0.0) + (wp.S_last > 1 ? (double)last * rest : 0.0));
-  return 8.3 + 2.4e-6 * M * n + grid_us(full, workgroup(WIDE_ROWS, wp.S), last, workgroup(rest, wp.S_last), cus) + 0.14e-6 * partials + 0.5e-6 * M * m;
+  return 4.6 + 2.1e-6 * M * n + grid_us(full, workgroup(WIDE_ROWS, wp.S), last, workgroup(rest, wp.S_last), num_cu()) + 0.14e-6 * partials +
+         0.15e-6 * M * m + 0.68e-9 * M * m * n;
 }
-// Launches; dequantization; product, its output, and its serial part by columns; float16 converts the weight once more.
+// Launches; dequantization; product, its output, and a serial part by columns, which is less for few tiles (of 128x128: the library then
+// splits the columns) and comes again with every round of 256x256 tiles over the chip; float16 converts the weight once more.
 inline double dequant_us(int m, int n, int M, int x_dtype) {
   const double weights = (double)m * n;
-  const bool converted = x_dtype != HTR_BF16;
-  return 9.6 + weights * 0.93e-6 + 2.0 * M * weights / 1.73e9 + 1.03e-6 * M * m + 0.00165 * n + (converted ? 3.7 + weights * 1.6e-6 : 0.0);
+  const int cus = num_cu();
+  const long few = (long)(m / 128) * ((M + 127) / 128), tiles = (long)((m + 255) / 256) * ((M + 255) / 256), rounds = (tiles + cus - 1) / cus;
+  const double columns = 1.22e-3 * n * (few < 50 ? few / 50.0 : 1.0) + 1.37e-3 * n * rounds;
+  return 9.7 + weights * 0.86e-6 + M * weights * 0.99e-9 + 1.17e-6 * M * m + columns + (x_dtype == HTR_BF16 ? 0.0 : 3.5 + weights * 1.6e-6);
 }
-// eager: the call is queued by itself.  The host then takes 25 us for dequantization and product (30 with the conversion), and 9 for a
-// wide launch; longer calls take what the GPU takes.
+// eager: the call is queued by itself.  The host then takes 23 to 25 us for dequantization and product (28 to 30 with the conversion), and
+// 9 for a wide launch; longer calls take what the GPU takes.
 inline bool wide_ahead(int m, int n, int K, int M, int x_dtype, const WidePlan& wp, bool eager) {
   double wide = wide_us(m, n, K, M, wp), dequant = dequant_us(m, n, M, x_dtype);
   if (eager) {
-    const double host = x_dtype == HTR_BF16 ? 25.0 : 30.0;
+    const double host = x_dtype == HTR_BF16 ? 23.5 : 28.5;
     if (wide < 9.0) wide = 9.0;
     if (dequant < host) dequant = host;
   }
-  return 1.1 * wide < dequant;
+  return 1.04 * wide < dequant;
 }
 
 struct BatchArgs { const uint32_t* qw; float* part; const void* x; const uint8_t* su; int m, n, M, flags; };

@@ -71,7 +71,6 @@ _MEASURED = [(256, 4352, 3, 1089, 1, (36.7, 26.0), (36.0, 29.6)),
              (768, 7168, 4, 934, 0, (41.5, 33.6), (41.9, 33.9)),
              (1152, 8960, 3, 347, 1, (34.5, 56.7), (34.4, 54.9)),
              (1408, 3456, 5, 746, 1, (34.5, 40.6), (33.9, 41.4)),
-             (2944, 256, 8, 1998, 1, (25.3, 21.2), (24.9, 29.5)),
              (3200, 384, 8, 194, 0, (17.1, 12.4), (16.5, 25.8)),
              (4736, 2304, 6, 1437, 1, (55.7, 68.9), (55.9, 68.8)),
              (5760, 256, 5, 254, 0, (17.8, 13.2), (17.8, 25.4)),
