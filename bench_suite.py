@@ -215,7 +215,8 @@ def prefill(dev):
 
             t1 = eager(one_launch)
             rec = {"M": M, "gemm_us": round(tg, 1), "dequant_plus_gemm_us": round(td + tg, 1), "one_fused_launch_us": round(t1, 1),
-                   "ops_rows_per_fused_launch": ops.fused_rows_per_launch(m, n, M)}       # 0: ops.linear dequantizes
+                   # 2**27: ops.linear takes the wide kernel, 0: the decode kernels, -1: it dequantizes
+                   "route": L.htr_linear_route(m, n, 4, M, _native.BF16, 1)}
             if M > 128:
                 old_max, old_rows = ops.GEMV_LOOP_MAX, ops.LAUNCH_MAX_M
                 ops.GEMV_LOOP_MAX, ops.LAUNCH_MAX_M = 10 ** 9, 128

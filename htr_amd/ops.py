@@ -27,10 +27,13 @@ NSPLIT = int(os.environ.get("HTR_NSPLIT", "0"))
 # the product, as the reference does for prefill (HTR_PREFILL="w", htr/ops.py:52-54,89-93); up to it, fused launches
 # run (the reference's HTR_GEMV_LOOP_MAX, htr/ops.py:59-61): up to 128 rows the decode kernels; beyond, ONE launch of a kernel that
 # decodes the weight once per tile of activation rows.
-# Which of the two is ahead beyond 128 rows says htr_linear_route, by a model of both (the wide kernel, tiles of 256 rows, against
-# dequantization and product).  The limits below are those of the kernel with tiles of 96 or 128 rows (htr_linear's own policy),
-# which still takes what the wide kernel may not: calls whose derivatives or transforms torch follows go on as they went before it.
-# HTR_GEMV_LOOP_MAX overrides the row limit for every shape (launches of LAUNCH_MAX_M rows up to it) and leaves the wide kernel out.
+# htr_linear_route says which beyond 128 rows, for the C++ host path and for this one.  Up to the limits below a call is always one launch of
+# the wide kernel (tiles of 256 rows); beyond them it is where models put it ahead of dequantization and product, for 16-bit
+# activations.  A call whose derivatives or transforms torch follows is never moved from the product to a launch: beyond the limits
+# it is dequantized; up to them it is a launch, without a derivative in the activations, as every packed linear.
+# The kernel with tiles of 96 or 128 rows (htr_linear's own policy beyond 128 rows) is what HTR_GEMV_LOOP_MAX asks for, which
+# overrides the limits for every shape (launches of LAUNCH_MAX_M rows up to it), what HTR_GEMV_MAX_M's chunks of more than 128 rows
+# and HTR_PREFILL=rot take up to the limits, and what a shared capture workspace falls back to that holds no more.
 # Measured on MI355X (K4, us; one launch with tiles of 96 or 128 rows / wide kernel / dequantize + GEMM, GPU time):
 #   14336x4096: 192 rows 43 / 37 / 85, 256 rows 51 / 44 / 80, 333 rows 76 / 60 / 86, 512 rows 95 / 72 / 94, 1024 rows 186 / 130 / 131
 #   4096x14336: 129 rows 45 / 37 / 79, 256 rows 61 / 52 / 90, 333 rows 75 / 65 / 102, 512 rows 95 / 83 / 118
