@@ -121,6 +121,73 @@ __device__ __forceinline__ void rotate4_mfma(const u4& xr, uint32_t sb, bool is_
   y[1][0] = w0 + w2; y[1][1] = w1 + w3; y[1][2] = w0 - w2; y[1][3] = w1 - w3;
 }
 
+// ---- the same for 16 activation rows of one block, transposed: the rows are the columns of the B operands (lane (gk = lane / 16,
+// row = lane % 16) brings the 8 consecutive elements 32 a + 8 gk .. + 7 of its row, x[a], and the su byte of their signs, sb[a]),
+// and the rows of the A operands, those of H32, are dealt so that lane (gk, row) ends up with y[a'][t] = elements 32 a' + 8 gk + 4 t
+// .. + 3 of its row: eight consecutive results leave in one 16-byte store, where rotate4_mfma's lanes hold every 16th.  Per 2048
+// elements about 210 vector instructions with conversion, sums and stores, 90 of them additions and multiplications that this chip
+// issues at 2.4 instead of 4.4 cycles, and 4 stores; rotate4_mfma 440 and 32.  Same sums in the same order.
+__device__ __forceinline__ void rotate16_mfma(const u4 (&x)[4], const uint32_t (&sb)[4], bool is_bf16, int lane, f4 (&y)[4][2]) {
+  const int i = lane & 15, gk = lane >> 4;
+  u4 xs[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const uint32_t two = sb[a] | (sb[a] << 15);                    // bit 2 d, 2 d + 1 of the byte at bits 2 d, 2 d + 16
+#pragma unroll
+    for (int d = 0; d < 4; ++d) xs[a][d] = x[a][d] ^ ((two << (15 - 2 * d)) & 0x80008000u);
+  }
+  // A operand t: row i = element e = 8 (i / 4) + 4 t + i % 4 of H32, k = 8 gk + kk: 16-bit ones, negative where popcount(e & k) is odd
+  const uint32_t one2 = is_bf16 ? 0x3F803F80u : 0x3C003C00u;
+  const uint32_t far = (((i >> 2) & gk & 1) ^ ((i >> 3) & (gk >> 1))) ? 0x80008000u : 0u;
+  const uint32_t b0 = one2 ^ far ^ ((i & 1) ? 0x80000000u : 0u), b1 = b0 ^ ((i & 2) ? 0x80008000u : 0u);
+  const u4 h0 = {b0, b1, b0, b1}, h1 = {b0, b1, b0 ^ 0x80008000u, b1 ^ 0x80008000u};
+  const f4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  f4 t[4][2];
+  if (is_bf16) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      t[a][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, h0), __builtin_bit_cast(b8, xs[a]), zero4, 0, 0, 0);
+      t[a][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, h1), __builtin_bit_cast(b8, xs[a]), zero4, 0, 0, 0);
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      t[a][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, h0), __builtin_bit_cast(h8, xs[a]), zero4, 0, 0, 0);
+      t[a][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, h1), __builtin_bit_cast(h8, xs[a]), zero4, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const f4 u0 = t[0][h] + t[1][h], u1 = t[0][h] - t[1][h], u2 = t[2][h] + t[3][h], u3 = t[2][h] - t[3][h];
+    y[0][h] = u0 + u2; y[1][h] = u1 + u3; y[2][h] = u0 - u2; y[3][h] = u1 - u3;
+  }
+}
+// largest sign-cleared 16-bit pattern of a lane's elements: |values| compare like their bits
+__device__ __forceinline__ uint32_t amax16(const u4 (&x)[4]) {
+  us2 m = {0, 0};
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, x[a][d] & 0x7FFF7FFFu));
+  return max((uint32_t)m.x, (uint32_t)m.y);
+}
+// over the four lanes lane % 16 + 0, 16, 32, 48
+__device__ __forceinline__ uint32_t max_over_groups(uint32_t v) {
+  u2s r = __builtin_amdgcn_permlane16_swap(v, v, false, false); v = max(r.x, r.y);
+  r = __builtin_amdgcn_permlane32_swap(v, v, false, false); return max(r.x, r.y);
+}
+__device__ __forceinline__ float sum_over_groups(float v) {
+  float e, o;
+  halves16(v, e, o); v = e + o;
+  halves32(v, e, o); return e + o;
+}
+// bit pattern of a row's largest |value| to its scale exponent (a NaN anywhere: treat the row as unbounded, scale 1)
+__device__ __forceinline__ int scale_exponent16(uint32_t m16, bool is_bf16) {
+  float amax = is_bf16 ? bf16_bits_to_float((uint16_t)m16) : f16_bits_to_float((uint16_t)m16);
+  if (amax != amax) amax = __uint_as_float(0x7F800000u);
+  return scale_exponent(amax);
+}
+
 // Rotation of all activation rows ahead of the linear kernel (used where every workgroup rotating its own column
 // blocks would repeat too much work, and for float32 activations).  Workgroup (g, row) rotates column blocks
 // 8g .. 8g + 7 of one activation row, one block per wave; every workgroup scans the whole row for max|x| itself

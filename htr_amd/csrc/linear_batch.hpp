@@ -226,9 +226,9 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
   // range: zeros), so every group of 16 rows is addressed alike.  With more than 64 rows the partial does not fit
   // behind the blocks and takes their place once the last step is done.
   // ROT (up to 16 rows over up to 16 column blocks per split, or up to 32 rows over up to 8): no rotation launch; the
-  // workgroup rotates the activations of its own column blocks at the start (wave w: rows 2 MG w .. 2 MG w + 2 MG - 1,
-  // four blocks per pass on the matrix unit, eight passes, one power-of-two scale per row from max|x| over the split's
-  // columns) and keeps all of them in LDS, [cb blocks][16 MG rows][136 halves] + [cb][16 MG][2] sums: no staging and no
+  // workgroup rotates the activations of its own column blocks at the start (on the matrix unit, in units of 16 rows of one
+  // block, two per wave, 13 rows of 4096x14336 at K3 14.6 -> 13.4 us and 32 rows of eight decoder layers 547 -> 529 against passes
+  // of four blocks of one row; one power-of-two scale per row from max|x| over the split's columns) and keeps all of them in LDS, [cb blocks][16 MG rows][136 halves] + [cb][16 MG][2] sums: no staging and no
   // barrier inside the loop.
   constexpr int ROWH = BATCH_ROWH, ROWS = 16 * MG, BUFH = ROWS * ROWH;
   constexpr bool FIN_OVER_BLOCKS = MG > 4;
@@ -276,29 +276,30 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
       if (has_piece) *(u4*)(xt + q * BUFH + piece_lds[i]) = xg[set][i];
     if (has_sum) s_xs[q * 2 * ROWS + tid] = xsg[set];
   };
-  // ROT: the raw activations of this wave's rows, eight passes of four blocks, all loads back to back
-  constexpr int RPASS = ROT ? 8 : 1;
-  constexpr int ROTR = 2 * MG, PPR = 8 / ROTR;          // rows a wave rotates, passes (of four blocks) per row
-  u4 rx[RPASS];
-  uint32_t rsb[RPASS];
+  // ROT: the raw activations of this wave's units (16 rows x one column block), all loads back to back: unit w + 8 i is block
+  // (w + 8 i) / MG of the split, rows 16 (w % MG) .. + 15
+  constexpr int UNITS = ROT ? 2 : 1;
+  const int g16 = lane >> 4, r16 = 16 * (w % MG) + (lane & 15);      // lane (k-group, activation row)
+  u4 rx[UNITS][4];
+  uint32_t rsb[UNITS][4];
   if constexpr (ROT) {
     const __amdgpu_buffer_rsrc_t rawsrc = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * n * 2, 0x00020000);
     const __amdgpu_buffer_rsrc_t sgnsrc = __builtin_amdgcn_make_buffer_rsrc((void*)su, 0, n >> 3, 0x00020000);
-    int xo[RPASS], so[RPASS];
+    int xo[UNITS], so[UNITS];
 #pragma unroll
-    for (int r = 0; r < RPASS; ++r) {
-      const int row = ROTR * w + r / PPR, bl = 4 * (r % PPR) + ((lane & 15) >> 2);      // block within the split
-      const int col = (c_begin + bl) * 128 + 32 * (lane & 3) + 8 * (lane >> 4);
-      const bool live = row < M && bl < nsteps;
-      xo[r] = live ? (row * n + col) * 2 : OUT_OF_RANGE;
-      so[r] = live ? col >> 3 : OUT_OF_RANGE;
+    for (int i = 0; i < UNITS; ++i) {
+      const int bl = (w + WG_WAVES * i) / MG, col = (c_begin + bl) * 128 + 8 * g16;
+      xo[i] = r16 < M && bl < nsteps ? (r16 * n + col) * 2 : OUT_OF_RANGE;
+      so[i] = bl < nsteps ? col >> 3 : OUT_OF_RANGE;
     }
     HTR_PIN();
 #pragma unroll
-    for (int r = 0; r < RPASS; ++r) {
-      rx[r] = __builtin_amdgcn_raw_buffer_load_b128(rawsrc, xo[r], 0, 0);
-      rsb[r] = (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(sgnsrc, so[r], 0, 0);
-    }
+    for (int i = 0; i < UNITS; ++i)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        rx[i][a] = __builtin_amdgcn_raw_buffer_load_b128(rawsrc, xo[i] + 64 * a, 0, 0);
+        rsb[i][a] = (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(sgnsrc, so[i] + 4 * a, 0, 0);
+      }
     HTR_PIN();
   } else {
     if (tid < ROWS) s_sc[tid] = tid < M ? t.sc_g[tid] : 0.f;
@@ -399,47 +400,47 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
   const int hist = history_lane_byteaddr(lane);
   DecodedStep<K> cur;
   if constexpr (ROT) {
-    // ---- rotation of this wave's rows.  Row scale from the raw values: |H128 x| / sqrt(128) <= sqrt(128) max|x|.
+    // ---- rotation of this wave's units.  Row scale from the raw values: |H128 x| / sqrt(128) <= sqrt(128) max|x| over the split's
+    // columns, which the waves tell each other through LDS (in the place of the partial)
     const bool is_bf16 = (flags & 3) == HTR_BF16;
-    const int j = lane & 15, gk = lane >> 4;
+    uint32_t* s_max = (uint32_t*)s_fin;                            // [block][row]
+    f4 y[UNITS][4][2];
 #pragma unroll
-    for (int rr = 0; rr < ROTR; ++rr) {
-      uint32_t m16 = 0u;
+    for (int i = 0; i < UNITS; ++i) {
+      const int bl = (w + WG_WAVES * i) / MG;
+      if (bl >= nsteps) continue;                                  // uniform
+      const uint32_t m16 = max_over_groups(amax16(rx[i]));
+      if (lane < 16) s_max[bl * ROWS + r16] = m16;
+      rotate16_mfma(rx[i], rsb[i], is_bf16, lane, y[i]);
+    }
+    __syncthreads();
+    uint32_t m16 = 0u;
+    for (int bl = g16; bl < nsteps; bl += 4) m16 = max(m16, s_max[bl * ROWS + r16]);
+    const int e = scale_exponent16(max_over_groups(m16), is_bf16);
+    const float f = pow2f(-e) * INV_SQRT128;
+    if (w < MG && lane < 16) s_sc[r16] = r16 < M ? pow2f(e) : 0.f;
 #pragma unroll
-      for (int q = 0; q < PPR; ++q) {
-        const uint32_t d[4] = {rx[PPR * rr + q].x, rx[PPR * rr + q].y, rx[PPR * rr + q].z, rx[PPR * rr + q].w};
+    for (int i = 0; i < UNITS; ++i) {
+      const int bl = (w + WG_WAVES * i) / MG;
+      if (bl >= nsteps) continue;
+      // columns 32 a + 8 g16 .. + 7 are piece 4 a + g16 of the block's sixteen
+      _Float16* dst = xt + (size_t)(bl * ROWS + r16) * ROWH + (g16 & 1) * 64 + (g16 >> 1) * 8;
+      float half_sum[2] = {0.f, 0.f};                              // of the rounded values: columns 0..63 | 64..127
+      const h2 ones = {(_Float16)1.f, (_Float16)1.f};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) m16 = max(m16, max(d[k] & 0x7FFFu, (d[k] >> 16) & 0x7FFFu));
-      }
-      m16 = wave_max_u32(m16);
-      float amax = is_bf16 ? bf16_bits_to_float((uint16_t)m16) : f16_bits_to_float((uint16_t)m16);
-      if (amax != amax) amax = __uint_as_float(0x7F800000u);      // a NaN anywhere: treat the row as unbounded (scale 1)
-      const int e = scale_exponent(amax);
-      const float f = pow2f(-e) * INV_SQRT128;
-      const int row = ROTR * w + rr;
-      if (lane == 0) s_sc[row] = row < M ? pow2f(e) : 0.f;
+      for (int a = 0; a < 4; ++a) {
+        u4 out;
 #pragma unroll
-      for (int q = 0; q < PPR; ++q) {
-        if (4 * q >= nsteps) continue;                             // uniform: none of the pass's blocks exists
-        float y[2][4];
-        rotate4_mfma(rx[PPR * rr + q], rsb[PPR * rr + q], is_bf16, lane, y);
-        const int bl = 4 * q + gk;                                 // lane (p = lane / 16, j) holds elements 32 a' + 16 h + j of block 4 q + p
-        const bool live_o = bl < nsteps;
-        _Float16* dst = xt + (size_t)(bl * ROWS + row) * ROWH + (j >> 3) * 64 + (j & 7);
-        float lo = 0.f, hi = 0.f;                                  // sums of the rounded values: columns 0..63 | 64..127
-        const h2 ones = {(_Float16)1.f, (_Float16)1.f};
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const h2 p01 = __builtin_convertvector(f2{y[h][0] * f, y[h][1] * f}, h2);
-          const h2 p23 = __builtin_convertvector(f2{y[h][2] * f, y[h][3] * f}, h2);
-          if (live_o) { dst[(0 + h) * 8] = p01.x; dst[(2 + h) * 8] = p01.y; dst[(4 + h) * 8] = p23.x; dst[(6 + h) * 8] = p23.y; }
-          lo = __builtin_amdgcn_fdot2(p01, ones, lo, false);
-          hi = __builtin_amdgcn_fdot2(p23, ones, hi, false);
+        for (int d = 0; d < 4; ++d) {
+          const f4 q = y[i][a][d >> 1];
+          const h2 pr = __builtin_convertvector(f2{((d & 1) ? q.z : q.x) * f, ((d & 1) ? q.w : q.y) * f}, h2);
+          out[d] = __builtin_bit_cast(uint32_t, pr);
+          half_sum[a >> 1] = __builtin_amdgcn_fdot2(pr, ones, half_sum[a >> 1], false);
         }
-        lo += dpp_mov<0xB1>(lo); lo += dpp_mov<0x4E>(lo); lo += dpp_mov<0x141>(lo); lo += dpp_mov<0x140>(lo);
-        hi += dpp_mov<0xB1>(hi); hi += dpp_mov<0x4E>(hi); hi += dpp_mov<0x141>(hi); hi += dpp_mov<0x140>(hi);
-        if (live_o && j == 0) { s_xs[(bl * ROWS + row) * 2] = lo; s_xs[(bl * ROWS + row) * 2 + 1] = hi; }
+        *(u4*)(dst + 16 * a) = out;
       }
+      const float lo = sum_over_groups(half_sum[0]), hi = sum_over_groups(half_sum[1]);
+      if (lane < 16) *(f2*)(s_xs + (bl * ROWS + r16) * 2) = f2{lo, hi};
     }
     decode_step<K>(buf[0], hist, cur);
     prefetch(buf[0]);

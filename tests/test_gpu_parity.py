@@ -830,3 +830,26 @@ def test_tiles_of_32_rows_over_long_splits(dev, oracle, K, m, n, M, S, dtype):
             assert _rel(ops.linear_f32out(x.to(dev), *w).cpu().numpy(), ref) <= REL_TOL
     finally:
         ops.NSPLIT = 0
+
+
+@pytest.mark.parametrize("m,n,M,S", [(128, 128, 9, 1), (256, 1920, 15, 1), (128, 2048, 16, 1), (256, 640, 17, 1), (128, 1024, 32, 1), (384, 2176, 31, 3), (256, 4096, 13, 2)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, m, n, M, S, dtype):
+    """9 to 32 rows rotated by the workgroups that multiply them: one unit of 16 rows and one block per wave and two, waves without
+    a unit, rows short of a unit, both 16-bit types.  Rows of very different size keep their own scale, and an infinity stays in its
+    row.  Max norm per row: 1e-3 as for every float32 result (float16 activations)."""
+    from htr_amd import ops
+    print(f"rotation by workgroups {m}x{n} M={M} S={S} {dtype}", flush=True)
+    qw, sc, su, sv, x = _case(m, n, 4, M, 3300 + M + n, torch.float32)
+    x = (x * torch.logspace(-3, 3, M)[:, None]).to(dtype)
+    w = [t.to(dev) for t in (qw, sc, su, sv)]
+    ref = _ref(oracle, qw, sc, su, sv, x)
+    ops.NSPLIT = (1 << 29) | S
+    try:
+        got = ops.linear_f32out(x.to(dev), *w).cpu().numpy()
+        assert np.all(np.abs(got - ref).max(axis=1) <= REL_TOL * np.abs(ref).max(axis=1))
+        x[M - 1, n - 1] = float("inf")
+        got = ops.linear_f32out(x.to(dev), *w).cpu().numpy()
+    finally:
+        ops.NSPLIT = 0
+    assert not np.any(np.isfinite(got[M - 1])) and np.all(np.abs(got - ref)[:M - 1].max(axis=1) <= REL_TOL * np.abs(ref).max(axis=1)[:M - 1])
