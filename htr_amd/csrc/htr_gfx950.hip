@@ -276,13 +276,14 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     t.chunk_magic = 0;
     t.group = nullptr; t.group_prerot_stride = 0; t.group_part_stride = 0; t.tiles = nullptr;
     hipStream_t st = (hipStream_t)stream;
-    // the workgroups rotate their own activations where the plan allows it (16-bit rows on 16-byte boundaries)
-    const bool rot = bp.rot && x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0;
+    // the workgroups rotate their own activations where the plan allows it or it is ahead (16-bit rows on 16-byte boundaries)
+    const bool whole = x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0;
+    const int rot = !whole ? 0 : bp.rot ? 1 : batch_rot_on() && batch_rot_long(K, M, bp.S, bp.cb, bp.wgs) ? 2 : 0;
     if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, bp.tile ? FRAG_FULL : 0));
     BatchArgs ba;
     ba.qw = (const uint32_t*)qweight; ba.part = (float*)((unsigned char*)workspace + WS_HEADER); ba.x = x; ba.su = (const uint8_t*)su;
     ba.m = m; ba.n = n; ba.M = M; ba.flags = x_dtype | (y_dtype << 2) | (bp.last_finishes ? FLAG_LAST_FINISHES : 0);
-    if (bp.rot && !rot) bp.lds = batch_lds_bytes(M, bp.tile);            // the layout of the kernel for pre-rotated activations
+    bp.lds = rot ? batch_rot_lds_bytes(M, bp.cb, rot) : batch_lds_bytes(M, bp.tile);
     HTR_FOR_K(K, return launch_batch_k<KK>(ba, rot, t, bp, st));
     return HTR_OK;
   }

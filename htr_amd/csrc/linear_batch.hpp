@@ -205,7 +205,7 @@ constexpr int BATCH_FIN_STRIDE = 128 + 4;    // floats per activation row of the
 // rows x 4 groups of 8 output rows) hit 64 different banks with each of their 8 values
 __device__ __forceinline__ int batch_fin_pos(int r) { return (r & 7) * 16 + (r >> 3); }
 
-template <int K, int MG, int P, bool ROT>
+template <int K, int MG, int P, int ROT>
 __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_batch(const uint32_t* __restrict__ qw, float* __restrict__ part,
                                                              const void* __restrict__ x, const uint8_t* __restrict__ su,
                                                              int m, int n, int M, int S, int flags, const LinearTail t) {
@@ -225,13 +225,13 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
   // [2 column halves][M][132] partial of the workgroup.  Rows M .. 16 MG - 1 are staged like the others (they read out of
   // range: zeros), so every group of 16 rows is addressed alike.  With more than 64 rows the partial does not fit
   // behind the blocks and takes their place once the last step is done.
-  // ROT (up to 16 rows over up to 16 column blocks per split, or up to 32 rows over up to 8): no rotation launch; the
-  // workgroup rotates the activations of its own column blocks at the start (on the matrix unit, in units of 16 rows of one
-  // block, two per wave, 13 rows of 4096x14336 at K3 14.6 -> 13.4 us and 32 rows of eight decoder layers 547 -> 529 against passes
-  // of four blocks of one row; one power-of-two scale per row from max|x| over the split's columns) and keeps all of them in LDS, [cb blocks][16 MG rows][136 halves] + [cb][16 MG][2] sums: no staging and no
-  // barrier inside the loop.
+  // ROT: no rotation launch; the workgroup rotates the activations of its own column blocks at the start (on the matrix unit, in
+  // units of 16 rows of one block; one power-of-two scale per row from max|x| over the split's columns) and keeps all of them in
+  // LDS, [cb blocks][16 MG rows][136 halves] + [cb][16 MG][2] sums: no staging and no barrier inside the loop.  1: up to two units
+  // per wave (16 rows over 16 column blocks per split, 32 rows over 8); 2: up to four, and the partial takes the place of the blocks.
+  // 13 rows of 4096x14336 at K3 14.6 -> 13.4 us and 32 rows of eight decoder layers 547 -> 529 against passes of four blocks of one row.
   constexpr int ROWH = BATCH_ROWH, ROWS = 16 * MG, BUFH = ROWS * ROWH;
-  constexpr bool FIN_OVER_BLOCKS = MG > 4;
+  constexpr bool FIN_OVER_BLOCKS = MG > 4 || ROT == 2;
   _Float16* xt = (_Float16*)lds;
   float* s_xs = (float*)(lds + (size_t)(ROT ? cb : 2) * BUFH * 2);
   float* s_sc = s_xs + (ROT ? cb * 2 * ROWS : 4 * ROWS);
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
   };
   // ROT: the raw activations of this wave's units (16 rows x one column block), all loads back to back: unit w + 8 i is block
   // (w + 8 i) / MG of the split, rows 16 (w % MG) .. + 15
-  constexpr int UNITS = ROT ? 2 : 1;
+  constexpr int UNITS = ROT ? 2 * ROT : 1;
   const int g16 = lane >> 4, r16 = 16 * (w % MG) + (lane & 15);      // lane (k-group, activation row)
   u4 rx[UNITS][4];
   uint32_t rsb[UNITS][4];
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(WG_THREADS, MG <= 2 && !ROT ? 4 : 2) void k_linear_
     // ---- rotation of this wave's units.  Row scale from the raw values: |H128 x| / sqrt(128) <= sqrt(128) max|x| over the split's
     // columns, which the waves tell each other through LDS (in the place of the partial)
     const bool is_bf16 = (flags & 3) == HTR_BF16;
-    uint32_t* s_max = (uint32_t*)s_fin;                            // [block][row]
+    uint32_t* s_max = (uint32_t*)(s_sc + ROWS);                    // [block][row]; ROT == 1: where the partial will be
     f4 y[UNITS][4][2];
 #pragma unroll
     for (int i = 0; i < UNITS; ++i) {

@@ -251,9 +251,25 @@ template <int K> int launch_linear_k(const LinearLaunch& a, bool prerot, int mb,
 
 // ---- batched kernel: split S of the column blocks per row block
 struct BatchPlan { int S, cb, wgs, mb, rot, last_finishes; bool tile; size_t lds; };      // tile: k_linear_tile, unless rot
-// rows x column blocks per split up to which a workgroup of the batched kernel rotates its own activations (256 pairs,
-// eight passes per wave) instead of a rotation launch: 16 x 16 or 32 x 8
+// rows x column blocks per split up to which a workgroup of the batched kernel always rotates its own activations (its ROT = 1: up to
+// two units of 16 rows and one block per wave) instead of a rotation launch: 16 x 16 or 32 x 8
 inline bool batch_rot_fits(int M, int cb) { return (M <= 16 && cb <= 16) || (M <= 32 && cb <= 8); }
+// Where it does so beyond that with up to four units per wave (ROT = 2).  Decided at the launch, by the activations it is given; the
+// plan is that of the rotation launch and of the kernel behind it, which all other activations take.  Measured on MI355X, us in
+// graphs over several weights, rotation launch / 2:
+//   up to 16 rows, everywhere (28672x4096, 16 rows K4 23.9 / 23.7, 9 rows K3 23.2 / 22.1, 12 rows K8 32.7 / 30.1; 20480x3072, 16 rows
+//     K4 19.5 / 19.0; 28672x2560, 8 rows K4 17.2 / 15.6; 4096x22528, 12 rows K4 22.0 / 18.9; 2048x32768, 16 rows K4 25.7 / 24.9)
+//   17 to 32 rows over 9 to 12 column blocks, everywhere (28672x1152, 32 rows K4 14.3 / 13.4; 10240x3840 15.7 / 14.9; 8704x3456, 17
+//     rows K8 17.7 / 14.8; 12288x3072, 32 rows K4 15.8 / 15.8) but on the smallest grids (128x12288 16.0 / 16.2)
+//   13 to 16 from five bits on, whose decode hides more of the rotation (4096x14336, 17 rows K5 19.8 / 17.6; 8192x8192 K8 24.9 / 23.6;
+//     12288x4096, 32 rows K5 19.9 / 19.8), and up to K4 13 and 14 on a grid of three splits and more that fills three quarters of the
+//     chip (4096x14336, 32 rows K4 19.3 / 18.6, 24 rows 18.8 / 17.3; 10240x5376 18.7 / 18.3): not 1024x14336, 17.4 / 17.7, nor
+//     10240x6144, 19.0 / 19.7, nor where k_linear_tile is what follows the launch (28672x2048 16.9 / 19.0, 12288x4096 18.3 / 18.9)
+inline bool batch_rot_long(int K, int M, int S, int cb, int wgs) {
+  const int cus = num_cu();
+  if (M > 32 || wgs > cus || (M <= 16 ? cb : 2 * cb) > 32) return false;
+  return M <= 16 || cb <= 10 || (cb <= 12 && 8 * wgs >= cus) || K >= 5 || (cb <= 14 && S >= 3 && 4 * wgs > 3 * cus);
+}
 constexpr int BATCH_MIN_M = 9;      // rows from which the library policy takes the batched kernel on every shape
 inline int batch_groups(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : 8)); }   // groups of 16 activation rows
 // k_linear_tile instead of k_linear_batch for 17 to 64 activation rows that were rotated ahead.  Measured on MI355X, us of the call
@@ -283,6 +299,16 @@ inline size_t batch_lds_bytes(int M, bool tile) {
   const int rows = 16 * batch_groups(M);
   const size_t blocks = (size_t)2 * rows * BATCH_ROWH * 2, small = (size_t)5 * rows * 4, fin = (size_t)2 * M * BATCH_FIN_STRIDE * 4;
   return M > 64 ? (blocks + small > fin ? blocks + small : fin) : blocks + small + fin;
+}
+// HTR_BATCH_ROT=0 switches the rotation by the workgroups off
+inline bool batch_rot_on() {
+  static const bool on = getenv("HTR_BATCH_ROT") == nullptr || atoi(getenv("HTR_BATCH_ROT")) != 0;
+  return on;
+}
+inline size_t batch_rot_lds_bytes(int M, int cb, int rot) {
+  const int rows = 16 * batch_groups(M);
+  return (size_t)cb * rows * BATCH_ROWH * 2 + (size_t)cb * 2 * rows * 4 + rows * 4 +
+         (rot == 1 ? (size_t)2 * M * BATCH_FIN_STRIDE * 4 : (size_t)cb * rows * 4);
 }
 inline bool make_batch_plan(int m, int n, int K, int M, int want_S, BatchPlan& bp) {
   const int nblk = n / 128, rbs = m / 128;
@@ -320,12 +346,9 @@ inline bool make_batch_plan(int m, int n, int K, int M, int want_S, BatchPlan& b
   // policy assumed) falls back to the last split finishing everything: it waits only for workgroups dispatched before it.
   bp.last_finishes = bp.wgs > cus ? 1 : 0;
   // Few rows over few column blocks per split, one workgroup per CU: every workgroup rotates its own slice.
-  // HTR_BATCH_ROT=0 switches it off.
-  static const bool rot_on = getenv("HTR_BATCH_ROT") == nullptr || atoi(getenv("HTR_BATCH_ROT")) != 0;
-  if (rot_on && batch_rot_fits(M, bp.cb) && bp.wgs <= cus) {
-    const int rows = 16 * bp.mb;
+  if (batch_rot_on() && batch_rot_fits(M, bp.cb) && bp.wgs <= cus) {
     bp.rot = 1;
-    bp.lds = (size_t)bp.cb * rows * BATCH_ROWH * 2 + (size_t)bp.cb * 2 * rows * 4 + rows * 4 + (size_t)2 * M * BATCH_FIN_STRIDE * 4;
+    bp.lds = batch_rot_lds_bytes(M, bp.cb, 1);
   }
   return true;
 }
@@ -507,7 +530,7 @@ inline bool wide_ahead(int m, int n, int K, int M, int x_dtype, const WidePlan& 
 }
 
 struct BatchArgs { const uint32_t* qw; float* part; const void* x; const uint8_t* su; int m, n, M, flags; };
-template <int K, int MB, bool ROT> int launch_batch_v(const BatchArgs& a, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
+template <int K, int MB, int ROT> int launch_batch_v(const BatchArgs& a, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
   const size_t lds = balanced_lds_request(bp.lds, bp.wgs);
   HTR_CHECK_HIP((allow_full_lds<k_linear_batch<K, MB, 4, ROT>>()));
   HTR_CHECK_HIP(launch_kernel(k_linear_batch<K, MB, 4, ROT>, dim3(bp.S, a.m / 128), dim3(WG_THREADS), lds, st, a.qw, a.part, a.x, a.su,
@@ -555,8 +578,9 @@ inline bool group_takes_tiles(int count, int m, int n, int K, int max_M) {
   const int nblk = n / 128, cus = num_cu(), grid = count * (m / 128), rounds = (grid + cus - 1) / cus;
   return rounds > 2 || nblk < (rounds == 1 ? 64 : 32) || 4 * grid > 3 * rounds * cus;
 }
-template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
-  if (rot) return bp.mb == 1 ? launch_batch_v<K, 1, true>(a, t, bp, st) : launch_batch_v<K, 2, true>(a, t, bp, st);
+template <int K> int launch_batch_k(const BatchArgs& a, int rot, const LinearTail& t, const BatchPlan& bp, hipStream_t st) {
+  if (rot == 1) return bp.mb == 1 ? launch_batch_v<K, 1, 1>(a, t, bp, st) : launch_batch_v<K, 2, 1>(a, t, bp, st);
+  if (rot == 2) return bp.mb == 1 ? launch_batch_v<K, 1, 2>(a, t, bp, st) : launch_batch_v<K, 2, 2>(a, t, bp, st);
   if (bp.tile) {
     // Grids beyond one workgroup per compute unit, us without / with ONE: K4, 64 rows 65536x4096 67.0 / 59.4, 40960x1024 28.7 /
     // 22.4, 33 rows 152064x4096 137.6 / 115.9; 17 rows 40960x2048 24.0 / 23.6, 32 rows 25.5 / 24.7, 65536x4096 45.4 / 44.9.  Up to one
@@ -566,10 +590,10 @@ template <int K> int launch_batch_k(const BatchArgs& a, bool rot, const LinearTa
     if constexpr (K <= 4) return a.M <= 32 ? launch_tile_v<K, 1, false>(a, t, bp.S, 1, st) : launch_tile_v<K, 2, false>(a, t, bp.S, 1, st);
   }
   switch (bp.mb) {
-    case 1: return launch_batch_v<K, 1, false>(a, t, bp, st);
-    case 2: return launch_batch_v<K, 2, false>(a, t, bp, st);
-    case 4: return launch_batch_v<K, 4, false>(a, t, bp, st);
-    default: return launch_batch_v<K, 8, false>(a, t, bp, st);
+    case 1: return launch_batch_v<K, 1, 0>(a, t, bp, st);
+    case 2: return launch_batch_v<K, 2, 0>(a, t, bp, st);
+    case 4: return launch_batch_v<K, 4, 0>(a, t, bp, st);
+    default: return launch_batch_v<K, 8, 0>(a, t, bp, st);
   }
 }
 // nsplit bit 29: batched kernel with the split in the low bits (0 = policy); otherwise the policy decides by M

@@ -111,6 +111,8 @@ unsigned long long htr_stream_capture_id(void* stream);
  * own (0: the workgroups rotate their own slices: up to 16 rows over at most 16 column blocks per split, or up to 32 rows
  * over at most 8), dynamic LDS bytes}.  Entries 4 and 5 assume bf16 / f16 activations on a 16-byte boundary; float32 or
  * otherwise aligned activations always take the rotation launch and the staged kernel's LDS layout.
+ * Where the plan says 1, up to 16 rows over 32 blocks and up to 32 rows over 16 may still be rotated by the workgroups, if that is
+ * faster and the activations are 16-bit rows on 16-byte boundaries: decided at the call, with more LDS than the plan says.
  * From 65 rows to HTR_MAX_ROWS_PER_TILE the wide kernel runs (tiles of up to 256 activation rows, which share what a workgroup
  * decodes), out6 as for the batched kernel; with bit 27 of nsplit it takes any row count, and out6[2] is the number of row tiles.
  * With more than HTR_MAX_ROWS_PER_TILE rows the fused decode -> matrix-unit (GEMM) kernel runs: the activations are

@@ -832,15 +832,16 @@ def test_tiles_of_32_rows_over_long_splits(dev, oracle, K, m, n, M, S, dtype):
         ops.NSPLIT = 0
 
 
-@pytest.mark.parametrize("m,n,M,S", [(128, 128, 9, 1), (256, 1920, 15, 1), (128, 2048, 16, 1), (256, 640, 17, 1), (128, 1024, 32, 1), (384, 2176, 31, 3), (256, 4096, 13, 2)])
+@pytest.mark.parametrize("K,m,n,M,S", [(4, 128, 128, 9, 1), (2, 256, 1920, 15, 1), (8, 128, 2048, 16, 1), (4, 256, 640, 17, 1), (3, 128, 1024, 32, 1), (5, 384, 2176, 31, 3), (4, 256, 4096, 13, 2),
+                                     (4, 4096, 2176, 9, 1), (3, 4096, 4096, 16, 1), (4, 4096, 1152, 17, 1), (2, 1408, 4608, 32, 3), (5, 4096, 1920, 29, 1), (8, 4096, 2048, 32, 1)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, m, n, M, S, dtype):
-    """9 to 32 rows rotated by the workgroups that multiply them: one unit of 16 rows and one block per wave and two, waves without
+def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, K, m, n, M, S, dtype):
+    """9 to 32 rows rotated by the workgroups that multiply them: one to four units of 16 rows and one block per wave, waves without
     a unit, rows short of a unit, both 16-bit types.  Rows of very different size keep their own scale, and an infinity stays in its
     row.  Max norm per row: 1e-3 as for every float32 result (float16 activations)."""
     from htr_amd import ops
-    print(f"rotation by workgroups {m}x{n} M={M} S={S} {dtype}", flush=True)
-    qw, sc, su, sv, x = _case(m, n, 4, M, 3300 + M + n, torch.float32)
+    print(f"rotation by workgroups K={K} {m}x{n} M={M} S={S} {dtype}", flush=True)
+    qw, sc, su, sv, x = _case(m, n, K, M, 3300 + M + n, torch.float32)
     x = (x * torch.logspace(-3, 3, M)[:, None]).to(dtype)
     w = [t.to(dev) for t in (qw, sc, su, sv)]
     ref = _ref(oracle, qw, sc, su, sv, x)
