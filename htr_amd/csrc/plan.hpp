@@ -106,7 +106,15 @@ inline bool search_plan(int m, int n, int M, int nsplit, int cus, Plan& pl) {
     if (ok && (nsplit & (1 << 30))) pl.prerot = 1;
     return ok;
   }
-  if (vtotal >= (long)64 * cus && nblk <= 64 && plan_for_chunk(m, n, M, nblk, pl)) return true;
+  // Large matrices: one row block per workgroup, or two equal chunks per compute unit.  The compute units take whole row blocks in
+  // rounds, so the last round is as long as the others however few row blocks are left; equal chunks cost 3 % more (partials, row
+  // ends inside a chunk; 10 % with five rows, which have no PACE there: 152064x4096 K3 71.8 / 72.8).  K4, 1 row, us with row blocks / chunks: 73728x4096 48.6 / 39.8, 102400x4096 62.0 / 51.8,
+  // 152064x4096 72.8 / 71.7 (another run 73.3 / 70.5), 128256x4096 61.8 / 61.3, 131072x4096 61.1 / 63.1; 73728x8192 K5 90.6 / 74.2.
+  if (vtotal >= (long)64 * cus && nblk <= 64) {
+    const int rounds = (rbs + cus - 1) / cus;
+    if ((M <= 4 ? 1.03 : 1.1) * rbs < (double)rounds * cus && plan_for_chunk(m, n, M, (int)((vtotal + 2 * cus - 1) / (2 * cus)), pl)) return true;
+    if (plan_for_chunk(m, n, M, nblk, pl)) return true;
+  }
   const double rows = M <= 8 ? 1.0 + 0.06 * (M - 1) : (M <= 16 ? 2.2 : 6.5);
   double best = 1e30;
   bool found = false;

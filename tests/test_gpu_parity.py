@@ -854,3 +854,16 @@ def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, K, m, n, 
     finally:
         ops.NSPLIT = 0
     assert not np.any(np.isfinite(got[M - 1])) and np.all(np.abs(got - ref)[:M - 1].max(axis=1) <= REL_TOL * np.abs(ref).max(axis=1)[:M - 1])
+
+
+@pytest.mark.parametrize("K,m,n,M", [(4, 33024, 8192, 1), (3, 65664, 4096, 4), (2, 131200, 2048, 5)])
+def test_large_matrices_in_equal_chunks(dev, oracle, K, m, n, M):
+    """One row block more than whole rounds over the compute units: two chunks per unit that cross row blocks.  A sample of the output
+    rows in float64, max norm 1e-3 as for every float32 result."""
+    from htr_amd import ops
+    print(f"large matrix in chunks K={K} {m}x{n} M={M}", flush=True)
+    qw, sc, su, sv, x = _case(m, n, K, M, 7700 + M)
+    y = ops.linear_f32out(x.to(dev), *[t.to(dev) for t in (qw, sc, su, sv)]).cpu().numpy()
+    for r0 in (0, m // 256 * 128, m - 128):                                  # a row block of the output by itself
+        ref = _ref(oracle, qw[r0 // 16:r0 // 16 + 8], sc[r0:r0 + 128], su, sv[r0 // 8:r0 // 8 + 16], x)
+        assert _rel(y[:, r0:r0 + 128], ref) <= REL_TOL

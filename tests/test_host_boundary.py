@@ -332,3 +332,15 @@ def test_limits_of_the_routed_expert_layer(L):
     assert need(1, inter=1 << 22) == 0 and need(1, hidden=1 << 23) == 0
     assert need(4000000) > 0 and need(4 << 20) == 0 and need(1 << 23, experts=4096) == 0 and need(1 << 24) == 0
     assert need(1, experts=4096) > 0 and need(1, experts=4097) == 0 and need(0) == 0 and need(1, top=0) == 0
+
+
+@pytest.mark.parametrize("m,n,M,chunk", [(73728, 4096, 1, 36), (152064, 4096, 4, 75), (152064, 4096, 5, 32), (131072, 4096, 1, 32), (128256, 4096, 2, 32),
+                                         (65664, 8192, 2, 65), (32768, 8192, 1, 64), (32896, 8192, 5, 33)])
+def test_large_matrices_take_row_blocks_or_equal_chunks(L, m, n, M, chunk):
+    """Up to five rows of matrices that give every compute unit 64 steps: whole row blocks where their rounds over 256 compute units are
+    nearly full, else two equal chunks per unit; either way the chunks tile the steps and the slots fit the workspace."""
+    out = (ctypes.c_int * 6)()
+    assert L.htr_linear_plan(m, n, 4, M, 0, out) == 0
+    steps = (m // 128) * (n // 128)
+    assert out[0] == chunk and out[1] == -(-steps // chunk) and (chunk == n // 128 or out[1] <= 512)
+    assert L.htr_workspace_bytes(m, n, 4, M, 0) >= 256 + out[1] * M * 512
