@@ -46,6 +46,8 @@ SIGNATURES = {
     "htr_stream_capture_id": (ctypes.c_ulonglong, [_vp]),
     "htr_viterbi_workspace_bytes": (_sz, [_i64, _i, _i]),
     "htr_viterbi": (_i, [_vp, _vp, _i64, _i, _i, _i, _vp, _vp, _sz, _vp]),
+    "htr_encode_targets": (_i, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp]),
+    "htr_encode_quantized": (_i, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _vp]),
     "htr_decode_raw": (_i, [_vp, _vp, _i64, _i, _vp]),
     "htr_dequant_q": (_i, [_vp, _vp, _vp, _i, _i, _i, _vp]),
     "htr_dequant_w": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),

@@ -668,6 +668,35 @@ int htr_viterbi(const void* x, const void* w, int64_t tiles, int T, int K, int t
   return HTR_OK;
 }
 
+static int encode_block_args(const void* const* pointers, int count, int64_t rows, int64_t n, int64_t col) {
+  for (int i = 0; i < count; ++i) {
+    if (!pointers[i]) return HTR_ERR_NULL;
+    if ((uintptr_t)pointers[i] & 15) return HTR_ERR_ALIGN;
+  }
+  if (rows <= 0 || rows % 16 || rows > ((int64_t)1 << 30) || n <= 0 || n % 16 || n > ((int64_t)1 << 30) || col < 0 || col % 16 || col >= n) return HTR_ERR_SHAPE;
+  return HTR_OK;
+}
+
+int htr_encode_targets(const void* W, const void* F, const void* scales, int64_t rows, int64_t n, int64_t col, void* x, void* stream) {
+  const void* pointers[] = {W, F, scales, x};
+  const int rc = encode_block_args(pointers, 4, rows, n, col);
+  if (rc != HTR_OK) return rc;
+  HTR_CHECK_HIP(launch_kernel(k_encode_targets, dim3((unsigned)((rows * 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (const float*)W,
+                              (const float*)F, (const float*)scales, rows, n, col, (float*)x));
+  return HTR_OK;
+}
+
+int htr_encode_quantized(const void* states_u16, const void* codebook, const void* W, const void* scales, int64_t rows, int64_t n, int64_t col,
+                         void* Q, void* err, void* states_i64, void* stream) {
+  const void* pointers[] = {states_u16, codebook, W, scales, Q, err, states_i64};
+  const int rc = encode_block_args(pointers, 7, rows, n, col);
+  if (rc != HTR_OK) return rc;
+  HTR_CHECK_HIP(launch_kernel(k_encode_quantized, dim3((unsigned)((rows * 4 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                              (const uint16_t*)states_u16, (const float*)codebook, (const float*)W, (const float*)scales, rows, n, col, (float*)Q,
+                              (float*)err, (int64_t*)states_i64));
+  return HTR_OK;
+}
+
 int htr_decode_raw(const void* qweight, void* out_i16, int64_t ntiles, int K, void* stream) {
   if (!qweight || !out_i16) return HTR_ERR_NULL;
   if (K < 2 || K > 8) return HTR_ERR_K;

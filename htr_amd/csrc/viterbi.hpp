@@ -302,3 +302,44 @@ __global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __r
     __syncthreads();                                    // xs, ws and the M arrays are free for the next tile
   }
 }
+
+// ------------------------------------------------------------------------------------------------ around the search
+// One 16-column block of the encoder's matrices before and after its search (htr/encode.py:69-88 of the reference): every thread
+// takes four consecutive elements of one row.  float32 and unfused, in the reference's order of operations.
+// targets: x = (W + F) / row scale, as the search wants its tiles.
+__global__ __launch_bounds__(256) void k_encode_targets(const float* __restrict__ W, const float* __restrict__ F, const float* __restrict__ rs,
+                                                        int64_t rows, int64_t ld, int64_t col, float* __restrict__ x) {
+#pragma clang fp contract(off)
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, row = i >> 2;
+  if (row >= rows) return;
+  const int64_t at = row * ld + col + 4 * (i & 3);
+  const f4 sum = *(const f4*)(W + at) + *(const f4*)(F + at);
+  const float r = rs[row];
+  *(f4*)(x + 4 * i) = f4{sum.x / r, sum.y / r, sum.z / r, sum.w / r};
+}
+// quantized: q = cb[s] * row scale into Q, W - q into err, the states as whole numbers into S [tile][blocks][256].  Bound: the launch;
+// with the kernel above two launches of 4 us where torch takes eleven, 0.9 MB each at 2816 rows.
+__global__ __launch_bounds__(256) void k_encode_quantized(const uint16_t* __restrict__ states, const float* __restrict__ cb, const float* __restrict__ W,
+                                                          const float* __restrict__ rs, int64_t rows, int64_t ld, int64_t col,
+                                                          float* __restrict__ Q, float* __restrict__ err, int64_t* __restrict__ S) {
+#pragma clang fp contract(off)
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, row = i >> 2;
+  if (row >= rows) return;
+  const int64_t at = row * ld + col + 4 * (i & 3);
+  const float r = rs[row];
+  const f4 w = *(const f4*)(W + at);
+  uint32_t s[4];
+  f4 q, e;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    s[k] = states[4 * i + k];
+    q[k] = cb[s[k]] * r;
+    e[k] = w[k] - q[k];
+  }
+  *(f4*)(Q + at) = q;
+  *(f4*)(err + 4 * i) = e;
+  typedef int64_t l2 __attribute__((ext_vector_type(2)));
+  l2* o = (l2*)(S + ((row >> 4) * (ld >> 4) + (col >> 4)) * 256 + (4 * i & 255));
+  o[0] = l2{(int64_t)s[0], (int64_t)s[1]};
+  o[1] = l2{(int64_t)s[2], (int64_t)s[3]};
+}

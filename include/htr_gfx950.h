@@ -262,6 +262,17 @@ int htr_viterbi(const void* x, const void* w, int64_t tiles, int T, int K, int t
                 void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * One 16-column block of the matrix encoder around its search (htr/encode.py:69-88), columns col .. col + 15 of float32 matrices
+ * [rows][n], rows, n and col multiples of 16, every pointer on a 16-byte boundary; float32 and unfused:
+ *   htr_encode_targets     x[rows / 16][256] = (W + F) / scales[row]
+ *   htr_encode_quantized   Q = codebook[s] * scales[row]; err[rows][16] = W - Q; states_i64[rows / 16][n / 16][256] = s
+ * for states_u16[rows / 16][256] as htr_viterbi leaves them (all T = 256 of a tile) and the float32 codebook of 65536 entries.
+ */
+int htr_encode_targets(const void* W, const void* F, const void* scales, int64_t rows, int64_t n, int64_t col, void* x, void* stream);
+int htr_encode_quantized(const void* states_u16, const void* codebook, const void* W, const void* scales, int64_t rows, int64_t n,
+                         int64_t col, void* Q, void* err, void* states_i64, void* stream);
+
+/*
  * Integer decode, tile order: out[tile, t] = v(s_t) as int16, tile = ti*(n/16)+tj, t = 16r+c.
  * Reference: decode_raw (htr/csrc/htr_kernels.cu:943-951, kernel :154-172).
  */

@@ -295,3 +295,36 @@ def test_codebook_check_is_not_fooled_by_a_reused_address(monkeypatch):
     for _ in range(40):
         encode._check_codebook(wire.codebook_f32("cpu").clone())
     assert len(encode._CHECKED_CB) <= 16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,sizes,n,shared,max_batch", [(2, [(128, 0)], 128, False, 8), (3, [(256, 0), (384, 0)], 256, True, 1024), (4, [(128, 0), (128, 1), (256, 1)], 384, True, 11),
+                                                       (5, [(1280, 0)], 128, True, 64)])
+def test_gpu_encoder_blocks_match_the_torch_lines(dev, monkeypatch, K, sizes, n, shared, max_batch):
+    """encode_group's launches around the search against its torch lines with the same search (which a hook selects): every output bit
+    for bit.  One and several matrices and Hessians, a dead input column, batches that do not divide the tiles."""
+    from htr_amd import encode
+    print(f"encoder blocks K={K} {sizes} n={n}", flush=True)
+    g = torch.Generator().manual_seed(K)
+    hessians = []
+    for i in range(2):
+        a = torch.randn(2 * n, n, generator=g) * torch.exp(0.5 * torch.randn(n, generator=g))
+        a[:, 5 + i] = 0
+        hessians.append((a.T @ a / (2 * n)).to(dev))
+    jobs = [dict(W=(0.02 * torch.randn(m, n, generator=g)).to(dev), H=hessians[h]) for m, h in sizes]
+    got = encode.encode_group(jobs, K, seed=7, shared_su=shared, max_batch=max_batch)
+    monkeypatch.setattr(encode, "VITERBI", lambda x, w, cb, k: encode.viterbi(x, w, cb, k))
+    want = encode.encode_group(jobs, K, seed=7, shared_su=shared, max_batch=max_batch)
+    for a, b in zip(got, want):
+        for name in b:
+            assert torch.equal(a[name], b[name]), name
+
+
+def test_encoder_block_launches_refuse_wrong_sizes():
+    from htr_amd import _native
+    L = _native.lib()
+    p = [1 << 12] * 7
+    assert L.htr_encode_targets(None, *p[1:3], 16, 16, 0, p[3], None) == 1 and L.htr_encode_targets(p[0] + 4, *p[1:3], 16, 16, 0, p[3], None) == L.htr_encode_targets(*p[:3], 16, 16, 0, p[3] + 8, None) != 0
+    for rows, n, col in ((0, 16, 0), (8, 16, 0), (16, 24, 0), (16, 16, 16), (16, 32, 8), (16, 16, -16), (1 << 31, 16, 0)):
+        bad = L.htr_encode_targets(*p[:3], rows, n, col, p[3], None)
+        assert bad == L.htr_encode_quantized(*p[:4], rows, n, col, *p[4:7], None) == L.htr_encode_targets(*p[:3], 8, 16, 0, p[3], None) != 0
