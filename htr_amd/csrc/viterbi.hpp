@@ -6,22 +6,23 @@
 // predecessors, M_t[low] = min_j cost_{t-1}[j * Sj + low] (Sj = 65536 >> K entries), need to live between steps, and
 // cost_t[s] = M_t[s >> K] + w_t (x_t - cb[s])^2, so two M arrays in LDS carry a whole tile (128 KB at K2, 32 KB at K4)
 // and no cost array ever goes to memory.
-// A thread owns 64 states for the whole launch and keeps their codebook values in registers (1024 threads x 64 = all
+// A thread owns 64 states for the whole launch and keeps their codebook values in registers over a tile's passes (1024 threads x 64 = all
 // 65536), so a candidate costs a subtraction, two multiplications and an addition, which this chip issues every 2.35
 // cycles from vector registers, and half a v_min3 (4.2).  (Looking the penalty up in a 1021-entry LDS table, as the first
-// version did, costs 5.4 cycles of the one LDS per 64 candidates plus the address arithmetic at the 4.2-cycle rate.)
+// version did, costs 5.4 cycles of the one LDS per 64 candidates plus the address arithmetic at the 4.2-cycle rate; even an eighth
+// of them from a table made two steps ahead, without that arithmetic, is 4 % slower than none: the M values are read through LDS too.)
 // The forward passes keep no backpointers at all: comparing and selecting an index costs 8.4 cycles per candidate against
 // 2.1 for the minimum alone.  Instead the deciding pass writes every C-th M array to memory, and the trace back
 // recomputes the C steps in between for the predecessors of the ONE state it is at (2^(K C) entries of M_{t-C}, 32 to 512
 // of them, one wave), with the same arithmetic, so the indices it finds are those the forward pass would have recorded.
 // Which array comes next does not depend on the state, so the other waves fetch it into LDS meanwhile.
 // Bound: vector issue in the forward passes (K4: 2890 cycles a step, 2944 by the rates above; 0.74 M cycles a pass), then
-// the trace back, 13 % of a tile: with every CU at it, the stored arrays (2 MB a tile) arrive at 5 TB/s.  C: a larger one
-// stores less and recomputes more (K3: C = 2 439 k cycles, C = 3 281 k; K5: C = 1 290 k, C = 2 327 k).
-// Registers: the trace back needs more than the 64 that the codebook values leave, so 8 (K6) to 111 (K7) of a lane's registers, 20
-// at K4, live in scratch, from K3 on outside the forward loop; at K2 (82) the trace back loads about 20 of them every turn.
-// 1024 tiles at K4: 7.46 ms with the table and one byte of backpointer per entry and step, 3.25 ms now; 176 tiles at K3,
-// one per CU: 2.60 -> 0.87 ms.
+// the trace back, 7 % of a tile at K4 and 10 % at K3: its stored arrays (2 MB a tile), then one wave's chain of LDS reads and lane
+// minima.  C: a larger one stores less and recomputes more (176 tiles, C - 1 instead: K2 929 us for 898, K3 823 / 763, K4 812 / 732).
+// Registers: the codebook values are read anew for every tile, so that none of what the trace back needs lies in scratch.  It did, 20 of
+// a lane's registers at K4, and loading them in every turn waited for all arrays in flight: 176 tiles, one per CU, at K2 / 3 / 4 / 5 / 7 / 8
+// took 1161 / 815 / 801 / 950 / 1067 / 955 us and take 900 / 763 / 735 / 857 / 888 / 844; 1024 at K4 3.25 -> 3.04 ms (7.46 with the
+// table and one byte of backpointer per entry and step, the first version).
 // Arithmetic and tie-breaking are the reference's: float32, d = (x - cb)^2, m + w * d without fusing, the first index
 // among equal values in every min / argmin.
 template <int K> struct VitCfg {
@@ -33,7 +34,7 @@ template <int K> struct VitCfg {
   static constexpr int NJ = NB / LANES;                               // predecessors a thread looks at: LOWS * NJ = 64
   static constexpr int C = K == 2 ? 4 : (K == 3 ? 3 : (K == 4 ? 2 : 1));  // steps per stored M array
   static constexpr int ROW = SJ + SJ / 16;                            // floats of an M array in LDS (the trace back shifts every 16)
-  static constexpr size_t LDS = ((size_t)2 * ROW + 1024 + 512 + 32) * 4;
+  static constexpr size_t LDS = ((size_t)2 * ROW + 1024 + 512 + 32 + 128) * 4;
 };
 // stored M arrays of one tile: M_t for t = T - 1 - C, T - 1 - 2 C, ... > 0
 inline __host__ __device__ int vit_rows(int T, int C) { return T >= 2 ? (T - 2) / C : 0; }
@@ -81,24 +82,28 @@ __global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __r
   uint32_t* red_i = (uint32_t*)(red_v + 16);
   const int tid = threadIdx.x, lane = tid & 63;
   // this thread's M entries low(r, i) and predecessors pj(j)
-  auto low = [&](int r, int i) { return LANES == 1 ? (r * THREADS + tid) * RUN + i : tid / LANES; };
-  auto pj = [&](int j) { return LANES == 1 ? j : j * LANES + tid % LANES; };
+  auto low_of = [](int r, int i, int id) { return LANES == 1 ? (r * THREADS + id) * RUN + i : id / LANES; };
+  auto pj_of = [](int j, int id) { return LANES == 1 ? j : j * LANES + id % LANES; };
+  auto low = [&](int r, int i) { return low_of(r, i, tid); };
+  auto pj = [&](int j) { return pj_of(j, tid); };
 
   for (int i = tid; i < 1024; i += THREADS) cbv[i] = i <= 1020 ? (float)((double)(i - 510) / rms) : 0.f;
   __syncthreads();
   auto cb_of = [&](uint32_t s) { return cbv[__builtin_amdgcn_sad_u8(s * GEN_A + GEN_B, 0u, 0u)]; };
-  float cb[RUNS][RUN][NJ];
-#pragma unroll
-  for (int r = 0; r < RUNS; ++r)
-#pragma unroll
-    for (int i = 0; i < RUN; ++i)
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) cb[r][i][j] = cb_of((uint32_t)(pj(j) * SJ + low(r, i)));
-
   const int nrows = vit_rows(T, C);
   float* my_rows = rows_g + (size_t)blockIdx.x * nrows * SJ;          // one set of stored arrays per workgroup, reused tile by tile
   for (size_t tile = blockIdx.x; tile < (size_t)tiles; tile += gridDim.x) {
     for (int i = tid; i < T; i += THREADS) { xs[i] = x[tile * T + i]; ws[i] = w[tile * T + i]; }
+    // the codebook values of this thread's states: read again for every tile (2 us of 800), so that the trace back has their registers
+    float cb[RUNS][RUN][NJ];
+    int own = tid;
+    asm volatile("" : "+v"(own));                         // or the compiler keeps the 64 addresses over the trace back instead
+#pragma unroll
+    for (int r = 0; r < RUNS; ++r)
+#pragma unroll
+      for (int i = 0; i < RUN; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) cb[r][i][j] = cb_of((uint32_t)(pj_of(j, own) * SJ + low_of(r, i, own)));
     uint32_t j0 = 0, final_state = 0;
     const int passes = tailbite ? 2 : 1;
     for (int pass = 0; pass < passes; ++pass) {
@@ -189,35 +194,38 @@ __global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __r
     // lowest bits (and the upper bits of j_n, if the lanes do not suffice, in PER registers): level n - 1 reads M_{t-n},
     // each level is a minimum over the lanes of one digit, which leaves the next level's values where they are needed.
     // The lanes that attain a level's minimum are kept as a mask, and the digits are read off the masks at the end.
-    uint16_t* st = states + tile * T;
+    uint16_t* st = (uint16_t*)red_v + 64;               // [256] in LDS, out at the end
     if (tid == 0) st[T - 1] = (uint16_t)final_state;
     if (T > 1) {
+      // in registers of their own: what the compiler derives from them and keeps is not kept over the forward passes
+      int id = tid, ln = lane;
+      asm volatile("" : "+v"(id), "+v"(ln));
       constexpr int RL = SJ >= THREADS ? SJ / THREADS : 1;             // row elements per thread
       auto lds_pos = [](uint32_t e) { return e + (e >> 4); };
-      const float* row = my_rows + (size_t)nrows * SJ;
-      int left = nrows;                                                // stored arrays not yet requested
-      auto request = [&](float (&reg)[RL]) {
-        if (left > 0) {
-          row -= SJ;
+      // The q-th array that the trace back reads: the stored ones from the last on, then M_0.  Nothing in the loop may make it wait for
+      // loads that it has just issued: no branch around a load (M_0 comes in where the array goes to LDS), no value in scratch.
+      auto request = [&](float (&reg)[RL], int q) {                    // beyond the last stored one: the first again, not looked at
+        const float* row = my_rows + (size_t)max(nrows - 1 - q, 0) * SJ;
 #pragma unroll
-          for (int i = 0; i < RL; ++i) if (SJ >= THREADS || tid < SJ) reg[i] = row[i * THREADS + tid];
-        } else {
-#pragma unroll
-          for (int i = 0; i < RL; ++i) reg[i] = (!tailbite || (uint32_t)(i * THREADS + tid) == j0) ? 0.f : __builtin_inff();      // M_0
-        }
-        --left;
+        for (int i = 0; i < RL; ++i) reg[i] = row[(i * THREADS + id) & (SJ - 1)];
       };
-      auto place = [&](const float (&reg)[RL], float* buf) {
+      auto place = [&](const float (&reg)[RL], int q, float* buf) {
+        auto first = [&](uint32_t e) { return !tailbite || e == j0 ? 0.f : __builtin_inff(); };      // M_0
 #pragma unroll
-        for (int i = 0; i < RL; ++i) if (SJ >= THREADS || tid < SJ) buf[lds_pos((uint32_t)(i * THREADS + tid))] = reg[i];
+        for (int i = 0; i < RL; ++i) {
+          const uint32_t e = (uint32_t)(i * THREADS + id);
+          if (SJ >= THREADS || id < SJ) buf[lds_pos(e)] = RL > 8 || q < nrows ? reg[i] : first(e);
+        }
+        // with 16 elements a thread the selections above would take longer than a second pass at the end (176 tiles at K2, 966 / 900 us)
+        if (RL > 8 && q >= nrows)
+          for (int e = id; e < SJ; e += THREADS) buf[lds_pos((uint32_t)e)] = first((uint32_t)e);
       };
       uint32_t s = final_state;
-      int t = T - 1;
-      auto turn = [&](auto nc, const float* buf) {
+      auto turn = [&](auto nc, const float* buf, int t) {
         constexpr int n = decltype(nc)::value;
         constexpr int PERB = K * n > 6 ? K * n - 6 : 0, PER = 1 << PERB, NBITS = K - PERB;      // lane bits of j_n
         const uint32_t p0 = s >> K;
-        auto digit = [&](int i) { return i == n ? (uint32_t)lane & ((1u << NBITS) - 1) : ((uint32_t)lane >> (NBITS + K * (n - 1 - i))) & ((1u << K) - 1); };
+        auto digit = [&](int i) { return i == n ? (uint32_t)ln & ((1u << NBITS) - 1) : ((uint32_t)ln >> (NBITS + K * (n - 1 - i))) & ((1u << K) - 1); };
         unsigned long long mask[n][PER];
         float v = 0.f;
 #pragma unroll
@@ -267,38 +275,38 @@ __global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __r
           }
           if (d < n - 1) base += j << shift;
           s = j * SJ + (s >> K);
-          if (lane == 0) st[t - d - 1] = (uint16_t)s;
+          if (ln == 0) st[t - d - 1] = (uint16_t)s;
         }
       };
-      // arrays travel three turns ahead, two in registers and one in the other LDS buffer (K = 2, whose arrays are the
-      // largest: two turns, one in registers)
-      constexpr bool TWO = RL <= 8;
-      float ra[RL], rb[TWO ? RL : 1];
-      request(ra);
-      place(ra, M0);
-      request(ra);
-      if constexpr (TWO) request(rb);
+      // arrays travel AHEAD turns ahead in registers, one more in the other LDS buffer
+      constexpr int AHEAD = RL <= 8 ? 4 : 1, UNROLL = AHEAD > 2 ? AHEAD : 2;
+      float set[AHEAD][RL];
+      request(set[0], 0);
+      place(set[0], 0, M0);
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) request(set[i], 1 + i);
       __syncthreads();
-      auto one = [&](float (&reg)[RL], float* cur, float* nxt) {
-        place(reg, nxt);
-        request(reg);
-        if (tid < 64) {
-          if (t >= C) turn(std::integral_constant<int, C>{}, cur);
-          else if (C >= 4 && t == 3) turn(std::integral_constant<int, (C >= 4 ? 3 : 1)>{}, cur);
-          else if (C >= 3 && t == 2) turn(std::integral_constant<int, (C >= 3 ? 2 : 1)>{}, cur);
-          else turn(std::integral_constant<int, 1>{}, cur);
-        }
-        t -= C;
-        __syncthreads();
-      };
-      while (t > 0) {
-        one(ra, M0, M1);
-        if (t > 0) {
-          if constexpr (TWO) one(rb, M1, M0);
-          else one(ra, M1, M0);
+      const int full = (T - 1) / C, rest = (T - 1) % C;
+      for (int k0 = 0; k0 < full; k0 += UNROLL) {
+#pragma unroll
+        for (int i = 0; i < UNROLL; ++i) {
+          const int k = k0 + i;
+          if (k >= full) break;                                        // uniform
+          place(set[i % AHEAD], k + 1, i & 1 ? M0 : M1);
+          request(set[i % AHEAD], k + 1 + AHEAD);
+          if (id < 64) turn(std::integral_constant<int, C>{}, i & 1 ? M1 : M0, T - 1 - C * k);
+          __syncthreads();
         }
       }
+      if (C > 1 && rest > 0 && id < 64) {                              // from M_0 itself
+        const float* buf = full & 1 ? M1 : M0;
+        if (C >= 4 && rest == 3) turn(std::integral_constant<int, (C >= 4 ? 3 : 1)>{}, buf, rest);
+        else if (C >= 3 && rest == 2) turn(std::integral_constant<int, (C >= 3 ? 2 : 1)>{}, buf, rest);
+        else turn(std::integral_constant<int, 1>{}, buf, rest);
+      }
     }
+    __syncthreads();
+    for (int i = tid; i < T; i += THREADS) states[tile * T + i] = st[i];
     __syncthreads();                                    // xs, ws and the M arrays are free for the next tile
   }
 }

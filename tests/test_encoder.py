@@ -328,3 +328,20 @@ def test_encoder_block_launches_refuse_wrong_sizes():
     for rows, n, col in ((0, 16, 0), (8, 16, 0), (16, 24, 0), (16, 16, 16), (16, 32, 8), (16, 16, -16), (1 << 31, 16, 0)):
         bad = L.htr_encode_targets(*p[:3], rows, n, col, p[3], None)
         assert bad == L.htr_encode_quantized(*p[:4], rows, n, col, *p[4:7], None) == L.htr_encode_targets(*p[:3], 8, 16, 0, p[3], None) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,lengths", [(2, (10, 13, 14, 17, 18, 21, 22)), (3, (9, 10, 11, 13, 14, 16, 17, 20)), (4, (7, 8, 9, 10, 11, 12, 13, 14, 256)),
+                                       (5, (4, 5, 6, 7, 8, 9, 10, 11)), (6, (5, 6, 9)), (7, (5, 6, 7, 10)), (8, (5, 7, 8, 256))])
+@pytest.mark.parametrize("tailbite", [True, False])
+def test_gpu_search_with_few_stored_arrays(dev, oracle, K, lengths, tailbite):
+    """Lengths with one to ten stored arrays, around the four that the trace back has in flight and its loop takes at a time, and the
+    longest.  Whole numbers: exact."""
+    from htr_amd import encode
+    for T in lengths:
+        print(f"viterbi K={K} T={T} tailbite={tailbite}", flush=True)
+        g = torch.Generator().manual_seed(91 * K + T)
+        x = torch.randn(2, T, generator=g)
+        w = torch.rand(2, T, generator=g) + 0.25
+        st = encode.viterbi(x.to(dev), w.to(dev), None, K, tailbite=tailbite).cpu().numpy()
+        assert np.array_equal(st.astype(np.uint32), oracle.c_viterbi(x.numpy(), w.numpy(), K, tailbite=tailbite))
