@@ -17,7 +17,7 @@
 // of them, one wave), with the same arithmetic, so the indices it finds are those the forward pass would have recorded.
 // Which array comes next does not depend on the state, so the other waves fetch it into LDS meanwhile.
 // Bound: vector issue in the forward passes (K4: 2890 cycles a step, 2944 by the rates above; 0.74 M cycles a pass), then
-// the trace back, 7 % of a tile at K4 and 10 % at K3: its stored arrays (2 MB a tile), then one wave's chain of LDS reads and lane
+// the trace back, 10 % of a tile at K3 and K4: its stored arrays (2 MB a tile), then one wave's chain of LDS reads and lane
 // minima.  C: a larger one stores less and recomputes more (176 tiles, C - 1 instead: K2 929 us for 898, K3 823 / 763, K4 812 / 732).
 // Registers: the codebook values are read anew for every tile, so that none of what the trace back needs lies in scratch.  It did, 20 of
 // a lane's registers at K4, and loading them in every turn waited for all arrays in flight: 176 tiles, one per CU, at K2 / 3 / 4 / 5 / 7 / 8
