@@ -235,7 +235,7 @@ class _NativeBlocks:
         self.G, self.cb, self.K, self.max_batch = G, cb, K, max_batch
         self.x = torch.empty_like(G.wg)
         self.states = torch.zeros(G.wg.shape, dtype=torch.int16, device=dev)
-        self.err = torch.empty((G.Wt.shape[0], 16), device=dev)
+        self.err = torch.empty((G.Wt.shape[0], 16), dtype=torch.float32, device=dev)      # not torch's default type: a kernel writes it
 
     def __call__(self, k):
         G, L, m, n = self.G, _native.lib(), self.G.Wt.shape[0], self.G.n

@@ -345,3 +345,19 @@ def test_gpu_search_with_few_stored_arrays(dev, oracle, K, lengths, tailbite):
         w = torch.rand(2, T, generator=g) + 0.25
         st = encode.viterbi(x.to(dev), w.to(dev), None, K, tailbite=tailbite).cpu().numpy()
         assert np.array_equal(st.astype(np.uint32), oracle.c_viterbi(x.numpy(), w.numpy(), K, tailbite=tailbite))
+
+
+@pytest.mark.parametrize("default", [torch.float64, torch.bfloat16])
+def test_buffers_of_the_encoder_blocks_do_not_follow_the_default_type(default):
+    """htr_encode_quantized writes float32 errors: a buffer of torch's default type would be read as other numbers, or be too short."""
+    from types import SimpleNamespace
+    from htr_amd import encode
+    G = SimpleNamespace(Wt=torch.zeros(32, 128), wg=torch.zeros(2, 256))
+    before = torch.get_default_dtype()
+    torch.set_default_dtype(default)
+    try:
+        blocks = encode._NativeBlocks(G, None, 4, 1024)
+    finally:
+        torch.set_default_dtype(before)
+    assert blocks.err.dtype == torch.float32 and blocks.err.shape == (32, 16)
+    assert blocks.x.dtype == torch.float32 and blocks.x.shape == (2, 256) and blocks.states.dtype == torch.int16
