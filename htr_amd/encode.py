@@ -160,8 +160,9 @@ def prep_H(H, W, damp=0.01):
     bit, and damping the diagonal in place, or before the dead columns are fixed, rounds differently."""
     H = H.clone().double()
     dead = torch.diag(H) == 0
-    torch.diagonal(H).masked_fill_(dead, 1.0)                     # masks, not index lists, which the GPU makes in a synchronisation
-    W = W.masked_fill(dead[None, :], 0)
+    H[dead, dead] = 1.0
+    W = W.clone()
+    W[:, dead] = 0
     H += damp * torch.diag(H).mean() * torch.eye(H.shape[0], device=H.device, dtype=H.dtype)
     return H, W
 

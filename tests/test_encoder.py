@@ -361,3 +361,22 @@ def test_buffers_of_the_encoder_blocks_do_not_follow_the_default_type(default):
         torch.set_default_dtype(before)
     assert blocks.err.dtype == torch.float32 and blocks.err.shape == (32, 16)
     assert blocks.x.dtype == torch.float32 and blocks.x.shape == (2, 256) and blocks.states.dtype == torch.int16
+
+
+@pytest.mark.parametrize("shape", [(6, 1), (6,), (6, 64), (6, 256), (1, 6)])
+def test_dead_columns_of_a_matrix_that_does_not_fit_the_hessian_are_refused(shape):
+    from htr_amd import encode
+    H = torch.diag(torch.arange(128).float())
+    with pytest.raises(IndexError):
+        encode.prep_H(H, torch.ones(shape))
+    with pytest.raises(IndexError):
+        encode.prep_H(H[:1], torch.ones(6, 128))
+
+
+def test_dead_columns_of_a_matrix_with_further_dimensions():
+    from htr_amd import encode
+    H = torch.diag((torch.arange(128) != 5).float())
+    W = torch.ones(6, 128, 3)
+    Hd, Wd = encode.prep_H(H, W, damp=0.0)
+    assert torch.equal(Wd[:, 5], torch.zeros(6, 3)) and int((Wd == 0).sum()) == 18 and bool((W == 1).all())
+    assert torch.equal(Hd, torch.eye(128, dtype=torch.float64))
