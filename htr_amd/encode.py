@@ -260,7 +260,7 @@ def encode_group(jobs, K, seed=1234, shared_su=True, damp=0.01, max_batch=1024, 
     G = _Group(jobs, seed, shared_su, damp)
     cb = wire.codebook_f32(G.Wt.device)
     ntiles = G.wg.shape[0]
-    native = VITERBI is None and G.Wt.is_cuda and all(t.is_contiguous() for t in (G.Wt, G.F, G.Q, G.rs, G.wg))
+    native = VITERBI is None and G.Wt.is_cuda and ntiles > 0 and all(t.is_contiguous() for t in (G.Wt, G.F, G.Q, G.rs, G.wg))
     quantize = _NativeBlocks(G, cb, K, max_batch) if native else None
     for k in range(G.nb - 1, -1, -1):
         cols = slice(16 * k, 16 * k + 16)

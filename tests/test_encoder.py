@@ -380,3 +380,20 @@ def test_dead_columns_of_a_matrix_with_further_dimensions():
     Hd, Wd = encode.prep_H(H, W, damp=0.0)
     assert torch.equal(Wd[:, 5], torch.zeros(6, 3)) and int((Wd == 0).sum()) == 18 and bool((W == 1).all())
     assert torch.equal(Hd, torch.eye(128, dtype=torch.float64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [(0,), (0, 128)])
+def test_gpu_encoder_takes_matrices_without_rows(dev, rows):
+    """A matrix of 0 rows, alone and beside another one: empty results, as on the CPU, and the other as by itself."""
+    from htr_amd import encode
+    print(f"encoder, matrices of {rows} rows", flush=True)
+    g = torch.Generator().manual_seed(3)
+    a = torch.randn(256, 128, generator=g)
+    H = (a.T @ a / 256).to(dev)
+    jobs = [dict(W=0.02 * torch.randn(m, 128, generator=g).to(dev), H=H) for m in rows]
+    got = encode.encode_group(jobs, 4, seed=5)
+    assert [tuple(r["qweight"].shape) for r in got] == [(m // 16, 8, 32) for m in rows] and got[0]["What"].shape == (0, 128)
+    if len(rows) > 1:
+        other = encode.encode_group([dict(W=jobs[0]["W"].new_zeros(128, 128), H=H), jobs[1]], 4, seed=5)[1]
+        assert torch.equal(got[1]["qweight"], other["qweight"]) and torch.equal(got[1]["What"], other["What"])
