@@ -226,10 +226,28 @@ class _Group:
         self.wg = wg / wg.mean(dim=1, keepdim=True)
 
 
+class _TorchBlocks:
+    """What encode_group does with a 16-column block: its targets, the search, and what follows from the states: scaled values, states
+    and the error, which is returned."""
+
+    def __init__(self, G, cb, K, max_batch):
+        self.G, self.cb, self.K, self.max_batch = G, cb, K, max_batch
+        self.search = VITERBI or (lambda x, w, cb, k: viterbi(x, w, cb, k))
+
+    def __call__(self, k):
+        G, cols = self.G, slice(16 * k, 16 * k + 16)
+        target = ((G.Wt[:, cols] + G.F[:, cols]) / G.rs[:, None]).reshape(-1, 256)
+        for b0 in range(0, G.wg.shape[0], self.max_batch):
+            part = slice(b0, b0 + self.max_batch)
+            G.S[part, k] = self.search(target[part].contiguous(), G.wg[part].contiguous(), self.cb, self.K)
+        q = self.cb[G.S[:, k]].reshape(-1, 16) * G.rs[:, None]
+        G.Q[:, cols] = q
+        return G.Wt[:, cols] - q
+
+
 class _NativeBlocks:
-    """What encode_group does with a 16-column block, on the GPU in three launches: targets, search, and what follows from the states
-    (scaled values, error, states).  The same float32 operations as the torch lines in encode_group, bit for bit: eleven launches of
-    torch's, 45 us of the 950 that a block of 2816 rows takes, are two."""
+    """The same on the GPU in three launches: targets, search, and what follows from the states.  The same float32 operations as
+    _TorchBlocks, bit for bit: eleven launches of torch's, 45 us of the 950 that a block of 2816 rows takes, are two."""
 
     def __init__(self, G, cb, K, max_batch):
         dev = G.Wt.device
@@ -256,31 +274,15 @@ def encode_group(jobs, K, seed=1234, shared_su=True, damp=0.01, max_batch=1024, 
     """jobs: list of dict(W=[m, n], H=[n, n]) sharing n.  Returns a list of dict(qweight, scales, su, sv, What, Q)
     (htr/encode.py:45-110): block LDLQ from the last 16-column block to the first, each block's tiles quantized by the
     trellis search against the row scales, the block's error fed forward through the feedback matrix."""
-    search = VITERBI or (lambda x, w, cb, k: viterbi(x, w, cb, k))
     G = _Group(jobs, seed, shared_su, damp)
     cb = wire.codebook_f32(G.Wt.device)
-    ntiles = G.wg.shape[0]
-    native = VITERBI is None and G.Wt.is_cuda and ntiles > 0 and all(t.is_contiguous() for t in (G.Wt, G.F, G.Q, G.rs, G.wg))
-    quantize = _NativeBlocks(G, cb, K, max_batch) if native else None
+    native = VITERBI is None and G.Wt.is_cuda and G.wg.shape[0] > 0 and all(t.is_contiguous() for t in (G.Wt, G.F, G.Q, G.rs, G.wg))
+    quantize = (_NativeBlocks if native else _TorchBlocks)(G, cb, K, max_batch)
     for k in range(G.nb - 1, -1, -1):
-        cols = slice(16 * k, 16 * k + 16)
-        if quantize is not None:
-            err = quantize(k)
-            if k > 0:
-                for first, last, Lb in G.factors:
-                    G.F[first:last, :16 * k] += err[first:last] @ Lb[cols, :16 * k]
-            if log and k % 32 == 0:
-                log(f"  block {k}/{G.nb}")
-            continue
-        target = ((G.Wt[:, cols] + G.F[:, cols]) / G.rs[:, None]).reshape(-1, 256)
-        for b0 in range(0, ntiles, max_batch):
-            G.S[b0:b0 + max_batch, k] = search(target[b0:b0 + max_batch].contiguous(), G.wg[b0:b0 + max_batch].contiguous(), cb, K)
-        q = cb[G.S[:, k]].reshape(-1, 16) * G.rs[:, None]
-        G.Q[:, cols] = q
+        err = quantize(k)
         if k > 0:
-            err = G.Wt[:, cols] - q
             for first, last, Lb in G.factors:
-                G.F[first:last, :16 * k] += err[first:last] @ Lb[cols, :16 * k]
+                G.F[first:last, :16 * k] += err[first:last] @ Lb[16 * k:16 * k + 16, :16 * k]
         if log and k % 32 == 0:
             log(f"  block {k}/{G.nb}")
     outs = []
