@@ -208,7 +208,11 @@ template <int K> struct Window {
 #pragma unroll
     for (int k = 0; k < K; ++k) mid[k] = __builtin_amdgcn_alignbit(V[k], V[k + 1], 16);
   }
-  template <int U> __device__ __forceinline__ uint32_t state() const { return (word<U>() >> shift<U>()) & 0xFFFFu; }
+  template <int U> __device__ __forceinline__ uint32_t state() const {
+    constexpr int b = 16 + (U + 1) * K, w = b >> 5, off = b & 31;
+    if constexpr (off <= 16) return (V[w] >> (16 - off)) & 0xFFFFu;
+    else return (mid[w] >> (32 - off)) & 0xFFFFu;
+  }
   // generator word x = s*A + B; s < 2^16 and A < 2^24 so this is one v_mad_u32_u24
   template <int U> __device__ __forceinline__ uint32_t genword() const { return state<U>() * GEN_A + GEN_B; }
   // two consecutive weights as packed halves (1534 + v(u), 1534 + v(u + 1))
@@ -219,51 +223,8 @@ template <int K> struct Window {
   template <int U> __device__ __forceinline__ int value() const {   // integer v(s)
     return (int)__builtin_amdgcn_sad_u8(genword<U>(), 0u, 0u) - 510;
   }
-  // dword that holds the window of state U, from bit shift<U>() on
-  template <int U> __device__ __forceinline__ uint32_t word() const {
-    constexpr int b = 16 + (U + 1) * K, w = b >> 5, off = b & 31;
-    if constexpr (off <= 16) return V[w]; else return mid[w];
-  }
-  template <int U> static constexpr int shift() {
-    constexpr int off = (16 + (U + 1) * K) & 31;
-    return off <= 16 ? 16 - off : 32 - off;
-  }
-  // Four weights, two pairs as above, with the instructions in an order of their own.  All three kinds issue every 4.4 cycles by
-  // themselves, but a multiplication overlaps with an extraction or a byte sum of the SIMD's other waves, and how often it does
-  // depends on the order: bfe mad bfe sad mad sad, the compiler's, 4.6 cycles per instruction with two waves on a SIMD and 3.95 with
-  // four, this one 4.0 and 3.7 (the best of 29; an `and` or a shift in the place of a bfe, 4 bytes of code less, spoils it).
-  // us before / after: 6144x4096 K3 1 row 8.5 / 8.1, 14336x4096 K5 1 row 13.2 / 12.5, 152064x4096 K4 71.9 / 70.9, 4096x14336 K3 13
-  // rows 14.2 / 13.8, 32 rows 18.3 / 17.9; 6144x4096 K3 32 rows 11.75 / 11.80.
-  template <int U> __device__ __forceinline__ void quad_f16(uint32_t& lo, uint32_t& hi) const {
-    uint32_t t0, t1, t2, t3;
-    asm("v_bfe_u32 %[t0], %[w0], %[o0], 16\n\t"
-        "v_bfe_u32 %[t1], %[w1], %[o1], 16\n\t"
-        "v_bfe_u32 %[t2], %[w2], %[o2], 16\n\t"
-        "v_bfe_u32 %[t3], %[w3], %[o3], 16\n\t"
-        "v_mad_u32_u24 %[t0], %[t0], %[a], %[b]\n\t"
-        "v_sad_u8 %[lo], %[t0], 0, %[base]\n\t"
-        "v_mad_u32_u24 %[t1], %[t1], %[a], %[b]\n\t"
-        "v_sad_hi_u8 %[lo], %[t1], 0, %[lo]\n\t"
-        "v_mad_u32_u24 %[t2], %[t2], %[a], %[b]\n\t"
-        "v_sad_u8 %[hi], %[t2], 0, %[base]\n\t"
-        "v_mad_u32_u24 %[t3], %[t3], %[a], %[b]\n\t"
-        "v_sad_hi_u8 %[hi], %[t3], 0, %[hi]"
-        : [lo] "=&v"(lo), [hi] "=&v"(hi), [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3)
-        : [w0] "v"(word<U>()), [w1] "v"(word<U + 1>()), [w2] "v"(word<U + 2>()), [w3] "v"(word<U + 3>()), [o0] "n"(shift<U>()),
-          [o1] "n"(shift<U + 1>()), [o2] "n"(shift<U + 2>()), [o3] "n"(shift<U + 3>()), [a] "s"(GEN_A), [b] "v"(GEN_B), [base] "v"(0x64006400u));
-  }
-  // 8 consecutive weights as an MFMA operand; QUADS: in that order (k_linear_wide, which decodes one block of its many this way, is
-  // 0.1 us slower with it: 640x512 97 rows 11.73 / 11.78)
-  template <int U0, bool QUADS = true> __device__ __forceinline__ h8 group8() const {
-    u4 v;
-    if constexpr (QUADS) {
-      uint32_t q[4];
-      quad_f16<U0>(q[0], q[1]);
-      quad_f16<U0 + 4>(q[2], q[3]);
-      v = u4{q[0], q[1], q[2], q[3]};
-    } else {
-      v = u4{pair_f16<U0>(), pair_f16<U0 + 2>(), pair_f16<U0 + 4>(), pair_f16<U0 + 6>()};
-    }
+  template <int U0> __device__ __forceinline__ h8 group8() const {   // 8 consecutive weights as an MFMA operand
+    u4 v = {pair_f16<U0>(), pair_f16<U0 + 2>(), pair_f16<U0 + 4>(), pair_f16<U0 + 6>()};
     return __builtin_bit_cast(h8, v);
   }
 };

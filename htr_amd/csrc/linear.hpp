@@ -360,7 +360,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_rotate_mfma(const void* __restri
 template <int K> struct DecodedStep { h8 a[4]; };   // MFMA A operands of one step: (row 2q | 2q+1) x (columns 0..7 | 8..15)
 
 // NODECODE (timing anchors only): the operands are the raw stream words, no arithmetic at all; results are meaningless
-template <int K, bool NODECODE = false, bool QUADS = true> __device__ __forceinline__ void decode_step(const StreamRegs<K>& r, int hist, DecodedStep<K>& d) {
+template <int K, bool NODECODE = false> __device__ __forceinline__ void decode_step(const StreamRegs<K>& r, int hist, DecodedStep<K>& d) {
   if constexpr (NODECODE) {
     const u4 raw = {r.d[0], r.d[1 % K], r.d[2 % K], r.d[3 % K]};
 #pragma unroll
@@ -373,12 +373,12 @@ template <int K, bool NODECODE = false, bool QUADS = true> __device__ __forceinl
   __builtin_amdgcn_sched_barrier(0);
   Window<K> win;
   win.build_tail(r);
-  d.a[1] = win.template group8<8, QUADS>();
-  d.a[2] = win.template group8<16, QUADS>();
-  d.a[3] = win.template group8<24, QUADS>();
+  d.a[1] = win.template group8<8>();
+  d.a[2] = win.template group8<16>();
+  d.a[3] = win.template group8<24>();
   __builtin_amdgcn_sched_barrier(0);
   win.build_head(prev);
-  d.a[0] = win.template group8<0, QUADS>();
+  d.a[0] = win.template group8<0>();
 }
 
 // The same with something to do at the fence between the two parts (a barrier and LDS reads, in the batched kernel)

@@ -182,7 +182,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_linear_wide(const uint32_t* __re
   };
   {
     DecodedStep<K> d0;
-    decode_step<K, false, false>(buf[0], hist, d0);
+    decode_step<K>(buf[0], hist, d0);
     prefetch(buf[0]);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
