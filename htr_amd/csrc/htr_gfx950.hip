@@ -95,7 +95,7 @@ size_t htr_workspace_bytes(int m, int n, int K, int M, int nsplit) {
   }
   if (M > HTR_MAX_GROUP_ROWS) return 0;          // the chunked kernel takes up to 32 rows
   Plan pl;
-  if (!make_plan(m, n, M, nsplit, pl)) return 0;
+  if (!make_plan(m, n, K, M, nsplit, pl)) return 0;
   return ws_need((size_t)pl.wgs * M * 128 * sizeof(float), prerot_bytes(n, M));
 }
 
@@ -125,7 +125,7 @@ int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
   }
   if (M > HTR_MAX_GROUP_ROWS) return HTR_ERR_BATCH;
   Plan pl;
-  if (!make_plan(m, n, M, nsplit, pl)) return HTR_ERR_SPLIT;
+  if (!make_plan(m, n, K, M, nsplit, pl)) return HTR_ERR_SPLIT;
   out6[0] = pl.chunk; out6[1] = pl.wgs; out6[2] = pl.segfin; out6[3] = pl.nbl; out6[4] = pl.prerot; out6[5] = (int)pl.lds;
   return HTR_OK;
 }
@@ -289,7 +289,7 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
   }
   if (M > HTR_MAX_GROUP_ROWS) return HTR_ERR_BATCH;          // an explicit chunked plan: that kernel takes up to 32 rows
   Plan pl;
-  if (!make_plan(m, n, M, nsplit, pl)) return HTR_ERR_SPLIT;
+  if (!make_plan(m, n, K, M, nsplit, pl)) return HTR_ERR_SPLIT;
   // the in-kernel rotation reads 16-bit elements in pairs: float32 activations, and rows that do not start on a
   // 4-byte boundary, take the pre-rotation
   const bool prerot = pl.prerot || x_dtype == HTR_F32 || ((uintptr_t)x & 3);
@@ -573,7 +573,7 @@ int htr_anchor_linear(int kind, const void* qweight, const void* scales, const v
   if (x_dtype == HTR_F32 || !dtype_ok(x_dtype) || !dtype_ok(y_dtype)) return HTR_ERR_DTYPE;
   if (((uintptr_t)qweight & 15) || ((uintptr_t)x & 3)) return HTR_ERR_ALIGN;
   Plan pl;
-  if (!make_plan(m, n, 1, 0, pl) || pl.prerot) return HTR_ERR_SPLIT;
+  if (!make_plan(m, n, K, 1, 0, pl) || pl.prerot) return HTR_ERR_SPLIT;
   const size_t need = htr_workspace_bytes(m, n, K, 1, 0);
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
   LinearLaunch a;

@@ -96,25 +96,9 @@ inline bool plan_for_chunk(int m, int n, int M, int chunk, Plan& pl) {
 // throughput bound, proportional to the load of the fullest CU, plus a set-up per workgroup); a penalty for chunks
 // that do not tile the rows of column blocks; the extra launch of a pre-rotation; and the growth of all per-step work
 // with the number of activation rows.
-inline bool search_plan(int m, int n, int M, int nsplit, int cus, Plan& pl) {
+inline bool search_chunk(int m, int n, int M, int cus, Plan& pl) {
   const int nblk = n / 128, rbs = m / 128;
   const long vtotal = (long)rbs * nblk;
-  pl.mb = M <= 8 ? 1 : (M <= 16 ? 2 : 4);
-  if (nsplit > 0) {                                                 // explicit plan (tuning): chunk length in the low
-    const int chunk = nsplit & 0xFFFFF;                             // 20 bits, bit 30 = force pre-rotation
-    bool ok = chunk > 0 ? plan_for_chunk(m, n, M, chunk, pl) : false;
-    if (ok && (nsplit & (1 << 30))) pl.prerot = 1;
-    return ok;
-  }
-  // Large matrices: one row block per workgroup, or two equal chunks per compute unit.  The compute units take whole row blocks in
-  // rounds, so the last round is as long as the others however few row blocks are left; equal chunks cost 3 % more (partials, row
-  // ends inside a chunk; 10 % with five rows, which have no PACE there: 152064x4096 K3 71.8 / 72.8).  K4, 1 row, us with row blocks / chunks: 73728x4096 48.6 / 39.8, 102400x4096 62.0 / 51.8,
-  // 152064x4096 72.8 / 71.7 (another run 73.3 / 70.5), 128256x4096 61.8 / 61.3, 131072x4096 61.1 / 63.1; 73728x8192 K5 90.6 / 74.2.
-  if (vtotal >= (long)64 * cus && nblk <= 64) {
-    const int rounds = (rbs + cus - 1) / cus;
-    if ((M <= 4 ? 1.03 : 1.1) * rbs < (double)rounds * cus && plan_for_chunk(m, n, M, (int)((vtotal + 2 * cus - 1) / (2 * cus)), pl)) return true;
-    if (plan_for_chunk(m, n, M, nblk, pl)) return true;
-  }
   const double rows = M <= 8 ? 1.0 + 0.06 * (M - 1) : (M <= 16 ? 2.2 : 6.5);
   double best = 1e30;
   bool found = false;
@@ -142,18 +126,62 @@ inline bool search_plan(int m, int n, int M, int nsplit, int cus, Plan& pl) {
   return found;
 }
 
+inline bool search_plan(int m, int n, int K, int M, int nsplit, int cus, Plan& pl) {
+  const int nblk = n / 128, rbs = m / 128;
+  const long vtotal = (long)rbs * nblk;
+  pl.mb = M <= 8 ? 1 : (M <= 16 ? 2 : 4);
+  if (nsplit > 0) {                                                 // explicit plan (tuning): chunk length in the low
+    const int chunk = nsplit & 0xFFFFF;                             // 20 bits, bit 30 = force pre-rotation
+    bool ok = chunk > 0 ? plan_for_chunk(m, n, M, chunk, pl) : false;
+    if (ok && (nsplit & (1 << 30))) pl.prerot = 1;
+    return ok;
+  }
+  // Large matrices: one row block per workgroup where that fits LDS
+  const bool large = vtotal >= (long)64 * cus && nblk <= 64;
+  bool found = false;
+  if (large) {
+    Plan whole;
+    whole.mb = pl.mb;
+    found = plan_for_chunk(m, n, M, nblk, whole);
+    if (found) pl = whole;
+  }
+  if (!found) found = search_chunk(m, n, M, cus, pl);
+  // ... or, instead of either, two equal chunks per compute unit.  The compute units take workgroups in rounds, so the last round is as
+  // long as the others however few are left; equal chunks fill it, at the price of partials, of row ends inside a chunk, and of PACE
+  // where the activations are rotated ahead.  They pay where the rounds hold `spare` times the steps that there are: later from five
+  // bits on, except over short rows, as whole row blocks then read at close to the memory's rate already (61184x6144 K5 4.4, K8 4.9 of
+  // the 5.0 TB/s of a copy; K4 3.7).  Measured on MI355X with margins from 1.005 to 1.5, n from 1536 to 8192; us with row blocks /
+  // chunks at a margin:
+  //   K4 1 row 61824x6144 (1.06) 50.6 / 50.6, 60032x6144 (1.09) 49.0 / 47.0, 152064x4096 (1.08) 72.8 / 71.7, 73728x4096 (1.33) 48.6 /
+  //   39.8; 3 rows 91776x4096 (1.07) 51.7 / 48.8; 5 rows, rotated ahead, 92672x4096 (1.06) 52.9 / 53.4, 90112x4096 (1.09) 52.5 / 50.9
+  //   K5 1 row 122496x2560 (1.07) 45.8 / 45.0, K6 153088x2048 (1.07) 54.1 / 51.6: short rows
+  //   K5 1 row 61184x6144 (1.07) 53.2 / 53.8, 3 rows, rotated ahead, 60032x6144 (1.09) 55.1 / 58.3, 5 rows 84736x4096 (1.16) 57.1 / 58.9
+  //   K6 1 row 61184x5120 (1.07) 51.1 / 52.8, 3 rows 112896x3072 (1.16) 60.4 / 56.5; K7 1 row 93568x4096 (1.05) 66.7 / 69.6; K8 3 rows
+  //   87680x3072 (1.12) 58.1 / 59.2
+  //   3 rows of 8192, whose row blocks do not fit, with the search's 32 steps: K4 61184 (1.07) 66.6 / 64.6, 43648 (1.12) 51.4 / 49.1; K6
+  //   46720 (1.05) 63.7 / 67.1, 50304 (1.30) 79.1 / 74.3; K7 46720 72.1 / 77.2
+  Plan even;
+  even.mb = pl.mb;
+  if (large && plan_for_chunk(m, n, M, (int)((vtotal + 2 * cus - 1) / (2 * cus)), even)) {
+    const bool early = K <= 4 || (K <= 6 && K * nblk <= 120);
+    const double spare = early ? (even.prerot && pl.chunk == nblk ? 1.1 : 1.06) : (even.prerot ? 1.2 : 1.15);
+    if (!found || spare * vtotal < (double)((pl.wgs + cus - 1) / cus) * pl.chunk * cus) { pl = even; found = true; }
+  }
+  return found;
+}
+
 // The search above walks every chunk length (up to 4096 of them): tens of microseconds on the host, more than the launch
-// it plans.  Plans depend only on (m, n, M, nsplit) and the device's CU count, so the last 64 distinct ones are kept.
-inline bool make_plan(int m, int n, int M, int nsplit, Plan& pl) {
+// it plans.  Plans depend only on (m, n, K, M, nsplit) and the device's CU count, so the last 64 distinct ones are kept.
+inline bool make_plan(int m, int n, int K, int M, int nsplit, Plan& pl) {
   const int cus = num_cu();
-  struct Entry { int m, n, M, nsplit, cus; bool ok; Plan pl; };
+  struct Entry { int m, n, K, M, nsplit, cus; bool ok; Plan pl; };
   static Entry cache[64];
   static int filled = 0, next = 0;
   static std::atomic_flag busy = ATOMIC_FLAG_INIT;
   while (busy.test_and_set(std::memory_order_acquire)) {}
   for (int i = 0; i < filled; ++i) {
     const Entry& e = cache[i];
-    if (e.m == m && e.n == n && e.M == M && e.nsplit == nsplit && e.cus == cus) {
+    if (e.m == m && e.n == n && e.K == K && e.M == M && e.nsplit == nsplit && e.cus == cus) {
       const bool ok = e.ok;
       pl = e.pl;
       busy.clear(std::memory_order_release);
@@ -162,10 +190,10 @@ inline bool make_plan(int m, int n, int M, int nsplit, Plan& pl) {
   }
   busy.clear(std::memory_order_release);
   Plan found = {};
-  const bool ok = search_plan(m, n, M, nsplit, cus, found);
+  const bool ok = search_plan(m, n, K, M, nsplit, cus, found);
   while (busy.test_and_set(std::memory_order_acquire)) {}
   Entry& e = cache[next];
-  e.m = m; e.n = n; e.M = M; e.nsplit = nsplit; e.cus = cus; e.ok = ok; e.pl = found;
+  e.m = m; e.n = n; e.K = K; e.M = M; e.nsplit = nsplit; e.cus = cus; e.ok = ok; e.pl = found;
   next = (next + 1) % 64;
   if (filled < 64) ++filled;
   busy.clear(std::memory_order_release);

@@ -344,3 +344,16 @@ def test_large_matrices_take_row_blocks_or_equal_chunks(L, m, n, M, chunk):
     steps = (m // 128) * (n // 128)
     assert out[0] == chunk and out[1] == -(-steps // chunk) and (chunk == n // 128 or out[1] <= 512)
     assert L.htr_workspace_bytes(m, n, 4, M, 0) >= 256 + out[1] * M * 512
+
+
+@pytest.mark.parametrize("K,m,n,M,chunk", [(3, 152064, 4096, 1, 75), (5, 152064, 4096, 1, 32), (8, 152064, 4096, 4, 32), (5, 73728, 4096, 1, 36), (6, 73728, 4096, 5, 36),
+                                           (7, 84736, 4096, 5, 32), (5, 122496, 2560, 1, 38), (6, 153088, 2048, 1, 38), (7, 153088, 2048, 1, 16), (4, 61184, 8192, 3, 60),
+                                           (4, 153600, 2048, 5, 38), (4, 63616, 6144, 1, 48), (8, 87680, 3072, 3, 24)])
+def test_large_matrices_of_more_bits_keep_whole_row_blocks_longer(L, K, m, n, M, chunk):
+    """From five bits on, and where the activations are rotated ahead, equal chunks wait for a shorter last round; short rows, and rows
+    whose whole blocks do not fit LDS, go over earlier."""
+    out = (ctypes.c_int * 6)()
+    assert L.htr_linear_plan(m, n, K, M, 0, out) == 0
+    steps = (m // 128) * (n // 128)
+    assert out[0] == chunk and out[1] == -(-steps // chunk)
+    assert L.htr_workspace_bytes(m, n, K, M, 0) >= 256 + out[1] * M * 512
