@@ -99,6 +99,23 @@ size_t htr_workspace_bytes(int m, int n, int K, int M, int nsplit) {
   return ws_need((size_t)pl.wgs * M * 128 * sizeof(float), prerot_bytes(n, M));
 }
 
+// the chunked kernel's own rotation reads 16-bit elements in pairs: float32 activations, and rows that do not start on a
+// 4-byte boundary, take the pre-rotation
+static bool chunks_prerotated(const Plan& pl, int x_dtype, const void* x) { return pl.prerot || x_dtype == HTR_F32 || ((uintptr_t)x & 3); }
+
+int htr_linear_rotation(int m, int n, int K, int M, int nsplit, int x_dtype, const void* x) {
+  int out6[6];
+  const int rc = htr_linear_plan(m, n, K, M, nsplit, out6);
+  if (rc != HTR_OK) return -rc;
+  if (!dtype_ok(x_dtype)) return -HTR_ERR_DTYPE;
+  if ((uintptr_t)x & (x_dtype == HTR_F32 ? 3 : 1)) return -HTR_ERR_ALIGN;
+  if (wants_wide(M, nsplit) || wants_gemm(M, nsplit)) return 0;
+  BatchPlan bp;
+  if (wants_batch(M, nsplit, m, n, K)) return make_batch_plan(m, n, K, M, nsplit > 0 ? nsplit & 0xFFFFF : 0, bp) ? batch_rot(K, M, x_dtype, x, bp) : -HTR_ERR_SPLIT;
+  Plan pl;
+  return make_plan(m, n, K, M, nsplit, pl) ? !chunks_prerotated(pl, x_dtype, x) : -HTR_ERR_SPLIT;
+}
+
 int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6) {
   if (!out6) return HTR_ERR_NULL;
   if (K < 2 || K > 8) return HTR_ERR_K;
@@ -276,9 +293,7 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
     t.chunk_magic = 0;
     t.group = nullptr; t.group_prerot_stride = 0; t.group_part_stride = 0; t.tiles = nullptr;
     hipStream_t st = (hipStream_t)stream;
-    // the workgroups rotate their own activations where the plan allows it or it is ahead (16-bit rows on 16-byte boundaries)
-    const bool whole = x_dtype != HTR_F32 && ((uintptr_t)x & 15) == 0;
-    const int rot = !whole ? 0 : bp.rot ? 1 : batch_rot_on() && batch_rot_long(K, M, bp.S, bp.cb, bp.wgs) ? 2 : 0;
+    const int rot = batch_rot(K, M, x_dtype, x, bp);
     if (!rot) HTR_CHECK_HIP(launch_rotation(x, (const uint8_t*)su, n, M, x_dtype, t, st, bp.tile ? FRAG_FULL : 0));
     BatchArgs ba;
     ba.qw = (const uint32_t*)qweight; ba.part = (float*)((unsigned char*)workspace + WS_HEADER); ba.x = x; ba.su = (const uint8_t*)su;
@@ -290,9 +305,7 @@ int htr_linear(const void* qweight, const void* scales, const void* su, const vo
   if (M > HTR_MAX_GROUP_ROWS) return HTR_ERR_BATCH;          // an explicit chunked plan: that kernel takes up to 32 rows
   Plan pl;
   if (!make_plan(m, n, K, M, nsplit, pl)) return HTR_ERR_SPLIT;
-  // the in-kernel rotation reads 16-bit elements in pairs: float32 activations, and rows that do not start on a
-  // 4-byte boundary, take the pre-rotation
-  const bool prerot = pl.prerot || x_dtype == HTR_F32 || ((uintptr_t)x & 3);
+  const bool prerot = chunks_prerotated(pl, x_dtype, x);
   const size_t need = htr_workspace_bytes(m, n, K, M, nsplit);
   if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return HTR_ERR_WORKSPACE;
 

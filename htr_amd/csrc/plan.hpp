@@ -341,6 +341,12 @@ inline bool batch_rot_on() {
   static const bool on = getenv("HTR_BATCH_ROT") == nullptr || atoi(getenv("HTR_BATCH_ROT")) != 0;
   return on;
 }
+// Who rotates a call's activations x: 0 a launch of its own, else the workgroups, as k_linear_batch's ROT says; 16-bit rows on 16-byte
+// boundaries only
+inline int batch_rot(int K, int M, int x_dtype, const void* x, const BatchPlan& bp) {
+  if (x_dtype == HTR_F32 || ((uintptr_t)x & 15)) return 0;
+  return bp.rot ? 1 : batch_rot_on() && batch_rot_long(K, M, bp.S, bp.cb, bp.wgs) ? 2 : 0;
+}
 inline size_t batch_rot_lds_bytes(int M, int cb, int rot) {
   const int rows = 16 * batch_groups(M);
   return (size_t)cb * rows * BATCH_ROWH * 2 + (size_t)cb * 2 * rows * 4 + rows * 4 +

@@ -112,7 +112,8 @@ unsigned long long htr_stream_capture_id(void* stream);
  * over at most 8), dynamic LDS bytes}.  Entries 4 and 5 assume bf16 / f16 activations on a 16-byte boundary; float32 or
  * otherwise aligned activations always take the rotation launch and the staged kernel's LDS layout.
  * Where the plan says 1, up to 16 rows over 32 blocks and up to 32 rows over 16 may still be rotated by the workgroups, if that is
- * faster and the activations are 16-bit rows on 16-byte boundaries: decided at the call, with more LDS than the plan says.
+ * faster and the activations are 16-bit rows on 16-byte boundaries: decided at the call, with more LDS than the plan says
+ * (htr_linear_rotation).
  * From 65 rows to HTR_MAX_ROWS_PER_TILE the wide kernel runs (tiles of up to 256 activation rows, which share what a workgroup
  * decodes), out6 as for the batched kernel; with bit 27 of nsplit it takes any row count, and out6[2] is the number of row tiles.
  * With more than HTR_MAX_ROWS_PER_TILE rows the fused decode -> matrix-unit (GEMM) kernel runs: the activations are
@@ -132,6 +133,14 @@ unsigned long long htr_stream_capture_id(void* stream);
  * that many column splits of every tile in the low bits (0 = its own policy; at most 8; any row count up to HTR_MAX_BATCH).
  */
 int htr_linear_plan(int m, int n, int K, int M, int nsplit, int* out6);
+
+/*
+ * Who rotates the activations in htr_linear's call with these arguments (x decides by its type and alignment, it is not read): 0 a
+ * launch of its own, 1 the workgroups that multiply, as planned, 2 the workgroups of the batched kernel where its plan is made for a
+ * rotation launch; below 0 minus the status that the call returns.  No reference counterpart: its prologue is always a launch
+ * (htr/csrc/htr_kernels.cu:972-987).
+ */
+int htr_linear_rotation(int m, int n, int K, int M, int nsplit, int x_dtype, const void* x);
 
 /*
  * How this call is best made: a value for htr_linear's nsplit (0, or 2^27, the wide kernel, beyond HTR_MAX_ROWS_PER_TILE rows), or

@@ -704,21 +704,26 @@ def test_seeded_random_cases_through_the_c_abi(dev, oracle):
 
 @pytest.mark.parametrize("M,S", [(12, 1), (16, 1), (16, 2), (32, 1), (32, 4), (10, 8)])
 def test_batched_kernel_with_explicit_splits(dev, oracle, M, S, monkeypatch):
-    """The batched kernel with an explicit number of column splits (nsplit bit 29): one split of 32 column blocks is more
-    than a workgroup rotates and keeps by itself, so those cases take the rotation launch and the staged blocks also at
-    few rows; the short splits take the in-kernel rotation.  Same result either way."""
+    """The batched kernel with an explicit number of column splits (nsplit bit 29).  One split of 32 column blocks is more than the plan
+    has a workgroup rotate by itself: up to 16 rows it still does (rotation 2), 32 rows take the rotation launch and the staged blocks;
+    the short splits take the in-kernel rotation of the plan.  Rows off a 16-byte boundary take the launch everywhere.  Same result."""
     import ctypes
     from htr_amd import _native, ops
     print(f"batched kernel, explicit splits M={M} S={S}", flush=True)
     m, n = 512, 4096
     out = (ctypes.c_int * 6)()
-    assert _native.lib().htr_linear_plan(m, n, 4, M, (1 << 29) | S, out) == 0
+    L, nsplit = _native.lib(), (1 << 29) | S
+    assert L.htr_linear_plan(m, n, 4, M, nsplit, out) == 0
     cb = out[0]
     assert cb == 32 // S and out[4] == (0 if (M <= 16 and cb <= 16) or cb <= 8 else 1)
     qw, sc, su, sv, x = _case(m, n, 4, M, 5200 + 10 * M + S)
-    monkeypatch.setattr(ops, "NSPLIT", (1 << 29) | S)
-    y = ops.linear_f32out(x.to(dev), *[t.to(dev) for t in (qw, sc, su, sv)]).cpu().numpy()
-    assert _rel(y, _ref(oracle, qw, sc, su, sv, x)) <= REL_TOL
+    monkeypatch.setattr(ops, "NSPLIT", nsplit)
+    w, ref = [t.to(dev) for t in (qw, sc, su, sv)], _ref(oracle, qw, sc, su, sv, x)
+    odd = torch.empty(M * n + 1, dtype=x.dtype, device=dev)[1:].view(M, n)
+    odd.copy_(x)
+    for xd, rotation in ((x.to(dev), 1 if out[4] == 0 else (2 if M <= 16 else 0)), (odd, 0)):
+        assert L.htr_linear_rotation(m, n, 4, M, nsplit, _native.BF16, xd.data_ptr()) == rotation
+        assert _rel(ops.linear_f32out(xd, *w).cpu().numpy(), ref) <= REL_TOL
 
 
 @pytest.mark.parametrize("M,S", [(12, 4), (24, 4), (32, 8), (64, 2), (100, 4), (128, 8)])
@@ -832,15 +837,17 @@ def test_tiles_of_32_rows_over_long_splits(dev, oracle, K, m, n, M, S, dtype):
         ops.NSPLIT = 0
 
 
-@pytest.mark.parametrize("K,m,n,M,S", [(4, 128, 128, 9, 1), (2, 256, 1920, 15, 1), (8, 128, 2048, 16, 1), (4, 256, 640, 17, 1), (3, 128, 1024, 32, 1), (5, 384, 2176, 31, 3), (4, 256, 4096, 13, 2),
-                                     (4, 4096, 2176, 9, 1), (3, 4096, 4096, 16, 1), (4, 4096, 1152, 17, 1), (2, 1408, 4608, 32, 3), (5, 4096, 1920, 29, 1), (8, 4096, 2048, 32, 1)])
+@pytest.mark.parametrize("rotation,K,m,n,M,S", [(1, 4, 128, 128, 9, 1), (1, 2, 256, 1920, 15, 1), (1, 8, 128, 2048, 16, 1), (1, 4, 256, 640, 17, 1), (1, 3, 128, 1024, 32, 1),
+                                              (1, 5, 384, 2176, 31, 3), (1, 4, 256, 4096, 13, 2), (2, 4, 4096, 2176, 9, 1), (2, 3, 4096, 4096, 16, 1), (2, 4, 4096, 1152, 17, 1),
+                                              (2, 2, 1408, 4608, 32, 3), (2, 5, 4096, 1920, 29, 1), (2, 8, 4096, 2048, 32, 1)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, K, m, n, M, S, dtype):
+def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, rotation, K, m, n, M, S, dtype):
     """9 to 32 rows rotated by the workgroups that multiply them: one to four units of 16 rows and one block per wave, waves without
     a unit, rows short of a unit, both 16-bit types.  Rows of very different size keep their own scale, and an infinity stays in its
     row.  Max norm per row: 1e-3 as for every float32 result (float16 activations)."""
-    from htr_amd import ops
+    from htr_amd import _native, ops
     print(f"rotation by workgroups K={K} {m}x{n} M={M} S={S} {dtype}", flush=True)
+    assert _native.lib().htr_linear_rotation(m, n, K, M, (1 << 29) | S, _native.BF16 if dtype == torch.bfloat16 else _native.F16, None) == rotation
     qw, sc, su, sv, x = _case(m, n, K, M, 3300 + M + n, torch.float32)
     x = (x * torch.logspace(-3, 3, M)[:, None]).to(dtype)
     w = [t.to(dev) for t in (qw, sc, su, sv)]

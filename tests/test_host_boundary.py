@@ -357,3 +357,15 @@ def test_large_matrices_of_more_bits_keep_whole_row_blocks_longer(L, K, m, n, M,
     steps = (m // 128) * (n // 128)
     assert out[0] == chunk and out[1] == -(-steps // chunk)
     assert L.htr_workspace_bytes(m, n, K, M, 0) >= 256 + out[1] * M * 512
+
+
+@pytest.mark.parametrize("args,rotation", [((4096, 4096, 4, 1, 0, 0, 16), 1), ((4096, 4096, 4, 1, 0, 0, 4), 1), ((4096, 4096, 4, 1, 0, 0, 2), 0), ((4096, 4096, 4, 1, 0, 2, 16), 0),
+                                           ((4096, 4096, 4, 1, 1 << 30 | 8, 0, 16), 0), ((4096, 4096, 4, 9, 0, 0, 16), 1), ((4096, 4096, 4, 9, 0, 0, 8), 0),
+                                           ((28672, 4096, 3, 13, 0, 1, 32), 2), ((28672, 4096, 3, 13, 0, 2, 32), 0), ((28672, 4096, 3, 13, 0, 0, 2), 0), ((28672, 4096, 3, 32, 0, 0, 16), 0),
+                                           ((4096, 4096, 4, 97, 0, 0, 16), 0), ((4096, 4096, 4, 333, 0, 0, 16), 0)])
+def test_who_rotates_the_activations(L, args, rotation):
+    """By plan, type and alignment: chunked, batched, wide and GEMM kernels; what the call refuses has no answer."""
+    assert L.htr_linear_rotation(*args) == rotation
+    m, n, K, M, nsplit, dtype, x = args
+    for bad in ((m, n, 9, M, nsplit, dtype, x), (m + 1, n, K, M, nsplit, dtype, x), (m, n, K, 0, nsplit, dtype, x), (m, n, K, M, nsplit, 3, x), (m, n, K, M, nsplit, dtype, x + 1)):
+        assert L.htr_linear_rotation(*bad) < 0
