@@ -291,20 +291,29 @@ struct BatchPlan { int S, cb, wgs, mb, rot, last_finishes; bool tile; size_t lds
 // two units of 16 rows and one block per wave) instead of a rotation launch: 16 x 16 or 32 x 8
 inline bool batch_rot_fits(int M, int cb) { return (M <= 16 && cb <= 16) || (M <= 32 && cb <= 8); }
 // Where it does so beyond that with up to four units per wave (ROT = 2).  Decided at the launch, by the activations it is given; the
-// plan is that of the rotation launch and of the kernel behind it, which all other activations take.  Measured on MI355X, us in
-// graphs over several weights, rotation launch / 2:
-//   up to 16 rows, everywhere (28672x4096, 16 rows K4 23.9 / 23.7, 9 rows K3 23.2 / 22.1, 12 rows K8 32.7 / 30.1; 20480x3072, 16 rows
-//     K4 19.5 / 19.0; 28672x2560, 8 rows K4 17.2 / 15.6; 4096x22528, 12 rows K4 22.0 / 18.9; 2048x32768, 16 rows K4 25.7 / 24.9)
-//   17 to 32 rows over 9 to 12 column blocks, everywhere (28672x1152, 32 rows K4 14.3 / 13.4; 10240x3840 15.7 / 14.9; 8704x3456, 17
-//     rows K8 17.7 / 14.8; 12288x3072, 32 rows K4 15.8 / 15.8) but on the smallest grids (128x12288 16.0 / 16.2)
-//   13 to 16 from five bits on, whose decode hides more of the rotation (4096x14336, 17 rows K5 19.8 / 17.6; 8192x8192 K8 24.9 / 23.6;
-//     12288x4096, 32 rows K5 19.9 / 19.8), and up to K4 13 and 14 on a grid of three splits and more that fills three quarters of the
-//     chip (4096x14336, 32 rows K4 19.3 / 18.6, 24 rows 18.8 / 17.3; 10240x5376 18.7 / 18.3): not 1024x14336, 17.4 / 17.7, nor
-//     10240x6144, 19.0 / 19.7, nor where k_linear_tile is what follows the launch (28672x2048 16.9 / 19.0, 12288x4096 18.3 / 18.9)
+// plan is that of the rotation launch and of the kernel behind it, which all other activations take.  The units are of 16 rows, so
+// what the workgroups spend does not grow from 17 to 32 rows, while what the launch and the kernel behind it take does not pay for
+// rows that are not there: the more rows, the fewer column blocks.  More bits hide more of it, and on the smallest grids, up to a few
+// row blocks, the launch is short.  Measured on MI355X, us in graphs over several weights, rotation launch / 2:
+//   up to 16 rows, everywhere (28672x4096, 16 rows K4 23.9 / 23.7, 9 rows K3 23.2 / 22.1; 4096x22528, 12 rows K4 22.0 / 18.9; 128x16384,
+//     16 rows K5 15.9 / 15.2)
+//   17 to 32 rows over 9 and 10 column blocks, everywhere (28672x1152, 32 rows K4 14.5 / 13.9; 10240x3840 16.2 / 15.4), and from seven
+//     bits on over up to 16 (128x16384, 32 rows K7 21.0 / 20.3; 20480x2048 K8 22.4 / 22.6)
+//   K5 and K6: up to 20 rows (20480x2048, 17 rows K5 18.9 / 18.7, 24 and 32 rows 18.9 / 19.3 and 19.6 / 20.2); beyond, on an eighth of
+//     the chip and more (128x11264, 32 rows K5 15.8 / 16.0), with four column splits and more (8192x8192, 24 rows 23.5 / 23.2, 32 rows
+//     24.4 / 24.1), else over up to 14 blocks to 24 rows and then with two splits over up to 12 (28672x1664, one split over 13, 24 rows
+//     17.5 / 17.4, 32 rows 18.2 / 18.4)
+//   up to K4: 20 rows over 11 and 12 (14336x3072, 17 / 24 / 32 rows K4 16.7 / 16.5, 17.0 / 17.0, 16.9 / 17.3; 20480x1408, 32 rows 14.8 /
+//     15.4), and 13 and 14 on a grid of three splits and more that fills three quarters of the chip (4096x14336, 24 rows K4 19.8 /
+//     19.3, K3 19.1 / 18.9; K2, whose decode hides least, 17.4 / 17.4 with 17, 18.3 / 18.7 with 32)
 inline bool batch_rot_long(int K, int M, int S, int cb, int wgs) {
   const int cus = num_cu();
   if (M > 32 || wgs > cus || (M <= 16 ? cb : 2 * cb) > 32) return false;
-  return M <= 16 || cb <= 10 || (cb <= 12 && 8 * wgs >= cus) || K >= 5 || (cb <= 14 && S >= 3 && 4 * wgs > 3 * cus);
+  if (M <= 16 || cb <= 10 || K >= 7) return true;
+  const bool eighth = 8 * wgs >= cus;
+  if (K >= 5) return M <= 20 || (eighth && (S >= 4 || (M <= 24 ? cb <= 14 : S > 1 && cb <= 12)));
+  if (cb <= 12) return M <= 20 && eighth;
+  return cb <= 14 && S >= 3 && 4 * wgs > 3 * cus && (K >= 3 || M <= 20);
 }
 constexpr int BATCH_MIN_M = 9;      // rows from which the library policy takes the batched kernel on every shape
 inline int batch_groups(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : 8)); }   // groups of 16 activation rows

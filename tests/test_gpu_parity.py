@@ -839,7 +839,8 @@ def test_tiles_of_32_rows_over_long_splits(dev, oracle, K, m, n, M, S, dtype):
 
 @pytest.mark.parametrize("rotation,K,m,n,M,S", [(1, 4, 128, 128, 9, 1), (1, 2, 256, 1920, 15, 1), (1, 8, 128, 2048, 16, 1), (1, 4, 256, 640, 17, 1), (1, 3, 128, 1024, 32, 1),
                                               (1, 5, 384, 2176, 31, 3), (1, 4, 256, 4096, 13, 2), (2, 4, 4096, 2176, 9, 1), (2, 3, 4096, 4096, 16, 1), (2, 4, 4096, 1152, 17, 1),
-                                              (2, 2, 1408, 4608, 32, 3), (2, 5, 4096, 1920, 29, 1), (2, 8, 4096, 2048, 32, 1)])
+                                              (2, 2, 1408, 4608, 20, 3), (2, 7, 4096, 1920, 29, 1), (2, 8, 4096, 2048, 32, 1),
+                                              (2, 5, 2048, 5632, 32, 4), (0, 2, 1408, 4608, 32, 3), (0, 5, 4096, 1920, 29, 1)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_workgroups_rotate_their_blocks_16_rows_at_a_time(dev, oracle, rotation, K, m, n, M, S, dtype):
     """9 to 32 rows rotated by the workgroups that multiply them: one to four units of 16 rows and one block per wave, waves without

@@ -369,3 +369,15 @@ def test_who_rotates_the_activations(L, args, rotation):
     m, n, K, M, nsplit, dtype, x = args
     for bad in ((m, n, 9, M, nsplit, dtype, x), (m + 1, n, K, M, nsplit, dtype, x), (m, n, K, 0, nsplit, dtype, x), (m, n, K, M, nsplit, 3, x), (m, n, K, M, nsplit, dtype, x + 1)):
         assert L.htr_linear_rotation(*bad) < 0
+
+
+@pytest.mark.parametrize("K,m,S,cb,rotation", [(4, 28672, 1, 9, "222"), (2, 10240, 3, 10, "222"), (7, 128, 8, 16, "222"), (8, 20480, 1, 16, "222"),                          # 17 | 24 | 32 rows
+                                                (5, 20480, 1, 16, "200"), (5, 128, 8, 11, "200"), (5, 28672, 1, 13, "220"), (6, 14336, 2, 12, "222"), (5, 4096, 8, 14, "222"), (6, 8192, 4, 16, "222"),
+                                                (4, 14336, 2, 12, "200"), (3, 512, 8, 11, "200"), (4, 128, 8, 11, "000"), (4, 4096, 8, 14, "222"), (2, 4096, 8, 14, "200"), (4, 2048, 8, 14, "000"),
+                                                (4, 14336, 2, 15, "000")])
+def test_where_the_workgroups_rotate_17_rows_and_more(L, K, m, S, cb, rotation):
+    """Column blocks per split, rows, bits and grid: where the rotation by the workgroups measured faster than the launch."""
+    got = "".join(str(L.htr_linear_rotation(m, 128 * cb * S, K, M, (1 << 29) | S, 0, None)) for M in (17, 24, 32))
+    assert got == rotation
+    assert all(L.htr_linear_rotation(m, 128 * cb * S, K, M, (1 << 29) | S, 0, None) in (1, 2) for M in (6, 16))
+    assert all(L.htr_linear_rotation(m, 128 * cb * S, K, M, (1 << 29) | S, 2, None) == 0 for M in (6, 17, 32))
