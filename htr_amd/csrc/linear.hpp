@@ -125,8 +125,8 @@ __device__ __forceinline__ void rotate4_mfma(const u4& xr, uint32_t sb, bool is_
 // row = lane % 16) brings the 8 consecutive elements 32 a + 8 gk .. + 7 of its row, x[a], and the su byte of their signs, sb[a]),
 // and the rows of the A operands, those of H32, are dealt so that lane (gk, row) ends up with y[a'][t] = elements 32 a' + 8 gk + 4 t
 // .. + 3 of its row: eight consecutive results leave in one 16-byte store, where rotate4_mfma's lanes hold every 16th.  Per 2048
-// elements about 210 vector instructions with conversion, sums and stores, 90 of them additions and multiplications that this chip
-// issues at 2.4 instead of 4.4 cycles, and 4 stores; rotate4_mfma 440 and 32.  Same sums in the same order.
+// elements about 230 vector instructions with the maximum, conversion and sums, 64 additions and 32 multiplications among them, which
+// this chip issues at 2.4 instead of 4.4 cycles, and 4 stores; rotate4_mfma 440 and 32.  Same sums in the same order.
 __device__ __forceinline__ void rotate16_mfma(const u4 (&x)[4], const uint32_t (&sb)[4], bool is_bf16, int lane, f4 (&y)[4][2]) {
   const int i = lane & 15, gk = lane >> 4;
   u4 xs[4];

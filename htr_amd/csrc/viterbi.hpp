@@ -19,10 +19,12 @@
 // Bound: vector issue in the forward passes (K4: 2890 cycles a step, 2944 by the rates above; 0.74 M cycles a pass), then
 // the trace back, 10 % of a tile at K3 and K4: its stored arrays (2 MB a tile), then one wave's chain of LDS reads and lane
 // minima.  C: a larger one stores less and recomputes more (176 tiles, C - 1 instead: K2 929 us for 898, K3 823 / 763, K4 812 / 732).
-// Registers: the codebook values are read anew for every tile, so that none of what the trace back needs lies in scratch.  It did, 20 of
-// a lane's registers at K4, and loading them in every turn waited for all arrays in flight: 176 tiles, one per CU, at K2 / 3 / 4 / 5 / 7 / 8
-// took 1161 / 815 / 801 / 950 / 1067 / 955 us and take 900 / 763 / 735 / 857 / 888 / 844; 1024 at K4 3.25 -> 3.04 ms (7.46 with the
-// table and one byte of backpointer per entry and step, the first version).
+// Registers: the codebook values are read anew for every tile, so that the trace back has their registers.  20 of a lane's lay in
+// scratch at K4, and loading them in every turn waited for all arrays in flight.  From K3 on its loop now loads nothing from scratch;
+// at K2, where 16 elements of an array are a lane's, it still loads seven registers in two turns.  Scratch bytes of a lane at K2 to K8:
+// 108, 60, 44, 68, 64, 404, 140 (332, 116, 68, 44, 36, 404, 136 then), loaded once a tile or once a pass, never in the steps.  176 tiles, one per CU, us at K2 to K8: 1226, 829, 823, 956, 850, 1078, 974 before, 979, 772, 743,
+// 858, 833, 895, 844 now; 1024 at K4 3.25 -> 3.03 ms (7.46 with the table and one byte of backpointer per entry and step, the first
+// version).
 // Arithmetic and tie-breaking are the reference's: float32, d = (x - cb)^2, m + w * d without fusing, the first index
 // among equal values in every min / argmin.
 template <int K> struct VitCfg {
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(VitCfg<K>::THREADS) void k_viterbi(const float* __r
       constexpr int RL = SJ >= THREADS ? SJ / THREADS : 1;             // row elements per thread
       auto lds_pos = [](uint32_t e) { return e + (e >> 4); };
       // The q-th array that the trace back reads: the stored ones from the last on, then M_0.  Nothing in the loop may make it wait for
-      // loads that it has just issued: no branch around a load (M_0 comes in where the array goes to LDS), no value in scratch.
+      // loads that it has just issued: no branch around a load (M_0 comes in where the array goes to LDS), from K3 on no value in scratch.
       auto request = [&](float (&reg)[RL], int q) {                    // beyond the last stored one: the first again, not looked at
         const float* row = my_rows + (size_t)max(nrows - 1 - q, 0) * SJ;
 #pragma unroll

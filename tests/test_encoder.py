@@ -301,8 +301,7 @@ def test_codebook_check_is_not_fooled_by_a_reused_address(monkeypatch):
 @pytest.mark.parametrize("K,sizes,n,shared,max_batch", [(2, [(128, 0)], 128, False, 8), (3, [(256, 0), (384, 0)], 256, True, 1024), (4, [(128, 0), (128, 1), (256, 1)], 384, True, 11),
                                                        (5, [(1280, 0)], 128, True, 64)])
 def test_gpu_encoder_blocks_match_the_torch_lines(dev, monkeypatch, K, sizes, n, shared, max_batch):
-    """encode_group's launches around the search against its torch lines with the same search (which a hook selects): every output bit
-    for bit.  One and several matrices and Hessians, a dead input column, batches that do not divide the tiles."""
+    """_NativeBlocks against _TorchBlocks with the same search (a hook selects them): every output bit for bit.  One and several matrices and Hessians, a dead input column, batches that do not divide the tiles."""
     from htr_amd import encode
     print(f"encoder blocks K={K} {sizes} n={n}", flush=True)
     g = torch.Generator().manual_seed(K)
@@ -336,7 +335,7 @@ def test_encoder_block_launches_refuse_wrong_sizes():
 @pytest.mark.parametrize("tailbite", [True, False])
 def test_gpu_search_with_few_stored_arrays(dev, oracle, K, lengths, tailbite):
     """Lengths with one to ten stored arrays, around the four that the trace back has in flight and its loop takes at a time, and the
-    longest.  Whole numbers: exact."""
+    longest.  The states are whole numbers: exact."""
     from htr_amd import encode
     for T in lengths:
         print(f"viterbi K={K} T={T} tailbite={tailbite}", flush=True)
