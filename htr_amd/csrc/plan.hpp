@@ -164,7 +164,10 @@ inline bool search_plan(int m, int n, int K, int M, int nsplit, int cus, Plan& p
   even.mb = pl.mb;
   if (large && plan_for_chunk(m, n, M, (int)((vtotal + 2 * cus - 1) / (2 * cus)), even)) {
     const bool early = K <= 4 || (K <= 6 && K * nblk <= 120);
-    const double spare = early ? (even.prerot && pl.chunk == nblk ? 1.1 : 1.06) : (even.prerot ? 1.2 : 1.15);
+    double spare = early ? (even.prerot && pl.chunk == nblk ? 1.1 : 1.06) : (even.prerot ? 1.2 : 1.15);
+    // partials beyond the library's own workspace (4 rows of 262144 and more): two slots per compute unit always fit.  us with row
+    // blocks / chunks: 437888x3584 K6 4 rows 278.8 / 251.9, 310272x4096 K4 171.9 / 161.4, 253952x4096 K8 5 rows 199.6 / 204.9
+    if (found && ws_need((size_t)pl.wgs * M * 128 * sizeof(float), prerot_bytes(n, M)) > HTR_STATIC_SCRATCH_BYTES) spare = 1.0;
     if (!found || spare * vtotal < (double)((pl.wgs + cus - 1) / cus) * pl.chunk * cus) { pl = even; found = true; }
   }
   return found;

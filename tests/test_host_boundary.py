@@ -381,3 +381,14 @@ def test_where_the_workgroups_rotate_17_rows_and_more(L, K, m, S, cb, rotation):
     assert got == rotation
     assert all(L.htr_linear_rotation(m, 128 * cb * S, K, M, (1 << 29) | S, 0, None) in (1, 2) for M in (6, 16))
     assert all(L.htr_linear_rotation(m, 128 * cb * S, K, M, (1 << 29) | S, 2, None) == 0 for M in (6, 17, 32))
+
+
+@pytest.mark.parametrize("K,m,n,M", [(6, 437888, 3584, 4), (8, 253952, 4096, 5), (4, 310272, 4096, 4), (5, 1100800, 2048, 1)])
+def test_large_matrices_whose_row_blocks_exceed_the_librarys_own_workspace_fit_it_in_chunks(L, K, m, n, M):
+    """One slot per row block is more than HTR_STATIC_SCRATCH_BYTES: with any room in the last round the call goes to equal chunks, at
+    margins from 1.01 on, where it would stay with row blocks otherwise."""
+    from htr_amd import _native
+    assert 2 * (m // 128) * M * 512 > _native.STATIC_SCRATCH_BYTES
+    out = (ctypes.c_int * 6)()
+    assert L.htr_linear_plan(m, n, K, M, 0, out) == 0 and out[1] <= 512
+    assert 0 < L.htr_workspace_bytes(m, n, K, M, 0) <= _native.STATIC_SCRATCH_BYTES
