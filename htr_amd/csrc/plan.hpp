@@ -149,25 +149,33 @@ inline bool search_plan(int m, int n, int K, int M, int nsplit, int cus, Plan& p
   // ... or, instead of either, two equal chunks per compute unit.  The compute units take workgroups in rounds, so the last round is as
   // long as the others however few are left; equal chunks fill it, at the price of partials, of row ends inside a chunk, and of PACE
   // where the activations are rotated ahead.  They pay where the rounds hold `spare` times the steps that there are: later from five
-  // bits on, except over short rows, as whole row blocks then read at close to the memory's rate already (61184x6144 K5 4.4, K8 4.9 of
-  // the 5.0 TB/s of a copy; K4 3.7).  Measured on MI355X with margins from 1.005 to 1.5, n from 1536 to 8192; us with row blocks /
-  // chunks at a margin:
-  //   K4 1 row 61824x6144 (1.06) 50.6 / 50.6, 60032x6144 (1.09) 49.0 / 47.0, 152064x4096 (1.08) 72.8 / 71.7, 73728x4096 (1.33) 48.6 /
-  //   39.8; 3 rows 91776x4096 (1.07) 51.7 / 48.8; 5 rows, rotated ahead, 92672x4096 (1.06) 52.9 / 53.4, 90112x4096 (1.09) 52.5 / 50.9
+  // bits on, as whole row blocks then read at close to the memory's rate already (61184x6144 K5 4.4, K8 4.9 of the 5.0 TB/s of a copy;
+  // K4 3.7), though up to K6 not over short rows, nor with more rounds, whose workgroups each pay for their ends.  Measured on MI355X
+  // with margins from 1.005 to 1.5, n from 1536 to 8192, two to eleven rounds; us with row blocks / chunks at a margin:
+  //   K4 1 row 63616x6144 (1.03) 48.8 / 50.8, 61824x6144 (1.06) 50.6 / 50.6, 60032x6144 (1.09) 49.0 / 47.0; five rounds 158976x4096
+  //   (1.03) 77.0 / 75.4, 152064x4096 (1.08) 72.8 / 71.7; three 73728x4096 (1.33) 48.6 / 39.8; 5 rows, rotated ahead, 92672x4096 (1.06)
+  //   52.9 / 53.4, 90112x4096 (1.09) 52.5 / 50.9
   //   K5 1 row 122496x2560 (1.07) 45.8 / 45.0, K6 153088x2048 (1.07) 54.1 / 51.6: short rows
   //   K5 1 row 61184x6144 (1.07) 53.2 / 53.8, 3 rows, rotated ahead, 60032x6144 (1.09) 55.1 / 58.3, 5 rows 84736x4096 (1.16) 57.1 / 58.9
   //   K6 1 row 61184x5120 (1.07) 51.1 / 52.8, 3 rows 112896x3072 (1.16) 60.4 / 56.5; K7 1 row 93568x4096 (1.05) 66.7 / 69.6; K8 3 rows
   //   87680x3072 (1.12) 58.1 / 59.2
+  //   five rounds, 1 row 151680x4096 (1.08) K5 83.3 / 81.4, K6 94.3 / 91.9, K7 104.2 / 106.5; K8 5 rows 116992x3072 (1.12) 75.4 / 79.1; K5 5
+  //   rows, rotated ahead, 151680x4096 89.3 / 91.5, 147584x4096 89.2 / 89.9
   //   3 rows of 8192, whose row blocks do not fit, with the search's 32 steps: K4 61184 (1.07) 66.6 / 64.6, 43648 (1.12) 51.4 / 49.1; K6
   //   46720 (1.05) 63.7 / 67.1, 50304 (1.30) 79.1 / 74.3; K7 46720 72.1 / 77.2
   Plan even;
   even.mb = pl.mb;
   if (large && plan_for_chunk(m, n, M, (int)((vtotal + 2 * cus - 1) / (2 * cus)), even)) {
-    const bool early = K <= 4 || (K <= 6 && K * nblk <= 120);
-    double spare = early ? (even.prerot && pl.chunk == nblk ? 1.1 : 1.06) : (even.prerot ? 1.2 : 1.15);
-    // partials beyond the library's own workspace (4 rows of 262144 and more): two slots per compute unit always fit.  us with row
-    // blocks / chunks: 437888x3584 K6 4 rows 278.8 / 251.9, 310272x4096 K4 171.9 / 161.4, 253952x4096 K8 5 rows 199.6 / 204.9
-    if (found && ws_need((size_t)pl.wgs * M * 128 * sizeof(float), prerot_bytes(n, M)) > HTR_STATIC_SCRATCH_BYTES) spare = 1.0;
+    const int rounds = (rbs + cus - 1) / cus;
+    double spare;
+    if (K <= 4) spare = rounds >= 3 ? 1.03 : 1.06;
+    else if (K <= 6 && K * nblk <= 120) spare = 1.03;
+    else spare = K <= 6 && rounds >= 4 ? 1.06 : 1.15;
+    if (even.prerot && (K > 4 || pl.chunk == nblk)) spare += 0.07;
+    // partials beyond the library's own workspace (4 rows of 262144 and more), which two slots per compute unit always fit: 437888x3584
+    // K6 4 rows 278.8 / 251.9, 310272x4096 K4 171.9 / 161.4
+    const double fitting = even.prerot && M > 4 ? 1.1 : 1.03;
+    if (found && spare > fitting && ws_need((size_t)pl.wgs * M * 128 * sizeof(float), prerot_bytes(n, M)) > HTR_STATIC_SCRATCH_BYTES) spare = fitting;
     if (!found || spare * vtotal < (double)((pl.wgs + cus - 1) / cus) * pl.chunk * cus) { pl = even; found = true; }
   }
   return found;

@@ -346,12 +346,12 @@ def test_large_matrices_take_row_blocks_or_equal_chunks(L, m, n, M, chunk):
     assert L.htr_workspace_bytes(m, n, 4, M, 0) >= 256 + out[1] * M * 512
 
 
-@pytest.mark.parametrize("K,m,n,M,chunk", [(3, 152064, 4096, 1, 75), (5, 152064, 4096, 1, 32), (8, 152064, 4096, 4, 32), (5, 73728, 4096, 1, 36), (6, 73728, 4096, 5, 36),
+@pytest.mark.parametrize("K,m,n,M,chunk", [(3, 152064, 4096, 1, 75), (5, 152064, 4096, 1, 75), (5, 152064, 4096, 5, 32), (7, 152064, 4096, 1, 32), (8, 152064, 4096, 4, 32), (5, 73728, 4096, 1, 36), (6, 73728, 4096, 5, 36),
                                            (7, 84736, 4096, 5, 32), (5, 122496, 2560, 1, 38), (6, 153088, 2048, 1, 38), (7, 153088, 2048, 1, 16), (4, 61184, 8192, 3, 60),
                                            (4, 153600, 2048, 5, 38), (4, 63616, 6144, 1, 48), (8, 87680, 3072, 3, 24)])
 def test_large_matrices_of_more_bits_keep_whole_row_blocks_longer(L, K, m, n, M, chunk):
-    """From five bits on, and where the activations are rotated ahead, equal chunks wait for a shorter last round; short rows, and rows
-    whose whole blocks do not fit LDS, go over earlier."""
+    """From five bits on, and where the activations are rotated ahead, equal chunks wait for a shorter last round; short rows, four
+    rounds and more, and rows whose whole blocks do not fit LDS, go over earlier."""
     out = (ctypes.c_int * 6)()
     assert L.htr_linear_plan(m, n, K, M, 0, out) == 0
     steps = (m // 128) * (n // 128)
@@ -383,10 +383,10 @@ def test_where_the_workgroups_rotate_17_rows_and_more(L, K, m, S, cb, rotation):
     assert all(L.htr_linear_rotation(m, 128 * cb * S, K, M, (1 << 29) | S, 2, None) == 0 for M in (6, 17, 32))
 
 
-@pytest.mark.parametrize("K,m,n,M", [(6, 437888, 3584, 4), (8, 253952, 4096, 5), (4, 310272, 4096, 4), (5, 1100800, 2048, 1)])
+@pytest.mark.parametrize("K,m,n,M", [(6, 437888, 3584, 4), (8, 317440, 2048, 4), (4, 310272, 4096, 4), (5, 1049600, 1024, 1)])
 def test_large_matrices_whose_row_blocks_exceed_the_librarys_own_workspace_fit_it_in_chunks(L, K, m, n, M):
-    """One slot per row block is more than HTR_STATIC_SCRATCH_BYTES: with any room in the last round the call goes to equal chunks, at
-    margins from 1.01 on, where it would stay with row blocks otherwise."""
+    """One slot per row block is more than HTR_STATIC_SCRATCH_BYTES: the call goes to equal chunks from a margin of 3 % on, where it would
+    stay with row blocks otherwise."""
     from htr_amd import _native
     assert 2 * (m // 128) * M * 512 > _native.STATIC_SCRATCH_BYTES
     out = (ctypes.c_int * 6)()
