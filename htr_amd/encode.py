@@ -160,9 +160,14 @@ def prep_H(H, W, damp=0.01):
     bit, and damping the diagonal in place, or before the dead columns are fixed, rounds differently."""
     H = H.clone().double()
     dead = torch.diag(H) == 0
-    H[dead, dead] = 1.0
-    W = W.clone()
-    W[:, dead] = 0
+    if W.dim() == 2 and H.shape == (W.shape[1], W.shape[1]) and W.device == H.device:
+        # by masks: the GPU makes index lists in a synchronisation (256x256 K4 13.56 ms by index, 13.47 by masks, two 1408x1024 K3 55.95 / 55.70)
+        torch.diagonal(H).masked_fill_(dead, 1.0)
+        W = W.clone().masked_fill_(dead, 0)
+    else:
+        H[dead, dead] = 1.0
+        W = W.clone()
+        W[:, dead] = 0
     H += damp * torch.diag(H).mean() * torch.eye(H.shape[0], device=H.device, dtype=H.dtype)
     return H, W
 

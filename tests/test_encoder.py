@@ -396,3 +396,22 @@ def test_gpu_encoder_takes_matrices_without_rows(dev, rows):
     if len(rows) > 1:
         other = encode.encode_group([dict(W=jobs[0]["W"].new_zeros(128, 128), H=H), jobs[1]], 4, seed=5)[1]
         assert torch.equal(got[1]["qweight"], other["qweight"]) and torch.equal(got[1]["What"], other["What"])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16])
+def test_dead_columns_by_masks_are_those_by_index(dtype):
+    """What is not a number, infinite or a negative zero in a dead column as well, and a matrix that is a transposed view."""
+    from htr_amd import encode
+    g = torch.Generator().manual_seed(11)
+    H = torch.randn(128, 128, generator=g)
+    W = torch.randn(128, 6, generator=g).to(dtype).T
+    for c, v in ((0, float("nan")), (7, -0.0), (127, float("inf"))):
+        H[c, c] = 0
+        W[2, c] = v
+    Hd, Wd = encode.prep_H(H, W, damp=0.0)
+    dead = torch.diag(H) == 0
+    want_H, want_W = H.double(), W.clone()
+    want_H[dead, dead] = 1.0
+    want_W[:, dead] = 0
+    assert torch.equal(Hd, want_H) and torch.equal(Wd, want_W) and Wd.dtype == dtype and Wd.stride() == want_W.stride()
+    assert not torch.signbit(Wd[:, dead]).any() and bool(torch.isnan(W[2, 0]))
